@@ -13,9 +13,24 @@
 //   RPY                 -- the point-tracer limit (target radius 0) of the RPY
 //                          pair tensor, <3,6> from segments and <3,3> from blobs.
 //
-// Two targets per lane, all sources streamed through LDS in batches of BLOCK;
-// the 4.2M-point plane is 8k workgroups, so no source splitting is needed.  FP32 evaluation uses double-float positions and
-// flushes FP32 partial sums into FP64 accumulators after every batch.
+// Sources are streamed through LDS in batches of BLOCK.  Two forms (flow_plan
+// picks one from the point count): each lane holds two targets of its own, or
+// (SHARED) the BLOCK/64 waves of a workgroup hold the same 64 targets and
+// divide every batch between them, adding their sums in LDS in wave order.
+// Either form may also divide the sources between gridDim.y workgroups, which
+// write FP64 partial sums that flow_finish_kernel adds in chunk order, so a
+// result does not change from run to run.  FP32 evaluation uses double-float
+// positions and flushes FP32 partial sums into FP64 accumulators after every
+// batch.
+//
+// Bound by VALU issue: at 4.2M points (FP32) the kernel's time equals the sum
+// of its instructions' issue times (about 97 cycles per segment source and 64
+// targets, 68 per blob).  What the divided forms give (MI355X): 10,007 points
+// x 2,320 sources in FP64, where 20 workgroups were left for 256 CUs, and 1M
+// points x 34,600 sources in FP32, where 1,954 workgroups made 7.6 per CU;
+// times at flow_plan.
+#include <algorithm>
+
 #include "rpy_pair.h"
 #include "tfs_internal.h"
 
@@ -56,23 +71,39 @@ __device__ __forceinline__ void blakelet(double* acc, double zi, double zj, doub
     acc[2] += g * (Dzx * fx + Dzy * fy + Dzz * fz);
 }
 
-template <typename T, int MODE, bool BLAKE, int FS, int BLOCK, int R>
-__device__ __forceinline__ void flow_sources(const FlowArgs& a, CView xsrc, CView fsrc, int nsrc, double aj,
+// 2/sqrt(x) from the v_rsq_f64 seed z by one Newton-Raphson step without its
+// factor 1/2, w = z (3 - x z^2): three operations instead of four; callers fold
+// the powers of two into their flush.  The same error as rsqrt_refined.
+__device__ __forceinline__ double rsqrt_twice(double x) {
+    const double z = __builtin_amdgcn_rsq(x);
+    return z * __builtin_fma(-x * z, z, 3.0);
+}
+
+// The sources [s_lo, s_hi) of one class added into acc.  SHARED: wave w takes
+// the w-th part of every batch.
+template <typename T, int MODE, bool BLAKE, int FS, int BLOCK, int R, bool SHARED>
+__device__ __forceinline__ void flow_sources(const FlowArgs& a, CView xsrc, CView fsrc, int s_lo, int s_hi, double aj,
                                              const double (&xi)[R][3], const T (&xh)[R][3],
                                              const T (&xl)[R][3], double (&acc)[R][3], T* lds) {
     constexpr int REC = flow_rec<T>();
     constexpr bool F32 = sizeof(T) == 4;
     const int tid = threadIdx.x;
-    const double PI = 3.14159265358979323846;
     const T s3 = T(aj * aj / 3.0);
-    const T c8 = T(1.0 / (8.0 * PI * a.mu));
+    const T m3s3 = T(-3) * s3;
     const T aj2 = T(aj * aj);
     T part[R][3];
-    // FP32 Stokeslet mode: the rotlet's negative cross-product halves, summed
-    // apart and subtracted at the flush (every operation an accumulate)
+    // FP32: the rotlet's negative cross-product halves, summed apart and
+    // subtracted at the flush (every operation an accumulate).  FP64: the
+    // terms in 1/r^3 (times 8), apart from the A f ones (times 2).
     T negp[R][3];
-    for (int s0 = 0; s0 < nsrc; s0 += BLOCK) {
-        const int n = (nsrc - s0) < BLOCK ? (nsrc - s0) : BLOCK;
+    for (int s0 = s_lo; s0 < s_hi; s0 += BLOCK) {
+        const int n = (s_hi - s0) < BLOCK ? (s_hi - s0) : BLOCK;
+        int j0 = 0, j1 = n;
+        if constexpr (SHARED) {  // uniform over the wave
+            const int per = (n + BLOCK / 64 - 1) / (BLOCK / 64);
+            j0 = __builtin_amdgcn_readfirstlane(tid >> 6) * per;
+            j1 = j0 + per < n ? j0 + per : n;
+        }
         __syncthreads();
         if (tid < n) {
             const int64_t s = s0 + tid;
@@ -98,7 +129,7 @@ __device__ __forceinline__ void flow_sources(const FlowArgs& a, CView xsrc, CVie
             part[r][0] = part[r][1] = part[r][2] = T(0);
             negp[r][0] = negp[r][1] = negp[r][2] = T(0);
         }
-        for (int j = 0; j < n; ++j) {
+        for (int j = j0; j < j1; ++j) {
             const T* rec = lds + j * REC;
             constexpr int F0 = F32 ? 6 : 3;
             T f[FS];
@@ -116,19 +147,35 @@ __device__ __forceinline__ void flow_sources(const FlowArgs& a, CView xsrc, CVie
                     dy = T(xi[r][1]) - rec[1];
                     dz = T(xi[r][2]) - rec[2];
                 }
-                const T r2 = dx * dx + dy * dy + dz * dz;
-                if constexpr (MODE == 0 && F32) {
-                    // Stokeslet (+ rotlet): flow_field_evaluator.cu:66-78, 119-124, written
-                    // as accumulates only: v += f/r + (d.f) d / r^3 + (tau x d) / r^3.
-                    const T rm1 = rsqrt_refined(r2);
-                    const T rm3 = rm1 * (rm1 * rm1);
-                    const T sd = rm3 * fma_t(dz, f[2], fma_t(dy, f[1], dx * f[0]));
-                    part[r][0] = fma_t(sd, dx, fma_t(rm1, f[0], part[r][0]));
-                    part[r][1] = fma_t(sd, dy, fma_t(rm1, f[1], part[r][1]));
-                    part[r][2] = fma_t(sd, dz, fma_t(rm1, f[2], part[r][2]));
+                const T r2 = fma_t(dz, dz, fma_t(dy, dy, dx * dx));
+                // Stokeslet (+ rotlet): flow_field_evaluator.cu:66-78, 119-124; RPY point
+                // tracer: the pair tensor with ai = 0.  Both are A f + Q (d.f) d / r^3 +
+                // (tau x d) / r^3, with A = 1/r, Q = 1 or A = 1/r + s3/r^3, Q = 1 - 3 s3/r^2.
+                // A tracer within the source's radius gets nothing here (its w = 0) and the
+                // inner form below.
+                bool inside = false;
+                if constexpr (MODE == 1) inside = !(r2 > aj2);
+                if constexpr (F32) {
+                    // accumulates only
+                    T rm1 = rsqrt_refined(r2);
+                    if constexpr (MODE == 1) rm1 = inside ? T(0) : rm1;
+                    const T rm2 = rm1 * rm1;
+                    const T rm3 = rm1 * rm2;
+                    const T A = MODE == 1 ? fma_t(s3, rm3, rm1) : rm1;
+                    T sd;
+                    T ex, ey, ez;
+                    if constexpr (FS == 6) {
+                        ex = rm3 * dx, ey = rm3 * dy, ez = rm3 * dz;
+                        sd = fma_t(ez, f[2], fma_t(ey, f[1], ex * f[0]));
+                    } else {
+                        sd = rm3 * fma_t(dz, f[2], fma_t(dy, f[1], dx * f[0]));
+                    }
+                    if constexpr (MODE == 1) sd = fma_t(m3s3 * rm2, sd, sd);
+                    part[r][0] = fma_t(sd, dx, fma_t(A, f[0], part[r][0]));
+                    part[r][1] = fma_t(sd, dy, fma_t(A, f[1], part[r][1]));
+                    part[r][2] = fma_t(sd, dz, fma_t(A, f[2], part[r][2]));
                     if constexpr (FS == 6) {
                         // (tau x d) / r^3 as + and - halves
-                        const T ex = rm3 * dx, ey = rm3 * dy, ez = rm3 * dz;
                         part[r][0] = fma_t(f[4], ez, part[r][0]);
                         negp[r][0] = fma_t(f[5], ey, negp[r][0]);
                         part[r][1] = fma_t(f[5], ex, part[r][1]);
@@ -136,44 +183,47 @@ __device__ __forceinline__ void flow_sources(const FlowArgs& a, CView xsrc, CVie
                         part[r][2] = fma_t(f[3], ey, part[r][2]);
                         negp[r][2] = fma_t(f[4], ex, negp[r][2]);
                     }
-                    if constexpr (BLAKE) {
-                        // Blakelet image system, flow_field_evaluator.cu:83-116, evaluated in
-                        // double (the image distance of a wall-adjacent pair is small).
-                        const double zi = xi[r][2];
-                        const double zj = double(rec[2]) + double(rec[5]);
-                        blakelet(acc[r], zi, zj, double(dx), double(dy), double(f[0]), double(f[1]), double(f[2]));
-                    }
-                } else if constexpr (MODE == 0) {
-                    // Stokeslet (+ rotlet): flow_field_evaluator.cu:66-78, 119-124
-                    const T rm1 = rsqrt_refined(r2);
-                    const T rm2 = rm1 * rm1;
-                    const T k = rm2 * (dx * f[0] + dy * f[1] + dz * f[2]);
-                    part[r][0] += rm1 * (f[0] + dx * k);
-                    part[r][1] += rm1 * (f[1] + dy * k);
-                    part[r][2] += rm1 * (f[2] + dz * k);
-                    if constexpr (FS == 6) {
-                        const T rm3 = rm1 * rm2;
-                        part[r][0] += rm3 * (f[4] * dz - f[5] * dy);
-                        part[r][1] += rm3 * (f[5] * dx - f[3] * dz);
-                        part[r][2] += rm3 * (f[3] * dy - f[4] * dx);
-                    }
-                    if constexpr (BLAKE) {
-                        // Blakelet image system, flow_field_evaluator.cu:83-116, evaluated in
-                        // double (the image distance of a wall-adjacent pair is small).
-                        const double zi = xi[r][2];
-                        double zj;
-                        if constexpr (F32) zj = double(rec[2]) + double(rec[5]);
-                        else zj = rec[2];
-                        blakelet(acc[r], zi, zj, double(dx), double(dy), double(f[0]), double(f[1]), double(f[2]));
-                    }
                 } else {
-                    // RPY point tracer: the pair tensor with ai = 0.
-                    if (r2 > aj2) {
-                        pair_far<T, 3, FS>(part[r], dx, dy, dz, rsqrt_refined(r2), f, s3, c8);
+                    // w = 2/r: part = 2 A f, negp = 8 [Q (d.f) d + tau x d] / r^3
+                    T w = rsqrt_twice(r2);
+                    if constexpr (MODE == 1) w = inside ? T(0) : w;
+                    const T w2 = w * w;
+                    const T w3 = w * w2;
+                    const T A = MODE == 1 ? fma_t(T(0.25) * s3, w3, w) : w;
+                    part[r][0] = fma_t(A, f[0], part[r][0]);
+                    part[r][1] = fma_t(A, f[1], part[r][1]);
+                    part[r][2] = fma_t(A, f[2], part[r][2]);
+                    T sd;
+                    T ex, ey, ez;
+                    if constexpr (FS == 6) {
+                        ex = w3 * dx, ey = w3 * dy, ez = w3 * dz;
+                        sd = fma_t(ez, f[2], fma_t(ey, f[1], ex * f[0]));
                     } else {
-                        double fd[FS];
-#pragma unroll
-                        for (int k = 0; k < FS; ++k) fd[k] = double(f[k]);
+                        sd = w3 * fma_t(dz, f[2], fma_t(dy, f[1], dx * f[0]));
+                    }
+                    if constexpr (MODE == 1) sd = fma_t(T(0.25) * m3s3 * w2, sd, sd);
+                    negp[r][0] = fma_t(sd, dx, negp[r][0]);
+                    negp[r][1] = fma_t(sd, dy, negp[r][1]);
+                    negp[r][2] = fma_t(sd, dz, negp[r][2]);
+                    if constexpr (FS == 6) {
+                        negp[r][0] = fma_t(f[4], ez, fma_t(-f[5], ey, negp[r][0]));
+                        negp[r][1] = fma_t(f[5], ex, fma_t(-f[3], ez, negp[r][1]));
+                        negp[r][2] = fma_t(f[3], ey, fma_t(-f[4], ex, negp[r][2]));
+                    }
+                }
+                if constexpr (BLAKE) {
+                    // Blakelet image system, flow_field_evaluator.cu:83-116, evaluated in
+                    // double (the image distance of a wall-adjacent pair is small).
+                    const double zi = xi[r][2];
+                    double zj;
+                    if constexpr (F32) zj = double(rec[2]) + double(rec[5]);
+                    else zj = rec[2];
+                    blakelet(acc[r], zi, zj, double(dx), double(dy), double(f[0]), double(f[1]), double(f[2]));
+                }
+                if constexpr (MODE == 1) {
+                    if (inside) {
+                        // rare: the rigid-body limit f / (6 pi mu aj) + tau x d / (8 pi mu aj^3)
+                        // (cuda_functions.cu:207-354 with ai = 0), before the common factor
                         double ddx, ddy, ddz;
                         if constexpr (F32) {
                             ddx = xi[r][0] - (double(rec[0]) + double(rec[3]));
@@ -182,7 +232,15 @@ __device__ __forceinline__ void flow_sources(const FlowArgs& a, CView xsrc, CVie
                         } else {
                             ddx = dx; ddy = dy; ddz = dz;
                         }
-                        pair_near<3, FS>(acc[r], ddx, ddy, ddz, fd, 0.0, aj, a.mu);
+                        const double ca = 4.0 / (3.0 * aj), cc = 1.0 / (aj * aj * aj);
+                        double u[3] = {ca * double(f[0]), ca * double(f[1]), ca * double(f[2])};
+                        if constexpr (FS == 6) {
+                            u[0] += cc * (double(f[4]) * ddz - double(f[5]) * ddy);
+                            u[1] += cc * (double(f[5]) * ddx - double(f[3]) * ddz);
+                            u[2] += cc * (double(f[3]) * ddy - double(f[4]) * ddx);
+                        }
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) acc[r][k] += u[k];
                     }
                 }
             }
@@ -190,21 +248,58 @@ __device__ __forceinline__ void flow_sources(const FlowArgs& a, CView xsrc, CVie
 #pragma unroll
         for (int r = 0; r < R; ++r)
 #pragma unroll
-            for (int k = 0; k < 3; ++k) acc[r][k] += double(part[r][k]) - double(negp[r][k]);
+            for (int k = 0; k < 3; ++k) {
+                if constexpr (!F32) acc[r][k] += 0.5 * part[r][k] + 0.125 * negp[r][k];
+                else acc[r][k] += double(part[r][k]) - double(negp[r][k]);
+            }
     }
 }
 
-template <typename T, int MODE, bool BLAKE, int BLOCK, int R>
+// Each body's total force as one Stokeslet at its centre, taken out of acc
+// (the per-source sums of flow_field_evaluator.cu:125-143, 191-209).
+__device__ __forceinline__ void take_out_net_force(const FlowArgs& a, const double* __restrict__ net,
+                                                   const double (&x)[3], double (&acc)[3]) {
+    for (int b = 0; b < a.num_bodies; ++b) {
+        const double dx = x[0] - a.x_bodies[3 * b], dy = x[1] - a.x_bodies[3 * b + 1],
+                     dz = x[2] - a.x_bodies[3 * b + 2];
+        const double fx = net[3 * b], fy = net[3 * b + 1], fz = net[3 * b + 2];
+        const double rm2 = 1.0 / (dx * dx + dy * dy + dz * dz);
+        const double rm1 = __builtin_sqrt(rm2);
+        const double k = rm2 * (dx * fx + dy * fy + dz * fz);
+        acc[0] -= rm1 * (fx + dx * k);
+        acc[1] -= rm1 * (fy + dy * k);
+        acc[2] -= rm1 * (fz + dz * k);
+    }
+}
+
+// The common factor of every term.
+__device__ __forceinline__ double flow_prefactor(double mu) { return 1.0 / (8.0 * 3.14159265358979323846 * mu); }
+
+// Finish stamp of a workgroup: the largest of them is the evaluation's end.
+__device__ __forceinline__ void stamp_end(unsigned long long* stamps) {
+    if (threadIdx.x == 0) atomicMax(stamps + 1, (unsigned long long)wall_clock64());
+}
+
+// blockIdx.x: a tile of targets (BLOCK x R, or 64 x R shared by the waves);
+// blockIdx.y: a chunk of a.chunk sources of the segments followed by the blobs.
+// With a.part the sums go to part[(blockIdx.y * 3 + k) * nt + t], otherwise
+// (one chunk) straight to the velocities.
+template <typename T, int MODE, bool BLAKE, int BLOCK, int R, bool SHARED>
 __global__ __launch_bounds__(BLOCK) void flow_kernel(FlowArgs a, const double* __restrict__ net) {
-    __shared__ __align__(16) T lds[BLOCK * flow_rec<T>()];
+    constexpr int LANES = SHARED ? 64 : BLOCK;
+    constexpr int SUMS = SHARED ? (BLOCK / 64 - 1) * 64 * R * 3 * (int)(sizeof(double) / sizeof(T)) : 0;
+    constexpr int BATCH = BLOCK * flow_rec<T>();
+    __shared__ __align__(16) T lds[BATCH > SUMS ? BATCH : SUMS];
     constexpr bool F32 = sizeof(T) == 4;
-    const int64_t t0 = (int64_t)blockIdx.x * (BLOCK * R) + threadIdx.x;
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) a.stamps[0] = (unsigned long long)wall_clock64();
+    const int lane = (int)threadIdx.x & (LANES - 1);
+    const int64_t t0 = (int64_t)blockIdx.x * (LANES * R) + lane;
     double xi[R][3];
     T xh[R][3], xl[R][3];
     double acc[R][3];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        int64_t t = t0 + (int64_t)r * BLOCK;
+        int64_t t = t0 + (int64_t)r * LANES;
         t = t < a.nt ? t : a.nt - 1;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
@@ -218,34 +313,73 @@ __global__ __launch_bounds__(BLOCK) void flow_kernel(FlowArgs a, const double* _
             acc[r][k] = 0.0;
         }
     }
-    if (a.ns_total > 0)
-        flow_sources<T, MODE, BLAKE, 6, BLOCK, R>(a, a.xs, a.fs, a.ns_total, a.a_seg, xi, xh, xl, acc, lds);
-    if (a.nb_total > 0)
-        flow_sources<T, MODE, false, 3, BLOCK, R>(a, a.xb, a.fb, a.nb_total, a.a_blob, xi, xh, xl, acc, lds);
-    const double PI = 3.14159265358979323846;
-    const double prefac = MODE == 0 ? 1.0 / (8.0 * PI * a.mu) : 1.0;
+    const int64_t total = (int64_t)a.ns_total + a.nb_total;
+    const int64_t c0 = (int64_t)blockIdx.y * a.chunk, c1 = c0 + a.chunk < total ? c0 + a.chunk : total;
+    if (c0 < a.ns_total)
+        flow_sources<T, MODE, BLAKE, 6, BLOCK, R, SHARED>(a, a.xs, a.fs, (int)c0,
+                                                          (int)(c1 < a.ns_total ? c1 : a.ns_total), a.a_seg, xi, xh,
+                                                          xl, acc, lds);
+    if (c1 > a.ns_total)
+        flow_sources<T, MODE, false, 3, BLOCK, R, SHARED>(a, a.xb, a.fb, (int)(c0 > a.ns_total ? c0 - a.ns_total : 0),
+                                                          (int)(c1 - a.ns_total), a.a_blob, xi, xh, xl, acc, lds);
+    bool writes = true;
+    if constexpr (SHARED && BLOCK > 64) {
+        double* buf = reinterpret_cast<double*>(lds);
+        const int w = (int)threadIdx.x >> 6;
+        __syncthreads();  // every wave is done with the last batch's records
+        if (w > 0) {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) buf[(((w - 1) * R + r) * 3 + k) * 64 + lane] = acc[r][k];
+        }
+        __syncthreads();
+        writes = w == 0;
+        if (writes) {
+            for (int v = 0; v < BLOCK / 64 - 1; ++v)
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) acc[r][k] += buf[((v * R + r) * 3 + k) * 64 + lane];
+        }
+    }
+    const double prefac = flow_prefactor(a.mu);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-        const int64_t t = t0 + (int64_t)r * BLOCK;
-        if (t >= a.nt) continue;
-        if (MODE == 0 && a.remove_net_force) {
-            // Each body's total force as one Stokeslet at its centre
-            // (the per-source sums of flow_field_evaluator.cu:125-143, 191-209).
-            for (int b = 0; b < a.num_bodies; ++b) {
-                const double dx = xi[r][0] - a.x_bodies[3 * b], dy = xi[r][1] - a.x_bodies[3 * b + 1],
-                             dz = xi[r][2] - a.x_bodies[3 * b + 2];
-                const double fx = net[3 * b], fy = net[3 * b + 1], fz = net[3 * b + 2];
-                const double rm2 = 1.0 / (dx * dx + dy * dy + dz * dz);
-                const double rm1 = __builtin_sqrt(rm2);
-                const double k = rm2 * (dx * fx + dy * fy + dz * fz);
-                acc[r][0] -= rm1 * (fx + dx * k);
-                acc[r][1] -= rm1 * (fy + dy * k);
-                acc[r][2] -= rm1 * (fz + dz * k);
-            }
+        const int64_t t = t0 + (int64_t)r * LANES;
+        if (!writes || t >= a.nt) continue;
+        if (a.part) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) a.part[((int64_t)blockIdx.y * 3 + k) * a.nt + t] = acc[r][k];
+            continue;
         }
+        if (MODE == 0 && a.remove_net_force) take_out_net_force(a, net, xi[r], acc[r]);
 #pragma unroll
         for (int k = 0; k < 3; ++k) a.vt.p[t * a.vt.ld_p + k * a.vt.ld_c] = prefac * acc[r][k];
     }
+    if (!a.part) stamp_end(a.stamps);
+}
+
+// Adds the chunks' partial sums of each target in chunk order.
+template <int MODE>
+__global__ __launch_bounds__(256) void flow_finish_kernel(FlowArgs a, int nchunk, const double* __restrict__ net) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (t < a.nt) {
+        double acc[3] = {0.0, 0.0, 0.0};
+#pragma unroll 4
+        for (int c = 0; c < nchunk; ++c)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) acc[k] += a.part[((int64_t)c * 3 + k) * a.nt + t];
+        if (MODE == 0 && a.remove_net_force) {
+            const double x[3] = {a.xt.p[t * a.xt.ld_p], a.xt.p[t * a.xt.ld_p + a.xt.ld_c],
+                                 a.xt.p[t * a.xt.ld_p + 2 * a.xt.ld_c]};
+            take_out_net_force(a, net, x, acc);
+        }
+        const double prefac = flow_prefactor(a.mu);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) a.vt.p[t * a.vt.ld_p + k * a.vt.ld_c] = prefac * acc[k];
+    }
+    stamp_end(a.stamps);
 }
 
 // Per-body total force (segments + blobs), one thread per body.
@@ -260,17 +394,25 @@ __global__ void net_force_kernel(FlowArgs a, double* __restrict__ net, int nbod)
     for (int k = 0; k < 3; ++k) net[3 * b + k] = f[k];
 }
 
+template <typename T, int MODE, bool BLAKE, int BLOCK>
+void launch_block(const FlowArgs& a, const double* net, const FlowPlan& p, hipStream_t s) {
+    const int64_t tile = p.shared ? 64 : 2 * BLOCK;
+    const dim3 grid((unsigned)((a.nt + tile - 1) / tile), (unsigned)p.chunks);
+    if (p.shared) hipLaunchKernelGGL((flow_kernel<T, MODE, BLAKE, BLOCK, 1, true>), grid, dim3(BLOCK), 0, s, a, net);
+    else hipLaunchKernelGGL((flow_kernel<T, MODE, BLAKE, BLOCK, 2, false>), grid, dim3(BLOCK), 0, s, a, net);
+}
+
 template <typename T, int MODE, bool BLAKE>
-hipError_t launch_typed(const FlowArgs& a, const double* net, int block, hipStream_t s) {
-    const int R = 2;  // two targets per lane share every LDS source read
-    const int64_t tile = (int64_t)block * R;
-    const dim3 grid((unsigned)((a.nt + tile - 1) / tile));
-    switch (block) {
-        case 64: hipLaunchKernelGGL((flow_kernel<T, MODE, BLAKE, 64, 2>), grid, dim3(64), 0, s, a, net); break;
-        case 128: hipLaunchKernelGGL((flow_kernel<T, MODE, BLAKE, 128, 2>), grid, dim3(128), 0, s, a, net); break;
-        case 256: hipLaunchKernelGGL((flow_kernel<T, MODE, BLAKE, 256, 2>), grid, dim3(256), 0, s, a, net); break;
+hipError_t launch_typed(const FlowArgs& a, const double* net, const FlowPlan& p, hipStream_t s) {
+    switch (p.block) {
+        case 64: launch_block<T, MODE, BLAKE, 64>(a, net, p, s); break;
+        case 128: launch_block<T, MODE, BLAKE, 128>(a, net, p, s); break;
+        case 256: launch_block<T, MODE, BLAKE, 256>(a, net, p, s); break;
         default: return hipErrorInvalidValue;
     }
+    if (a.part)
+        hipLaunchKernelGGL(flow_finish_kernel<MODE>, dim3((unsigned)((a.nt + 255) / 256)), dim3(256), 0, s, a, p.chunks,
+                           net);
     return hipGetLastError();
 }
 
@@ -282,15 +424,50 @@ hipError_t launch_flow_net(const FlowArgs& a, double* net, int nbod, hipStream_t
     return hipGetLastError();
 }
 
-hipError_t launch_flow_eval(int precision, const FlowArgs& a, const double* net, int block, hipStream_t s) {
+// The launch form for nt points and nsrc sources on num_cus CUs.
+//
+// Each lane two targets of its own (every LDS read of a source serves both)
+// where that form, with chunks of at least four batches, gives every CU 16
+// workgroups, or undivided four; below, one target per lane, shared by the
+// workgroup's waves.  Then the sources are divided until every CU has ~32
+// (own targets) or ~12 (shared) workgroups of four waves, chunks at least
+// four batches (own: the partial sums then cost under 1%) or half a batch
+// (shared), partial sums within 256 MB.  Measured (MI355X, call of 320
+// segments + 2,000 blobs at 10,007 points, FP64): 334 us undivided, own
+// targets; 32 us shared and divided.  13,000 sources at 300,000 points, FP32:
+// 3,240 and 2,140 us (own targets both).  34,600 sources at 1M points, FP32:
+// 22.2 and 19.6 ms.
+FlowPlan flow_plan(int64_t nt, int64_t nsrc, int block, int num_cus, bool may_divide) {
+    FlowPlan p;
+    p.block = block;
+    const int64_t own = (nt + 2 * block - 1) / (2 * block);
+    const int64_t least_own = 4LL * block;
+    p.shared = own < 4LL * num_cus && own * (nsrc / least_own) < 16LL * num_cus;
+    const int64_t tiles = p.shared ? (nt + 63) / 64 : own;
+    const int64_t unit = p.shared ? 64 : block;                       // chunks are multiples of this
+    const int64_t least = p.shared ? std::max(64, block / 2) : least_own;
+    const int64_t waves = block / 64;
+    const int64_t want = (p.shared ? 48LL : 128LL) * num_cus / waves;  // workgroups
+    int64_t n = may_divide && tiles > 0 ? (want + tiles - 1) / tiles : 1;
+    n = std::min<int64_t>(n, std::max<int64_t>(nsrc / least, 1));
+    n = std::min<int64_t>(n, std::max<int64_t>((256LL << 20) / (24 * std::max<int64_t>(nt, 1)), 1));
+    n = std::max<int64_t>(std::min<int64_t>(n, 65535), 1);
+    int64_t chunk = (nsrc + n - 1) / n;
+    if (n > 1) chunk = (chunk + unit - 1) / unit * unit;
+    p.chunk = (int)std::max<int64_t>(std::min<int64_t>(chunk, INT32_MAX), 1);
+    p.chunks = (int)std::max<int64_t>((nsrc + p.chunk - 1) / p.chunk, 1);
+    return p;
+}
+
+hipError_t launch_flow_eval(int precision, const FlowArgs& a, const double* net, const FlowPlan& plan, hipStream_t s) {
     if (a.nt <= 0) return hipSuccess;
     const bool blake = a.mode == 0 && a.nb_per_body == 0 && a.ns_total > 0;
     if (precision == 0) {
-        if (a.mode == 1) return launch_typed<double, 1, false>(a, net, block, s);
-        return blake ? launch_typed<double, 0, true>(a, net, block, s) : launch_typed<double, 0, false>(a, net, block, s);
+        if (a.mode == 1) return launch_typed<double, 1, false>(a, net, plan, s);
+        return blake ? launch_typed<double, 0, true>(a, net, plan, s) : launch_typed<double, 0, false>(a, net, plan, s);
     }
-    if (a.mode == 1) return launch_typed<float, 1, false>(a, net, block, s);
-    return blake ? launch_typed<float, 0, true>(a, net, block, s) : launch_typed<float, 0, false>(a, net, block, s);
+    if (a.mode == 1) return launch_typed<float, 1, false>(a, net, plan, s);
+    return blake ? launch_typed<float, 0, true>(a, net, plan, s) : launch_typed<float, 0, false>(a, net, plan, s);
 }
 
 }  // namespace tfs

@@ -21,16 +21,6 @@
 
 namespace tfs {
 
-// Pair-independent constants, computed once on the host for given radii and mu.
-template <typename T>
-struct PairConsts {
-    T sum_a2;      // (ai + aj)^2          far-field threshold on r^2
-    T s3;          // (ai^2 + aj^2)/3
-    T c8;          // 1/(8 pi mu)
-    // overlap / inner branch (evaluated in double for both evaluation types)
-    double ai, aj, mu;
-};
-
 __device__ __forceinline__ double rsqrt_refined(double x) {
     // v_rsq_f64 seed (measured on gfx950: relative error <= 5.3e-8 over
     // x in [4, 4e6]), then one Newton-Raphson step y <- y + y/2 (1 - x y^2),
@@ -44,44 +34,6 @@ __device__ __forceinline__ float rsqrt_refined(float x) {
     return __builtin_amdgcn_rsqf(x);
 }
 
-// Far field, r^2 > (ai+aj)^2.  rm1 = 1/r.
-template <typename T, int VT, int FS>
-__device__ __forceinline__ void pair_far(T* __restrict__ v, T dx, T dy, T dz, T rm1,
-                                         const T* __restrict__ f, T s3, T c8) {
-    const T rm2 = rm1 * rm1;
-    const T c = c8 * rm1;                       // 1/(8 pi mu r)
-    const T A = c + (c * s3) * rm2;             // (1 + (ai^2+aj^2)/(3 r^2)) / (8 pi mu r)
-    const T B = (c - T(3) * (c * s3) * rm2) * rm2;
-    const T dF = dx * f[0] + dy * f[1] + dz * f[2];
-    const T Bd = B * dF;
-    v[0] += A * f[0] + Bd * dx;
-    v[1] += A * f[1] + Bd * dy;
-    v[2] += A * f[2] + Bd * dz;
-    if constexpr (FS == 6 || VT == 6) {
-        const T C = c * rm2;                    // 1/(8 pi mu r^3)
-        if constexpr (FS == 6) {
-            // translation-rotation: v += C (tau x d)
-            v[0] += C * (f[4] * dz - f[5] * dy);
-            v[1] += C * (f[5] * dx - f[3] * dz);
-            v[2] += C * (f[3] * dy - f[4] * dx);
-        }
-        if constexpr (VT == 6) {
-            // rotation-translation: w += C (F x d)
-            v[3] += C * (f[1] * dz - f[2] * dy);
-            v[4] += C * (f[2] * dx - f[0] * dz);
-            v[5] += C * (f[0] * dy - f[1] * dx);
-            if constexpr (FS == 6) {
-                // rotation-rotation: w += -C/2 [tau - 3 (tau.d) d / r^2]
-                const T Ar = T(-0.5) * C;
-                const T Br = T(-3) * Ar * rm2 * (dx * f[3] + dy * f[4] + dz * f[5]);
-                v[3] += Ar * f[3] + Br * dx;
-                v[4] += Ar * f[4] + Br * dy;
-                v[5] += Ar * f[5] + Br * dz;
-            }
-        }
-    }
-}
-
 __device__ __forceinline__ float fmax_t(float a, float b) { return __builtin_fmaxf(a, b); }
 __device__ __forceinline__ double fmax_t(double a, double b) { return __builtin_fmax(a, b); }
 __device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
@@ -89,8 +41,7 @@ __device__ __forceinline__ double fma_t(double a, double b, double c) { return _
 
 // Far field with the source strengths already multiplied by 1/(8 pi mu), in
 // the fewest VALU operations: A = 1/r + s3/r^3, B = (1 - 3 s3/r^2)/r^3,
-// C = 1/r^3, and every term is fused into the accumulators.  The same tensor
-// as pair_far.
+// C = 1/r^3, and every term is fused into the accumulators.
 // fneg (FP32 only, else unused): the negated torque (FS = 6) followed by the
 // negated force (VT = 6) of the source, so that the cross products are
 // accumulates.

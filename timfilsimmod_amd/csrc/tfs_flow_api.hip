@@ -24,7 +24,12 @@ struct tfs_flow {
            *net = nullptr;
     double* pts = nullptr;     // staging for host callers: points | velocities
     int64_t pts_cap = 0;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    double* part = nullptr;    // partial sums of divided sources
+    int64_t part_len = 0;
+    int num_cus = 256;
+    int clock_khz = 0;
+    unsigned long long* stamps = nullptr;  // start and finish of the last evaluation (wall clock ticks)
+    bool stamped = false;
     tfs::F32Stage f32;         // FP32 entry points (tfs_flow_*_f32)
 };
 
@@ -68,8 +73,13 @@ int tfs_flow_create(const tfs_flow_desc* desc, tfs_flow** out) {
     for (int64_t l : lens) total += ((std::max<int64_t>(l, 1) + 31) / 32) * 32;
     if (e == hipSuccess) e = hipMalloc(&h->src, total * 8);
     if (e == hipSuccess) e = hipMemsetAsync(h->src, 0, total * 8, h->stream);
-    if (e == hipSuccess) e = hipEventCreate(&h->ev0);
-    if (e == hipSuccess) e = hipEventCreate(&h->ev1);
+    if (e == hipSuccess) e = hipMalloc(&h->stamps, 16);
+    if (e == hipSuccess) e = hipMemsetAsync(h->stamps, 0, 16, h->stream);
+    int dev = 0, cus = 0;
+    if (e == hipSuccess) e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&h->clock_khz, hipDeviceAttributeWallClockRate, dev);
+    if (e == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
+        h->num_cus = cus;
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) {
         tfs_flow_destroy(h);
@@ -90,9 +100,9 @@ int tfs_flow_destroy(tfs_flow* h) {
     if (h->stream) hipStreamSynchronize(h->stream);
     if (h->src) hipFree(h->src);
     if (h->pts) hipFree(h->pts);
+    if (h->part) hipFree(h->part);
+    if (h->stamps) hipFree(h->stamps);
     free_stage(h->f32);
-    if (h->ev0) hipEventDestroy(h->ev0);
-    if (h->ev1) hipEventDestroy(h->ev1);
     if (h->own_stream) hipStreamDestroy(h->stream);
     delete h;
     return TFS_OK;
@@ -105,14 +115,23 @@ int tfs_flow_set_sources(tfs_flow* h, const double* x_segs, const double* f_segs
     const int64_t ns = (int64_t)D.num_bodies * D.segs_per_body, nb = (int64_t)D.num_bodies * D.blobs_per_body;
     if ((ns && (!x_segs || !f_segs)) || (nb && (!x_blobs || !f_blobs)) || (D.remove_net_force && !x_bodies))
         return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_flow_set_sources: missing array");
-    const hipMemcpyKind k = D.memory == TFS_MEMORY_HOST ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
+    if (D.memory == TFS_MEMORY_DEVICE) {
+        CopyList list;
+        list.add(x_segs, h->x_segs, 3 * ns);
+        list.add(f_segs, h->f_segs, 6 * ns);
+        list.add(x_blobs, h->x_blobs, 3 * nb);
+        list.add(f_blobs, h->f_blobs, 3 * nb);
+        if (x_bodies) list.add(x_bodies, h->x_bodies, 3LL * D.num_bodies);
+        return check(copy_list(list, h->stream), "tfs_flow_set_sources");
+    }
+    const hipMemcpyKind k = hipMemcpyHostToDevice;
     hipError_t e = hipSuccess;
     if (ns) e = hipMemcpyAsync(h->x_segs, x_segs, 24 * ns, k, h->stream);
     if (e == hipSuccess && ns) e = hipMemcpyAsync(h->f_segs, f_segs, 48 * ns, k, h->stream);
     if (e == hipSuccess && nb) e = hipMemcpyAsync(h->x_blobs, x_blobs, 24 * nb, k, h->stream);
     if (e == hipSuccess && nb) e = hipMemcpyAsync(h->f_blobs, f_blobs, 24 * nb, k, h->stream);
     if (e == hipSuccess && x_bodies) e = hipMemcpyAsync(h->x_bodies, x_bodies, 24LL * D.num_bodies, k, h->stream);
-    if (e == hipSuccess && D.memory == TFS_MEMORY_HOST) e = hipStreamSynchronize(h->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     return check(e, "tfs_flow_set_sources");
 }
 
@@ -166,11 +185,35 @@ hipError_t run_flow(tfs_flow* h, int64_t num_points, const double* xp, double* v
     a.a_seg = D.seg_radius;
     a.a_blob = D.blob_radius;
     a.mu = D.mu;
+    a.stamps = h->stamps;
+    a.part = nullptr;
     hipError_t e = hipSuccess;
+    // A captured evaluation keeps the undivided form: a graph must not hold the
+    // partial-sum buffer, which a later call may replace.
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    (void)hipStreamIsCapturing(h->stream, &capture);
+    const bool may_divide = capture == hipStreamCaptureStatusNone;
+    const int64_t nsrc = (int64_t)a.ns_total + a.nb_total;
+    FlowPlan plan = flow_plan(num_points, nsrc, h->block, h->num_cus, may_divide);
+    if (plan.chunks > 1) {
+        const int64_t need = 3LL * plan.chunks * num_points;
+        if (need > h->part_len) {
+            if (h->part) {
+                (void)hipStreamSynchronize(h->stream);
+                (void)hipFree(h->part);
+            }
+            h->part = nullptr;
+            h->part_len = 0;
+            if (hipMalloc(&h->part, 8 * need) == hipSuccess) h->part_len = need;
+            else (void)hipGetLastError();  // no room: undivided
+        }
+        if (h->part) a.part = h->part;
+        else plan = flow_plan(num_points, nsrc, h->block, h->num_cus, false);
+    }
+    a.chunk = plan.chunk;
     if (a.remove_net_force) e = launch_flow_net(a, h->net, D.num_bodies, h->stream);
-    if (e == hipSuccess) e = hipEventRecord(h->ev0, h->stream);
-    if (e == hipSuccess) e = launch_flow_eval(D.precision, a, h->net, h->block, h->stream);
-    if (e == hipSuccess) e = hipEventRecord(h->ev1, h->stream);
+    if (e == hipSuccess) e = launch_flow_eval(D.precision, a, h->net, plan, h->stream);
+    h->stamped = e == hipSuccess;
     return e;
 }
 
@@ -249,10 +292,11 @@ int tfs_flow_set_block(tfs_flow* h, int32_t block) {
 
 int tfs_flow_last_kernel_ms(tfs_flow* h, double* ms) {
     if (!h || !ms) return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_flow_last_kernel_ms: null argument");
-    hipError_t e = hipEventSynchronize(h->ev1);
-    float f = 0.0f;
-    if (e == hipSuccess) e = hipEventElapsedTime(&f, h->ev0, h->ev1);
-    *ms = f;
+    if (!h->stamped) return hip_fail(hipErrorInvalidHandle, "tfs_flow_last_kernel_ms: no evaluation yet");
+    unsigned long long t[2] = {0, 0};
+    hipError_t e = hipMemcpyAsync(t, h->stamps, sizeof(t), hipMemcpyDeviceToHost, h->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    *ms = t[1] > t[0] && h->clock_khz > 0 ? double(t[1] - t[0]) / h->clock_khz : 0.0;
     return check(e, "tfs_flow_last_kernel_ms");
 }
 

@@ -238,10 +238,42 @@ struct FlowArgs {
     int remove_net_force;
     int mode;          // 0 Stokeslet + rotlet (+ Blakelet without blobs), 1 RPY point tracer
     double a_seg, a_blob, mu;
+    int chunk;               // sources per workgroup (segments, then blobs)
+    double* part;            // several chunks: their partial sums, chunks x 3 x nt; else null
+    unsigned long long* stamps;  // start and finish of the evaluation (wall_clock64 ticks)
 };
+// Launch form of an evaluation: threads per workgroup, whether a workgroup's
+// waves share its targets, and the division of the sources.
+struct FlowPlan {
+    int block = 256;
+    bool shared = false;
+    int chunk = 1;
+    int chunks = 1;
+};
+FlowPlan flow_plan(int64_t nt, int64_t nsrc, int block, int num_cus, bool may_divide);
 // net[3*b..] = total force on body b (segments + blobs).
 hipError_t launch_flow_net(const FlowArgs& a, double* net, int nbod, hipStream_t stream);
-hipError_t launch_flow_eval(int precision, const FlowArgs& a, const double* net, int block, hipStream_t stream);
+hipError_t launch_flow_eval(int precision, const FlowArgs& a, const double* net, const FlowPlan& plan,
+                            hipStream_t stream);
+
+// Device-to-device copies of arrays of doubles in one launch (a small
+// hipMemcpyAsync occupies the stream for ~5 us each, the launch for ~5 in all).
+struct CopyList {
+    static constexpr int kMax = 8;
+    double* dst[kMax];
+    const double* src[kMax];
+    int64_t n[kMax];
+    int count = 0;
+    int64_t longest = 0;
+    void add(const double* from, double* to, int64_t len) {
+        if (from == to || len <= 0) return;
+        src[count] = from;
+        dst[count] = to;
+        n[count++] = len;
+        longest = longest > len ? longest : len;
+    }
+};
+hipError_t copy_list(const CopyList& list, hipStream_t stream);
 
 }  // namespace tfs
 

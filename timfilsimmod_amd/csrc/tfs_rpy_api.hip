@@ -35,6 +35,19 @@ int hip_fail(hipError_t e, const char* where) {
 
 int hip_fail_if(hipError_t e, const char* where) { return e == hipSuccess ? TFS_OK : hip_fail(e, where); }
 
+__global__ __launch_bounds__(256) static void copy_list_kernel(CopyList L) {
+    for (int k = 0; k < L.count; ++k)
+        for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < L.n[k]; i += (int64_t)gridDim.x * 256)
+            L.dst[k][i] = L.src[k][i];
+}
+
+hipError_t copy_list(const CopyList& list, hipStream_t stream) {
+    if (list.count == 0) return hipSuccess;
+    const int64_t g = (list.longest + 255) / 256;
+    hipLaunchKernelGGL(copy_list_kernel, dim3((unsigned)(g < 1024 ? g : 1024)), dim3(256), 0, stream, list);
+    return hipGetLastError();
+}
+
 // s.chunk for ~per_cu items per CU over a body of ns segments and nb blobs
 // (a multiple of the block).
 static void size_chunk(TileShape& s, int ns, int nb, int num_cus, long per_cu) {

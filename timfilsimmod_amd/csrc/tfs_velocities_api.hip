@@ -221,36 +221,6 @@ __global__ __launch_bounds__(256) void free_direct_forces_kernel(const double* _
     for (int c = 0; c < 3; ++c) out[3 * m + c] = R[3 * c] * b[0] + R[3 * c + 1] * b[1] + R[3 * c + 2] * b[2];
 }
 
-// Up to eight device-to-device copies of doubles in one launch.
-struct CopyList {
-    const double* src[8];
-    double* dst[8];
-    int64_t n[8];
-    int count = 0;
-    int64_t longest = 0;
-    void add(const double* s, double* d, int64_t len) {
-        if (s == d || len <= 0) return;
-        src[count] = s;
-        dst[count] = d;
-        n[count] = len;
-        ++count;
-        longest = len > longest ? len : longest;
-    }
-};
-
-__global__ __launch_bounds__(256) void copy_list_kernel(CopyList L) {
-    for (int k = 0; k < L.count; ++k)
-        for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < L.n[k]; i += (int64_t)gridDim.x * 256)
-            L.dst[k][i] = L.src[k][i];
-}
-
-hipError_t copy_list(const CopyList& L, hipStream_t st) {
-    if (L.count == 0) return hipSuccess;
-    const int64_t g = (L.longest + 255) / 256;
-    hipLaunchKernelGGL(copy_list_kernel, dim3((unsigned)(g < 1024 ? g : 1024)), dim3(256), 0, st, L);
-    return hipGetLastError();
-}
-
 // flag = 1 if a[i] != b[i] for some i (every writer stores the same value).
 __global__ __launch_bounds__(256) void differs_kernel(const double* __restrict__ a, const double* __restrict__ b,
                                                      int64_t n, int32_t* __restrict__ flag) {
