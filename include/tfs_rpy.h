@@ -185,17 +185,20 @@ int tfs_rpy_get_source_split(tfs_rpy *h, int32_t precision, int32_t *split);
  * ordered pair, cuda_functions.cu:362-757): the far-field tensor of a pair is
  * the same seen from either particle, so each unordered pair is evaluated once
  * and its term added to both particles' sums -- one 1/r, A and B for two
- * terms.  64-particle tiles in groups of four per workgroup of 256 threads;
+ * terms.  Tiles of 64 particles, four or eight to a workgroup of 256 threads;
  * results agree with the other shapes to FP32 rounding and are the same on
  * every run.  Independent bodies (tfs_rpy_set_bodies) pair within a body only,
  * and the items of bodies whose stop flag is set return at once.  Both
- * precisions; 3-DOF segments only (refused otherwise); evaluations whose
- * blocks lack SS, SB
- * or BS, and the half-space domain, take the default source-split shape
- * instead.  No persistent form.  The default shape (both precisions) of a
- * handle with 3-DOF segments whose (largest) body's groups of four tiles pair
- * into at least four items per CU (e.g. 12,800 segments + 9,000 blobs: 3,741
- * items); enable = 0 selects the source-split default instead. */
+ * precisions; set for 3-DOF segments only (refused otherwise); evaluations whose
+ * blocks lack SS, SB or BS, and the half-space domain, take the default
+ * source-split shape instead.  No persistent form.  The default shape (both
+ * precisions) of a handle with 3-DOF segments whose (largest) body's groups of
+ * four tiles pair into at least four items per CU (e.g. 12,800 segments + 9,000
+ * blobs: 3,741 items); enable = 0 selects the source-split default instead.
+ * Handles that no shape was set for also evaluate this way, with either kind of
+ * segments, wherever their size favours it (from about 4,100 particles on);
+ * the shape that the functions here report is then the one such a handle falls
+ * back to, and setting any shape ends it. */
 int tfs_rpy_set_symmetric(tfs_rpy *h, int32_t precision, int32_t enable);
 /* 1 if the precision's current shape is the symmetric form. */
 int tfs_rpy_get_symmetric(tfs_rpy *h, int32_t precision, int32_t *enabled);

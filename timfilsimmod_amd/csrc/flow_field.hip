@@ -71,14 +71,6 @@ __device__ __forceinline__ void blakelet(double* acc, double zi, double zj, doub
     acc[2] += g * (Dzx * fx + Dzy * fy + Dzz * fz);
 }
 
-// 2/sqrt(x) from the v_rsq_f64 seed z by one Newton-Raphson step without its
-// factor 1/2, w = z (3 - x z^2): three operations instead of four; callers fold
-// the powers of two into their flush.  The same error as rsqrt_refined.
-__device__ __forceinline__ double rsqrt_twice(double x) {
-    const double z = __builtin_amdgcn_rsq(x);
-    return z * __builtin_fma(-x * z, z, 3.0);
-}
-
 // The sources [s_lo, s_hi) of one class added into acc.  SHARED: wave w takes
 // the w-th part of every batch.
 template <typename T, int MODE, bool BLAKE, int FS, int BLOCK, int R, bool SHARED>

@@ -322,187 +322,424 @@ __global__ __launch_bounds__(BLOCK) void rpy_pairs_kernel(const MatvecItem* __re
     }
 }
 
-// ---- symmetric form (3-DOF particles) -----------------------------------------
+// ---- symmetric form ------------------------------------------------------------
 //
-// The far-field tensor of a pair is the same seen from either particle: the
-// separation enters twice (its sign cancels) and the radii symmetrically, so
-// M_ji = M_ij and one evaluation of 1/r, A and B serves both.  Tiles of 64
-// particles are grouped kSymTiles to a workgroup; item (ga, gb), ga <= gb,
-// evaluates the tile pairs of groups ga and gb, wave w owning tile w of group
-// ga.  In stage t the wave takes source tile (w + t) mod kSymTiles of group gb
-// from LDS, lane l pairing its particle with source (l + kSymRot k) mod 64 at
-// step k: the lane's own sum gets the source's term and the source's sum gets
-// the lane's term.  The source sums live in one register per component that
-// moves one lane per step (a DPP wave rotation ahead of the accumulates), so
-// after 64 steps lane l holds the sum of source (l + 63 kSymRot) mod 64.  Each stage
-// adds those sums into the source tile's FP64 LDS sums; the stages are fenced
-// by barriers and the writer of a tile's sums in stage t is wave
-// (tile - t) mod kSymTiles, a fixed order.  A pair of distinct groups is
-// evaluated once for both tiles; in a diagonal item (ga == gb) the pairs with
-// tile a < tile b are evaluated once, a == b one-sided (the self pair and the
-// overlapping pairs take the clamped far field, which the reduce kernel swaps
-// for the exact value), and a > b not at all.
+// The mobility of a pair is symmetric (M_ji = M_ij^T): the translational and
+// rotational tensors are the same seen from either particle, the couplings
+// change sign with the separation.  One evaluation of 1/r and its powers so
+// serves both particles.  Tiles hold 64 particles of one class of one body; a
+// panel is kSymWaves x R tiles.  An item pairs a panel with a run of tiles from
+// the panel's first on: wave w owns the panel's tiles w, w + kSymWaves, ... (R
+// particles per lane) and meets each tile of the run from LDS, lane l pairing
+// its particles with source (l + k) mod 64 at step k: the lane's own sums get
+// the source's term and the source's sums get the lane's terms.  The source
+// sums live in one register per component that moves one lane per step (a DPP
+// wave rotation ahead of the accumulates; the R particles of a lane share it),
+// so after step k lane l holds the sum of source (l + k) mod 64.  The waves'
+// sums of a source tile meet in LDS and are added in wave order.  Tile pairs
+// a < b are evaluated once, a == b one-sided (the self pair and the overlapping
+// pairs take the clamped far field, which the reduce kernel swaps for the exact
+// value), and a > b not at all.  Within a body the segment tiles come first, so
+// a blob target never meets a segment source.
 //
-// Partial slots: tile t of group g has one slot per group q its body overlaps
-// (groups run body after body; tile pairs of different bodies are skipped),
-// holding the sums it received from group q (its own sums when q > g, the
-// source sums when q < g, both added for q == g), each written once per
-// launch, so the reduce kernel sums them in slot order.
-constexpr int kSymTiles = kSymGroupTiles;
-constexpr int kSymRot = 1;  // DPP wave_rol:1 -- lane l reads lane l + 1 (mod 64)
+// Partial slots: tile t of panel P has one slot per panel A < P its body
+// overlaps (its sums as a source of panel A), then one per run of P from the
+// one that holds t up to its body's last (its own sums; in its own run the sums
+// it received as a source from its panel added), each written once per launch,
+// so the reduce kernel sums them in slot order.
+//
+// Bound by VALU issue.  Cycles per wave instruction measured on MI355X (nominal
+// 2.4 GHz): FP32 add, subtract, multiply 2.3-2.5, multiply-accumulate 2.7-3.1;
+// maximum, int-to-float, DPP move, three-operand fma 4.3; rsq 8.2; FP64 4.4-5.6,
+// its rsq 16.2 (FP32 and FP64 MFMA occupy the same pipes: their time adds to the
+// VALU's, so moving sums there gains nothing).  Per launch at 12,800 segments +
+// 9,000 blobs: 3 components FP32 195 us, FP64 320 (one particle per lane, items
+// of 4 x 4 tiles: 212 and 354); 6 components FP32 325, FP64 540 (every ordered
+// pair with the source split: 384 and 690).  Two particles per lane halve the
+// rotations and the LDS reads; the three-operation Newton step saves one FP64
+// operation; runs that shorten towards the end keep the CUs evenly loaded
+// (FP32, 6 components: 355 us with two tiles per item throughout).
+constexpr int kSymRot = 0x134;  // DPP wave_rol:1 -- lane l reads lane l + 1 (mod 64)
 __device__ __forceinline__ float rotate_lanes(float x) {
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), kSymRot > 0 ? 0x134 : 0x13C, 0xF, 0xF, false));
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), kSymRot, 0xF, 0xF, false));
 }
 __device__ __forceinline__ double rotate_lanes(double x) {
-    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), kSymRot > 0 ? 0x134 : 0x13C, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), kSymRot > 0 ? 0x134 : 0x13C, 0xF, 0xF, false);
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), kSymRot, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), kSymRot, 0xF, 0xF, false);
     return __hiloint2double(hi, lo);
 }
 
-// LDS records of one source tile, twice over (index j and j + 64 hold
-// particle j, so that lane l reads record l + kSymRot k + (kSymRot < 0 ? 64 :
-// 0) without a wrap), split into arrays of 16 or 8 bytes per record so that
-// consecutive lanes, reading consecutive records, share no banks within a
-// read phase.  FP32: X Y Z (fixed-point integers as their bits) and the first
-// strength, then the other two strengths.  FP64: x y, z and the first
-// strength, the other two.
-template <typename T>
+// LDS records of one source tile, split into arrays of 16 (or 8) bytes per
+// record so that consecutive lanes, reading consecutive records, share no banks
+// within a read phase.  FP32 positions are fixed-point integers as their bits.
+// 3 components: held twice over (index j and j + 64 hold particle j), so that
+// lane l reads record l + k without a wrap (the two index instructions per
+// step cost more than the LDS).  6 components: held once, the index masked (of
+// ~100 instructions per step two more matter less than a workgroup per CU),
+// every array 16 bytes wide so that one address serves all.
+template <typename T, int DOF>
 struct SymTileLds;
 template <>
-struct SymTileLds<float> {
+struct SymTileLds<float, 3> {
+    static constexpr bool kTwice = true;
     float4 xf[128];
     float2 yz[128];
+    __device__ __forceinline__ void get(int j, float (&X)[3], float (&f)[3]) const {
+        const float4 a = xf[j];
+        const float2 b = yz[j];
+        X[0] = a.x, X[1] = a.y, X[2] = a.z;
+        f[0] = a.w, f[1] = b.x, f[2] = b.y;
+    }
+    __device__ __forceinline__ void put(int j, const int32_t (&X)[3], const float (&f)[3]) {
+        xf[j] = make_float4(__int_as_float(X[0]), __int_as_float(X[1]), __int_as_float(X[2]), f[0]);
+        yz[j] = make_float2(f[1], f[2]);
+    }
 };
 template <>
-struct SymTileLds<double> {
+struct SymTileLds<double, 3> {
+    static constexpr bool kTwice = true;
     double2 xy[128];
     double2 zf[128];
     double2 gh[128];
+    __device__ __forceinline__ void get(int j, double (&X)[3], double (&f)[3]) const {
+        const double2 a = xy[j], b = zf[j], c = gh[j];
+        X[0] = a.x, X[1] = a.y, X[2] = b.x;
+        f[0] = b.y, f[1] = c.x, f[2] = c.y;
+    }
+    __device__ __forceinline__ void put(int j, const double (&X)[3], const double (&f)[3]) {
+        xy[j] = make_double2(X[0], X[1]);
+        zf[j] = make_double2(X[2], f[0]);
+        gh[j] = make_double2(f[1], f[2]);
+    }
+};
+template <>
+struct SymTileLds<float, 6> {
+    static constexpr bool kTwice = false;
+    float4 a[64], b[64], c[64];
+    template <int N>
+    __device__ __forceinline__ void get(int j, float (&X)[3], float (&f)[N]) const {
+        const float4 p = a[j], q = b[j];
+        X[0] = p.x, X[1] = p.y, X[2] = p.z;
+        f[0] = p.w, f[1] = q.x, f[2] = q.y;
+        if constexpr (N == 6) f[3] = q.z, f[4] = q.w, f[5] = c[j].x;
+    }
+    __device__ __forceinline__ void put(int j, const int32_t (&X)[3], const float (&f)[6]) {
+        a[j] = make_float4(__int_as_float(X[0]), __int_as_float(X[1]), __int_as_float(X[2]), f[0]);
+        b[j] = make_float4(f[1], f[2], f[3], f[4]);
+        c[j].x = f[5];
+    }
+};
+template <>
+struct SymTileLds<double, 6> {
+    static constexpr bool kTwice = false;
+    double2 a[64], b[64], c[64], d[64], e[64];
+    template <int N>
+    __device__ __forceinline__ void get(int j, double (&X)[3], double (&f)[N]) const {
+        const double2 p = a[j], q = b[j], r = c[j];
+        X[0] = p.x, X[1] = p.y, X[2] = q.x;
+        f[0] = q.y, f[1] = r.x, f[2] = r.y;
+        if constexpr (N == 6) {
+            const double2 s = d[j];
+            f[3] = s.x, f[4] = s.y, f[5] = e[j].x;
+        }
+    }
+    __device__ __forceinline__ void put(int j, const double (&X)[3], const double (&f)[6]) {
+        a[j] = make_double2(X[0], X[1]);
+        b[j] = make_double2(X[2], f[0]);
+        c[j] = make_double2(f[1], f[2]);
+        d[j] = make_double2(f[3], f[4]);
+        e[j].x = f[5];
+    }
 };
 
-__device__ __forceinline__ void sym_record(const SymTileLds<float>& L, int j, float (&rec)[3], float (&f)[3]) {
-    const float4 q = L.xf[j];
-    const float2 g = L.yz[j];
-    rec[0] = q.x;
-    rec[1] = q.y;
-    rec[2] = q.z;
-    f[0] = q.w;
-    f[1] = g.x;
-    f[2] = g.y;
-}
-__device__ __forceinline__ void sym_record(const SymTileLds<double>& L, int j, double (&rec)[3], double (&f)[3]) {
-    const double2 a = L.xy[j], b = L.zf[j], c = L.gh[j];
-    rec[0] = a.x;
-    rec[1] = a.y;
-    rec[2] = b.x;
-    f[0] = b.y;
-    f[1] = c.x;
-    f[2] = c.y;
-}
-__device__ __forceinline__ void sym_put(SymTileLds<float>& L, int j, const int32_t (&X)[3], const float (&f)[3]) {
-    L.xf[j] = make_float4(__int_as_float(X[0]), __int_as_float(X[1]), __int_as_float(X[2]), f[0]);
-    L.yz[j] = make_float2(f[1], f[2]);
-}
-__device__ __forceinline__ void sym_put(SymTileLds<double>& L, int j, const double (&X)[3], const double (&f)[3]) {
-    L.xy[j] = make_double2(X[0], X[1]);
-    L.zf[j] = make_double2(X[2], f[0]);
-    L.gh[j] = make_double2(f[1], f[2]);
+// Pair constants of one class pair.  FP32 tiles work in the fixed-point frame
+// (separation from integer coordinates, s3 and (ai+aj)^2 scaled by lambda^2)
+// with 1/r from the rsq instruction; FP64 with w = 2/r (one Newton-Raphson
+// step without its factor 1/2, three operations), the powers of two folded
+// into these constants and the staged strengths (sym_scale).
+template <typename T>
+struct SymConsts {
+    T sum_a2;  // (ai + aj)^2
+    T s3;      // s3, or s3/4
+    T m3s3;    // -3 s3, or -3 s3/16
+};
+template <typename T>
+__device__ __forceinline__ SymConsts<T> sym_consts(double ai, double aj, double lam) {
+    const double s3 = lam * lam * ((ai * ai + aj * aj) / 3.0);
+    SymConsts<T> c;
+    c.sum_a2 = T(lam * lam * ((ai + aj) * (ai + aj)));
+    c.s3 = sizeof(T) == 4 ? T(s3) : T(0.25 * s3);
+    c.m3s3 = sizeof(T) == 4 ? T(-3) * T(s3) : T(-3.0 / 16.0 * s3);
+    return c;
 }
 
-// The 64 steps of one stage.  BOTH: add the lane's terms into the rotating
-// source sums pj as well (an off-diagonal tile pair); otherwise only the
-// lane's own sum pi (the tile against itself).  FP32 tiles work in the
-// fixed-point frame (separation from integer coordinates, s3 and (ai+aj)^2
-// scaled by lambda^2).
-template <bool BOTH, typename T>
-__device__ __forceinline__ void sym_stage(const SymTileLds<T>& recs, int lane, const TargetT<T> (&Xi)[3],
-                                          const T (&fi)[3], T sum_a2, T s3, T m3s3, T (&pi)[3], T (&pj)[3]) {
-    const int j0 = lane + (kSymRot > 0 ? 0 : 64);
-    // Not unrolled: FP32 48 VGPRs, eight waves per SIMD to hide the LDS and
-    // dependency latency (measured on MI355X, production body: 0.212 ms per
-    // launch, against 0.219 unrolled twice (59 VGPRs) and 0.239 eight times
-    // (119 VGPRs, four waves per SIMD)).
-#pragma unroll 1
-    for (int k = 0; k < 64; ++k) {
-        T rec[3], fj[3];
-        sym_record(recs, j0 + kSymRot * k, rec, fj);
-        T dx, dy, dz;
-        const T r2 = separation(Xi, rec, dx, dy, dz);
-        const T rm1 = rsqrt_refined(fmax_t(r2, sum_a2));
-        const T rm2 = rm1 * rm1;
-        const T rm3 = rm1 * rm2;
-        const T A = fma_t(s3, rm3, rm1);
-        const T u = m3s3 * rm2;
-        const T B = fma_t(u, rm3, rm3);
+// Factors of the staged forces and torques, and of the rotational sums as they
+// are stored.  FP32: forces lambda c8, torques lambda^2 c8 (c8 = 1/(8 pi mu)):
+// rotational sums come out divided by lambda.  FP64: forces c8/2, torques
+// c8/8: rotational sums come out times 4.
+template <typename T>
+__device__ __forceinline__ void sym_scale(const MatvecArgs& a, double& force, double& torque, double& rot) {
+    const double c8 = 1.0 / (8.0 * 3.14159265358979323846 * a.mu);
+    if constexpr (sizeof(T) == 4) {
+        force = a.lam * c8;
+        torque = a.lam * a.lam * c8;
+        rot = a.lam;
+    } else {
+        force = 0.5 * c8;
+        torque = 0.125 * c8;
+        rot = 0.25;
+    }
+}
+
+// The pair term at separation d: pi += (i's velocity from fj), and with BOTH
+// pj += (j's velocity from fi).  IT, JT: components of the target and source
+// (6: force and torque in, velocity and angular velocity out).  `neg` is -1,
+// opaque to the compiler in FP32 so that negated products stay two-operand
+// accumulates (half the issue time of the three-operand form).
+template <bool BOTH, typename T, int IT, int JT>
+__device__ __forceinline__ void sym_pair(T dx, T dy, T dz, T r2, const SymConsts<T>& c, T neg, const T (&fi)[IT],
+                                         const T (&fj)[JT], T (&pi)[IT], T (&pj)[JT]) {
+    constexpr bool F32 = sizeof(T) == 4;
+    r2 = fmax_t(r2, c.sum_a2);
+    T w;
+    if constexpr (F32) {
+        w = rsqrt_refined(r2);
+    } else {
+        w = rsqrt_twice(r2);
+    }
+    const T w2 = w * w;
+    const T w3 = w * w2;
+    const T A = fma_t(c.s3, w3, w);
+    // (1 - 3 s3 / r^2) as a factor: FP32 1 + u, FP64 u = a quarter of it
+    const T u = F32 ? c.m3s3 * w2 : fma_t(c.m3s3, w2, T(0.25));
+    if constexpr (IT == 3 && JT == 3) {
+        const T B = F32 ? fma_t(u, w3, w3) : u * w3;
         const T Bd = B * fma_t(dz, fj[2], fma_t(dy, fj[1], dx * fj[0]));
         pi[0] = fma_t(Bd, dx, fma_t(A, fj[0], pi[0]));
         pi[1] = fma_t(Bd, dy, fma_t(A, fj[1], pi[1]));
         pi[2] = fma_t(Bd, dz, fma_t(A, fj[2], pi[2]));
         if constexpr (BOTH) {
-            // the source's term: the same A, B and separation (d_ji = -d
-            // enters twice), the lane's strengths
             const T Be = B * fma_t(dz, fi[2], fma_t(dy, fi[1], dx * fi[0]));
-            pj[0] = fma_t(Be, dx, fma_t(A, fi[0], rotate_lanes(pj[0])));
-            pj[1] = fma_t(Be, dy, fma_t(A, fi[1], rotate_lanes(pj[1])));
-            pj[2] = fma_t(Be, dz, fma_t(A, fi[2], rotate_lanes(pj[2])));
+            pj[0] = fma_t(Be, dx, fma_t(A, fi[0], pj[0]));
+            pj[1] = fma_t(Be, dy, fma_t(A, fi[1], pj[1]));
+            pj[2] = fma_t(Be, dz, fma_t(A, fi[2], pj[2]));
+        }
+    } else {
+        const T ex = w3 * dx, ey = w3 * dy, ez = w3 * dz;
+        const T nw3 = neg * w3;
+        const T nx = nw3 * dx, ny = nw3 * dy, nz = nw3 * dz;
+        T s = fma_t(ez, fj[2], fma_t(ey, fj[1], ex * fj[0]));
+        s = F32 ? fma_t(u, s, s) : u * s;
+        pi[0] = fma_t(s, dx, fma_t(A, fj[0], pi[0]));
+        pi[1] = fma_t(s, dy, fma_t(A, fj[1], pi[1]));
+        pi[2] = fma_t(s, dz, fma_t(A, fj[2], pi[2]));
+        if constexpr (BOTH) {
+            T t = fma_t(ez, fi[2], fma_t(ey, fi[1], ex * fi[0]));
+            t = F32 ? fma_t(u, t, t) : u * t;
+            pj[0] = fma_t(t, dx, fma_t(A, fi[0], pj[0]));
+            pj[1] = fma_t(t, dy, fma_t(A, fi[1], pj[1]));
+            pj[2] = fma_t(t, dz, fma_t(A, fi[2], pj[2]));
+        }
+        if constexpr (JT == 6) {
+            // v_i += tau_j x d / r^3
+            pi[0] = fma_t(fj[5], ny, fma_t(fj[4], ez, pi[0]));
+            pi[1] = fma_t(fj[3], nz, fma_t(fj[5], ex, pi[1]));
+            pi[2] = fma_t(fj[4], nx, fma_t(fj[3], ey, pi[2]));
+            if constexpr (BOTH) {
+                // omega_j -= F_i x d / r^3
+                pj[3] = fma_t(fi[2], ey, fma_t(fi[1], nz, pj[3]));
+                pj[4] = fma_t(fi[0], ez, fma_t(fi[2], nx, pj[4]));
+                pj[5] = fma_t(fi[1], ex, fma_t(fi[0], ny, pj[5]));
+            }
+        }
+        if constexpr (IT == 6) {
+            // omega_i += F_j x d / r^3
+            pi[3] = fma_t(fj[2], ny, fma_t(fj[1], ez, pi[3]));
+            pi[4] = fma_t(fj[0], nz, fma_t(fj[2], ex, pi[4]));
+            pi[5] = fma_t(fj[1], nx, fma_t(fj[0], ey, pi[5]));
+            if constexpr (BOTH) {
+                // v_j -= tau_i x d / r^3
+                pj[0] = fma_t(fi[5], ey, fma_t(fi[4], nz, pj[0]));
+                pj[1] = fma_t(fi[3], ez, fma_t(fi[5], nx, pj[1]));
+                pj[2] = fma_t(fi[4], ex, fma_t(fi[3], ny, pj[2]));
+            }
+        }
+        if constexpr (IT == 6 && JT == 6) {
+            // omega_i += -tau_j / (2 r^3) + 3 (tau_j . d) d / (2 r^5), and with i and j swapped
+            const T Ar = (F32 ? T(-0.5) : T(-2)) * w3;
+            const T h = T(1.5) * w2;
+            const T q = h * fma_t(ez, fj[5], fma_t(ey, fj[4], ex * fj[3]));
+            pi[3] = fma_t(q, dx, fma_t(Ar, fj[3], pi[3]));
+            pi[4] = fma_t(q, dy, fma_t(Ar, fj[4], pi[4]));
+            pi[5] = fma_t(q, dz, fma_t(Ar, fj[5], pi[5]));
+            if constexpr (BOTH) {
+                const T p = h * fma_t(ez, fi[5], fma_t(ey, fi[4], ex * fi[3]));
+                pj[3] = fma_t(p, dx, fma_t(Ar, fi[3], pj[3]));
+                pj[4] = fma_t(p, dy, fma_t(Ar, fi[4], pj[4]));
+                pj[5] = fma_t(p, dz, fma_t(Ar, fi[5], pj[5]));
+            }
         }
     }
 }
 
-// One particle of a tile for the symmetric form: its position (FP32 tiles:
-// fixed-point) and strengths scaled by fsc (zero, with the tile's first
-// position, for lanes past the tile's end).
-__device__ __forceinline__ void sym_particle(const MatvecTile& tl, const MatvecArgs& a, int lane, double fsc,
-                                             int32_t (&X)[3], float (&f)[3]) {
-    const int s = tl.t_begin + lane;
-    const bool ok = s < tl.t_end;
-    const int sc = ok ? s : tl.t_begin;
-    const int4 q = a.xfx[(tl.cls == 0 ? 0 : a.ns) + sc];
-    X[0] = q.x;
-    X[1] = q.y;
-    X[2] = q.z;
-    const CView fv = tl.cls == 0 ? a.fs : a.fb;
+// Steps [k0, k1) of one stage: R target particles of the lane (IT of their DOF
+// components) against the tile's sources (JT components).  BOTH: the sources'
+// sums pj rotate and gather the lanes' terms (an off-diagonal tile pair);
+// otherwise only the lane's own sums (the tile against itself).
+template <bool BOTH, int IT, int JT, int R, typename T, int DOF>
+__device__ __forceinline__ void sym_stage(const SymTileLds<T, DOF>& recs, int lane, int k0, int k1,
+                                          const TargetT<T> (&Xi)[R][3], const T (&fi)[R][IT], const SymConsts<T>& c,
+                                          T neg, T (&pi)[R][IT], T (&pj)[JT]) {
+    // Not unrolled: more waves hide the LDS and dependency latency better than
+    // a longer body (3 components, R = 1, FP32: 0.212 ms per launch of the
+    // production body, 0.219 unrolled twice, 0.239 eight times).
+#pragma unroll 1
+    for (int k = k0; k < k1; ++k) {
+        T X[3], fj[JT];
+        recs.get(SymTileLds<T, DOF>::kTwice ? lane + k : (lane + k) & 63, X, fj);
+        if constexpr (BOTH) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) f[k] = ok ? float(fsc * fv.p[(int64_t)sc * fv.ld_p + k * fv.ld_c]) : 0.0f;
-}
-__device__ __forceinline__ void sym_particle(const MatvecTile& tl, const MatvecArgs& a, int lane, double fsc,
-                                             double (&X)[3], double (&f)[3]) {
-    const int s = tl.t_begin + lane;
-    const bool ok = s < tl.t_end;
-    const int sc = ok ? s : tl.t_begin;
-    const CView xv = tl.cls == 0 ? a.xs : a.xb;
-    const CView fv = tl.cls == 0 ? a.fs : a.fb;
+            for (int q = 0; q < JT; ++q) pj[q] = rotate_lanes(pj[q]);
+        }
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        X[k] = xv.p[(int64_t)sc * xv.ld_p + k * xv.ld_c];
-        f[k] = ok ? fsc * fv.p[(int64_t)sc * fv.ld_p + k * fv.ld_c] : 0.0;
+        for (int r = 0; r < R; ++r) {
+            T dx, dy, dz;
+            const T r2 = separation(Xi[r], X, dx, dy, dz);
+            sym_pair<BOTH, T, IT, JT>(dx, dy, dz, r2, c, neg, fi[r], fj, pi[r], pj);
+        }
     }
 }
 
-// One workgroup of kSymTiles waves per item (tile = ga, src_cls = gb).
+// One particle of a tile: its position (FP32 tiles: fixed-point) and strengths
+// scaled by fsc and tsc (zero, with the tile's first position, for lanes past
+// the tile's end; no torque for blobs).
+template <typename T, int DOF>
+__device__ __forceinline__ void sym_particle(const MatvecTile& tl, const MatvecArgs& a, int lane, double fsc,
+                                             double tsc, TargetT<T> (&X)[3], T (&f)[DOF]) {
+    const int s = tl.t_begin + lane;
+    const bool ok = s < tl.t_end;
+    const int sc = ok ? s : tl.t_begin;
+    load_target(a, tl.cls, sc, X);
+    const CView fv = tl.cls == 0 ? a.fs : a.fb;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) f[k] = ok ? T(fsc * fv.p[(int64_t)sc * fv.ld_p + k * fv.ld_c]) : T(0);
+    if constexpr (DOF == 6) {
+        const bool tq = ok && tl.cls == 0;
+#pragma unroll
+        for (int k = 3; k < 6; ++k) f[k] = tq ? T(tsc * fv.p[(int64_t)sc * fv.ld_p + k * fv.ld_c]) : T(0);
+    }
+}
+
+// Parts of a stage after each of which the sums are put down into FP64: an FP32
+// sum of the sources takes at most 64 particles' terms, and a lane's own at
+// most 64 (32 with rotations, whose terms add four times to a component and
+// not twice).  The length of these chains sets the FP32 error: 12,800 segments
+// + 9,000 blobs with rotations, 2.1e-7 with one part, 1.2e-7 with four (5%
+// slower).
+template <typename T, int DOF, int R>
+constexpr int sym_parts() {
+    return sizeof(T) == 4 ? (DOF == 6 ? 2 : R) : 1;
+}
+
+// R tiles of the lane against one source tile: own sums into acc, the sources'
+// sums (BOTH) of every part to the wave's LDS sets js[part] (added to what they
+// hold with `add`).
+template <bool BOTH, int IT, int JT, int R, int PARTS, typename T, int DOF>
+__device__ __forceinline__ void sym_tiles(const SymTileLds<T, DOF>& recs, int lane, const TargetT<T> (&Xi)[R][3],
+                                          const T (&fi)[R][DOF], const SymConsts<T>& c, T neg, double (&acc)[R][DOF],
+                                          T (*js)[DOF][64], bool add) {
+    constexpr bool F32 = sizeof(T) == 4;
+    T fv[R][IT];
+    double sum[R][IT];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int k = 0; k < IT; ++k) {
+            fv[r][k] = fi[r][k];
+            sum[r][k] = acc[r][k];
+        }
+#pragma unroll 1
+    for (int p = 0; p < PARTS; ++p) {
+        T pi[R][IT], pj[JT];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int k = 0; k < IT; ++k) {
+                if constexpr (F32) pi[r][k] = T(0);
+                else pi[r][k] = sum[r][k];
+            }
+#pragma unroll
+        for (int k = 0; k < JT; ++k) pj[k] = T(0);
+        const int k0 = p * (64 / PARTS), k1 = k0 + 64 / PARTS;
+        sym_stage<BOTH, IT, JT, R, T, DOF>(recs, lane, k0, k1, Xi, fv, c, neg, pi, pj);
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int k = 0; k < IT; ++k) {
+                if constexpr (F32) sum[r][k] += double(pi[r][k]);
+                else sum[r][k] = pi[r][k];
+            }
+        if constexpr (BOTH) {
+            const int j = (lane + k1 - 1) & 63;  // the source whose sums the lane holds now
+#pragma unroll
+            for (int k = 0; k < JT; ++k) js[p][k][j] = add ? js[p][k][j] + pj[k] : pj[k];
+        }
+    }
+    // every component is written, also the ones that this class pair leaves as
+    // they are: the instances then end in the same stores and the array stays
+    // in registers
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int k = 0; k < DOF; ++k) acc[r][k] = k < IT ? sum[r][k < IT ? k : 0] : acc[r][k] + 0.0;
+}
+
+// The class pair's instance of sym_tiles.
+template <bool BOTH, int R, int PARTS, typename T, int DOF>
+__device__ __forceinline__ void sym_classes(int cls_a, int cls_b, const SymTileLds<T, DOF>& recs, int lane,
+                                            const TargetT<T> (&Xi)[R][3], const T (&fi)[R][DOF],
+                                            const SymConsts<T>& c, T neg, double (&acc)[R][DOF], T (*js)[DOF][64],
+                                            bool add) {
+    if constexpr (DOF == 3) {
+        sym_tiles<BOTH, 3, 3, R, PARTS, T, DOF>(recs, lane, Xi, fi, c, neg, acc, js, add);
+    } else if (cls_a == 1) {
+        sym_tiles<BOTH, 3, 3, R, PARTS, T, DOF>(recs, lane, Xi, fi, c, neg, acc, js, add);
+    } else if (cls_b == 0) {
+        sym_tiles<BOTH, 6, 6, R, PARTS, T, DOF>(recs, lane, Xi, fi, c, neg, acc, js, add);
+    } else {
+        // a segment tile against a blob tile: never the tile itself
+        if constexpr (BOTH) sym_tiles<true, 6, 3, R, PARTS, T, DOF>(recs, lane, Xi, fi, c, neg, acc, js, add);
+    }
+}
+
+template <typename T, int DOF, int R>
+constexpr int sym_min_waves() {
+    if (R == 1) return DOF == 3 ? (sizeof(T) == 4 ? 8 : 6) : (sizeof(T) == 4 ? 6 : 4);
+    return DOF == 3 ? (sizeof(T) == 4 ? 6 : 4) : (sizeof(T) == 4 ? 4 : 3);
+}
+
+// One workgroup of kSymWaves waves per item (tile = panel, source tiles
+// [src_cls, s_begin), s_end = the run's number within the panel).
 // `bb`: blob-blob pairs are evaluated (off when an overwriting BS block
 // replaces BB).  Tile pairs of different bodies are skipped, and so is an item
 // whose bodies all have their stop flag set; with `stamps`, thread 0 stores
 // the item's start and finish (wall_clock64 ticks).
-template <typename T>
-__global__ __launch_bounds__(64 * kSymTiles) void rpy_pairs_sym_kernel(const MatvecItem* __restrict__ items,
-                                                                        const MatvecTile* __restrict__ tiles,
-                                                                        int n_tiles, int bb, MatvecArgs a,
-                                                                        T* __restrict__ partial,
-                                                                        int64_t* __restrict__ stamps) {
+template <typename T, int DOF, int R>
+__global__ __launch_bounds__(64 * kSymWaves, (sym_min_waves<T, DOF, R>())) void rpy_pairs_sym_kernel(
+    const MatvecItem* __restrict__ items, const MatvecTile* __restrict__ tiles, int n_tiles, int bb, MatvecArgs a,
+    T* __restrict__ partial, int64_t* __restrict__ stamps) {
     constexpr bool F32 = sizeof(T) == 4;
-    __shared__ SymTileLds<T> recs[kSymTiles];
-    __shared__ double jsum[kSymTiles][3][64];
+    constexpr int NW = kSymWaves, PANEL = NW * R, PARTS = sym_parts<T, DOF, R>();
+    __shared__ SymTileLds<T, DOF> recs;
+    __shared__ T jsum[NW * PARTS][DOF][64];
     if (a.skip && *a.skip) return;
     const int64_t t_start = stamps ? (int64_t)wall_clock64() : 0;
     const int w = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
     const MatvecItem it = items[blockIdx.x];
-    const int ga = it.tile, gb = it.src_cls;
+    const int pa = it.tile, q0 = it.src_cls, q1 = it.s_begin;
     if (a.body_skip) {
         // the bodies of the item's tiles are a contiguous range
-        const int b0 = tiles[kSymTiles * ga].body;
-        const int tl_last = kSymTiles * gb + kSymTiles < n_tiles ? kSymTiles * gb + kSymTiles : n_tiles;
-        const int b1 = tiles[tl_last - 1].body;
+        const int b0 = tiles[PANEL * pa].body, b1 = tiles[q1 - 1].body;
         bool any = false;
         for (int b = b0; b <= b1 && !any; ++b) any = a.body_skip[b] == 0;
         if (!any) {
@@ -513,90 +750,121 @@ __global__ __launch_bounds__(64 * kSymTiles) void rpy_pairs_sym_kernel(const Mat
             return;
         }
     }
-    const double PI = 3.14159265358979323846;
     const double lam = F32 ? a.lam : 1.0;
-    const double fsc = lam / (8.0 * PI * a.mu);
-    // wave w stages source tile w of group gb (twice: records lane and lane + 64)
-    {
-        const int tb = kSymTiles * gb + w;
-        if (tb < n_tiles) {
+    double fsc, tsc, rot;
+    sym_scale<T>(a, fsc, tsc, rot);
+    T neg = T(-1);
+    if constexpr (F32 && DOF == 6) asm volatile("" : "+v"(neg));
+    TargetT<T> Xi[R][3];
+    T fi[R][DOF];
+    double acc[R][DOF];
+    int cls[R], body[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int ta = PANEL * pa + NW * r + w;
+        cls[r] = 0;
+        body[r] = -1;  // nothing to evaluate
+#pragma unroll
+        for (int k = 0; k < 3; ++k) Xi[r][k] = 0;
+#pragma unroll
+        for (int k = 0; k < DOF; ++k) {
+            fi[r][k] = T(0);
+            acc[r][k] = 0.0;
+        }
+        if (ta < n_tiles) {
+            const MatvecTile tl = tiles[ta];
+            cls[r] = tl.cls;
+            if (!(a.body_skip && a.body_skip[tl.body])) body[r] = tl.body;
+            sym_particle<T, DOF>(tl, a, lane, fsc, tsc, Xi[r], fi[r]);
+        }
+    }
+    for (int tb = q0; tb < q1; ++tb) {
+        const MatvecTile tlb = tiles[tb];
+        if (w == (tb & (NW - 1))) {
             TargetT<T> X[3];
-            T f[3];
-            sym_particle(tiles[tb], a, lane, fsc, X, f);
-            sym_put(recs[w], lane, X, f);
-            sym_put(recs[w], lane + 64, X, f);
+            T f[DOF];
+            sym_particle<T, DOF>(tlb, a, lane, fsc, tsc, X, f);
+            recs.put(lane, X, f);
+            if constexpr (SymTileLds<T, DOF>::kTwice) recs.put(lane + 64, X, f);
         }
+        __syncthreads();  // the records are in, the sums of the tile before are taken
+        int mode[R];      // 0 nothing, 1 one-sided, 2 both particles
+        bool all2 = true;
 #pragma unroll
-        for (int k = 0; k < 3; ++k) jsum[w][k][lane] = 0.0;
-    }
-    const int ta = kSymTiles * ga + w;
-    const bool has_a = ta < n_tiles;
-    TargetT<T> Xi[3] = {0, 0, 0};
-    T fi[3] = {T(0), T(0), T(0)};
-    MatvecTile tla{};
-    bool run_a = false;
-    if (has_a) {
-        tla = tiles[ta];
-        run_a = !(a.body_skip && a.body_skip[tla.body]);
-        sym_particle(tla, a, lane, fsc, Xi, fi);
-    }
-    __syncthreads();
-    double acc[3] = {0.0, 0.0, 0.0};
-    for (int t = 0; t < kSymTiles; ++t) {
-        const int bq = (w + t) & (kSymTiles - 1);
-        const int tb = kSymTiles * gb + bq;
-        int mode = 0;  // 0 nothing, 1 one-sided, 2 both particles
-        int cls_b = 0;
-        if (run_a && tb < n_tiles) {
-            const MatvecTile tlb = tiles[tb];
-            cls_b = tlb.cls;
-            mode = (ga < gb || ta < tb) ? 2 : (ta == tb ? 1 : 0);
-            if ((tla.cls == 1 && cls_b == 1 && !bb) || tlb.body != tla.body) mode = 0;
+        for (int r = 0; r < R; ++r) {
+            const int ta = PANEL * pa + NW * r + w;
+            mode[r] = ta < tb ? 2 : (ta == tb ? 1 : 0);
+            if (body[r] != tlb.body || (cls[r] == 1 && tlb.cls == 1 && !bb)) mode[r] = 0;
+            all2 = all2 && mode[r] == 2 && cls[r] == cls[0];
         }
-        if (mode) {
-            const double ai = tla.cls == 0 ? a.a_seg : a.a_blob;
-            const double aj = cls_b == 0 ? a.a_seg : a.a_blob;
-            const T sum_a2 = T(lam * lam * ((ai + aj) * (ai + aj)));
-            const T s3 = T(lam * lam * ((ai * ai + aj * aj) / 3.0));
-            const T m3s3 = T(-3) * s3;
-            T pi[3] = {T(0), T(0), T(0)}, pj[3] = {T(0), T(0), T(0)};
-            if (mode == 2) sym_stage<true, T>(recs[bq], lane, Xi, fi, sum_a2, s3, m3s3, pi, pj);
-            else sym_stage<false, T>(recs[bq], lane, Xi, fi, sum_a2, s3, m3s3, pi, pj);
+        const double aj = tlb.cls == 0 ? a.a_seg : a.a_blob;
+        T(*js)[DOF][64] = jsum + w * PARTS;  // this wave's sets
+        if (!all2) {
 #pragma unroll
-            for (int k = 0; k < 3; ++k) acc[k] += double(pi[k]);
-            if (mode == 2) {
-                const int j = (lane + 63 * kSymRot) & 63;
+            for (int p = 0; p < PARTS; ++p)
 #pragma unroll
-                for (int k = 0; k < 3; ++k) jsum[bq][k][j] += double(pj[k]);
+                for (int k = 0; k < DOF; ++k) js[p][k][lane] = T(0);
+        }
+        if (all2) {
+            const SymConsts<T> c = sym_consts<T>(cls[0] == 0 ? a.a_seg : a.a_blob, aj, lam);
+            sym_classes<true, R, PARTS, T, DOF>(cls[0], tlb.cls, recs, lane, Xi, fi, c, neg, acc, js, false);
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                if (mode[r] == 0) continue;
+                const SymConsts<T> c = sym_consts<T>(cls[r] == 0 ? a.a_seg : a.a_blob, aj, lam);
+                TargetT<T> X1[1][3];
+                T f1[1][DOF];
+                double a1[1][DOF];
+#pragma unroll
+                for (int k = 0; k < 3; ++k) X1[0][k] = Xi[r][k];
+#pragma unroll
+                for (int k = 0; k < DOF; ++k) {
+                    f1[0][k] = fi[r][k];
+                    a1[0][k] = acc[r][k];
+                }
+                if (R > 1 && mode[r] == 2)  // R = 1: all2
+                    sym_classes<true, 1, PARTS, T, DOF>(cls[r], tlb.cls, recs, lane, X1, f1, c, neg, a1, js, true);
+                else
+                    sym_classes<false, 1, PARTS, T, DOF>(cls[r], tlb.cls, recs, lane, X1, f1, c, neg, a1, js, true);
+#pragma unroll
+                for (int k = 0; k < DOF; ++k) acc[r][k] = a1[0][k];
             }
         }
-        __syncthreads();  // this stage's source sums are in before the next writer's
+        __syncthreads();  // every wave's sums are in
+        auto source_sum = [&](int k) {
+            double v = 0.0;
+#pragma unroll
+            for (int h = 0; h < NW * PARTS; ++h) v += double(jsum[h][k][lane]);
+            return v;
+        };
+        if (tb < PANEL * pa + PANEL) {
+            // one of the panel's own tiles: into its owner's sums
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (tb == PANEL * pa + NW * r + w) {
+#pragma unroll
+                    for (int k = 0; k < DOF; ++k)
+                        if (k < 3 || tlb.cls == 0) acc[r][k] += source_sum(k);
+                }
+        } else {
+            T* s = partial + (size_t)(tlb.first_item + pa - tlb.panel0) * (DOF * 64);
+            const int ncomp = tlb.cls == 0 ? DOF : 3;
+            for (int k = w; k < ncomp; k += NW) s[k * 64 + lane] = T(k < 3 ? source_sum(k) : rot * source_sum(k));
+        }
     }
-    // slot of (tile, partner group q) if q is one of the groups of the tile's
-    // body: 3 x 64 values
-    auto slot = [&](const MatvecTile& tl, int q) -> T* {
-        return (q >= tl.group0 && q < tl.group0 + tl.n_items)
-                   ? partial + ((size_t)tl.first_item + (q - tl.group0)) * (kSymSlotDof * 64)
-                   : nullptr;
-    };
-    if (ga < gb) {
-        if (has_a) {
-            if (T* s = slot(tla, gb)) {
+    // own sums: the slot of this run, if one of the tile's own to its body's last
 #pragma unroll
-                for (int k = 0; k < 3; ++k) s[k * 64 + lane] = T(acc[k]);
-            }
-        }
-        const int tb = kSymTiles * gb + w;
-        if (tb < n_tiles) {
-            if (T* s = slot(tiles[tb], ga)) {
+    for (int r = 0; r < R; ++r) {
+        const int ta = PANEL * pa + NW * r + w;
+        if (ta >= n_tiles) continue;
+        const MatvecTile tl = tiles[ta];
+        const int slot = (pa - tl.panel0) + it.s_end - tl.run0;  // after the panels before the tile's
+        if (it.s_end < tl.run0 || slot >= tl.n_items) continue;
+        T* s = partial + (size_t)(tl.first_item + slot) * (DOF * 64);
 #pragma unroll
-                for (int k = 0; k < 3; ++k) s[k * 64 + lane] = T(jsum[w][k][lane]);
-            }
-        }
-    } else if (has_a) {
-        T* s = slot(tla, ga);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) s[k * 64 + lane] = T(acc[k] + jsum[w][k][lane]);
+        for (int k = 0; k < DOF; ++k)
+            if (k < 3 || tl.cls == 0) s[k * 64 + lane] = T(k < 3 ? acc[r][k] : rot * acc[r][k]);
     }
     if (stamps && threadIdx.x == 0) {
         stamps[2 * (int64_t)blockIdx.x] = t_start;
@@ -1166,22 +1434,28 @@ __device__ void saddle_filament_rows(const SaddleEpilogue& e, int m, int lane) {
 
 // Adds the partial slots of each tile and the overlapping pairs, and applies
 // the write rule.  A slot holds slot_dof x tile_targets values (component k
-// of target l at k * tile_targets + l).  A workgroup covers 64 targets of one tile with four groups
-// of 64 threads: group g sums the items g, g+4, g+8, ... (loads of four items
-// issued together) and then the near-list entries g, g+4, ... of its target
-// (the lists are sorted when built); the four group sums are added in group
-// order, so the result is the same on every run.  Workgroups past
-// `tile_blocks` write the filament rows of the saddle-point operator.
-template <int SEGDOF, typename P>
-__global__ __launch_bounds__(256) void rpy_reduce_kernel(const MatvecTile* __restrict__ tiles,
-                                                         const P* __restrict__ partial, int tile_targets,
-                                                         int tile_blocks, int merge_k, int slot_dof, OutArgs o,
-                                                         MatvecArgs a, NearList near) {
-    __shared__ double grp_acc[3][6][64];
+// of target l at k * tile_targets + l).  A workgroup covers 64 targets of one
+// tile with GR groups of 64 threads: group g sums the items g, g+GR, g+2 GR,
+// ... (loads of four items issued together) and then the near-list entries g,
+// g+GR, ... of its target (the lists are sorted when built); the group sums
+// are added in group order, so the result is the same on every run.
+// Workgroups past `tile_blocks` write the filament rows of the saddle-point
+// operator.
+//
+// Bound by latency and the slots' bytes: few tiles with many slots each want
+// many loads in flight (reduce_groups: 12,800 segments + 9,000 blobs, 6
+// components FP32, 28 MB of slots: 36 us with the component count a condition
+// on every load, 13 without).
+template <int SEGDOF, typename P, int GR>
+__global__ __launch_bounds__(64 * GR) void rpy_reduce_kernel(const MatvecTile* __restrict__ tiles,
+                                                             const P* __restrict__ partial, int tile_targets,
+                                                             int tile_blocks, int merge_k, int slot_dof, OutArgs o,
+                                                             MatvecArgs a, NearList near) {
+    __shared__ double grp_acc[GR - 1][6][64];
     if (a.skip && *a.skip) return;
     const int grp = threadIdx.x >> 6;
     if ((int)blockIdx.x >= tile_blocks) {
-        const int m = ((int)blockIdx.x - tile_blocks) * 4 + grp;
+        const int m = ((int)blockIdx.x - tile_blocks) * GR + grp;
         if (m < o.sad.nfil && !(a.body_skip && o.sad.fil_body && a.body_skip[o.sad.fil_body[m]]))
             saddle_filament_rows(o.sad, m, threadIdx.x & 63);
         return;
@@ -1204,23 +1478,29 @@ __global__ __launch_bounds__(256) void rpy_reduce_kernel(const MatvecTile* __res
                                                      : tl.n_items;
     auto slot_of = [&](int q) { return merge_k > 0 ? (q == 0 ? 0 : (q0 + q) * merge_k - tl.first_item) : q; };
     double acc[6] = {0, 0, 0, 0, 0, 0};
-    for (int m0 = grp; m0 < nslots; m0 += 16) {
-        double v[4][6];
+    // one instance per component count: with the count a condition on each load
+    // the loads of an iteration would wait for one another
+    auto sum_slots = [&](auto comps) {
+        constexpr int VT = decltype(comps)::value;
+        for (int m0 = grp; m0 < nslots; m0 += 4 * GR) {
+            double v[4][VT];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int m = m0 + 4 * u;
-            const int mm = slot_of(m < nslots ? m : grp);
+            for (int u = 0; u < 4; ++u) {
+                const int m = m0 + GR * u;
+                const P* q = p + (size_t)slot_of(m < nslots ? m : grp) * slot_len;
 #pragma unroll
-            for (int k = 0; k < 6; ++k)
-                v[u][k] = k < vt ? double(p[(size_t)mm * slot_len + (size_t)k * tile_targets]) : 0.0;
+                for (int k = 0; k < VT; ++k) v[u][k] = double(q[(size_t)k * tile_targets]);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const bool in = m0 + GR * u < nslots;
+#pragma unroll
+                for (int k = 0; k < VT; ++k) acc[k] += in ? v[u][k] : 0.0;
+            }
         }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const bool in = m0 + 4 * u < nslots;
-#pragma unroll
-            for (int k = 0; k < 6; ++k) acc[k] += in ? v[u][k] : 0.0;
-        }
-    }
+    };
+    if (SEGDOF == 6 && seg_t) sum_slots(std::integral_constant<int, 6>{});
+    else sum_slots(std::integral_constant<int, 3>{});
     // Active source classes for this target class: bit 0 segments, bit 1 blobs.
     const uint32_t cls_mask = seg_t ? ((o.blocks & 1u) ? 1u : 0u) | ((o.blocks & 2u) ? 2u : 0u)
                                     : ((o.blocks & 8u) ? 1u : 0u) | ((o.blocks & 4u) ? 2u : 0u);
@@ -1232,7 +1512,7 @@ __global__ __launch_bounds__(256) void rpy_reduce_kernel(const MatvecTile* __res
         const double xi[3] = {xv.p[(int64_t)t * xv.ld_p], xv.p[(int64_t)t * xv.ld_p + xv.ld_c],
                               xv.p[(int64_t)t * xv.ld_p + 2 * xv.ld_c]};
         const double ai = seg_t ? a.a_seg : a.a_blob;
-        for (int q = grp; q < c; q += 4) {
+        for (int q = grp; q < c; q += GR) {
             if (seg_t && SEGDOF == 6) add_near<6>(acc, e[q], xi, ai, a, SEGDOF, cls_mask);
             else add_near<3>(acc, e[q], xi, ai, a, SEGDOF, cls_mask);
         }
@@ -1244,7 +1524,7 @@ __global__ __launch_bounds__(256) void rpy_reduce_kernel(const MatvecTile* __res
     __syncthreads();
     if (grp > 0 || !active) return;
 #pragma unroll
-    for (int g = 0; g < 3; ++g)
+    for (int g = 0; g < GR - 1; ++g)
 #pragma unroll
         for (int k = 0; k < 6; ++k) acc[k] += grp_acc[g][k][threadIdx.x];
     if (seg_t && o.sad.in && (o.sad.dyn_phase || o.sad.dyn_angle)) {
@@ -1368,6 +1648,20 @@ hipError_t dispatch_shape(const TileShape& sh, const MatvecArgs& a, const Matvec
     return hipErrorInvalidValue;
 }
 
+template <typename T, int DOF>
+hipError_t launch_sym(int kind, const MatvecArgs& a, const MatvecItem* d_items, int n_items, const MatvecTile* d_tiles,
+                      int n_tiles, int bb, double* partial, const PersistState& ps, hipStream_t stream) {
+    T* part = reinterpret_cast<T*>(partial);
+    const dim3 grid((unsigned)n_items), block(64 * kSymWaves);
+    if (kind == kSymWide)
+        hipLaunchKernelGGL((rpy_pairs_sym_kernel<T, DOF, 2>), grid, block, 0, stream, d_items, d_tiles, n_tiles, bb, a,
+                           part, ps.item_stamps);
+    else
+        hipLaunchKernelGGL((rpy_pairs_sym_kernel<T, DOF, 1>), grid, block, 0, stream, d_items, d_tiles, n_tiles, bb, a,
+                           part, ps.item_stamps);
+    return hipGetLastError();
+}
+
 }  // namespace
 
 void build_worklist(const std::vector<BodyRange>& bodies, int tile_targets, int chunk, bool ss, bool sb,
@@ -1444,8 +1738,8 @@ void build_worklist(const std::vector<BodyRange>& bodies, int tile_targets, int 
     }
 }
 
-size_t build_sym_worklist(const std::vector<BodyRange>& bodies, int seg_write, int blob_write,
-                          std::vector<MatvecTile>& tiles, std::vector<MatvecItem>& items) {
+size_t build_sym_worklist(const std::vector<BodyRange>& bodies, int kind, int seg_dof, int num_cus, int seg_write,
+                          int blob_write, std::vector<MatvecTile>& tiles, std::vector<MatvecItem>& items) {
     tiles.clear();
     items.clear();
     for (size_t b = 0; b < bodies.size(); ++b) {
@@ -1464,29 +1758,75 @@ size_t build_sym_worklist(const std::vector<BodyRange>& bodies, int seg_write, i
         add_tiles(1, bodies[b].blob_begin, bodies[b].blob_end, blob_write);
     }
     const int n_tiles = (int)tiles.size();
-    const int n_groups = (n_tiles + kSymTiles - 1) / kSymTiles;
-    // each body's groups [gfirst, glast]; each group's bodies [blo, bhi]
-    std::vector<int> gfirst(bodies.size(), -1), glast(bodies.size(), -1), blo(n_groups), bhi(n_groups);
-    for (int t = 0; t < n_tiles; ++t) {
-        const int b = tiles[t].body, g = t / kSymTiles;
-        if (gfirst[b] < 0) gfirst[b] = g;
-        glast[b] = g;
-        if (t % kSymTiles == 0) blo[g] = b;
-        bhi[g] = b;
+    const int panel = sym_panel(kind), n_panels = (n_tiles + panel - 1) / panel;
+    std::vector<int> first(bodies.size(), 0), last(bodies.size(), -1);  // each body's tiles
+    for (int t = n_tiles - 1; t >= 0; --t) {
+        first[tiles[t].body] = t;
+        if (last[tiles[t].body] < 0) last[tiles[t].body] = t;
+    }
+    // Source tiles of panel A: its own, then the rest of its last body's.
+    auto end_of = [&](int A) { return last[tiles[std::min(panel * A + panel, n_tiles) - 1].body] + 1; };
+    // Cost of a panel's tiles against one source tile, in 3-component tile pairs;
+    // beyond the panel it depends on the source's class only.
+    auto pair_cost = [&](int ta, int tb) {
+        if (ta > tb || tiles[ta].body != tiles[tb].body) return 0.0;
+        const bool sa = tiles[ta].cls == 0, sb = tiles[tb].cls == 0;
+        return (seg_dof == 6 ? (sa && sb ? 2.2 : sa || sb ? 1.4 : 1.0) : 1.0) * (ta == tb ? 0.6 : 1.0);
+    };
+    auto cost_of = [&](int A, int tb) {
+        double c = 0.0;
+        for (int ta = panel * A; ta < std::min(panel * A + panel, n_tiles); ++ta) c += pair_cost(ta, tb);
+        return c;
+    };
+    std::vector<double> cost(n_tiles);  // of the current panel's source tiles
+    auto panel_costs = [&](int A) {
+        const int own_end = std::min(panel * A + panel, n_tiles), end = end_of(A);
+        double sum = 0.0;
+        for (int q = panel * A; q < end; ++q) {
+            const bool as_before = q > own_end && tiles[q].cls == tiles[q - 1].cls;
+            cost[q] = as_before ? cost[q - 1] : cost_of(A, q);
+            sum += cost[q];
+        }
+        return sum;
+    };
+    double left = 0.0;
+    for (int A = 0; A < n_panels; ++A) left += panel_costs(A);
+    // Runs: about half of what is left shared by the workgroups that fit the
+    // device, so that the last ones are single tiles and the launch ends evenly
+    // without every tile costing its panel a slot.
+    const double resident = 5.0 * (num_cus > 0 ? num_cus : 256);
+    std::vector<int> run_of;                       // of the panel's source tiles
+    for (int A = 0; A < n_panels; ++A) {
+        const int q_lo = panel * A, q_hi = end_of(A);
+        run_of.assign(q_hi - q_lo, 0);
+        panel_costs(A);
+        int run = 0;
+        for (int q = q_lo; q < q_hi;) {
+            const double want = std::max(left / (2.0 * resident), 1.0);
+            int e = q;
+            double c = 0.0;
+            while (e < q_hi && e - q < kSymMaxRun && (e == q || c + 0.5 * cost[e] <= want)) {
+                c += cost[e];
+                run_of[e - q_lo] = run;
+                ++e;
+            }
+            items.push_back({A, q, e, run});
+            left -= c;
+            q = e;
+            ++run;
+        }
+        for (int t = q_lo; t < std::min(q_lo + panel, n_tiles); ++t) {
+            MatvecTile& tl = tiles[t];
+            tl.panel0 = first[tl.body] / panel;
+            tl.run0 = run_of[t - q_lo];
+            tl.n_items = (A - tl.panel0) + (run_of[last[tl.body] - q_lo] - tl.run0 + 1);
+        }
     }
     size_t slots = 0;
     for (MatvecTile& tl : tiles) {
-        tl.group0 = gfirst[tl.body];
         tl.first_item = (int32_t)slots;
-        tl.n_items = glast[tl.body] - gfirst[tl.body] + 1;
         slots += (size_t)tl.n_items;
     }
-    // off-diagonal items (both tiles' sums, the costlier ones) first; groups
-    // are in body order, so ga < gb share a body when gb starts no later than
-    // the last body of ga
-    for (int ga = 0; ga < n_groups; ++ga)
-        for (int gb = ga + 1; gb < n_groups && blo[gb] <= bhi[ga]; ++gb) items.push_back({ga, gb, 0, 0});
-    for (int g = 0; g < n_groups; ++g) items.push_back({g, g, 0, 0});
     return slots;
 }
 
@@ -1617,12 +1957,56 @@ hipError_t launch_barrier(const MatvecArgs& a, NearGrid& grid, const BarrierPara
     return hipGetLastError();
 }
 
+// Groups of a reduce workgroup: sixteen (eight with rotations, whose near-pair
+// terms take too many registers for sixteen) where the tiles are few and have
+// many slots each, else four.
+template <int SEGDOF>
+static int reduce_groups(int tile_blocks, int n_tiles, int n_slots) {
+    return tile_blocks <= 1024 && n_slots >= 24 * n_tiles ? (SEGDOF == 6 ? 8 : 16) : 4;
+}
+
+template <int SEGDOF, typename P>
+static void launch_reduce_typed(const MatvecArgs& a, const OutArgs& o, const MatvecTile* d_tiles, int n_tiles, int n_slots,
+                                int tile_targets, int merge_k, int slot_dof, const P* partial, const NearList& near,
+                                hipStream_t stream) {
+    const int tile_blocks = n_tiles * ((tile_targets + 63) / 64);
+    const int gr = reduce_groups<SEGDOF>(tile_blocks, n_tiles, n_slots);
+    const int fil_blocks = o.sad.in ? (o.sad.nfil + gr - 1) / gr : 0;
+    const dim3 grid((unsigned)(tile_blocks + fil_blocks));
+    constexpr int MANY = SEGDOF == 6 ? 8 : 16;
+    if (gr == MANY)
+        hipLaunchKernelGGL((rpy_reduce_kernel<SEGDOF, P, MANY>), grid, dim3(64 * MANY), 0, stream, d_tiles, partial,
+                           tile_targets, tile_blocks, merge_k, slot_dof, o, a, near);
+    else
+        hipLaunchKernelGGL((rpy_reduce_kernel<SEGDOF, P, 4>), grid, dim3(256), 0, stream, d_tiles, partial,
+                           tile_targets, tile_blocks, merge_k, slot_dof, o, a, near);
+}
+
+// The reduce kernel over n_slots partial slots of the evaluation type.
+static hipError_t launch_reduce(int precision, int seg_dof, const MatvecArgs& a, const OutArgs& o,
+                                const MatvecTile* d_tiles, int n_tiles, int n_slots, int tile_targets, int merge_k,
+                                int slot_dof, const double* partial, const NearList& near, hipStream_t stream) {
+    const float* pf = reinterpret_cast<const float*>(partial);
+    if (precision == 0) {
+        if (seg_dof == 6)
+            launch_reduce_typed<6>(a, o, d_tiles, n_tiles, n_slots, tile_targets, merge_k, slot_dof, partial, near, stream);
+        else
+            launch_reduce_typed<3>(a, o, d_tiles, n_tiles, n_slots, tile_targets, merge_k, slot_dof, partial, near, stream);
+    } else {
+        if (seg_dof == 6)
+            launch_reduce_typed<6>(a, o, d_tiles, n_tiles, n_slots, tile_targets, merge_k, slot_dof, pf, near, stream);
+        else
+            launch_reduce_typed<3>(a, o, d_tiles, n_tiles, n_slots, tile_targets, merge_k, slot_dof, pf, near, stream);
+    }
+    return hipGetLastError();
+}
+
 hipError_t launch_matvec_wall(int precision, int seg_dof, const MatvecArgs& a, const OutArgs& o,
                               const MatvecTile* d_tiles, int n_tiles, const MatvecItem* d_items, int n_items,
                               double* partial, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end) {
     if (n_tiles == 0) return hipSuccess;
-    float* pf = reinterpret_cast<float*>(partial);
     if (n_items > 0) {
+        float* pf = reinterpret_cast<float*>(partial);
         if (ev_begin) TFS_HIP_CHECK(hipEventRecord(ev_begin, stream));
         const dim3 grid((unsigned)n_items), block(kWallBlock);
         if (precision == 0) {
@@ -1641,46 +2025,27 @@ hipError_t launch_matvec_wall(int precision, int seg_dof, const MatvecArgs& a, c
         TFS_HIP_CHECK(hipGetLastError());
         if (ev_end) TFS_HIP_CHECK(hipEventRecord(ev_end, stream));
     }
-    const int tile_blocks = n_tiles * ((kWallBlock + 63) / 64);
-    const int fil_blocks = o.sad.in ? (o.sad.nfil + 3) / 4 : 0;
-    const NearList none{};
-    const dim3 grid((unsigned)(tile_blocks + fil_blocks));
-    if (precision == 0) {
-        if (seg_dof == 6)
-            hipLaunchKernelGGL((rpy_reduce_kernel<6, double>), grid, dim3(256), 0, stream, d_tiles,
-                               (const double*)partial, kWallBlock, tile_blocks, 0, kMaxDof, o, a, none);
-        else
-            hipLaunchKernelGGL((rpy_reduce_kernel<3, double>), grid, dim3(256), 0, stream, d_tiles,
-                               (const double*)partial, kWallBlock, tile_blocks, 0, kMaxDof, o, a, none);
-    } else {
-        if (seg_dof == 6)
-            hipLaunchKernelGGL((rpy_reduce_kernel<6, float>), grid, dim3(256), 0, stream, d_tiles, (const float*)pf,
-                               kWallBlock, tile_blocks, 0, kMaxDof, o, a, none);
-        else
-            hipLaunchKernelGGL((rpy_reduce_kernel<3, float>), grid, dim3(256), 0, stream, d_tiles, (const float*)pf,
-                               kWallBlock, tile_blocks, 0, kMaxDof, o, a, none);
-    }
-    return hipGetLastError();
+    return launch_reduce(precision, seg_dof, a, o, d_tiles, n_tiles, n_items, kWallBlock, 0, kMaxDof, partial, NearList{},
+                         stream);
 }
 
 hipError_t launch_matvec(int precision, int seg_dof, const TileShape& shape, const MatvecArgs& a,
                          const OutArgs& o, const MatvecTile* d_tiles, int n_tiles,
-                         const MatvecItem* d_items, int n_items, double* partial, const NearList& near,
+                         const MatvecItem* d_items, int n_items, int n_slots, double* partial, const NearList& near,
                          const PersistState& ps, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end) {
     if (n_tiles == 0) return hipSuccess;
-    if (shape.symmetric && (seg_dof != 3 || (precision == 1 && !a.xfx))) return hipErrorInvalidValue;
+    if (shape.symmetric && precision == 1 && !a.xfx) return hipErrorInvalidValue;
     if (n_items > 0) {
         hipError_t e;
         if (ev_begin) TFS_HIP_CHECK(hipEventRecord(ev_begin, stream));
         if (shape.symmetric) {
             const int bb = (o.blocks & 4u) ? 1 : 0;
-            if (precision == 1)
-                hipLaunchKernelGGL(rpy_pairs_sym_kernel<float>, dim3((unsigned)n_items), dim3(64 * kSymTiles), 0, stream,
-                                   d_items, d_tiles, n_tiles, bb, a, reinterpret_cast<float*>(partial), ps.item_stamps);
+            if (precision == 0)
+                e = seg_dof == 6 ? launch_sym<double, 6>(shape.symmetric, a, d_items, n_items, d_tiles, n_tiles, bb, partial, ps, stream)
+                                 : launch_sym<double, 3>(shape.symmetric, a, d_items, n_items, d_tiles, n_tiles, bb, partial, ps, stream);
             else
-                hipLaunchKernelGGL(rpy_pairs_sym_kernel<double>, dim3((unsigned)n_items), dim3(64 * kSymTiles), 0,
-                                   stream, d_items, d_tiles, n_tiles, bb, a, partial, ps.item_stamps);
-            e = hipGetLastError();
+                e = seg_dof == 6 ? launch_sym<float, 6>(shape.symmetric, a, d_items, n_items, d_tiles, n_tiles, bb, partial, ps, stream)
+                                 : launch_sym<float, 3>(shape.symmetric, a, d_items, n_items, d_tiles, n_tiles, bb, partial, ps, stream);
         } else if (precision == 0) {
             e = seg_dof == 6 ? dispatch_shape<double, 6>(shape, a, d_items, n_items, d_tiles, partial, ps, stream)
                              : dispatch_shape<double, 3>(shape, a, d_items, n_items, d_tiles, partial, ps, stream);
@@ -1691,31 +2056,12 @@ hipError_t launch_matvec(int precision, int seg_dof, const TileShape& shape, con
         if (e != hipSuccess) return e;
         if (ev_end) TFS_HIP_CHECK(hipEventRecord(ev_end, stream));
     }
-    const int tt = tile_targets(shape);
-    const int tile_blocks = n_tiles * ((tt + 63) / 64);
-    const int fil_blocks = o.sad.in ? (o.sad.nfil + 3) / 4 : 0;
-    const dim3 grid((unsigned)(tile_blocks + fil_blocks));
     // The partial slots hold the evaluation type (FP32 sums for FP32 tiles);
     // the persistent form fills only its tile segments' first slots.
     const int merge_k = shape.persistent > 0 && n_items > 0 ? persistent_items(shape, n_items, ps.num_cus) : 0;
-    const int slot_dof = shape.symmetric ? kSymSlotDof : kMaxDof;
-    const float* pf = reinterpret_cast<const float*>(partial);
-    if (precision == 0) {
-        if (seg_dof == 6)
-            hipLaunchKernelGGL((rpy_reduce_kernel<6, double>), grid, dim3(256), 0, stream, d_tiles,
-                               (const double*)partial, tt, tile_blocks, merge_k, slot_dof, o, a, near);
-        else
-            hipLaunchKernelGGL((rpy_reduce_kernel<3, double>), grid, dim3(256), 0, stream, d_tiles,
-                               (const double*)partial, tt, tile_blocks, merge_k, slot_dof, o, a, near);
-    } else {
-        if (seg_dof == 6)
-            hipLaunchKernelGGL((rpy_reduce_kernel<6, float>), grid, dim3(256), 0, stream, d_tiles, pf, tt,
-                               tile_blocks, merge_k, slot_dof, o, a, near);
-        else
-            hipLaunchKernelGGL((rpy_reduce_kernel<3, float>), grid, dim3(256), 0, stream, d_tiles, pf, tt,
-                               tile_blocks, merge_k, slot_dof, o, a, near);
-    }
-    return hipGetLastError();
+    const int slots = shape.symmetric ? n_slots : n_items;
+    return launch_reduce(precision, seg_dof, a, o, d_tiles, n_tiles, slots, tile_targets(shape), merge_k,
+                         shape.symmetric ? seg_dof : kMaxDof, partial, near, stream);
 }
 
 }  // namespace tfs

@@ -30,11 +30,24 @@ __device__ __forceinline__ double rsqrt_refined(double x) {
     return __builtin_fma(0.5 * y, e, y);
 }
 
+// 2/sqrt(x): the same step without its factor 1/2, w = z (3 - x z^2) -- three
+// operations instead of four; callers fold the powers of two into constants.
+__device__ __forceinline__ double rsqrt_twice(double x) {
+    const double z = __builtin_amdgcn_rsq(x);
+    return z * __builtin_fma(-x * z, z, 3.0);
+}
+
 __device__ __forceinline__ float rsqrt_refined(float x) {
     return __builtin_amdgcn_rsqf(x);
 }
 
-__device__ __forceinline__ float fmax_t(float a, float b) { return __builtin_fmaxf(a, b); }
+// The instruction itself: where the compiler cannot see that b is canonical (a
+// loop invariant) it would put a second maximum before each.
+__device__ __forceinline__ float fmax_t(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
 __device__ __forceinline__ double fmax_t(double a, double b) { return __builtin_fmax(a, b); }
 __device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }

@@ -33,7 +33,8 @@ struct Plan {
     MatvecTile* d_tiles = nullptr;
     MatvecItem* d_items = nullptr;
     uint32_t blocks = 0;  // blocks actually evaluated (after the reference's overwrite rule)
-    bool symmetric = false;  // items are pairs of tile groups (the symmetric form)
+    int symmetric = 0;    // the symmetric form's kind (items are a panel and a run of tiles), or 0
+    int slots = 0;        // partial slots
 };
 
 }  // namespace tfs
@@ -90,6 +91,12 @@ struct tfs_rpy {
     // Tile shape set by tfs_rpy_set_tile_shape or tfs_rpy_autotune (else the
     // default follows the body list).
     bool shape_chosen[2] = {false, false};
+    // The symmetric form in evaluations that a non-symmetric `shape` would
+    // take: -1 while the shape is the default, where the handle may choose it
+    // by its size, else 0 (off) or the kind that the autotuner found fastest.
+    int sym_pick[2] = {-1, -1};
+    bool graph_made = false;        // a captured graph may hold `partial`: replaced buffers stay
+    std::vector<double*> retired;   // until the handle goes
     // Stop flag passed to the kernels of later evaluations (set by a solver
     // around its speculative Krylov iterations; null otherwise).
     const int32_t* skip_flag = nullptr;
@@ -174,11 +181,11 @@ int hip_fail(hipError_t e, const char* where);
 int hip_fail_if(hipError_t e, const char* where);
 TileShape default_shape(int precision, int ns, int nb, int num_cus, int seg_dof, int num_bodies);
 Plan* get_plan(tfs_rpy* h, uint32_t blocks, const TileShape& sh, int* err);
-// Whether the symmetric form can evaluate `blocks` of this handle in
-// `precision` (3-DOF segments, unbounded domain, the SS, SB and BS blocks all
-// active).
-bool symmetric_applies(const tfs_rpy* h, int precision, uint32_t blocks);
-// The launch shape of one evaluation: the handle's shape, or its default
+// Whether the symmetric form can evaluate `blocks` of this handle (unbounded
+// domain, the SS, SB and BS blocks all active).
+bool symmetric_applies(const tfs_rpy* h, uint32_t blocks);
+// The launch shape of one evaluation: the handle's shape, the symmetric form
+// where the handle has no chosen shape and its size favours it, or the default
 // source-split shape where a symmetric shape does not apply.
 TileShape effective_shape(const tfs_rpy* h, int precision, uint32_t blocks);
 // Positions changed: the near-pair lists must be rebuilt before the next matvec.

@@ -48,8 +48,8 @@ struct MatvecTile {
     int32_t n_items;
     int32_t write_mode;  // 0 overwrite, 1 accumulate into the output
     int32_t body;        // index into the body list
-    int32_t group0;      // symmetric form: first tile group of the body (slot of group q:
-                         // first_item + q - group0)
+    int32_t panel0;      // symmetric form: first panel of tiles of the body, and the run of its
+    int32_t run0;        // own panel's source tiles that holds the tile
 };
 
 // Overlapping pairs (r^2 <= (ai+aj)^2 as evaluated by the pair kernel of one
@@ -103,20 +103,23 @@ struct TileShape {
                      // taking a contiguous range of the work list
     int split = 0;   // 1: the block/64 waves share one tile of 64 x per_thread targets and
                      // split every LDS batch of sources between them
-    int symmetric = 0;  // 1: each pair once for both particles (FP32 tiles, 3-DOF, one
-                        // body; 64-particle tiles in groups of four, 256 threads)
+    int symmetric = 0;  // each pair once for both particles: kSymWide or kSymNarrow
 };
 
 // Up to this many particles the near-pair lists test every pair (bit masks of
 // n^2 / 8 bytes) instead of sorting the particles into a hashed grid.
 constexpr int kNearPairsMax = 6144;
 
-// Tiles of 64 particles per group (and waves per workgroup) of the symmetric
-// form; values per particle in its partial slots (3 x 64 per slot); the
-// largest partial buffer its default shape may take (the slots grow as
-// tiles x groups).
-constexpr int kSymGroupTiles = 4;
-constexpr int kSymSlotDof = 3;
+// The symmetric form's kinds, two target particles per lane or one (bodies
+// where two would leave too few workgroups); the waves of its workgroups, and
+// the 64-particle tiles of a panel; the longest run of source tiles of one
+// item; the largest partial buffer that a handle's own choice may take (the
+// slots grow as tiles x panels).
+constexpr int kSymWide = 1;
+constexpr int kSymNarrow = 2;
+constexpr int kSymWaves = 4;
+constexpr int kSymMaxRun = 8;
+constexpr int sym_panel(int kind) { return kind == kSymWide ? 2 * kSymWaves : kSymWaves; }
 constexpr double kSymMaxPartialBytes = 4.0 * (1 << 30);
 
 // Targets per tile (and per partial slot) of a launch shape.
@@ -185,12 +188,11 @@ void build_worklist(const std::vector<BodyRange>& bodies, int tile_targets, int 
                     bool bb, bool bs, int seg_write, int blob_write, std::vector<MatvecTile>& tiles,
                     std::vector<MatvecItem>& items);
 // The symmetric form's work list: 64-particle tiles (each body's segments,
-// then its blobs, body after body) in groups of four, one item (tile = ga,
-// src_cls = gb) per pair of groups ga <= gb that share a body, the diagonal
-// ones last; every tile one partial slot per group its body overlaps.
-// Returns the number of partial slots.
-size_t build_sym_worklist(const std::vector<BodyRange>& bodies, int seg_write, int blob_write,
-                          std::vector<MatvecTile>& tiles, std::vector<MatvecItem>& items);
+// then its blobs, body after body), one item (tile = panel, source tiles
+// [src_cls, s_begin), s_end = run) per panel and run of tiles from the panel's
+// first on that share a body with it.  Returns the number of partial slots.
+size_t build_sym_worklist(const std::vector<BodyRange>& bodies, int kind, int seg_dof, int num_cus, int seg_write,
+                          int blob_write, std::vector<MatvecTile>& tiles, std::vector<MatvecItem>& items);
 
 // Rebuilds `near` for the given precision: every pair of particles of one
 // body whose squared separation, in the pair kernel's own arithmetic for that
@@ -207,12 +209,13 @@ hipError_t launch_barrier(const MatvecArgs& a, NearGrid& grid, const BarrierPara
                           hipStream_t stream);
 
 // Launches pair kernel + reduce on `stream`.  d_tiles/d_items/partial are device
-// buffers sized for the work list; precision 0 = fp64, 1 = fp32 tiles with fp64
+// buffers sized for the work list (n_slots partial slots in the symmetric form,
+// one per item otherwise); precision 0 = fp64, 1 = fp32 tiles with fp64
 // accumulation.  ev_begin/ev_end (may be null) are recorded around the pair
 // kernel only.
 hipError_t launch_matvec(int precision, int seg_dof, const TileShape& shape, const MatvecArgs& a,
                          const OutArgs& o, const MatvecTile* d_tiles, int n_tiles,
-                         const MatvecItem* d_items, int n_items, double* partial, const NearList& near,
+                         const MatvecItem* d_items, int n_items, int n_slots, double* partial, const NearList& near,
                          const PersistState& ps, hipStream_t stream, hipEvent_t ev_begin = nullptr,
                          hipEvent_t ev_end = nullptr);
 

@@ -92,26 +92,49 @@ TileShape default_shape(int precision, int ns, int nb, int num_cus, int seg_dof,
     return s;
 }
 
-// The default launch shape of a handle: the symmetric form for 3-DOF
-// segments when the (largest) body alone gives every CU ~4 items (measured on
-// MI355X, 12,800 segments + 9,000 blobs: 0.212 ms per FP32 launch against
-// 0.266 for the best source-split shape, 0.358 ms per FP64 launch against
-// 0.432; 64 uneven bodies in lock-step, a mixed timestep in 831 ms against
-// 1,027), else default_shape.
-// `sym_slots`: the symmetric form's partial slots over all bodies (its buffer
-// takes 3 x 64 doubles each), which must stay below kSymMaxPartialBytes.
-static TileShape preferred_shape(int precision, int ns, int nb, int num_cus, int seg_dof, int num_bodies,
-                                 double sym_slots) {
-    if (seg_dof == 3 && sym_slots * kSymSlotDof * 64 * sizeof(double) <= kSymMaxPartialBytes) {
-        const long tiles = (ns + 63L) / 64 + (nb + 63L) / 64;
-        const long groups = (tiles + 3) / 4;
-        if (groups * (groups + 1) / 2 >= 4L * (num_cus > 0 ? num_cus : 256)) {
-            TileShape s{256, 1, 0, 0, 0};
-            s.symmetric = 1;
-            return s;
-        }
+// Whether bodies of these sizes give every CU ~4 items of the symmetric form's
+// panels (12,800 segments + 9,000 blobs: 3,741 pairs of groups of four tiles
+// for 256 CUs).
+static bool panels_fill(const std::vector<BodyRange>& bodies, int num_cus) {
+    double items = 0.0;
+    for (const BodyRange& b : bodies) {
+        const long tiles = (b.seg_end - b.seg_begin + 63L) / 64 + (b.blob_end - b.blob_begin + 63L) / 64;
+        const double groups = double((tiles + 3) / 4);
+        items += groups * (groups + 1.0) / 2.0;
     }
-    return default_shape(precision, ns, nb, num_cus, seg_dof, num_bodies);
+    return items >= 4.0 * (num_cus > 0 ? num_cus : 256);
+}
+
+// The symmetric form's partial slots for these bodies, at most.
+static double sym_slot_count(const std::vector<BodyRange>& bodies, int kind) {
+    double slots = 0.0;
+    const int panel = sym_panel(kind);
+    for (const BodyRange& b : bodies) {
+        const double t = double((b.seg_end - b.seg_begin + 63) / 64 + (b.blob_end - b.blob_begin + 63) / 64);
+        slots += t * (t + 0.5 * (t / panel) + 2.0) * 0.6;
+    }
+    return slots;
+}
+
+static bool sym_fits(const std::vector<BodyRange>& bodies, int kind, int seg_dof) {
+    return sym_slot_count(bodies, kind) * seg_dof * 64 * sizeof(double) <= kSymMaxPartialBytes;
+}
+
+// The shape of a handle that none was set for: the symmetric form for 3-DOF
+// segments when the largest body alone fills the device with its items
+// (measured on MI355X, 12,800 segments + 9,000 blobs: 0.212 ms per FP32 launch
+// against 0.266 for the best source-split shape, 0.358 ms per FP64 launch
+// against 0.432; 64 uneven bodies in lock-step, a mixed timestep in 831 ms
+// against 1,027), else default_shape.
+static TileShape preferred_shape(int precision, int ns, int nb, int num_cus, int seg_dof,
+                                 const std::vector<BodyRange>& bodies) {
+    if (seg_dof == 3 && sym_fits(bodies, kSymWide, seg_dof) &&
+        panels_fill({BodyRange{0, ns, 0, nb}}, num_cus)) {
+        TileShape s{256, 1, 0, 0, 0};
+        s.symmetric = kSymWide;
+        return s;
+    }
+    return default_shape(precision, ns, nb, num_cus, seg_dof, (int)bodies.size());
 }
 
 // Without the split: 512-target tiles, ~16 items per CU (short items even
@@ -140,17 +163,6 @@ static void largest_body(const tfs_rpy* h, int* ns, int* nb) {
     }
 }
 
-// The symmetric form's partial slots for these bodies (each tile one per
-// group of four tiles its body overlaps).
-static double sym_slot_count(const std::vector<BodyRange>& bodies) {
-    double slots = 0.0;
-    for (const BodyRange& b : bodies) {
-        const double t = double((b.seg_end - b.seg_begin + 63) / 64 + (b.blob_end - b.blob_begin + 63) / 64);
-        slots += t * (std::ceil(t / kSymGroupTiles) + 1.0);
-    }
-    return slots;
-}
-
 Plan* get_plan(tfs_rpy* h, uint32_t blocks, const TileShape& sh, int* err) {
     bool ss = blocks & TFS_BLOCK_SS, sb = blocks & TFS_BLOCK_SB;
     bool bb = blocks & TFS_BLOCK_BB, bs = blocks & TFS_BLOCK_BS;
@@ -168,12 +180,14 @@ Plan* get_plan(tfs_rpy* h, uint32_t blocks, const TileShape& sh, int* err) {
     p.blocks = eff;
     size_t slots = 0;
     if (sh.symmetric) {
-        slots = build_sym_worklist(h->bodies, seg_write, blob_write, p.tiles, p.items);
-        p.symmetric = true;
+        slots = build_sym_worklist(h->bodies, sh.symmetric, h->desc.seg_dof, h->num_cus, seg_write, blob_write, p.tiles,
+                                   p.items);
+        p.symmetric = sh.symmetric;
     } else {
         build_worklist(h->bodies, tile_targets(sh), sh.chunk, ss, sb, bb, bs, seg_write, blob_write, p.tiles, p.items);
         slots = p.items.size();
     }
+    p.slots = (int)slots;
     if (!p.tiles.empty()) {
         hipError_t e = hipMalloc(&p.d_tiles, sizeof(MatvecTile) * p.tiles.size());
         if (e == hipSuccess && !p.items.empty())
@@ -190,9 +204,11 @@ Plan* get_plan(tfs_rpy* h, uint32_t blocks, const TileShape& sh, int* err) {
             *err = hip_fail(e, "work list upload");
             return nullptr;
         }
-        const size_t need = slots * (size_t)(sh.symmetric ? kSymSlotDof : 6) * (size_t)tile_targets(sh);
+        const size_t need = slots * (size_t)(sh.symmetric ? h->desc.seg_dof : 6) * (size_t)tile_targets(sh);
         if (need > h->partial_len) {
-            if (h->partial) {
+            if (h->partial && h->graph_made) {
+                h->retired.push_back(h->partial);
+            } else if (h->partial) {
                 hipStreamSynchronize(h->stream);
                 hipFree(h->partial);
             }
@@ -210,15 +226,43 @@ Plan* get_plan(tfs_rpy* h, uint32_t blocks, const TileShape& sh, int* err) {
     return &res.first->second;
 }
 
-bool symmetric_applies(const tfs_rpy* h, int precision, uint32_t blocks) {
-    (void)precision;
-    return h->desc.seg_dof == 3 && h->domain == TFS_DOMAIN_UNBOUNDED && (blocks & TFS_BLOCK_SS) &&
-           (blocks & TFS_BLOCK_SB) && (blocks & TFS_BLOCK_BS);
+bool symmetric_applies(const tfs_rpy* h, uint32_t blocks) {
+    return h->domain == TFS_DOMAIN_UNBOUNDED && (blocks & TFS_BLOCK_SS) && (blocks & TFS_BLOCK_SB) &&
+           (blocks & TFS_BLOCK_BS);
+}
+
+// The symmetric form's kind that a handle without a chosen shape takes by its
+// size, or 0.  Two particles per lane where the bodies' panels fill the device;
+// one per lane (twice as many, smaller items) from 8 pairs of tiles per CU on,
+// about 4,100 particles in one body; below that the launch is bound by its
+// longest item and the finest directed shape (one wave per 64 x 32 pairs) is
+// as fast.  Measured on MI355X per evaluation, directed / symmetric, us, with
+// rotations: 1,600 + 2,600 particles FP32 31 / 30, FP64 41 / 40; 2,461 + 3,333
+// 44 / 42, 64 / 57; 6,000 + 4,500 109 / 100, 171 / 155; 12,800 + 9,000 392 /
+// 340, 693 / 560; twelve uneven bodies 3,480 / 2,830, 6,250 / 4,750.
+static int sym_by_size(const tfs_rpy* h) {
+    const double cus = h->num_cus > 0 ? h->num_cus : 256;
+    if (panels_fill(h->bodies, h->num_cus) && sym_fits(h->bodies, kSymWide, h->desc.seg_dof)) return kSymWide;
+    double pairs = 0.0;
+    for (const BodyRange& b : h->bodies) {
+        const double t = double((b.seg_end - b.seg_begin + 63) / 64 + (b.blob_end - b.blob_begin + 63) / 64);
+        pairs += t * (t + 1.0) / 2.0;
+    }
+    return pairs >= 8.0 * cus && sym_fits(h->bodies, kSymNarrow, h->desc.seg_dof) ? kSymNarrow : 0;
 }
 
 TileShape effective_shape(const tfs_rpy* h, int precision, uint32_t blocks) {
     const TileShape& sh = h->shape[precision];
-    if (!sh.symmetric || symmetric_applies(h, precision, blocks)) return sh;
+    const bool applies = symmetric_applies(h, blocks);
+    if (!sh.symmetric) {
+        const int pick = h->sym_pick[precision];
+        const int kind = !applies || sh.persistent > 0 ? 0 : pick < 0 ? sym_by_size(h) : pick;
+        if (!kind) return sh;
+        TileShape s{64 * kSymWaves, 1, 0, 0, 0};
+        s.symmetric = kind;
+        return s;
+    }
+    if (applies) return sh;
     int ns = 0, nb = 0;
     largest_body(h, &ns, &nb);
     return default_shape(precision, ns, nb, h->num_cus, h->desc.seg_dof, (int)h->bodies.size());
@@ -580,7 +624,7 @@ int run_matvec(tfs_rpy* h, uint32_t blocks, int precision, CView fs, CView fb, V
     hipError_t e = wall ? launch_matvec_wall(precision, h->desc.seg_dof, a, o, p->d_tiles, (int)p->tiles.size(), p->d_items,
                                              (int)p->items.size(), h->partial, h->stream, eb, ee)
                         : launch_matvec(precision, h->desc.seg_dof, sh, a, o, p->d_tiles, (int)p->tiles.size(),
-                                        p->d_items, (int)p->items.size(), h->partial, h->near[precision], ps,
+                                        p->d_items, (int)p->items.size(), p->slots, h->partial, h->near[precision], ps,
                                         h->stream, eb, ee);
     if (e != hipSuccess) return hip_fail(e, "matvec launch");
     return TFS_OK;
@@ -657,8 +701,8 @@ int tfs_rpy_create(const tfs_rpy_desc* desc, tfs_rpy** out) {
         return hip_fail(e, "tfs_rpy_create: clear");
     }
     for (int pr = 0; pr < 2; ++pr)
-        h->shape[pr] = preferred_shape(pr, desc->num_segs, desc->num_blobs, cus, desc->seg_dof, 1,
-                                       sym_slot_count({BodyRange{0, desc->num_segs, 0, desc->num_blobs}}));
+        h->shape[pr] = preferred_shape(pr, desc->num_segs, desc->num_blobs, cus, desc->seg_dof,
+                                       {BodyRange{0, desc->num_segs, 0, desc->num_blobs}});
     h->bodies.push_back(BodyRange{0, desc->num_segs, 0, desc->num_blobs});
     e = hipHostMalloc((void**)&h->host_int, 64, hipHostMallocDefault);
     if (e != hipSuccess) {
@@ -682,6 +726,7 @@ int tfs_rpy_destroy(tfs_rpy* h) {
             hipEventDestroy(pr.end);
         }
     if (h->partial) hipFree(h->partial);
+    for (double* p : h->retired) hipFree(p);
     if (h->arena) hipFree(h->arena);
     for (auto& nl : h->near) free_near(nl);
     free_grid(h->grid);
@@ -884,6 +929,7 @@ static int set_shape(tfs_rpy* h, const char* fn, int32_t precision, int32_t bloc
         return fail(TFS_ERR_INVALID_ARGUMENT, std::string(fn) + ": the source split has no persistent form");
     h->shape[precision] = TileShape{block, per_thread, chunk, pers, split};
     h->shape_chosen[precision] = true;
+    h->sym_pick[precision] = 0;
     return TFS_OK;
 }
 
@@ -901,6 +947,7 @@ int tfs_rpy_set_symmetric(tfs_rpy* h, int32_t precision, int32_t enable) {
     if (precision != 0 && precision != 1)
         return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_set_symmetric: unknown precision");
     if (!enable) {
+        h->sym_pick[precision] = 0;
         if (h->shape[precision].symmetric) {
             int ns = 0, nb = 0;
             largest_body(h, &ns, &nb);
@@ -913,8 +960,8 @@ int tfs_rpy_set_symmetric(tfs_rpy* h, int32_t precision, int32_t enable) {
         return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_set_symmetric: the symmetric form needs 3-DOF segments");
     if (h->shape[precision].persistent > 0)
         return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_set_symmetric: the symmetric form has no persistent form");
-    TileShape sh{64 * 4, 1, 0, 0, 0};
-    sh.symmetric = 1;
+    TileShape sh{256, 1, 0, 0, 0};
+    sh.symmetric = kSymWide;
     h->shape[precision] = sh;
     h->shape_chosen[precision] = true;
     return TFS_OK;
@@ -923,7 +970,7 @@ int tfs_rpy_set_symmetric(tfs_rpy* h, int32_t precision, int32_t enable) {
 int tfs_rpy_get_symmetric(tfs_rpy* h, int32_t precision, int32_t* enabled) {
     if (!h || !enabled || (precision != 0 && precision != 1))
         return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_get_symmetric: bad arguments");
-    *enabled = h->shape[precision].symmetric;
+    *enabled = h->shape[precision].symmetric ? 1 : 0;
     return TFS_OK;
 }
 
@@ -959,8 +1006,7 @@ int tfs_rpy_set_bodies(tfs_rpy* h, int32_t num_bodies, const int32_t* segs_per_b
     largest_body(h, &lns, &lnb);
     for (int pr = 0; pr < 2; ++pr)
         if (!h->shape_chosen[pr])
-            h->shape[pr] = preferred_shape(pr, lns, lnb, h->num_cus, h->desc.seg_dof, (int)h->bodies.size(),
-                                           sym_slot_count(h->bodies));
+            h->shape[pr] = preferred_shape(pr, lns, lnb, h->num_cus, h->desc.seg_dof, h->bodies);
     return TFS_OK;
 }
 
@@ -982,6 +1028,7 @@ int tfs_rpy_graph_create(tfs_rpy* h, uint32_t blocks, int32_t evaluations, tfs_g
     if (e != hipSuccess) return hip_fail(e, "tfs_rpy_graph_create: warm-up");
     const bool prof = h->profiling;
     h->profiling = false;
+    h->graph_made = true;
     tfs_graph* g = new tfs_graph();
     g->stream = h->stream;
     e = hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal);
@@ -1041,6 +1088,8 @@ int tfs_rpy_autotune(tfs_rpy* h, int32_t precision, uint32_t blocks, int32_t rep
     int ns = 0, nb = 0;
     largest_body(h, &ns, &nb);
     const double pairs = double(ns + nb) * double(ns + nb);
+    h->sym_pick[precision] = 0;
+    int best_pick = 0;
     auto time_shape = [&](const TileShape& sh) {
         h->shape[precision] = sh;
         rc = tfs_rpy_evaluate(h, blocks);  // builds the plan; warm-up
@@ -1055,12 +1104,24 @@ int tfs_rpy_autotune(tfs_rpy* h, int32_t precision, uint32_t blocks, int32_t rep
         if (ms / reps < best_t) {
             best_t = ms / reps;
             best = h->shape[precision];
+            best_pick = h->sym_pick[precision];
         }
     };
-    if (symmetric_applies(h, precision, blocks)) {
-        TileShape sym{256, 1, 0, 0, 0};
-        sym.symmetric = 1;
-        time_shape(sym);
+    // The symmetric form: as the shape of 3-DOF handles, behind the default
+    // shape of 6-DOF ones.
+    if (symmetric_applies(h, blocks) && sym_fits(h->bodies, kSymWide, h->desc.seg_dof)) {
+        if (h->desc.seg_dof == 3) {
+            TileShape sym{256, 1, 0, 0, 0};
+            sym.symmetric = kSymWide;
+            time_shape(sym);
+        } else {
+            for (int kind : {kSymWide, kSymNarrow}) {
+                if (rc || !sym_fits(h->bodies, kind, h->desc.seg_dof)) continue;
+                h->sym_pick[precision] = kind;
+                time_shape(default_shape(precision, ns, nb, h->num_cus, h->desc.seg_dof, (int)h->bodies.size()));
+            }
+            h->sym_pick[precision] = 0;
+        }
     }
     for (int cand = 0; cand < 8 && !rc; ++cand) {
         const int split = cand / 4, block = 64 << (cand % 4);
@@ -1095,6 +1156,7 @@ int tfs_rpy_autotune(tfs_rpy* h, int32_t precision, uint32_t blocks, int32_t rep
     h->desc.precision = saved_precision;
     h->shape[precision] = best;
     h->shape_chosen[precision] = true;
+    h->sym_pick[precision] = best_pick;
     if (best_ms) *best_ms = best_t;
     return rc;
 }
@@ -1113,6 +1175,7 @@ int tfs_rpy_set_persistent(tfs_rpy* h, int32_t precision, int32_t workgroups_per
         largest_body(h, &ns, &nb);
         h->shape[precision] = plain_shape(ns, nb, h->num_cus);
         h->shape_chosen[precision] = true;
+        h->sym_pick[precision] = 0;
     }
     h->shape[precision].persistent = workgroups_per_cu;
     return TFS_OK;
@@ -1161,11 +1224,10 @@ int tfs_rpy_body_times(tfs_rpy* h, double* ms_per_body) {
     const int nt = (int)p->tiles.size();
     for (size_t i = 0; i < ni; ++i) {
         if (p->symmetric) {
-            // an item pairs tile groups ga <= gb: the bodies both hold
-            const int ga = p->items[i].tile, gb = p->items[i].src_cls;
-            const int g = kSymGroupTiles;
-            const int lo = std::max(p->tiles[g * ga].body, p->tiles[g * gb].body);
-            const int hi = std::min(p->tiles[std::min(g * ga + g, nt) - 1].body, p->tiles[std::min(g * gb + g, nt) - 1].body);
+            // an item pairs a panel and a run of tiles: the bodies both hold
+            const int n = sym_panel(p->symmetric), pa = p->items[i].tile;
+            const int lo = std::max(p->tiles[n * pa].body, p->tiles[p->items[i].src_cls].body);
+            const int hi = std::min(p->tiles[std::min(n * pa + n, nt) - 1].body, p->tiles[p->items[i].s_begin - 1].body);
             for (int b = lo; b <= hi; ++b) done[b] = std::max(done[b], st[2 * i + 1]);
         } else {
             const int b = p->tiles[p->items[i].tile].body;
@@ -1520,7 +1582,7 @@ int tfs_rpy_apply_noalloc(const tfs_rpy_desc* desc, uint32_t blocks, const doubl
     o.blocks = eff;
     const TileShape sh{kStaticTile, 1, chunk, 0};
     PersistState ps;
-    e = launch_matvec(D.precision, D.seg_dof, sh, a, o, tiles, ts + tb, items, n_items,
+    e = launch_matvec(D.precision, D.seg_dof, sh, a, o, tiles, ts + tb, items, n_items, n_items,
                       reinterpret_cast<double*>(base + kOffPartial), near, ps, st);
     return e == hipSuccess ? TFS_OK : hip_fail(e, w);
 }
