@@ -1,0 +1,121 @@
+"""New positions: the fixed-point frame of FP32 tiles and the overlapping-pair
+lists against the FP64 oracle, from one particle on: particles by the hundred
+in one place (lists sorted from LDS, by rank and by insertion, capacities
+grown), independent bodies in the same place and bodies without particles, positions that are refused and the ones after
+them, lists rebuilt while an earlier capacity is in use.
+
+Tolerances: the matvec's bars, 1e-12 (FP64 sums of n terms in another order)
+and 1e-6 (FP32 tiles)."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+from timfilsimmod_amd import _lib as L
+from timfilsimmod_amd.mobility import RpyHandle
+
+pytestmark = pytest.mark.gpu
+
+P32, P64 = L.PRECISION_FP32_ACC64, L.PRECISION_FP64
+TOLS = {P32: 1e-6, P64: 1e-12}
+
+
+def rel(a, b):
+    return np.linalg.norm(a - b) / np.linalg.norm(b)
+
+
+def cloud(ns, nb, cluster, seed, centre=(0.0, 0.0, 0.0)):
+    """ns + nb particles at about one per 8 cubic radii, the first `cluster` of
+    the segments and of the blobs within one radius of the centre."""
+    rng = np.random.default_rng(seed)
+    box = (ns + nb) ** (1 / 3) + 2.0
+    c = np.asarray(centre)
+    xs, xb = rng.uniform(-box, box, (ns, 3)) + c, rng.uniform(-box, box, (nb, 3)) + c
+    for x in (xs, xb):
+        m = min(cluster, len(x))
+        x[:m] = rng.uniform(-0.55, 0.55, (m, 3)) + c
+    return xs.ravel(), xb.ravel(), rng.normal(size=6 * ns), rng.normal(size=3 * nb)
+
+
+def evaluate(h, ns, nb, xs, xb, fs, fb):
+    for what, a in ((L.SEG_POSITIONS, xs), (L.BLOB_POSITIONS, xb), (L.SEG_FORCES, fs), (L.BLOB_FORCES, fb)):
+        if a.size:
+            h.upload(what, a)
+    h.evaluate()
+    vs, vb = np.zeros(6 * ns), np.zeros(3 * nb)
+    if ns:
+        h.download(L.SEG_VELOCITIES, vs)
+    if nb:
+        h.download(L.BLOB_VELOCITIES, vb)
+    h.sync()
+    return np.concatenate([vs, vb])
+
+
+def oracle_all(xs, xb, fs, fb):
+    return np.concatenate(O.full_mobility(xs, xb, fs, fb, seg_dof=6, bs_accumulate=True, a_seg=1.0, a_blob=1.2))
+
+
+def handle(ns, nb, precision):
+    return RpyHandle(ns, nb, seg_dof=6, precision=precision, bs_accumulate=True, seg_radius=1.0, blob_radius=1.2)
+
+
+@pytest.mark.parametrize("precision", [P32, P64])
+@pytest.mark.parametrize("ns,nb,cluster", [(1, 0, 0), (0, 3, 2), (130, 71, 20), (700, 500, 170), (511, 1, 30),
+                                           (6100, 45, 30), (3300, 3100, 60), (4000, 2600, 170)])
+def test_sizes_and_clusters(ns, nb, cluster, precision):
+    print(f"case ns={ns} nb={nb} cluster={cluster} precision={precision}", flush=True)
+    h = handle(ns, nb, precision)
+    try:
+        for k, m in enumerate((0, cluster, 3)):      # grown capacities stay for the lists after them
+            case = cloud(ns, nb, m, 7 * ns + nb + k)
+            err = rel(evaluate(h, ns, nb, *case), oracle_all(*case))
+            print(f"  cluster {m}: rel err {err:.2e}", flush=True)
+            assert err <= TOLS[precision]
+    finally:
+        h.close()
+
+
+@pytest.mark.parametrize("precision", [P32, P64])
+@pytest.mark.parametrize("sizes", [[(40, 30), (0, 0), (1, 0), (0, 129), (300, 200)],
+                                   [(2000, 900), (0, 0), (1300, 1700), (40, 900)], [(3, 2)] * 300])
+def test_bodies_in_one_place(sizes, precision):
+    print(f"case bodies={len(sizes)} precision={precision}", flush=True)
+    cases = [cloud(ns, nb, 5, 11 + b, (0.3 * b, 0.0, 0.0)) for b, (ns, nb) in enumerate(sizes)]
+    ns, nb = sum(s for s, _ in sizes), sum(b for _, b in sizes)
+    h = handle(ns, nb, precision)
+    try:
+        h.set_bodies([s for s, _ in sizes], [b for _, b in sizes])
+        got = evaluate(h, ns, nb, *(np.concatenate([c[k] for c in cases]) for k in range(4)))
+        parts = [oracle_all(*c) if c[0].size + c[1].size else np.zeros(0) for c in cases]
+        want = np.concatenate([p[:6 * s] for p, (s, _) in zip(parts, sizes)] +
+                              [p[6 * s:] for p, (s, _) in zip(parts, sizes)])
+        err = rel(got, want)
+        print(f"  rel err {err:.2e}", flush=True)
+        assert err <= TOLS[precision]
+    finally:
+        h.close()
+
+
+@pytest.mark.parametrize("ns,nb", [(200, 100), (5000, 1500)])
+def test_refused_positions_and_the_ones_after_them(ns, nb):
+    print(f"case ns={ns} nb={nb}", flush=True)
+    xs, xb, fs, fb = cloud(ns, nb, 4, 5)
+    h = handle(ns, nb, P32)
+    try:
+        want = oracle_all(xs, xb, fs, fb)
+        assert rel(evaluate(h, ns, nb, xs, xb, fs, fb), want) <= TOLS[P32]
+        for value, where in ((np.nan, 0), (np.inf, 3 * ns - 1), (-1.1e4, 4), (1e308, 7)):
+            bad = xs.copy()
+            bad[where] = value
+            with pytest.raises(Exception) as err:
+                evaluate(h, ns, nb, bad, xb, fs, fb)
+            assert ("finite" if not np.isfinite(value) else "1024") in str(err.value)
+            assert rel(evaluate(h, ns, nb, xs, xb, fs, fb), want) <= TOLS[P32]
+    finally:
+        h.close()
+    # the frame far from the origin: the centre goes, the step stays
+    far = xs + 1e5
+    h = handle(ns, nb, P32)
+    try:
+        assert rel(evaluate(h, ns, nb, far, xb + 1e5, fs, fb), oracle_all(far, xb + 1e5, fs, fb)) <= TOLS[P32]
+    finally:
+        h.close()

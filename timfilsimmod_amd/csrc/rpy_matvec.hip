@@ -176,7 +176,7 @@ __device__ __forceinline__ void accumulate_item(const MatvecItem it, const Matve
     const double ai = tl.cls == 0 ? a.a_seg : a.a_blob;
     const double aj = it.src_cls == 0 ? a.a_seg : a.a_blob;
     const double PI = 3.14159265358979323846;
-    const double lam = F32 ? a.lam : 1.0;
+    const double lam = F32 ? *a.lam : 1.0;
     const T sum_a2 = T(lam * lam * ((ai + aj) * (ai + aj)));
     const T s3 = T(lam * lam * ((ai * ai + aj * aj) / 3.0));
     // -3 s3 as its own value (a negated operand would force the VOP3 form of the fma)
@@ -287,7 +287,7 @@ __device__ __forceinline__ void run_item(const MatvecItem it, const MatvecTile t
         combine_waves<VT, BLOCK, R, VT>(acc, reinterpret_cast<double*>(lds));
         if (threadIdx.x >= 64) return;
     }
-    store_slot<VT, T, LANES, R, VT>(slot, acc, sizeof(T) == 4 ? a.lam : 1.0);
+    store_slot<VT, T, LANES, R, VT>(slot, acc, sizeof(T) == 4 ? *a.lam : 1.0);
 }
 
 // One workgroup per item.  With `stamps`, thread 0 stores the item's start
@@ -481,9 +481,10 @@ template <typename T>
 __device__ __forceinline__ void sym_scale(const MatvecArgs& a, double& force, double& torque, double& rot) {
     const double c8 = 1.0 / (8.0 * 3.14159265358979323846 * a.mu);
     if constexpr (sizeof(T) == 4) {
-        force = a.lam * c8;
-        torque = a.lam * a.lam * c8;
-        rot = a.lam;
+        const double lam = *a.lam;
+        force = lam * c8;
+        torque = lam * lam * c8;
+        rot = lam;
     } else {
         force = 0.5 * c8;
         torque = 0.125 * c8;
@@ -750,7 +751,7 @@ __global__ __launch_bounds__(64 * kSymWaves, (sym_min_waves<T, DOF, R>())) void 
             return;
         }
     }
-    const double lam = F32 ? a.lam : 1.0;
+    const double lam = F32 ? *a.lam : 1.0;
     double fsc, tsc, rot;
     sym_scale<T>(a, fsc, tsc, rot);
     T neg = T(-1);
@@ -896,7 +897,7 @@ __device__ void run_item_wall(const MatvecItem it, const MatvecTile tl, const Ma
     if constexpr (F32) load_target(a, tl.cls, t, Xi);
     else load_target(a, tl.cls, t, xi);
     const T zi = T(zi_d);
-    const T inv_lam = T(F32 ? 1.0 / a.lam : 1.0);
+    const T inv_lam = T(F32 ? 1.0 / *a.lam : 1.0);
     const int tg = (tl.cls == 0 ? 0 : a.ns) + t;
     const int src_base = it.src_cls == 0 ? 0 : a.ns;
     const CView xsrc = it.src_cls == 0 ? a.xs : a.xb;
@@ -988,7 +989,7 @@ __global__ __launch_bounds__(BLOCK) void rpy_pairs_persistent_kernel(const Matve
     if (a.skip && *a.skip) return;
     const int i0 = blockIdx.x * k;
     const int i1 = i0 + k < n_items ? i0 + k : n_items;
-    const double lam = sizeof(T) == 4 ? a.lam : 1.0;
+    const double lam = sizeof(T) == 4 ? *a.lam : 1.0;
     TargetT<T> xi[R][3];
     double acc[R][SEGDOF];
     int cur = -1, cur_cls = 0, seg = 0;
@@ -1029,14 +1030,24 @@ __global__ __launch_bounds__(BLOCK) void rpy_pairs_persistent_kernel(const Matve
 }
 
 // ---------------------------------------------------------------------------
-// Near-pair listing on a hashed uniform grid.  Cells have side h >= (1 + 1e-5)
-// max(ai + aj), so every pair that either arithmetic (FP64, or FP32 fixed
-// point, whose r^2 errs by well under 1e-5 relative) could classify as
-// overlapping lies in neighbouring cells; each candidate is then classified
-// with the pair kernel's own staging and separation functions for the
-// requested precision, so the lists and the pair loop's clamp agree bit for
-// bit.  One thread per target, entries appended in visiting order (the
-// reduce kernel's order comes from near_sort_kernel).
+// New positions: the fixed-point frame of FP32 tiles and the near-pair lists.
+//
+// Bound by the launches and the round trips to the host between them, not by
+// the particles: three launches (clear + bounding boxes, place, list) and one
+// read-back that the caller takes while the pair kernel runs.  What new
+// positions add to an FP32 evaluation, two uploads included: 30 us for one body
+// of 12,800 + 9,000 particles and 74 us for twelve of 1,000-29,000 (164 and 620
+// with one workgroup per body for the boxes and the conversion, the frame
+// computed on the host, and a counting sort with a one-workgroup scan for the
+// cells).  Small problems take the same path: testing every pair instead (bit
+// masks) was 26 against 45 us at 5,794 particles and no faster at 64.
+//
+// Cells have side h >= (1 + 1e-5) max(ai + aj), so every pair that either
+// arithmetic (FP64, or FP32 fixed point, whose r^2 errs by well under 1e-5
+// relative) could classify as overlapping lies in neighbouring cells; each
+// candidate is then classified with the pair kernel's own staging and
+// separation functions for the requested precision, so the lists and the pair
+// loop's clamp agree bit for bit.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void particle_pos(const MatvecArgs& a, int p, double* x) {
     const CView v = p < a.ns ? a.xs : a.xb;
@@ -1052,13 +1063,6 @@ __device__ __forceinline__ int cell_coord(double x, double inv_h) {
 
 __device__ __forceinline__ uint32_t cell_hash(int cx, int cy, int cz, uint32_t mask) {
     return ((uint32_t)cx * 73856093u ^ (uint32_t)cy * 19349663u ^ (uint32_t)cz * 83492791u) & mask;
-}
-
-__global__ __launch_bounds__(256) void grid_body_kernel(const int4* __restrict__ ranges, int ns,
-                                                       int32_t* __restrict__ body_of) {
-    const int4 r = ranges[blockIdx.x];
-    for (int i = r.x + threadIdx.x; i < r.y; i += 256) body_of[i] = blockIdx.x;
-    for (int i = r.z + threadIdx.x; i < r.w; i += 256) body_of[ns + i] = blockIdx.x;
 }
 
 __global__ __launch_bounds__(256) void grid_count_kernel(MatvecArgs a, int n, double inv_h, uint32_t mask,
@@ -1173,138 +1177,278 @@ __global__ __launch_bounds__(256) void grid_sort_buckets_kernel(int table, const
     }
 }
 
+// Particle t of body range r (its segments, then its blobs).
+__device__ __forceinline__ int body_particle(const int4& r, int ns, int t) {
+    const int segs = r.y - r.x;
+    return t < segs ? r.x + t : ns + r.z + (t - segs);
+}
+
+// Bucket of a cell of one body: bodies that overlap in space (independent
+// bodies solved together) keep to buckets of their own.
+__device__ __forceinline__ uint32_t body_cell_hash(int cx, int cy, int cz, int body, uint32_t mask) {
+    return cell_hash((int)((uint32_t)cx + (uint32_t)body * 2654435761u), cy, cz, mask);
+}
+
+// Empties the grid (head, table entries, may be null), clears *max_cnt and,
+// with BOX, writes box[blockIdx.y gridDim.x + blockIdx.x]: the bounds (min
+// xyz, max xyz) of the workgroup's share of body blockIdx.y, NaN if any of its
+// coordinates is not finite.  Workgroups of 256.
+template <bool BOX>
+__global__ __launch_bounds__(256) void geometry_clear_kernel(MatvecArgs a, const int4* __restrict__ ranges,
+                                                            double* __restrict__ box, int32_t* __restrict__ head,
+                                                            int table, int32_t* __restrict__ max_cnt) {
+    const int tid = (int)threadIdx.x;
+    const int block = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+    if (head)
+        for (int i = (block * 256 + tid) * 4; i < table; i += (int)(gridDim.x * gridDim.y) * 1024)
+            *reinterpret_cast<int4*>(head + i) = make_int4(-1, -1, -1, -1);
+    if (block == 0 && tid == 0) *max_cnt = 0;
+    if constexpr (BOX) {
+        __shared__ double red[4][6];
+        const int4 r = ranges[blockIdx.y];
+        const int m = (r.y - r.x) + (r.w - r.z);
+        double lo[3] = {__builtin_inf(), __builtin_inf(), __builtin_inf()};
+        double hi[3] = {-__builtin_inf(), -__builtin_inf(), -__builtin_inf()};
+        bool bad = false;
+        for (int t = (int)blockIdx.x * 256 + tid; t < m; t += (int)gridDim.x * 256) {
+            double x[3];
+            particle_pos(a, body_particle(r, a.ns, t), x);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                bad |= !__builtin_isfinite(x[k]);
+                lo[k] = __builtin_fmin(lo[k], x[k]);
+                hi[k] = __builtin_fmax(hi[k], x[k]);
+            }
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                lo[k] = __builtin_fmin(lo[k], __shfl_xor(lo[k], off, 64));
+                hi[k] = __builtin_fmax(hi[k], __shfl_xor(hi[k], off, 64));
+            }
+        if ((tid & 63) == 0)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                red[tid >> 6][k] = lo[k];
+                red[tid >> 6][3 + k] = hi[k];
+            }
+        const bool any_bad = __syncthreads_or(bad);
+        if (tid < 6) {
+            double v = red[0][tid];
+            for (int w = 1; w < 4; ++w) v = tid < 3 ? __builtin_fmin(v, red[w][tid]) : __builtin_fmax(v, red[w][tid]);
+            box[6 * (int64_t)block + tid] = any_bad ? __builtin_nan("") : v;
+        }
+    }
+}
+
+// The fixed-point frame of the bodies' boxes (`shares` per body): each body is
+// centred on its bounding box; lambda = 2^k is the largest power of two with
+// lambda * (largest half-extent) <= 2^30 - 2, so every coordinate and every
+// difference of two fits an int32, and lambda amin < 2^40, so that the third
+// power of 1/r at the clamp r = ai + aj is no denormal float (a particle on
+// its own, bodies of coincident particles).  Returns lambda, 0
+// with *status set where the positions are not finite or the step 1/lambda is
+// not below 2^-19 amin, and the centre of body `own`.  Every workgroup of the
+// launch works it out for itself from the few hundred boxes.
+__device__ double fixed_frame(const double* __restrict__ box, int nbody, int shares, int own, double amin,
+                              double* centre, int* status) {
+    __shared__ double wave_ext[4], own_centre[3];
+    const int tid = (int)threadIdx.x;
+    int width = 1;  // lanes per body
+    while (width < shares && width < 64) width <<= 1;
+    double ext = 0.0;
+    bool bad = false;
+    for (int b = tid / width; b < nbody; b += 256 / width) {
+        double lo[3] = {__builtin_inf(), __builtin_inf(), __builtin_inf()};
+        double hi[3] = {-__builtin_inf(), -__builtin_inf(), -__builtin_inf()};
+        for (int g = tid % width; g < shares; g += width) {
+            const double* q = box + 6 * ((int64_t)b * shares + g);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                bad |= q[k] != q[k];
+                lo[k] = __builtin_fmin(lo[k], q[k]);
+                hi[k] = __builtin_fmax(hi[k], q[3 + k]);
+            }
+        }
+        for (int off = width >> 1; off > 0; off >>= 1)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                lo[k] = __builtin_fmin(lo[k], __shfl_xor(lo[k], off, width));
+                hi[k] = __builtin_fmax(hi[k], __shfl_xor(hi[k], off, width));
+            }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const bool some = lo[k] <= hi[k];  // a body without particles has no box
+            const double c = some ? 0.5 * (lo[k] + hi[k]) : 0.0;
+            ext = some ? __builtin_fmax(ext, __builtin_fmax(hi[k] - c, c - lo[k])) : ext;
+            if (b == own && tid % width == 0) own_centre[k] = c;
+        }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) ext = __builtin_fmax(ext, __shfl_xor(ext, off, 64));
+    if ((tid & 63) == 0) wave_ext[tid >> 6] = ext;
+    const bool any_bad = __syncthreads_or(bad);
+    for (int w = 0; w < 4; ++w) ext = __builtin_fmax(ext, wave_ext[w]);
+    for (int k = 0; k < 3; ++k) centre[k] = own_centre[k];
+    *status = any_bad ? kFrameNonFinite : ext < 1e300 ? 0 : kFrameTooLarge;
+    if (*status) return 0.0;
+    int k = 1000;
+    if (ext > 0.0) {
+        int e;
+        const double m = frexp(ext, &e);  // ext = m 2^e, 1/2 <= m < 1
+        k = m <= 1073741822.0 / 1073741824.0 ? 30 - e : 29 - e;
+    }
+    int ea;
+    (void)frexp(amin, &ea);
+    k = k < 40 - ea ? k : 40 - ea;
+    if (ldexp(1.0, -k) > ldexp(amin, -19)) {
+        *status = kFrameTooLarge;
+        return 0.0;
+    }
+    return ldexp(1.0, k);
+}
+
+// FIXED: X = rint(lambda (x - c_body)) of every particle, and the frame.
+// head not null: every particle into the grid, each bucket a list linked
+// through nodes[p] = (cell, next particle or -1), newest first (the order
+// varies between runs; near_grid_kernel sorts what it finds).  body_of (may be
+// null) gets each particle's body.  Grid (workgroups per body, bodies).
+template <bool FIXED>
+__global__ __launch_bounds__(256) void geometry_place_kernel(MatvecArgs a, const int4* __restrict__ ranges,
+                                                            const double* __restrict__ box, int shares, double amin,
+                                                            int4* __restrict__ fixed, GeomFrame* __restrict__ frame,
+                                                            double inv_h, uint32_t mask, int32_t* __restrict__ head,
+                                                            int4* __restrict__ nodes, int32_t* __restrict__ body_of) {
+    const int body = (int)blockIdx.y;
+    const int4 r = ranges[body];
+    const int m = (r.y - r.x) + (r.w - r.z);
+    double centre[3] = {0.0, 0.0, 0.0}, lam = 0.0;
+    if constexpr (FIXED) {
+        int status;
+        lam = fixed_frame(box, (int)gridDim.y, shares, body, amin, centre, &status);
+        if (blockIdx.x == 0 && body == 0 && threadIdx.x == 0) {
+            frame->lam = lam;
+            frame->status = status;
+        }
+        if (status) return;  // the same in every workgroup
+    }
+    for (int t = (int)(blockIdx.x * 256 + threadIdx.x); t < m; t += (int)gridDim.x * 256) {
+        const int p = body_particle(r, a.ns, t);
+        double x[3];
+        particle_pos(a, p, x);
+        if constexpr (FIXED)
+            fixed[p] = make_int4((int)__builtin_rint((x[0] - centre[0]) * lam),
+                                 (int)__builtin_rint((x[1] - centre[1]) * lam),
+                                 (int)__builtin_rint((x[2] - centre[2]) * lam), 0);
+        if (body_of) body_of[p] = body;
+        if (head) {
+            const int cx = cell_coord(x[0], inv_h), cy = cell_coord(x[1], inv_h), cz = cell_coord(x[2], inv_h);
+            const int32_t next = atomicExch(head + body_cell_hash(cx, cy, cz, body, mask), p);
+            nodes[p] = make_int4(cx, cy, cz, next);
+        }
+    }
+}
+
+// 32 lanes per target, lane l < 27 visiting neighbour cell l; the near sources
+// are appended in any order and then put into increasing order by rank (the
+// entries are distinct), from LDS for up to 64 of them, so the lists are the
+// same on every run.  cnt is the full count, entries past cap are dropped and
+// *max_cnt gets any count above cap.
+constexpr int kNearLds = 64, kRankPer = 8;
 template <typename T>
 __global__ __launch_bounds__(256) void near_grid_kernel(MatvecArgs a, int n, double inv_h, uint32_t mask,
-                                                       const int32_t* __restrict__ start,
-                                                       const int32_t* __restrict__ order,
-                                                       const int32_t* __restrict__ body_of,
-                                                       int32_t* __restrict__ cnt, int32_t* __restrict__ idx,
-                                                       int cap) {
-    // 32 lanes per target, lane l < 27 visiting neighbour cell l; near sources
-    // are appended in any order (near_rank_sort_kernel orders them).  cnt must
-    // start at zero and ends as the full count, entries past cap dropped.
+                                                       const int32_t* __restrict__ head,
+                                                       const int4* __restrict__ nodes,
+                                                       const int32_t* __restrict__ body_of, int32_t* __restrict__ cnt,
+                                                       int32_t* idx, int cap, int32_t* __restrict__ max_cnt) {
     constexpr bool F32 = sizeof(T) == 4;
     constexpr int REC = rec_len<T, 3>();
-    const int tg = blockIdx.x * 8 + (int)(threadIdx.x >> 5);
+    __shared__ int32_t found[8];
+    __shared__ int32_t list[8][kNearLds + 1];
+    const int s = (int)(threadIdx.x >> 5);
+    const int tg = (int)blockIdx.x * 8 + s;
     const int lane = (int)(threadIdx.x & 31);
-    if (tg >= n || lane >= 27) return;
-    const int cls = tg < a.ns ? 0 : 1;
-    const int t = cls == 0 ? tg : tg - a.ns;
-    using XT = typename std::conditional<F32, int32_t, double>::type;
-    XT xi[3];
-    load_target(a, cls, t, xi);
-    double xd[3];
-    particle_pos(a, tg, xd);
-    const int nx = cell_coord(xd[0], inv_h) + lane % 3 - 1;
-    const int ny = cell_coord(xd[1], inv_h) + (lane / 3) % 3 - 1;
-    const int nz = cell_coord(xd[2], inv_h) + lane / 9 - 1;
-    const int body = body_of[tg];
-    const double ai = cls == 0 ? a.a_seg : a.a_blob;
-    const double lam = F32 ? a.lam : 1.0;
-    const uint32_t b = cell_hash(nx, ny, nz, mask);
-    for (int q = start[b]; q < start[b + 1]; ++q) {
-        const int j = order[q];
-        if (body_of[j] != body) continue;
-        double xj[3];
-        particle_pos(a, j, xj);
-        // the bucket may also hold other cells: visit j from its own cell only
-        if (cell_coord(xj[0], inv_h) != nx || cell_coord(xj[1], inv_h) != ny || cell_coord(xj[2], inv_h) != nz)
-            continue;
-        const int jcls = j < a.ns ? 0 : 1;
-        T rec[REC];
-        stage_source<T, 3>(rec, a, jcls, jcls == 0 ? j : j - a.ns, false);
-        const double aj = jcls == 0 ? a.a_seg : a.a_blob;
-        const T sum_a2 = T(lam * lam * ((ai + aj) * (ai + aj)));
-        T ddx, ddy, ddz;
-        const T r2 = separation(xi, rec, ddx, ddy, ddz);
-        if (!(r2 > sum_a2)) {
-            const int k = atomicAdd(cnt + tg, 1);
-            if (k < cap) idx[(int64_t)tg * cap + k] = j;
+    const double lam = F32 ? *a.lam : 1.0;
+    if (!(lam > 0.0)) return;  // no frame: uniform over the launch
+    if (threadIdx.x < 8) found[threadIdx.x] = 0;
+    __syncthreads();
+    int32_t* e = idx + (int64_t)tg * cap;
+    if (tg < n && lane < 27) {
+        const int cls = tg < a.ns ? 0 : 1;
+        using XT = typename std::conditional<F32, int32_t, double>::type;
+        XT xi[3];
+        load_target(a, cls, cls == 0 ? tg : tg - a.ns, xi);
+        const int4 own = nodes[tg];
+        const int nx = own.x + lane % 3 - 1, ny = own.y + (lane / 3) % 3 - 1, nz = own.z + lane / 9 - 1;
+        const int body = body_of ? body_of[tg] : 0;
+        const double ai = cls == 0 ? a.a_seg : a.a_blob;
+        const T sum_seg = T(lam * lam * ((ai + a.a_seg) * (ai + a.a_seg)));
+        const T sum_blob = T(lam * lam * ((ai + a.a_blob) * (ai + a.a_blob)));
+        for (int j = head[body_cell_hash(nx, ny, nz, body, mask)]; j >= 0;) {
+            const int4 nd = nodes[j];
+            // the bucket may also hold other cells (and bodies): visit j from its own only
+            if (nd.x == nx && nd.y == ny && nd.z == nz && (!body_of || body_of[j] == body)) {
+                const int jcls = j < a.ns ? 0 : 1;
+                T rec[REC];
+                stage_source<T, 3>(rec, a, jcls, jcls == 0 ? j : j - a.ns, false);
+                T ddx, ddy, ddz;
+                const T r2 = separation(xi, rec, ddx, ddy, ddz);
+                if (!(r2 > (jcls == 0 ? sum_seg : sum_blob))) {
+                    const int k = atomicAdd(&found[s], 1);
+                    if (k < kNearLds) list[s][k] = j;
+                    if (k < cap) e[k] = j;
+                }
+            }
+            j = nd.w;
         }
-    }
-}
-
-// All pairs, for problems of a few thousand particles: one wave per 64
-// targets x 64 sources sets bit k of mask[c n + t] when source 64 c + k
-// overlaps target t, classified exactly as near_grid_kernel does (the pair
-// kernel's staging and separation, the same r^2 bound); body_of null: one
-// body.  Workgroup (0, 0) clears max_cnt for near_emit_kernel.
-template <typename T>
-__global__ __launch_bounds__(64) void near_pairs_kernel(MatvecArgs a, int n, const int32_t* __restrict__ body_of,
-                                                       uint64_t* __restrict__ mask, int32_t* __restrict__ max_cnt) {
-    constexpr bool F32 = sizeof(T) == 4;
-    constexpr int REC = rec_len<T, 3>();
-    __shared__ __align__(16) T recs[64 * REC];
-    __shared__ int32_t sbody[64];
-    __shared__ int32_t scls[64];
-    const int lane = (int)threadIdx.x;
-    if (blockIdx.x == 0 && blockIdx.y == 0 && lane == 0) *max_cnt = 0;
-    const int j0 = (int)blockIdx.y * 64;
-    const int jl = j0 + lane;
-    if (jl < n) {
-        const int jcls = jl < a.ns ? 0 : 1;
-        stage_source<T, 3>(recs + lane * REC, a, jcls, jcls == 0 ? jl : jl - a.ns, false);
-        sbody[lane] = body_of ? body_of[jl] : 0;
-        scls[lane] = jcls;
     }
     __syncthreads();
-    const int tg = (int)blockIdx.x * 64 + lane;
-    if (tg >= n) return;
-    const int cls = tg < a.ns ? 0 : 1;
-    using XT = typename std::conditional<F32, int32_t, double>::type;
-    XT xi[3];
-    load_target(a, cls, cls == 0 ? tg : tg - a.ns, xi);
-    const int body = body_of ? body_of[tg] : 0;
-    const double ai = cls == 0 ? a.a_seg : a.a_blob;
-    const double lam = F32 ? a.lam : 1.0;
-    const T sum_seg = T(lam * lam * ((ai + a.a_seg) * (ai + a.a_seg)));
-    const T sum_blob = T(lam * lam * ((ai + a.a_blob) * (ai + a.a_blob)));
-    const int m = n - j0 < 64 ? n - j0 : 64;
-    uint64_t bits = 0;
-#pragma unroll 8
-    for (int k = 0; k < m; ++k) {
-        T ddx, ddy, ddz;
-        const T r2 = separation(xi, recs + k * REC, ddx, ddy, ddz);
-        const bool near = !(r2 > (scls[k] == 0 ? sum_seg : sum_blob)) && sbody[k] == body;
-        bits |= near ? uint64_t(1) << k : uint64_t(0);
+    const int total = tg < n ? found[s] : 0;
+    if (tg < n && lane == 0) {
+        cnt[tg] = total;
+        if (total > cap) atomicMax(max_cnt, total);
     }
-    mask[(int64_t)blockIdx.y * n + tg] = bits;
-}
-
-// One wave per target: lane q takes the masks of chunks q, q + 64, ...; an
-// exclusive scan of the lanes' bit counts places each lane's sources, so the
-// list comes out in increasing source order (entries past cap dropped, cnt
-// the full count, max_cnt the largest count past cap).
-__global__ __launch_bounds__(256) void near_emit_kernel(const uint64_t* __restrict__ mask, int n, int nchunk,
-                                                       int32_t* __restrict__ cnt, int32_t* __restrict__ idx, int cap,
-                                                       int32_t* __restrict__ max_cnt) {
-    const int tg = (int)blockIdx.x * 4 + ((int)threadIdx.x >> 6);
-    const int lane = (int)threadIdx.x & 63;
-    if (tg >= n) return;  // uniform over the wave
-    int32_t* e = idx + (int64_t)tg * cap;
-    int base = 0;
-    for (int q0 = 0; q0 < nchunk; q0 += 64) {
-        const int q = q0 + lane;
-        uint64_t b = q < nchunk ? mask[(int64_t)q * n + tg] : uint64_t(0);
-        const int pc = __popcll(b);
-        int incl = pc;  // inclusive scan over the wave
+    const int c = total < cap ? total : cap;
+    if (total <= kNearLds) {
+        for (int i = lane; i < total; i += 32) {
+            const int32_t v = list[s][i];
+            int r = 0;
+            for (int j = 0; j < total; ++j) r += list[s][j] < v ? 1 : 0;
+            if (r < cap) e[r] = v;
+        }
+    }
+    if (!__syncthreads_or(total > kNearLds)) return;
+    // longer lists: ranked against what the barrier above made readable
+    int32_t val[kRankPer];
+    int rank[kRankPer];
 #pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int t = __shfl_up(incl, off, 64);
-            incl += lane >= off ? t : 0;
+    for (int q = 0; q < kRankPer; ++q) {
+        const int i = lane + 32 * q;
+        val[q] = 0;
+        rank[q] = -1;
+        if (total > kNearLds && c <= 32 * kRankPer && i < c) {
+            const int32_t v = e[i];
+            int r = 0;
+            for (int j = 0; j < c; ++j) r += e[j] < v ? 1 : 0;
+            val[q] = v;
+            rank[q] = r;
         }
-        int c = base + incl - pc;
-        while (b) {
-            const int k = __builtin_ctzll(b);
-            b &= b - 1;
-            if (c < cap) e[c] = q * 64 + k;
-            ++c;
-        }
-        base += __shfl(incl, 63, 64);
     }
-    if (lane == 0) {
-        cnt[tg] = base;
-        if (base > cap) atomicMax(max_cnt, base);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kRankPer; ++q)
+        if (rank[q] >= 0) e[rank[q]] = val[q];
+    if (total > kNearLds && c > 32 * kRankPer && lane == 0) {
+        for (int i = 1; i < c; ++i) {
+            const int32_t v = e[i];
+            int j = i - 1;
+            while (j >= 0 && e[j] > v) {
+                e[j + 1] = e[j];
+                --j;
+            }
+            e[j + 1] = v;
+        }
     }
 }
 
@@ -1554,64 +1698,6 @@ __global__ __launch_bounds__(64 * GR) void rpy_reduce_kernel(const MatvecTile* _
     }
 }
 
-// Sorts every target's near list into increasing source order, 32 lanes per
-// target: each lane ranks up to kRankPer entries against the whole list (the
-// entries are distinct source indices), then all write after a barrier.
-// Lists up to 32 kRankPer long; *max_cnt gets any count above cap.
-constexpr int kRankPer = 8;
-__global__ __launch_bounds__(256) void near_rank_sort_kernel(const int32_t* __restrict__ cnt,
-                                                             int32_t* __restrict__ idx, int cap, int64_t n,
-                                                             int32_t* __restrict__ max_cnt) {
-    const int64_t tg = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);
-    const int lane = (int)(threadIdx.x & 31);
-    int c = 0;
-    int32_t* e = idx;
-    if (tg < n) {
-        const int k = cnt[tg];
-        c = k < cap ? k : cap;
-        e = idx + tg * cap;
-        if (lane == 0 && k > cap) atomicMax(max_cnt, k);
-    }
-    int32_t val[kRankPer];
-    int rank[kRankPer];
-#pragma unroll
-    for (int s = 0; s < kRankPer; ++s) {
-        const int i = lane + 32 * s;
-        val[s] = 0;
-        rank[s] = -1;
-        if (i < c) {
-            const int32_t v = e[i];
-            int r = 0;
-            for (int j = 0; j < c; ++j) r += e[j] < v ? 1 : 0;
-            val[s] = v;
-            rank[s] = r;
-        }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int s = 0; s < kRankPer; ++s)
-        if (rank[s] >= 0) e[rank[s]] = val[s];
-}
-
-// The same for longer lists (insertion sort, one thread per target).
-__global__ __launch_bounds__(256) void near_sort_kernel(const int32_t* __restrict__ cnt, int32_t* __restrict__ idx,
-                                                        int cap, int64_t n, int32_t* __restrict__ max_cnt) {
-    const int64_t tg = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (tg >= n) return;
-    if (cnt[tg] > cap) atomicMax(max_cnt, cnt[tg]);
-    const int c = cnt[tg] < cap ? cnt[tg] : cap;
-    int32_t* e = idx + tg * cap;
-    for (int i = 1; i < c; ++i) {
-        const int32_t v = e[i];
-        int j = i - 1;
-        while (j >= 0 && e[j] > v) {
-            e[j + 1] = e[j];
-            --j;
-        }
-        e[j + 1] = v;
-    }
-}
-
 // Items per workgroup of the persistent form: the work list over
 // persistent x CUs workgroups, as contiguous ranges.
 int persistent_items(const TileShape& sh, int n_items, int num_cus) {
@@ -1831,28 +1917,32 @@ size_t build_sym_worklist(const std::vector<BodyRange>& bodies, int kind, int se
 }
 
 void free_grid(NearGrid& g) {
-    for (int32_t* p : {g.start, g.fill, g.bucket_of, g.order, g.body_of, g.pair_body})
+    for (int32_t* p : {g.start, g.fill, g.bucket_of, g.order, g.body_of})
         if (p) (void)hipFree(p);
-    if (g.mask) (void)hipFree(g.mask);
-    const bool may_alloc = g.may_alloc;
+    if (g.nodes) (void)hipFree(g.nodes);
     g = NearGrid{};
-    g.may_alloc = may_alloc;
+}
+
+// The grid's size for n particles; arrays made for another go.
+static void size_grid(NearGrid& grid, int n) {
+    int table = 1024;
+    while (table < 2 * n) table <<= 1;
+    if (grid.n == n && grid.table == table) return;
+    free_grid(grid);
+    grid.n = n;
+    grid.table = table;
 }
 
 // Sorts the n particles (segments, then blobs) into the grid's buckets for
 // cells of side 1 / inv_h: start (exclusive bucket offsets) and order.
 static hipError_t sort_into_grid(const MatvecArgs& a, NearGrid& grid, int n, double inv_h, hipStream_t stream) {
-    int table = 1024;
-    while (table < 2 * n) table <<= 1;
-    if (grid.n != n || grid.table != table) {
-        free_grid(grid);
-        TFS_HIP_CHECK(hipMalloc(&grid.start, sizeof(int32_t) * (table + 1)));
-        TFS_HIP_CHECK(hipMalloc(&grid.fill, sizeof(int32_t) * table));
-        TFS_HIP_CHECK(hipMalloc(&grid.bucket_of, sizeof(int32_t) * n));
+    size_grid(grid, n);
+    const int table = grid.table;
+    if (!grid.fill) TFS_HIP_CHECK(hipMalloc(&grid.fill, sizeof(int32_t) * table));
+    if (!grid.order) {
+        if (!grid.start) TFS_HIP_CHECK(hipMalloc(&grid.start, sizeof(int32_t) * (table + 1)));
+        if (!grid.bucket_of) TFS_HIP_CHECK(hipMalloc(&grid.bucket_of, sizeof(int32_t) * n));
         TFS_HIP_CHECK(hipMalloc(&grid.order, sizeof(int32_t) * n));
-        TFS_HIP_CHECK(hipMalloc(&grid.body_of, sizeof(int32_t) * n));
-        grid.n = n;
-        grid.table = table;
     }
     const uint32_t mask = (uint32_t)table - 1;
     const unsigned gn = (unsigned)((n + 255) / 256);
@@ -1867,82 +1957,64 @@ static hipError_t sort_into_grid(const MatvecArgs& a, NearGrid& grid, int n, dou
     return hipGetLastError();
 }
 
-hipError_t build_near_list(int precision, const MatvecArgs& a, NearGrid& grid, const int32_t* body_ranges, int nbody,
-                           NearList& near, int n_targets, int* max_count, int* host_scratch, hipStream_t stream) {
-    const int n = n_targets;
-    if (max_count) *max_count = 0;
+int box_shares(int nbody, int largest) {
+    const int fit = nbody < kBoxShares ? kBoxShares / nbody : 1;
+    return std::max(1, std::min(fit, (largest + 255) / 256));
+}
+
+// Clears (and with `fixed` the bounding boxes), then places: the fixed-point
+// positions and, with nodes, the grid.
+static void launch_geometry(const MatvecArgs& a, const GeometryArgs& g, bool fixed, NearGrid* grid, double inv_h,
+                            int32_t* max_cnt, hipStream_t stream) {
+    const int4* ranges = reinterpret_cast<const int4*>(g.ranges);
+    int32_t* head = grid ? grid->fill : nullptr;
+    const int table = grid ? grid->table : 0;
+    const int shares = box_shares(g.nbody, g.largest);
+    if (fixed)
+        hipLaunchKernelGGL(geometry_clear_kernel<true>, dim3((unsigned)shares, (unsigned)g.nbody), dim3(256), 0, stream,
+                           a, ranges, g.box, head, table, max_cnt);
+    else
+        hipLaunchKernelGGL(geometry_clear_kernel<false>, dim3((unsigned)std::max(1, table / 4096)), dim3(256), 0,
+                           stream, a, ranges, g.box, head, table, max_cnt);
+    const int per_body = std::max(1, std::min((g.largest + 255) / 256, std::max(1, 4096 / g.nbody)));
+    const dim3 place((unsigned)per_body, (unsigned)g.nbody);
+    const uint32_t mask = (uint32_t)table - 1;
+    int4* nodes = grid ? grid->nodes : nullptr;
+    int32_t* body_of = grid && g.nbody > 1 ? grid->body_of : nullptr;
+    if (fixed)
+        hipLaunchKernelGGL(geometry_place_kernel<true>, place, dim3(256), 0, stream, a, ranges, (const double*)g.box,
+                           shares, std::min(a.a_seg, a.a_blob), g.fixed, g.frame, inv_h, mask, head, nodes, body_of);
+    else
+        hipLaunchKernelGGL(geometry_place_kernel<false>, place, dim3(256), 0, stream, a, ranges, (const double*)g.box,
+                           shares, 0.0, g.fixed, g.frame, inv_h, mask, head, nodes, body_of);
+}
+
+hipError_t launch_fixed(const MatvecArgs& a, const GeometryArgs& g, hipStream_t stream) {
+    launch_geometry(a, g, true, nullptr, 0.0, &g.frame->max_cnt[1], stream);
+    return hipGetLastError();
+}
+
+hipError_t build_near_list(int precision, const MatvecArgs& a, const GeometryArgs& g, bool fixed, NearGrid& grid,
+                           const NearList& near, hipStream_t stream) {
+    const int n = a.ns + a.nb;
     if (n <= 0) return hipSuccess;
-    const int nchunk = (n + 63) / 64;
-    if (n <= kNearPairsMax && (grid.may_alloc || grid.mask_len >= (int64_t)nchunk * n)) {
-        if (grid.mask_len < (int64_t)nchunk * n) {
-            TFS_HIP_CHECK(hipStreamSynchronize(stream));
-            if (grid.mask) (void)hipFree(grid.mask);
-            grid.mask = nullptr;
-            grid.mask_len = 0;
-            TFS_HIP_CHECK(hipMalloc(&grid.mask, sizeof(uint64_t) * (size_t)nchunk * n));
-            grid.mask_len = (int64_t)nchunk * n;
-        }
-        const int32_t* body_of = nullptr;
-        if (nbody > 1) {
-            if (grid.pair_body_len < n) {
-                TFS_HIP_CHECK(hipStreamSynchronize(stream));
-                if (grid.pair_body) (void)hipFree(grid.pair_body);
-                grid.pair_body = nullptr;
-                grid.pair_body_len = 0;
-                TFS_HIP_CHECK(hipMalloc(&grid.pair_body, sizeof(int32_t) * n));
-                grid.pair_body_len = n;
-            }
-            hipLaunchKernelGGL(grid_body_kernel, dim3((unsigned)nbody), dim3(256), 0, stream,
-                               reinterpret_cast<const int4*>(body_ranges), a.ns, grid.pair_body);
-            body_of = grid.pair_body;
-        }
-        const dim3 g2((unsigned)nchunk, (unsigned)nchunk);
-        if (precision == 0)
-            hipLaunchKernelGGL(near_pairs_kernel<double>, g2, dim3(64), 0, stream, a, n, body_of, grid.mask,
-                               near.max_cnt);
-        else
-            hipLaunchKernelGGL(near_pairs_kernel<float>, g2, dim3(64), 0, stream, a, n, body_of, grid.mask,
-                               near.max_cnt);
-        hipLaunchKernelGGL(near_emit_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, stream,
-                           (const uint64_t*)grid.mask, n, nchunk, near.cnt, near.idx, near.cap, near.max_cnt);
-        TFS_HIP_CHECK(hipGetLastError());
-        if (!host_scratch) return hipSuccess;  // no capacity check wanted
-        TFS_HIP_CHECK(hipMemcpyAsync(host_scratch, near.max_cnt, sizeof(int32_t), hipMemcpyDeviceToHost, stream));
-        if (!max_count) return hipSuccess;
-        TFS_HIP_CHECK(hipStreamSynchronize(stream));
-        *max_count = *host_scratch;
-        return hipSuccess;
-    }
+    size_grid(grid, n);
+    if (!grid.fill) TFS_HIP_CHECK(hipMalloc(&grid.fill, sizeof(int32_t) * grid.table));
+    if (!grid.nodes) TFS_HIP_CHECK(hipMalloc(&grid.nodes, sizeof(int4) * n));
+    if (g.nbody > 1 && !grid.body_of) TFS_HIP_CHECK(hipMalloc(&grid.body_of, sizeof(int32_t) * n));
     const double h = 2.0 * std::max(a.a_seg, a.a_blob) * (1.0 + 1e-5);
     const double inv_h = 1.0 / h;
-    TFS_HIP_CHECK(sort_into_grid(a, grid, n, inv_h, stream));
+    launch_geometry(a, g, fixed, &grid, inv_h, near.max_cnt, stream);
     const uint32_t mask = (uint32_t)grid.table - 1;
-    const unsigned gn = (unsigned)((n + 255) / 256);
     const unsigned gl = (unsigned)((n + 7) / 8);   // 8 targets of 32 lanes per workgroup
-    hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, stream, near.max_cnt, 0, (int64_t)1);
-    hipLaunchKernelGGL(fill_int_kernel, dim3(gn), dim3(256), 0, stream, near.cnt, 0, (int64_t)n);
-    hipLaunchKernelGGL(grid_body_kernel, dim3((unsigned)nbody), dim3(256), 0, stream,
-                       reinterpret_cast<const int4*>(body_ranges), a.ns, grid.body_of);
+    const int32_t* body_of = g.nbody > 1 ? grid.body_of : nullptr;
     if (precision == 0)
-        hipLaunchKernelGGL(near_grid_kernel<double>, dim3(gl), dim3(256), 0, stream, a, n, inv_h, mask, grid.start,
-                           grid.order, grid.body_of, near.cnt, near.idx, near.cap);
+        hipLaunchKernelGGL(near_grid_kernel<double>, dim3(gl), dim3(256), 0, stream, a, n, inv_h, mask, grid.fill,
+                           grid.nodes, body_of, near.cnt, near.idx, near.cap, near.max_cnt);
     else
-        hipLaunchKernelGGL(near_grid_kernel<float>, dim3(gl), dim3(256), 0, stream, a, n, inv_h, mask, grid.start,
-                           grid.order, grid.body_of, near.cnt, near.idx, near.cap);
-    TFS_HIP_CHECK(hipGetLastError());
-    if (near.cap <= 32 * kRankPer)
-        hipLaunchKernelGGL(near_rank_sort_kernel, dim3(gl), dim3(256), 0, stream, near.cnt, near.idx, near.cap,
-                           (int64_t)n, near.max_cnt);
-    else
-        hipLaunchKernelGGL(near_sort_kernel, dim3(gn), dim3(256), 0, stream, near.cnt, near.idx, near.cap,
-                           (int64_t)n, near.max_cnt);
-    TFS_HIP_CHECK(hipGetLastError());
-    if (!host_scratch) return hipSuccess;  // no capacity check wanted
-    TFS_HIP_CHECK(hipMemcpyAsync(host_scratch, near.max_cnt, sizeof(int32_t), hipMemcpyDeviceToHost, stream));
-    if (!max_count) return hipSuccess;  // the caller reads host_scratch after its own wait
-    TFS_HIP_CHECK(hipStreamSynchronize(stream));
-    *max_count = *host_scratch;
-    return hipSuccess;
+        hipLaunchKernelGGL(near_grid_kernel<float>, dim3(gl), dim3(256), 0, stream, a, n, inv_h, mask, grid.fill,
+                           grid.nodes, body_of, near.cnt, near.idx, near.cap, near.max_cnt);
+    return hipGetLastError();
 }
 
 hipError_t launch_barrier(const MatvecArgs& a, NearGrid& grid, const BarrierParams& bp, double* fs, double* fb,
@@ -2001,11 +2073,10 @@ static hipError_t launch_reduce(int precision, int seg_dof, const MatvecArgs& a,
     return hipGetLastError();
 }
 
-hipError_t launch_matvec_wall(int precision, int seg_dof, const MatvecArgs& a, const OutArgs& o,
-                              const MatvecTile* d_tiles, int n_tiles, const MatvecItem* d_items, int n_items,
-                              double* partial, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end) {
-    if (n_tiles == 0) return hipSuccess;
-    if (n_items > 0) {
+hipError_t launch_wall_pairs(int precision, int seg_dof, const MatvecArgs& a, const MatvecTile* d_tiles, int n_tiles,
+                             const MatvecItem* d_items, int n_items, double* partial, hipStream_t stream,
+                             hipEvent_t ev_begin, hipEvent_t ev_end) {
+    if (n_tiles > 0 && n_items > 0) {
         float* pf = reinterpret_cast<float*>(partial);
         if (ev_begin) TFS_HIP_CHECK(hipEventRecord(ev_begin, stream));
         const dim3 grid((unsigned)n_items), block(kWallBlock);
@@ -2025,21 +2096,27 @@ hipError_t launch_matvec_wall(int precision, int seg_dof, const MatvecArgs& a, c
         TFS_HIP_CHECK(hipGetLastError());
         if (ev_end) TFS_HIP_CHECK(hipEventRecord(ev_end, stream));
     }
+    return hipSuccess;
+}
+
+hipError_t launch_wall_reduce(int precision, int seg_dof, const MatvecArgs& a, const OutArgs& o,
+                              const MatvecTile* d_tiles, int n_tiles, int n_items, const double* partial,
+                              hipStream_t stream) {
+    if (n_tiles == 0) return hipSuccess;
     return launch_reduce(precision, seg_dof, a, o, d_tiles, n_tiles, n_items, kWallBlock, 0, kMaxDof, partial, NearList{},
                          stream);
 }
 
-hipError_t launch_matvec(int precision, int seg_dof, const TileShape& shape, const MatvecArgs& a,
-                         const OutArgs& o, const MatvecTile* d_tiles, int n_tiles,
-                         const MatvecItem* d_items, int n_items, int n_slots, double* partial, const NearList& near,
-                         const PersistState& ps, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end) {
-    if (n_tiles == 0) return hipSuccess;
-    if (shape.symmetric && precision == 1 && !a.xfx) return hipErrorInvalidValue;
-    if (n_items > 0) {
+hipError_t launch_matvec_pairs(int precision, int seg_dof, const TileShape& shape, const MatvecArgs& a,
+                               uint32_t blocks, const MatvecTile* d_tiles, int n_tiles, const MatvecItem* d_items,
+                               int n_items, double* partial, const PersistState& ps, hipStream_t stream,
+                               hipEvent_t ev_begin, hipEvent_t ev_end) {
+    if (precision == 1 && (!a.xfx || !a.lam)) return hipErrorInvalidValue;
+    if (n_tiles > 0 && n_items > 0) {
         hipError_t e;
         if (ev_begin) TFS_HIP_CHECK(hipEventRecord(ev_begin, stream));
         if (shape.symmetric) {
-            const int bb = (o.blocks & 4u) ? 1 : 0;
+            const int bb = (blocks & 4u) ? 1 : 0;
             if (precision == 0)
                 e = seg_dof == 6 ? launch_sym<double, 6>(shape.symmetric, a, d_items, n_items, d_tiles, n_tiles, bb, partial, ps, stream)
                                  : launch_sym<double, 3>(shape.symmetric, a, d_items, n_items, d_tiles, n_tiles, bb, partial, ps, stream);
@@ -2056,6 +2133,14 @@ hipError_t launch_matvec(int precision, int seg_dof, const TileShape& shape, con
         if (e != hipSuccess) return e;
         if (ev_end) TFS_HIP_CHECK(hipEventRecord(ev_end, stream));
     }
+    return hipSuccess;
+}
+
+hipError_t launch_matvec_reduce(int precision, int seg_dof, const TileShape& shape, const MatvecArgs& a,
+                                const OutArgs& o, const MatvecTile* d_tiles, int n_tiles, int n_items, int n_slots,
+                                const double* partial, const NearList& near, const PersistState& ps,
+                                hipStream_t stream) {
+    if (n_tiles == 0) return hipSuccess;
     // The partial slots hold the evaluation type (FP32 sums for FP32 tiles);
     // the persistent form fills only its tile segments' first slots.
     const int merge_k = shape.persistent > 0 && n_items > 0 ? persistent_items(shape, n_items, ps.num_cus) : 0;

@@ -71,15 +71,15 @@ struct tfs_rpy {
     bool near_pending[2] = {false, false};
     tfs::NearGrid grid;
     int domain = 0;  // TFS_DOMAIN_UNBOUNDED or TFS_DOMAIN_HALF_SPACE
-    // Fixed-point positions for FP32 tiles (valid with the near lists):
-    // per-body centres c_b (bounding-box centres) and one lambda = 2^k.
+    // Fixed-point positions for FP32 tiles (valid with the near lists), their
+    // frame, and the event after its read-back into host_int[0..5].
     int4* x_fx = nullptr;
-    double fx_lambda = 1.0;
     bool fx_valid = false;
-    double* d_body_box = nullptr;    // 6 per body: min xyz, max xyz
+    tfs::GeomFrame* d_frame = nullptr;  // carved out of `arena`
+    hipEvent_t frame_read = nullptr;
+    double* d_body_box = nullptr;    // kBoxShares, or one per body: min xyz, max xyz
     int32_t* d_body_range = nullptr; // 4 per body (BodyRange), for the box and conversion kernels
     size_t body_cap = 0;
-    std::vector<double> fx_centre;   // 3 per body
     int32_t* host_int = nullptr;  // pinned scratch
     double* blob_rep = nullptr;   // device blob repulsion staging (tfs_rpy_barrier_forces, host memory)
     // Persistent launches with timing: per-item stamps of the last launch and

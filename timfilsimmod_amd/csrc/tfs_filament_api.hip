@@ -1793,9 +1793,9 @@ int tfs_elastic_step(tfs_elastic* e, int32_t nt, tfs_elastic_stats* stats) {
     defer.saved = rpyh->defer_near_check;
     rpyh->defer_near_check = true;
     // captured iterations are replayed several per wait when no near list can
-    // overflow: a capacity of every particle (all-pairs lists, small bodies)
+    // overflow: a capacity of every particle (small bodies)
     if (e->graphs && s_fil == s_vel && s_vel == s_bro && rpyh->desc.precision == TFS_PRECISION_FP64 &&
-        rpyh->desc.num_segs + rpyh->desc.num_blobs <= kNearPairsMax) {
+        rpyh->desc.num_segs + rpyh->desc.num_blobs <= kNearRoomyMax) {
         const int rc0 = tfs::rpy_near_reserve(rpyh, 0, rpyh->desc.num_segs + rpyh->desc.num_blobs);
         if (rc0) return rc0;
     }

@@ -60,29 +60,53 @@ struct MatvecTile {
 struct NearList {
     int32_t* cnt = nullptr;
     int32_t* idx = nullptr;
-    int32_t* max_cnt = nullptr;
+    int32_t* max_cnt = nullptr;  // in the handle's GeomFrame
     int cap = 0;
 };
 
-// Hashed uniform grid over every particle (segments, then blobs) that
-// build_near_list sorts the particles into: buckets of cells of side
-// >= max(ai + aj), a power-of-two table.  Device arrays, owned by the handle.
+// What the host reads back after new positions: the fixed-point scale lambda
+// (0 where there is no frame), why there is none, and per precision the
+// largest near-pair count past the lists' capacity (0: none is).  The pair
+// kernels read lambda where it is, so nothing waits for the read-back.
+constexpr int kFrameNonFinite = 1;  // a coordinate is not finite
+constexpr int kFrameTooLarge = 2;   // a body is too wide for FP32 tiles
+struct GeomFrame {
+    double lam;
+    int32_t status;
+    int32_t max_cnt[2];
+    int32_t pad;
+};
+
+// Hashed uniform grid over every particle (segments, then blobs): buckets of
+// cells of side >= max(ai + aj), a power-of-two table.  build_near_list links
+// the particles of a bucket, the barrier forces sort them.  Device arrays,
+// owned by the handle.
 struct NearGrid {
+    int32_t* fill = nullptr;       // table: per bucket the first particle, or a counter
+    int4* nodes = nullptr;         // n: cell of each particle, next particle of its bucket
     int32_t* start = nullptr;      // table + 1: first particle of each bucket in `order`
-    int32_t* fill = nullptr;       // table: per-bucket counters
     int32_t* bucket_of = nullptr;  // n
     int32_t* order = nullptr;      // n: particles by bucket
-    int32_t* body_of = nullptr;    // n: body index of each particle
+    int32_t* body_of = nullptr;    // n: body index of each particle (several bodies)
     int table = 0;
     int n = 0;
-    // Small problems (build_near_list's all-pairs form): overlap bit masks,
-    // 64 sources per word, and a body index per particle of its own.
-    uint64_t* mask = nullptr;
-    int64_t mask_len = 0;
-    int32_t* pair_body = nullptr;
-    int pair_body_len = 0;
-    bool may_alloc = false;        // the all-pairs form may allocate its buffers
 };
+
+// The bodies and buffers of a launch over new positions: BodyRange records and
+// the largest body's particle count, box_shares(nbody, largest) bounding boxes
+// per body (6 doubles each), the fixed-point positions (FP32 tiles).
+struct GeometryArgs {
+    const int32_t* ranges = nullptr;
+    int nbody = 1;
+    int largest = 0;
+    double* box = nullptr;
+    int4* fixed = nullptr;
+    GeomFrame* frame = nullptr;
+};
+// Workgroups per body that take bounding boxes: at most kBoxShares in all, or
+// one per body.
+constexpr int kBoxShares = 256;
+int box_shares(int nbody, int largest);
 
 // Barrier forces (cuda_functions.cu:1240-1436): strength
 // REPULSIVE_FORCE_FACTOR * END_FORCE_MAGNITUDE, NSEG for the neighbour
@@ -106,9 +130,9 @@ struct TileShape {
     int symmetric = 0;  // each pair once for both particles: kSymWide or kSymNarrow
 };
 
-// Up to this many particles the near-pair lists test every pair (bit masks of
-// n^2 / 8 bytes) instead of sorting the particles into a hashed grid.
-constexpr int kNearPairsMax = 6144;
+// Up to this many particles near-pair lists may be given room for every
+// particle (n^2 entries of 4 bytes), so that none can overflow.
+constexpr int kNearRoomyMax = 6144;
 
 // The symmetric form's kinds, two target particles per lane or one (bodies
 // where two would leave too few workgroups); the waves of its workgroups, and
@@ -142,9 +166,9 @@ struct MatvecArgs {
     // return at once (iterations a Krylov solver enqueued past convergence).
     const int32_t* skip = nullptr;
     // FP32 tiles: fixed-point positions X = rint(lambda (x - c_body)), segments
-    // then blobs (w unused), with lambda = 2^k and |X| < 2^30.
+    // then blobs (w unused), with *lam = lambda = 2^k and |X| < 2^30.
     const int4* xfx = nullptr;
-    double lam = 1.0;
+    const double* lam = nullptr;
     // Per-body stop flags (may be null): items and tiles of a body whose flag
     // is nonzero do nothing (independent bodies solved in lock-step, whose
     // converged members drop out).
@@ -196,11 +220,14 @@ size_t build_sym_worklist(const std::vector<BodyRange>& bodies, int kind, int se
 
 // Rebuilds `near` for the given precision: every pair of particles of one
 // body whose squared separation, in the pair kernel's own arithmetic for that
-// precision, is <= (ai+aj)^2, found through a hashed uniform grid (O(n)).
-// body_ranges: nbody BodyRange records on the device.  Grows `grid` as
-// needed; returns the largest per-target count in *max_count (synchronises).
-hipError_t build_near_list(int precision, const MatvecArgs& a, NearGrid& grid, const int32_t* body_ranges, int nbody,
-                           NearList& near, int n_targets, int* max_count, int* host_scratch, hipStream_t stream);
+// precision, is <= (ai+aj)^2.  With `fixed` the bodies' fixed-point frame and
+// positions are made first (precision 1).  Enqueues only: *near.max_cnt and
+// the frame are on the device once the stream gets there.  Allocates what
+// `grid` lacks.
+hipError_t build_near_list(int precision, const MatvecArgs& a, const GeometryArgs& g, bool fixed, NearGrid& grid,
+                           const NearList& near, hipStream_t stream);
+// The fixed-point frame and positions alone.
+hipError_t launch_fixed(const MatvecArgs& a, const GeometryArgs& g, hipStream_t stream);
 void free_grid(NearGrid& g);
 // Barrier forces of the positions in `a` (xs, xb, ns, nb, radii): fs += on
 // segment slots 0-2 (stride 6), fb = (stride 3, may be null).  Uses `grid`
@@ -208,25 +235,31 @@ void free_grid(NearGrid& g);
 hipError_t launch_barrier(const MatvecArgs& a, NearGrid& grid, const BarrierParams& bp, double* fs, double* fb,
                           hipStream_t stream);
 
-// Launches pair kernel + reduce on `stream`.  d_tiles/d_items/partial are device
+// Launch the pair kernel, then the reduce kernel, on `stream`.  d_tiles/d_items/partial are device
 // buffers sized for the work list (n_slots partial slots in the symmetric form,
 // one per item otherwise); precision 0 = fp64, 1 = fp32 tiles with fp64
 // accumulation.  ev_begin/ev_end (may be null) are recorded around the pair
-// kernel only.
-hipError_t launch_matvec(int precision, int seg_dof, const TileShape& shape, const MatvecArgs& a,
-                         const OutArgs& o, const MatvecTile* d_tiles, int n_tiles,
-                         const MatvecItem* d_items, int n_items, int n_slots, double* partial, const NearList& near,
-                         const PersistState& ps, hipStream_t stream, hipEvent_t ev_begin = nullptr,
-                         hipEvent_t ev_end = nullptr);
+// kernel only.  The pair kernel does not look at the near-pair lists.
+hipError_t launch_matvec_pairs(int precision, int seg_dof, const TileShape& shape, const MatvecArgs& a,
+                               uint32_t blocks, const MatvecTile* d_tiles, int n_tiles, const MatvecItem* d_items,
+                               int n_items, double* partial, const PersistState& ps, hipStream_t stream,
+                               hipEvent_t ev_begin = nullptr, hipEvent_t ev_end = nullptr);
+hipError_t launch_matvec_reduce(int precision, int seg_dof, const TileShape& shape, const MatvecArgs& a,
+                                const OutArgs& o, const MatvecTile* d_tiles, int n_tiles, int n_items, int n_slots,
+                                const double* partial, const NearList& near, const PersistState& ps,
+                                hipStream_t stream);
 
 // Half-space domain (no-slip wall at z = 0): the wall pair kernel (FP64, or
 // FP32 tiles from fixed-point separations) over a work list of
 // kWallBlock-target tiles (one target per lane), then the reduce kernel
 // without near-pair terms.
 constexpr int kWallBlock = 256;
-hipError_t launch_matvec_wall(int precision, int seg_dof, const MatvecArgs& a, const OutArgs& o,
-                              const MatvecTile* d_tiles, int n_tiles, const MatvecItem* d_items, int n_items,
-                              double* partial, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end);
+hipError_t launch_wall_pairs(int precision, int seg_dof, const MatvecArgs& a, const MatvecTile* d_tiles, int n_tiles,
+                             const MatvecItem* d_items, int n_items, double* partial, hipStream_t stream,
+                             hipEvent_t ev_begin, hipEvent_t ev_end);
+hipError_t launch_wall_reduce(int precision, int seg_dof, const MatvecArgs& a, const OutArgs& o,
+                              const MatvecTile* d_tiles, int n_tiles, int n_items, const double* partial,
+                              hipStream_t stream);
 
 // Flow-field evaluation (Stokeslet + rotlet mode and RPY mode).
 struct FlowArgs {

@@ -273,80 +273,8 @@ void invalidate_near(tfs_rpy* h) {
     h->fx_valid = false;
 }
 
-namespace {
-
-// Bounding box of each body's segments and blobs (min xyz, max xyz); a
-// non-finite coordinate makes the box NaN.  One workgroup per body.
-__global__ __launch_bounds__(256) void body_box_kernel(const double* __restrict__ xs, const double* __restrict__ xb,
-                                                       const int4* __restrict__ ranges, double* __restrict__ box) {
-    __shared__ double red[6][256];
-    __shared__ int bad_any;
-    const int4 r = ranges[blockIdx.x];
-    const int tid = threadIdx.x;
-    if (tid == 0) bad_any = 0;
-    double lo[3] = {__builtin_inf(), __builtin_inf(), __builtin_inf()};
-    double hi[3] = {-__builtin_inf(), -__builtin_inf(), -__builtin_inf()};
-    bool bad = false;
-    for (int i = r.x + tid; i < r.y; i += 256)
-        for (int k = 0; k < 3; ++k) {
-            const double v = xs[3 * (int64_t)i + k];
-            bad |= !__builtin_isfinite(v);
-            lo[k] = __builtin_fmin(lo[k], v);
-            hi[k] = __builtin_fmax(hi[k], v);
-        }
-    for (int i = r.z + tid; i < r.w; i += 256)
-        for (int k = 0; k < 3; ++k) {
-            const double v = xb[3 * (int64_t)i + k];
-            bad |= !__builtin_isfinite(v);
-            lo[k] = __builtin_fmin(lo[k], v);
-            hi[k] = __builtin_fmax(hi[k], v);
-        }
-    for (int k = 0; k < 3; ++k) {
-        red[k][tid] = lo[k];
-        red[3 + k][tid] = hi[k];
-    }
-    __syncthreads();
-    if (bad) bad_any = 1;
-    for (int w = 128; w > 0; w >>= 1) {
-        if (tid < w)
-            for (int k = 0; k < 3; ++k) {
-                red[k][tid] = __builtin_fmin(red[k][tid], red[k][tid + w]);
-                red[3 + k][tid] = __builtin_fmax(red[3 + k][tid], red[3 + k][tid + w]);
-            }
-        __syncthreads();
-    }
-    if (tid < 6) box[6 * blockIdx.x + tid] = bad_any ? __builtin_nan("") : red[tid][0];
-}
-
-// X = rint(lambda (x - c_body)) for every segment and blob of body blockIdx.x.
-__global__ __launch_bounds__(256) void to_fixed_kernel(const double* __restrict__ xs, const double* __restrict__ xb,
-                                                       const int4* __restrict__ ranges,
-                                                       const double* __restrict__ centre, double lam, int ns,
-                                                       int4* __restrict__ out) {
-    const int4 r = ranges[blockIdx.x];
-    const double c0 = centre[3 * blockIdx.x], c1 = centre[3 * blockIdx.x + 1], c2 = centre[3 * blockIdx.x + 2];
-    for (int i = r.x + threadIdx.x; i < r.y; i += 256) {
-        const double* x = xs + 3 * (int64_t)i;
-        out[i] = make_int4((int)__builtin_rint((x[0] - c0) * lam), (int)__builtin_rint((x[1] - c1) * lam),
-                           (int)__builtin_rint((x[2] - c2) * lam), 0);
-    }
-    for (int i = r.z + threadIdx.x; i < r.w; i += 256) {
-        const double* x = xb + 3 * (int64_t)i;
-        out[ns + i] = make_int4((int)__builtin_rint((x[0] - c0) * lam), (int)__builtin_rint((x[1] - c1) * lam),
-                                (int)__builtin_rint((x[2] - c2) * lam), 0);
-    }
-}
-
-}  // namespace
-
-// Fixed-point coordinates for FP32 tiles.  Each body is centred on its
-// bounding box; lambda = 2^k is the largest power of two with
-// lambda * (largest half-extent) <= 2^30 - 2, so every coordinate and every
-// difference of two fits an int32.  The quantisation step 1/lambda must stay
-// below 2^-19 of the smallest radius (a body within ~1024 radii of its
-// centre); larger bodies are refused in FP32.  Synchronises the stream.
-// The body table on the device (BodyRange records, plus room for 6 doubles
-// per body), uploaded on the handle's stream from h->bodies.
+// The body table on the device (BodyRange records, plus room for the bounding
+// boxes), uploaded on the handle's stream from h->bodies.
 int ensure_body_table(tfs_rpy* h) {
     if (h->body_table_valid) return TFS_OK;
     const size_t nbody = h->bodies.size();
@@ -356,7 +284,7 @@ int ensure_body_table(tfs_rpy* h) {
         if (h->d_body_range) (void)hipFree(h->d_body_range);
         h->d_body_box = nullptr;
         h->d_body_range = nullptr;
-        e = hipMalloc(&h->d_body_box, sizeof(double) * 6 * nbody);
+        e = hipMalloc(&h->d_body_box, sizeof(double) * 6 * std::max<size_t>(nbody, kBoxShares));
         if (e == hipSuccess) e = hipMalloc(&h->d_body_range, sizeof(int4) * nbody);
         h->body_cap = e == hipSuccess ? nbody : 0;
     }
@@ -366,79 +294,6 @@ int ensure_body_table(tfs_rpy* h) {
     if (e != hipSuccess) return hip_fail(e, "body table");
     h->body_table_valid = true;
     return TFS_OK;
-}
-
-// The fixed-point frame of the bodies' bounding boxes (6 per body: min xyz,
-// max xyz): each body's centre and one lambda = 2^k for all of them.
-static int fixed_point_frame(const double* box, size_t nbody, double amin, double* centre, double* lam) {
-    double ext = 0.0;
-    for (size_t b = 0; b < nbody; ++b) {
-        for (int k = 0; k < 3; ++k) {
-            const double lo = box[6 * b + k], hi = box[6 * b + 3 + k];
-            if (std::isnan(lo) || std::isnan(hi)) return fail(TFS_ERR_NON_FINITE, "positions are not finite");
-            centre[3 * b + k] = 0.0;
-            if (!(lo <= hi)) continue;  // body without particles
-            const double c = 0.5 * (lo + hi);
-            centre[3 * b + k] = c;
-            ext = std::max(ext, std::max(hi - c, c - lo));
-        }
-    }
-    const double lim = 1073741822.0;  // 2^30 - 2
-    int k = 60;
-    if (ext > 0.0) {
-        k = (int)std::floor(std::log2(lim / ext));
-        while (k > -1000 && std::ldexp(ext, k) > lim) --k;
-        while (k < 60 && std::ldexp(ext, k + 1) <= lim) ++k;
-        k = std::min(k, 60);
-    }
-    if (std::ldexp(1.0, -k) > std::ldexp(amin, -19))
-        return fail(TFS_ERR_INVALID_ARGUMENT,
-                    "FP32 tiles: a body extends more than about 1024 particle radii from its centre (use FP64)");
-    *lam = std::ldexp(1.0, k);
-    return TFS_OK;
-}
-
-int ensure_fixed(tfs_rpy* h) {
-    if (h->fx_valid) return TFS_OK;
-    const int ns = h->desc.num_segs, nb = h->desc.num_blobs;
-    const size_t nbody = h->bodies.size();
-    hipError_t e = hipSuccess;
-    if (!h->x_fx) e = hipMalloc(&h->x_fx, sizeof(int4) * (size_t)std::max(ns + nb, 1));
-    if (e != hipSuccess) return fail(TFS_ERR_OUT_OF_MEMORY, "fixed-point positions");
-    int rc = ensure_body_table(h);
-    if (rc) return rc;
-    std::vector<double> box(6 * nbody), centre(3 * nbody, 0.0);
-    {
-        hipLaunchKernelGGL(body_box_kernel, dim3((unsigned)nbody), dim3(256), 0, h->stream, h->x_segs, h->x_blobs,
-                           (const int4*)h->d_body_range, h->d_body_box);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(box.data(), h->d_body_box, sizeof(double) * 6 * nbody, hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (e != hipSuccess) return hip_fail(e, "fixed-point positions: bounding boxes");
-    int rc2 = fixed_point_frame(box.data(), nbody, std::min(h->desc.seg_radius, h->desc.blob_radius), centre.data(),
-                                &h->fx_lambda);
-    if (rc2) return rc2;
-    h->fx_centre = centre;
-    e = hipMemcpyAsync(h->d_body_box, h->fx_centre.data(), sizeof(double) * 3 * nbody, hipMemcpyHostToDevice,
-                       h->stream);
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(to_fixed_kernel, dim3((unsigned)nbody), dim3(256), 0, h->stream, h->x_segs, h->x_blobs,
-                           (const int4*)h->d_body_range, (const double*)h->d_body_box, h->fx_lambda, ns, h->x_fx);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (e != hipSuccess) return hip_fail(e, "fixed-point positions");
-    h->fx_valid = true;
-    return TFS_OK;
-}
-
-void free_near(NearList& nl) {
-    hipFree(nl.cnt);
-    hipFree(nl.idx);
-    hipFree(nl.max_cnt);
-    nl = NearList{};
 }
 
 MatvecArgs matvec_args(tfs_rpy* h, CView fs, CView fb) {
@@ -455,59 +310,151 @@ MatvecArgs matvec_args(tfs_rpy* h, CView fs, CView fb) {
     a.skip = h->skip_flag;
     a.body_skip = h->body_skip;
     a.xfx = h->x_fx;
-    a.lam = h->fx_lambda;
+    a.lam = &h->d_frame->lam;
     return a;
 }
 
-// Lists the overlapping pairs of the current positions for `precision`,
-// growing the per-target capacity until every list fits.
-int ensure_near(tfs_rpy* h, int precision) {
+// Device error of a launch over new positions.
+static int frame_error(int status) {
+    if (status == kFrameNonFinite) return fail(TFS_ERR_NON_FINITE, "positions are not finite");
+    return fail(TFS_ERR_INVALID_ARGUMENT,
+                "FP32 tiles: a body extends more than about 1024 particle radii from its centre (use FP64)");
+}
+
+static GeometryArgs geometry_args(const tfs_rpy* h) {
+    GeometryArgs g;
+    g.ranges = h->d_body_range;
+    g.nbody = (int)h->bodies.size();
+    for (const BodyRange& b : h->bodies)
+        g.largest = std::max(g.largest, (b.seg_end - b.seg_begin) + (b.blob_end - b.blob_begin));
+    g.box = h->d_body_box;
+    g.fixed = h->x_fx;
+    g.frame = h->d_frame;
+    return g;
+}
+
+// Enqueues the read-back of the frame into pinned memory.
+static hipError_t read_frame(tfs_rpy* h) {
+    return hipMemcpyAsync(h->host_int, h->d_frame, sizeof(GeomFrame), hipMemcpyDeviceToHost, h->stream);
+}
+
+static const GeomFrame& frame_of(const tfs_rpy* h) { return *reinterpret_cast<const GeomFrame*>(h->host_int); }
+
+static int alloc_fixed(tfs_rpy* h) {
+    const int n = h->desc.num_segs + h->desc.num_blobs;
+    if (!h->x_fx && hipMalloc(&h->x_fx, sizeof(int4) * (size_t)std::max(n, 1)) != hipSuccess)
+        return fail(TFS_ERR_OUT_OF_MEMORY, "fixed-point positions");
+    return TFS_OK;
+}
+
+// Fixed-point coordinates for FP32 tiles.  Each body is centred on its
+// bounding box; lambda = 2^k is the largest power of two with
+// lambda * (largest half-extent) <= 2^30 - 2, so every coordinate and every
+// difference of two fits an int32 (2^40 / the smallest radius where the bodies
+// are smaller than that).  The quantisation step 1/lambda must stay
+// below 2^-19 of the smallest radius (a body within ~1024 radii of its
+// centre); larger bodies are refused in FP32.  Synchronises the stream.
+int ensure_fixed(tfs_rpy* h) {
+    if (h->fx_valid) return TFS_OK;
+    int rc = alloc_fixed(h);
+    if (!rc) rc = ensure_body_table(h);
+    if (rc) return rc;
+    hipError_t e = launch_fixed(matvec_args(h, CView{h->f_segs, 6, 1}, CView{h->f_blobs, 3, 1}), geometry_args(h), h->stream);
+    if (e == hipSuccess) e = read_frame(h);
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    if (e != hipSuccess) return hip_fail(e, "fixed-point positions");
+    if (frame_of(h).status) return frame_error(frame_of(h).status);
+    h->fx_valid = true;
+    return TFS_OK;
+}
+
+void free_near(NearList& nl) {
+    hipFree(nl.cnt);
+    hipFree(nl.idx);
+    nl = NearList{};
+}
+
+// Enqueues the lists of the overlapping pairs of the current positions for
+// `precision` if they are not there (FP32: with the fixed-point positions), and
+// sets *open where near_close has to look at the read-back before they may be
+// used.  A caller that defers the capacity check (defer_near_check) looks for
+// itself and has nothing to close.
+static int near_open(tfs_rpy* h, int precision, bool* open) {
+    *open = false;
     if (h->near_valid[precision] && (precision == 0 || h->fx_valid)) return TFS_OK;
     const int nt = h->desc.num_segs + h->desc.num_blobs;
     if (nt == 0) {
         h->near_valid[precision] = true;
         return TFS_OK;
     }
-    int err = precision == 1 ? ensure_fixed(h) : ensure_body_table(h);
+    int err = ensure_body_table(h);
+    if (!err && precision == 1) err = h->defer_near_check ? ensure_fixed(h) : alloc_fixed(h);
     if (err) return err;
     NearList& nl = h->near[precision];
-    MatvecArgs a = matvec_args(h, CView{h->f_segs, 6, 1}, CView{h->f_blobs, 3, 1});
-    for (int attempt = 0; attempt < 8; ++attempt) {
-        if (!nl.cnt) {
-            if (nl.cap == 0) nl.cap = 32;
-            hipError_t e = hipMalloc(&nl.cnt, sizeof(int32_t) * nt);
-            if (e == hipSuccess) e = hipMalloc(&nl.idx, sizeof(int32_t) * (size_t)nt * nl.cap);
-            if (e == hipSuccess) e = hipMalloc(&nl.max_cnt, sizeof(int32_t));
-            if (e != hipSuccess) {
-                free_near(nl);
-                return fail(TFS_ERR_OUT_OF_MEMORY, "near-pair lists");
-            }
+    if (!nl.cnt) {
+        if (nl.cap == 0) nl.cap = 32;
+        hipError_t e = hipMalloc(&nl.cnt, sizeof(int32_t) * nt);
+        if (e == hipSuccess) e = hipMalloc(&nl.idx, sizeof(int32_t) * (size_t)nt * nl.cap);
+        if (e != hipSuccess) {
+            free_near(nl);
+            return fail(TFS_ERR_OUT_OF_MEMORY, "near-pair lists");
         }
-        if (h->defer_near_check && nl.cnt) {
-            // a capacity of every particle cannot overflow: nothing to check
-            const bool roomy = nl.cap >= nt;
-            hipError_t e = build_near_list(precision, a, h->grid, h->d_body_range, (int)h->bodies.size(), nl, nt,
-                                           nullptr, roomy ? nullptr : h->host_int + 8 + precision, h->stream);
-            if (e != hipSuccess) return hip_fail(e, "near-pair lists");
-            h->near_valid[precision] = true;
-            h->near_pending[precision] = !roomy;
-            return TFS_OK;
-        }
-        int max_count = 0;
-        hipError_t e = build_near_list(precision, a, h->grid, h->d_body_range, (int)h->bodies.size(), nl, nt,
-                                       &max_count, h->host_int, h->stream);
+    }
+    nl.max_cnt = &h->d_frame->max_cnt[precision];
+    const bool fixed = precision == 1 && !h->fx_valid;
+    hipError_t e = build_near_list(precision, matvec_args(h, CView{h->f_segs, 6, 1}, CView{h->f_blobs, 3, 1}),
+                                   geometry_args(h), fixed, h->grid, nl, h->stream);
+    if (h->defer_near_check) {
+        // a capacity of every particle cannot overflow: nothing to check
+        const bool roomy = nl.cap >= nt;
+        if (e == hipSuccess && !roomy)
+            e = hipMemcpyAsync(h->host_int + 8 + precision, nl.max_cnt, sizeof(int32_t), hipMemcpyDeviceToHost, h->stream);
         if (e != hipSuccess) return hip_fail(e, "near-pair lists");
-        if (max_count <= nl.cap) {
+        h->near_valid[precision] = true;
+        h->near_pending[precision] = !roomy;
+        return TFS_OK;
+    }
+    if (e == hipSuccess && !h->frame_read) e = hipEventCreateWithFlags(&h->frame_read, hipEventDisableTiming);
+    if (e == hipSuccess) e = read_frame(h);
+    if (e == hipSuccess) e = hipEventRecord(h->frame_read, h->stream);
+    if (e != hipSuccess) return hip_fail(e, "near-pair lists");
+    *open = true;
+    return TFS_OK;
+}
+
+// Waits for the read-back of near_open and checks it; lists that did not fit
+// are made again with room for the longest.
+static int near_close(tfs_rpy* h, int precision) {
+    NearList& nl = h->near[precision];
+    for (int attempt = 0; attempt < 8; ++attempt) {
+        hipError_t e = hipEventSynchronize(h->frame_read);
+        if (e != hipSuccess) return hip_fail(e, "near-pair lists");
+        const GeomFrame& f = frame_of(h);
+        if (precision == 1) {
+            if (!h->fx_valid && f.status) return frame_error(f.status);
+            h->fx_valid = true;
+        }
+        const int longest = f.max_cnt[precision];
+        if (longest <= nl.cap) {
             h->near_valid[precision] = true;
             return TFS_OK;
         }
         int cap = nl.cap;
-        while (cap < max_count) cap *= 2;
+        while (cap < longest) cap *= 2;
         hipStreamSynchronize(h->stream);
         free_near(nl);
         nl.cap = cap;
+        bool open = false;
+        const int rc = near_open(h, precision, &open);
+        if (rc) return rc;
     }
     return fail(TFS_ERR_INVALID_ARGUMENT, "near-pair lists: too many overlapping neighbours");
+}
+
+int ensure_near(tfs_rpy* h, int precision) {
+    bool open = false;
+    const int rc = near_open(h, precision, &open);
+    return rc || !open ? rc : near_close(h, precision);
 }
 
 int rpy_near_reserve(tfs_rpy* h, int precision, int cap) {
@@ -587,7 +534,9 @@ int run_matvec(tfs_rpy* h, uint32_t blocks, int precision, CView fs, CView fb, V
     Plan* p = get_plan(h, blocks, sh, &err);
     if (!p) return err;
     if (p->tiles.empty()) return TFS_OK;
-    if (!wall) err = ensure_near(h, precision);
+    // new positions: the pair kernel runs while the host reads back whether the lists fit
+    bool near_unread = false;
+    if (!wall) err = near_open(h, precision, &near_unread);
     else if (precision == TFS_PRECISION_FP32_ACC64) err = ensure_fixed(h);  // separations in fixed point
     if (err) return err;
     MatvecArgs a = matvec_args(h, fs, fb);
@@ -621,11 +570,19 @@ int run_matvec(tfs_rpy* h, uint32_t blocks, int precision, CView fs, CView fb, V
         ps.item_stamps = h->d_item_stamps;
         h->stamped_plan = p;
     }
-    hipError_t e = wall ? launch_matvec_wall(precision, h->desc.seg_dof, a, o, p->d_tiles, (int)p->tiles.size(), p->d_items,
-                                             (int)p->items.size(), h->partial, h->stream, eb, ee)
-                        : launch_matvec(precision, h->desc.seg_dof, sh, a, o, p->d_tiles, (int)p->tiles.size(),
-                                        p->d_items, (int)p->items.size(), p->slots, h->partial, h->near[precision], ps,
-                                        h->stream, eb, ee);
+    const int n_tiles = (int)p->tiles.size(), n_items = (int)p->items.size();
+    hipError_t e = wall ? launch_wall_pairs(precision, h->desc.seg_dof, a, p->d_tiles, n_tiles, p->d_items, n_items,
+                                            h->partial, h->stream, eb, ee)
+                        : launch_matvec_pairs(precision, h->desc.seg_dof, sh, a, o.blocks, p->d_tiles, n_tiles,
+                                              p->d_items, n_items, h->partial, ps, h->stream, eb, ee);
+    if (e == hipSuccess && near_unread) {
+        err = near_close(h, precision);
+        if (err) return err;
+    }
+    if (e == hipSuccess)
+        e = wall ? launch_wall_reduce(precision, h->desc.seg_dof, a, o, p->d_tiles, n_tiles, n_items, h->partial, h->stream)
+                 : launch_matvec_reduce(precision, h->desc.seg_dof, sh, a, o, p->d_tiles, n_tiles, n_items, p->slots,
+                                        h->partial, h->near[precision], ps, h->stream);
     if (e != hipSuccess) return hip_fail(e, "matvec launch");
     return TFS_OK;
 }
@@ -660,7 +617,6 @@ int tfs_rpy_create(const tfs_rpy_desc* desc, tfs_rpy** out) {
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1)
         return fail(TFS_ERR_NO_DEVICE, "tfs_rpy_create: no HIP device visible");
     tfs_rpy* h = new tfs_rpy();
-    h->grid.may_alloc = true;
     h->desc = *desc;
     hipGetDevice(&h->device);
     hipDeviceProp_t prop;
@@ -683,6 +639,7 @@ int tfs_rpy_create(const tfs_rpy_desc* desc, tfs_rpy** out) {
     const size_t lens[6] = {3 * ns, 6 * ns, 3 * nb, 3 * nb, 6 * ns, 3 * nb};
     size_t total = 0;
     for (size_t l : lens) total += std::max<size_t>(l, 1) + 32;  // keep 256-B alignment
+    total += 32;                                                  // d_frame
     hipError_t e = hipMalloc(&h->arena, total * sizeof(double));
     if (e != hipSuccess) {
         tfs_rpy_destroy(h);
@@ -694,6 +651,7 @@ int tfs_rpy_create(const tfs_rpy_desc* desc, tfs_rpy** out) {
         *dst[i] = p;
         p += ((std::max<size_t>(lens[i], 1) + 31) / 32) * 32;
     }
+    h->d_frame = reinterpret_cast<GeomFrame*>(p);
     e = hipMemsetAsync(h->arena, 0, total * sizeof(double), h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) {
@@ -733,6 +691,7 @@ int tfs_rpy_destroy(tfs_rpy* h) {
     if (h->x_fx) hipFree(h->x_fx);
     if (h->d_body_box) hipFree(h->d_body_box);
     if (h->d_body_range) hipFree(h->d_body_range);
+    if (h->frame_read) hipEventDestroy(h->frame_read);
     if (h->host_int) hipHostFree(h->host_int);
     if (h->blob_rep) hipFree(h->blob_rep);
     free_stage(h->f32);
@@ -1386,16 +1345,13 @@ constexpr size_t align256(size_t x) { return (x + 255) / 256 * 256; }
 constexpr size_t kOffPartial = 0;
 constexpr size_t kOffNearIdx = align256(kOffPartial + kStaticPartialBytes);
 constexpr size_t kOffNearCnt = align256(kOffNearIdx + sizeof(int32_t) * kStaticMaxParticles * kStaticNearCap);
-constexpr size_t kOffNearMax = align256(kOffNearCnt + sizeof(int32_t) * kStaticMaxParticles);
-constexpr size_t kOffStart = align256(kOffNearMax + sizeof(int32_t));
-constexpr size_t kOffFill = align256(kOffStart + sizeof(int32_t) * (kStaticTable + 1));
-constexpr size_t kOffBucket = align256(kOffFill + sizeof(int32_t) * kStaticTable);
-constexpr size_t kOffOrder = align256(kOffBucket + sizeof(int32_t) * kStaticMaxParticles);
-constexpr size_t kOffBodyOf = align256(kOffOrder + sizeof(int32_t) * kStaticMaxParticles);
-constexpr size_t kOffFixed = align256(kOffBodyOf + sizeof(int32_t) * kStaticMaxParticles);
+constexpr size_t kOffFrame = align256(kOffNearCnt + sizeof(int32_t) * kStaticMaxParticles);
+constexpr size_t kOffFill = align256(kOffFrame + sizeof(GeomFrame));
+constexpr size_t kOffNodes = align256(kOffFill + sizeof(int32_t) * kStaticTable);
+constexpr size_t kOffFixed = align256(kOffNodes + sizeof(int4) * kStaticMaxParticles);
 constexpr size_t kOffBody = align256(kOffFixed + sizeof(int4) * kStaticMaxParticles);
 constexpr size_t kOffBox = align256(kOffBody + sizeof(int4));
-constexpr size_t kOffTiles = align256(kOffBox + 6 * sizeof(double));
+constexpr size_t kOffTiles = align256(kOffBox + 6 * sizeof(double) * kBoxShares);
 constexpr size_t kOffItems = align256(kOffTiles + sizeof(MatvecTile) * kStaticMaxTiles);
 constexpr size_t kScratchBytes = align256(kOffItems + sizeof(MatvecItem) * kStaticMaxItems);
 
@@ -1454,17 +1410,6 @@ __global__ __launch_bounds__(256) void static_worklist_kernel(int ns, int nb, in
         for (int s0 = 0; s0 < ns; s0 += chunk) items[k++] = MatvecItem{t, 0, s0, s0 + chunk < ns ? s0 + chunk : ns};
     if (seg ? sb : bb)
         for (int s0 = 0; s0 < nb; s0 += chunk) items[k++] = MatvecItem{t, 1, s0, s0 + chunk < nb ? s0 + chunk : nb};
-}
-
-// X = rint(lambda (x - c)) for the one body of the call.
-__global__ __launch_bounds__(256) void static_fixed_kernel(const double* __restrict__ xs, const double* __restrict__ xb,
-                                                           int ns, int nb, double c0, double c1, double c2, double lam,
-                                                           int4* __restrict__ out) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= ns + nb) return;
-    const double* x = i < ns ? xs + 3 * (int64_t)i : xb + 3 * (int64_t)(i - ns);
-    out[i] = make_int4((int)__builtin_rint((x[0] - c0) * lam), (int)__builtin_rint((x[1] - c1) * lam),
-                       (int)__builtin_rint((x[2] - c2) * lam), 0);
 }
 
 int static_items(int ns, int nb, int chunk, int ts, int tb, bool ss, bool sb, bool bs, bool bb, int* is_, int* ib) {
@@ -1534,45 +1479,39 @@ int tfs_rpy_apply_noalloc(const tfs_rpy_desc* desc, uint32_t blocks, const doubl
     a.a_blob = D.blob_radius;
     a.mu = D.mu;
     const int n = ns + nb;
-    if (D.precision == TFS_PRECISION_FP32_ACC64) {
-        // fixed-point frame of the body's bounding box (read back to the stack)
-        double* box = reinterpret_cast<double*>(base + kOffBox);
-        hipLaunchKernelGGL(body_box_kernel, dim3(1), dim3(256), 0, st, x_segs, x_blobs, (const int4*)body, box);
-        double hbox[6], centre[3], lam = 1.0;
-        e = hipGetLastError();
-        if (e == hipSuccess) e = hipMemcpyAsync(hbox, box, sizeof(hbox), hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
-        if (e != hipSuccess) return hip_fail(e, w);
-        rc = fixed_point_frame(hbox, 1, std::min(D.seg_radius, D.blob_radius), centre, &lam);
-        if (rc) return rc;
-        int4* fx = reinterpret_cast<int4*>(base + kOffFixed);
-        hipLaunchKernelGGL(static_fixed_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x_segs, x_blobs,
-                           ns, nb, centre[0], centre[1], centre[2], lam, fx);
-        e = hipGetLastError();
-        if (e != hipSuccess) return hip_fail(e, w);
-        a.xfx = fx;
-        a.lam = lam;
+    // the fixed-point frame and positions (FP32 tiles) and the overlapping
+    // pairs, on the grid kept in scratch (sized for n: no allocation); the
+    // frame is read back to the stack
+    GeomFrame* frame = reinterpret_cast<GeomFrame*>(base + kOffFrame);
+    const bool f32 = D.precision == TFS_PRECISION_FP32_ACC64;
+    GeometryArgs g;
+    g.ranges = reinterpret_cast<const int32_t*>(body);
+    g.largest = n;
+    g.box = reinterpret_cast<double*>(base + kOffBox);
+    g.frame = frame;
+    g.fixed = reinterpret_cast<int4*>(base + kOffFixed);
+    if (f32) {
+        a.xfx = g.fixed;
+        a.lam = &frame->lam;
     }
-    // overlapping pairs, on the grid kept in scratch (sized for n: no allocation)
     NearList near;
     near.cnt = reinterpret_cast<int32_t*>(base + kOffNearCnt);
     near.idx = reinterpret_cast<int32_t*>(base + kOffNearIdx);
-    near.max_cnt = reinterpret_cast<int32_t*>(base + kOffNearMax);
+    near.max_cnt = &frame->max_cnt[D.precision];
     near.cap = kStaticNearCap;
     NearGrid grid;
-    grid.start = reinterpret_cast<int32_t*>(base + kOffStart);
     grid.fill = reinterpret_cast<int32_t*>(base + kOffFill);
-    grid.bucket_of = reinterpret_cast<int32_t*>(base + kOffBucket);
-    grid.order = reinterpret_cast<int32_t*>(base + kOffOrder);
-    grid.body_of = reinterpret_cast<int32_t*>(base + kOffBodyOf);
+    grid.nodes = reinterpret_cast<int4*>(base + kOffNodes);
     grid.n = n;
     grid.table = 1024;
     while (grid.table < 2 * n) grid.table <<= 1;
-    int max_count = 0, host_count = 0;
-    e = build_near_list(D.precision, a, grid, reinterpret_cast<const int32_t*>(body), 1, near, n, &max_count, &host_count,
-                        st);
+    GeomFrame host{};
+    e = build_near_list(D.precision, a, g, f32, grid, near, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(&host, frame, sizeof(host), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) return hip_fail(e, w);
-    if (max_count > kStaticNearCap)
+    if (f32 && host.status) return frame_error(host.status);
+    if (host.max_cnt[D.precision] > kStaticNearCap)
         return fail(TFS_ERR_INVALID_ARGUMENT, std::string(w) + ": a particle overlaps more than " +
                                                   std::to_string(kStaticNearCap) + " others; use tfs_rpy_apply");
     OutArgs o;
@@ -1582,8 +1521,10 @@ int tfs_rpy_apply_noalloc(const tfs_rpy_desc* desc, uint32_t blocks, const doubl
     o.blocks = eff;
     const TileShape sh{kStaticTile, 1, chunk, 0};
     PersistState ps;
-    e = launch_matvec(D.precision, D.seg_dof, sh, a, o, tiles, ts + tb, items, n_items, n_items,
-                      reinterpret_cast<double*>(base + kOffPartial), near, ps, st);
+    double* partial = reinterpret_cast<double*>(base + kOffPartial);
+    e = launch_matvec_pairs(D.precision, D.seg_dof, sh, a, eff, tiles, ts + tb, items, n_items, partial, ps, st);
+    if (e == hipSuccess)
+        e = launch_matvec_reduce(D.precision, D.seg_dof, sh, a, o, tiles, ts + tb, n_items, n_items, partial, near, ps, st);
     return e == hipSuccess ? TFS_OK : hip_fail(e, w);
 }
 

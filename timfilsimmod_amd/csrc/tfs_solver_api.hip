@@ -695,7 +695,7 @@ int ens_enqueue_steps(tfs_solver* s, int precision, int j0, int j1) {
 
 // The m steps of a cycle as one hipGraph, captured again only when something
 // the launches hold by value or pointer changed (the work list, partial
-// buffer, near-pair lists, fixed-point positions and their scale).
+// buffer, near-pair lists, fixed-point positions).
 int ens_cycle_graph(tfs_solver* s, int precision) {
     EnsState& E = *s->ens;
     tfs_rpy* h = s->rpy;
@@ -705,8 +705,6 @@ int ens_cycle_graph(tfs_solver* s, int precision) {
     const TileShape sh = effective_shape(h, precision, TFS_BLOCK_ALL);
     const Plan* p = get_plan(h, TFS_BLOCK_ALL, sh, &err);
     if (!p) return err;
-    uint64_t lam_bits = 0;
-    std::memcpy(&lam_bits, &h->fx_lambda, 8);
     const std::vector<uintptr_t> key = {(uintptr_t)p->d_tiles,
                                         (uintptr_t)p->d_items,
                                         (uintptr_t)h->partial,
@@ -714,7 +712,6 @@ int ens_cycle_graph(tfs_solver* s, int precision) {
                                         (uintptr_t)h->near[precision].idx,
                                         (uintptr_t)h->near[precision].cap,
                                         (uintptr_t)h->x_fx,
-                                        (uintptr_t)(precision == 1 ? lam_bits : 0),
                                         (uintptr_t)sh.block,
                                         (uintptr_t)sh.per_thread,
                                         (uintptr_t)sh.chunk,
