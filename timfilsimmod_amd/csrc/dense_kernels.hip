@@ -104,6 +104,132 @@ __global__ __launch_bounds__(256) void block_gauss_jordan_kernel(double* __restr
     if (tid == 0) status[b] = 0;
 }
 
+// The same for blocks of up to WAVES x ROWS rows and 64 x COLS columns: the
+// block stays in registers, lane l holding columns l, l + 64, ... of rows w,
+// w + WAVES, ... of its wave w.  Rows are not moved: each step takes the
+// largest entry of its column (by its first 12 bits, the lowest row among
+// equals) among the rows that were no pivot yet, and the block is written back
+// by the order in which they were.  Two barriers a step: the wave that holds
+// the pivot row puts it, scaled, into LDS; after the update the lane that holds
+// the next column puts that there and its rows' largest into a maximum over
+// the waves (keys of three steps in turn, the one after next cleared).
+//
+// Bound by the steps' latency and by what every wave does again (the search,
+// the barriers).  Sixteen blocks of 120 x 120: 182 us with sixteen waves (209
+// with eight, 358 with four; 370 with the division and the search over the
+// waves' maxima in every wave), 2,140 for the form above, which goes to global
+// memory for each of the 120 x 120 updates of a step.
+template <int WAVES, int ROWS, int COLS>
+__global__ __launch_bounds__(64 * WAVES) void block_inverse_kernel(double* __restrict__ A,
+                                                                  const int64_t* __restrict__ mat_off,
+                                                                  const int32_t* __restrict__ sizes,
+                                                                  int32_t* __restrict__ status) {
+    constexpr int NR = WAVES * ROWS, NC = 64 * COLS;
+    static_assert(NR < 256, "a key holds the row in its last 8 bits");
+    __shared__ double col[NR], row[NC];
+    __shared__ uint32_t key[3];
+    __shared__ int32_t pivot[NR], step_of[NR];
+    const int b = blockIdx.x;
+    const int n = sizes[b];
+    double* M = A + mat_off[b];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    double a[ROWS][COLS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) {
+            const int i = w + WAVES * r, j = lane + 64 * c;
+            a[r][c] = i < n && j < n ? M[(int64_t)i * n + j] : 0.0;
+        }
+    uint32_t left = 0;  // bit r: row w + WAVES r was no pivot yet
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) left |= w + WAVES * r < n ? 1u << r : 0u;
+    auto put_column = [&](int k) {
+        uint32_t best = 0;
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) {
+            if (c != k >> 6) continue;  // uniform
+            if (lane == (k & 63)) {
+#pragma unroll
+                for (int r = 0; r < ROWS; ++r) {
+                    col[w + WAVES * r] = a[r][c];
+                    const uint32_t hi = (uint32_t)__double2hiint(a[r][c]) & 0x7fffff00u;
+                    const uint32_t q = hi | (uint32_t)(255 - (w + WAVES * r));
+                    best = (left >> r & 1u) && q > best ? q : best;
+                }
+                atomicMax(&key[k % 3], best);
+            }
+        }
+    };
+    if (threadIdx.x < 3) key[threadIdx.x] = 0;
+    __syncthreads();
+    put_column(0);
+    __syncthreads();
+    bool bad = false;
+    for (int k = 0; k < n; ++k) {
+        const int p = 255 - (int)(__builtin_amdgcn_readfirstlane(key[k % 3]) & 255u);
+        const double d = col[p];
+        if (!(fabs(d) > 0.0) || !isfinite(d)) {
+            bad = true;  // uniform over the workgroup: every thread read the same d
+            break;
+        }
+        double f[ROWS];
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) f[r] = col[w + WAVES * r];
+        const bool own = p % WAVES == w;
+        if (own) {
+            const double inv = 1.0 / d;
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                if (r != p / WAVES) continue;  // uniform
+#pragma unroll
+                for (int c = 0; c < COLS; ++c) {
+                    const int j = lane + 64 * c;
+                    a[r][c] = j == k ? inv : a[r][c] * inv;
+                    row[j] = a[r][c];
+                }
+                f[r] = 0.0;
+            }
+            left &= ~(1u << p / WAVES);
+            if (lane == 0) {
+                pivot[k] = p;
+                step_of[p] = k;
+            }
+        }
+        if (threadIdx.x == 0) key[(k + 2) % 3] = 0;
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) {
+            if (c != k >> 6) continue;
+            if (lane == (k & 63)) {
+#pragma unroll
+                for (int r = 0; r < ROWS; ++r) a[r][c] = own && r == p / WAVES ? a[r][c] : 0.0;
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) {
+            const double v = row[lane + 64 * c];
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) a[r][c] -= f[r] * v;
+        }
+        if (k + 1 < n) put_column(k + 1);
+        __syncthreads();
+    }
+    if (bad) {
+        if (threadIdx.x == 0) status[b] = 1;
+        return;
+    }
+    // row i was pivot of step step_of[i]; column j belongs to row pivot[j]
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) {
+            const int i = w + WAVES * r, j = lane + 64 * c;
+            if (i < n && j < n) M[(int64_t)step_of[i] * n + pivot[j]] = a[r][c];
+        }
+    if (threadIdx.x == 0) status[b] = 0;
+}
+
 // In-place inverse of symmetric positive definite row-major blocks of at most
 // 64 rows by Gauss-Jordan elimination without pivoting (SPD: every pivot is
 // positive), one workgroup per block: the block sits in LDS, and each of the
@@ -341,6 +467,20 @@ hipError_t k_batched_inverse_spd(double* A, const int64_t* off, const int32_t* s
 hipError_t k_batched_inverse(double* A, const int64_t* off, const int32_t* sizes, int nblocks, int max_size,
                              int32_t* piv, const int32_t* piv_off, int32_t* status, hipStream_t stream) {
     if (nblocks <= 0) return hipSuccess;
+    const dim3 grid((unsigned)nblocks);
+    // in registers while the block fits them (192 rows: 72 entries per lane)
+    if (max_size <= 64) {
+        hipLaunchKernelGGL((block_inverse_kernel<8, 8, 1>), grid, dim3(512), 0, stream, A, off, sizes, status);
+        return hipGetLastError();
+    }
+    if (max_size <= 128) {
+        hipLaunchKernelGGL((block_inverse_kernel<16, 8, 2>), grid, dim3(1024), 0, stream, A, off, sizes, status);
+        return hipGetLastError();
+    }
+    if (max_size <= 192) {
+        hipLaunchKernelGGL((block_inverse_kernel<8, 24, 3>), grid, dim3(512), 0, stream, A, off, sizes, status);
+        return hipGetLastError();
+    }
     const size_t lds = sizeof(double) * 2 * (size_t)max_size;
     hipLaunchKernelGGL(block_gauss_jordan_kernel, dim3((unsigned)nblocks), dim3(256), lds, stream, A, off, sizes, piv,
                        piv_off, status);
