@@ -44,7 +44,7 @@ hipError_t k_spd_inverse_blocked(double* A, int n_pad, const DenseWork& work, hi
 // of n_pad entries) from its lower triangle: per 64 x 64 tile the row sums
 // and, off the diagonal, the column sums into partial (chunks x n_pad,
 // chunks = n_pad / 64), then summed in a fixed order.
-hipError_t k_symv_dense(const double* A, int n_pad, const double* x, double* y, double* partial, int chunks,
+hipError_t k_symv_dense(const double* A, int n_pad, const double* x, double* y, int n_out, double* partial, int chunks,
                         hipStream_t stream);
 
 }  // namespace tfs

@@ -433,8 +433,8 @@ __global__ __launch_bounds__(256) void symv_tiles_kernel(const double* __restric
 
 // y[R 64 + l] = sum over K of partial[(R nt + K) 64 + l]: workgroup R, wave
 // w summing K in [w q, (w + 1) q) (q = ceil(nt / 4)), the four quarters added
-// in order through LDS.
-__global__ __launch_bounds__(256) void symv_tiles_sum_kernel(const double* __restrict__ partial, int n_pad,
+// in order through LDS; the first n_out entries are written.
+__global__ __launch_bounds__(256) void symv_tiles_sum_kernel(const double* __restrict__ partial, int n_pad, int n_out,
                                                             double* __restrict__ y) {
     __shared__ double quarter[4][64];
     const int nt = n_pad / 64, R = (int)blockIdx.x;
@@ -451,7 +451,7 @@ __global__ __launch_bounds__(256) void symv_tiles_sum_kernel(const double* __res
     if (K < k1) a0 += p[(int64_t)K * 64];
     quarter[w][l] = a0 + a1;
     __syncthreads();
-    if (w == 0) y[R * 64 + l] = (quarter[0][l] + quarter[1][l]) + (quarter[2][l] + quarter[3][l]);
+    if (w == 0 && R * 64 + l < n_out) y[R * 64 + l] = (quarter[0][l] + quarter[1][l]) + (quarter[2][l] + quarter[3][l]);
 }
 
 }  // namespace
@@ -508,14 +508,14 @@ hipError_t k_spd_inverse_blocked(double* A, int n_pad, const DenseWork& w, hipSt
     return hipSuccess;
 }
 
-hipError_t k_symv_dense(const double* A, int n_pad, const double* x, double* y, double* partial, int chunks,
+hipError_t k_symv_dense(const double* A, int n_pad, const double* x, double* y, int n_out, double* partial, int chunks,
                         hipStream_t stream) {
     const int nt = n_pad / 64;
-    if (n_pad % 64 || chunks != nt) return hipErrorInvalidValue;
+    if (n_pad % 64 || chunks != nt || !A || !x || !y || !partial || n_out > n_pad) return hipErrorInvalidValue;
     hipLaunchKernelGGL(symv_tiles_kernel, dim3((unsigned)(nt * (nt + 1) / 2)), dim3(256), 0, stream, A, n_pad, x,
                        partial);
     hipLaunchKernelGGL(symv_tiles_sum_kernel, dim3((unsigned)nt), dim3(256), 0, stream, (const double*)partial,
-                       n_pad, y);
+                       n_pad, n_out, y);
     return hipGetLastError();
 }
 

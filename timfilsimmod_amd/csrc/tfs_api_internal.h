@@ -153,6 +153,13 @@ int broyden_dev_find_update(tfs_broyden* b, double* update);
 // pending (device, may be null): the end of iteration runs only while it is
 // nonzero, and clears it.
 int broyden_dev_end_of_iter(tfs_broyden* b, int32_t* pending);
+// end_of_iter and the next find_update in two launches, for at most 8,192
+// unknowns and loops of at most the engine's iterations: with an iteration
+// pending both, otherwise the update for the residual in slot 1, where
+// step_begin puts the engine's error before a loop's first.
+bool broyden_dev_step_supported(const tfs_broyden* b, int max_iter);
+int broyden_dev_step_begin(tfs_broyden* b);
+int broyden_dev_step(tfs_broyden* b, int32_t* pending, double* update);
 void broyden_dev_finish(tfs_broyden* b, int32_t iter, int32_t latest);
 // tfs_broyden_compute_errors in two halves: the launches and (copy_flags)
 // the copy of the flags to the host (no wait), and the flags once the stream

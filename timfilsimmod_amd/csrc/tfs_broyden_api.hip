@@ -189,17 +189,14 @@ __global__ __launch_bounds__(256) void coupling_apply_kernel(const double* __res
     }
 }
 
-// As block_gemv_kernel for blocks of 64 rows or more: 1024 threads per
-// block, eight column groups of 128 rows each, the groups added in a fixed
+// As block_gemv_kernel for blocks of 64 rows or more: 1024 threads for
+// block b, eight column groups of 128 rows each, the groups added in a fixed
 // order through LDS.
-__global__ __launch_bounds__(1024) void block_gemv_wide_kernel(const double* __restrict__ A,
-                                                               const int64_t* __restrict__ mat_off,
-                                                               const int32_t* __restrict__ row_off,
-                                                               const int32_t* __restrict__ sizes,
-                                                               const double* __restrict__ x, double* __restrict__ y,
-                                                               double alpha) {
+__device__ __forceinline__ void block_gemv_wide(const double* __restrict__ A, const int64_t* __restrict__ mat_off,
+                                                const int32_t* __restrict__ row_off, const int32_t* __restrict__ sizes,
+                                                const double* __restrict__ x, double* __restrict__ y, double alpha,
+                                                int b) {
     __shared__ double part[8][128];
-    const int b = blockIdx.x;
     const int bs = sizes[b];
     const double* Ab = A + mat_off[b];
     const int r0 = row_off[b];
@@ -230,6 +227,15 @@ __global__ __launch_bounds__(1024) void block_gemv_wide_kernel(const double* __r
                                  ((part[4][rl] + part[5][rl]) + (part[6][rl] + part[7][rl])));
         __syncthreads();
     }
+}
+
+__global__ __launch_bounds__(1024) void block_gemv_wide_kernel(const double* __restrict__ A,
+                                                               const int64_t* __restrict__ mat_off,
+                                                               const int32_t* __restrict__ row_off,
+                                                               const int32_t* __restrict__ sizes,
+                                                               const double* __restrict__ x, double* __restrict__ y,
+                                                               double alpha) {
+    block_gemv_wide(A, mat_off, row_off, sizes, x, y, alpha, (int)blockIdx.x);
 }
 
 // h[c] = D(:, c) . e for c < k: workgroup c, its four waves over rows
@@ -366,6 +372,128 @@ __global__ __launch_bounds__(1024) void end_small_kernel(const double* __restric
     if (tid == 0 && d_iter) {
         *d_iter = it + 1;
         if (pending) *pending = 0;
+    }
+}
+
+// First half of a device-counted step (the end of one iteration and the update
+// of the next): everything that reads the whole residual e = slot1 at once.
+// Workgroups by number: the nblocks blocks of y = alpha J0^{-1} e, the kmax
+// dots h[c] = D(:, c) . e (those of c < *d_iter), and one more for
+// sums = {||e - slot0||^2, (e - slot0) . e}.
+__global__ __launch_bounds__(1024) void step_parts_kernel(const double* __restrict__ A,
+                                                          const int64_t* __restrict__ mat_off,
+                                                          const int32_t* __restrict__ row_off,
+                                                          const int32_t* __restrict__ sizes, int nblocks,
+                                                          const double* __restrict__ e, double* __restrict__ y,
+                                                          double alpha, const double* __restrict__ D, int64_t ld,
+                                                          int kmax, int n, double* __restrict__ h,
+                                                          const int32_t* __restrict__ d_iter,
+                                                          const double* __restrict__ slot0,
+                                                          double* __restrict__ sums) {
+    const int b = (int)blockIdx.x;
+    if (b < nblocks) {
+        block_gemv_wide(A, mat_off, row_off, sizes, e, y, alpha, b);
+        return;
+    }
+    __shared__ double wsum[2][16];
+    const int c = b - nblocks, tid = (int)threadIdx.x;
+    const bool norm = c == kmax;
+    if (!norm && c >= *d_iter) return;
+    const double* d = D + (int64_t)c * ld;  // (norm: not read)
+    double s0 = 0.0, s1 = 0.0;
+    for (int r = tid; r < n; r += 1024) {
+        const double er = e[r];
+        const double dr = norm ? er - slot0[r] : d[r];
+        s0 += dr * er;
+        s1 += dr * dr;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        s0 += __shfl_down(s0, off, 64);
+        s1 += __shfl_down(s1, off, 64);
+    }
+    if ((tid & 63) == 0) {
+        wsum[0][tid >> 6] = s0;
+        wsum[1][tid >> 6] = s1;
+    }
+    __syncthreads();
+    if (tid != 0) return;
+    double t0 = 0.0, t1 = 0.0;
+    for (int w = 0; w < 16; ++w) {
+        t0 += wsum[0][w];
+        t1 += wsum[1][w];
+    }
+    if (norm) {
+        sums[0] = t1;
+        sums[1] = t0;
+    } else {
+        h[c] = t0;
+    }
+}
+
+// Second half.  v = y - C(:, 0:k) h is the update that the columns so far give
+// for the new residual, and the next column is C(:, k) = v / ||tD||, D(:, k) =
+// tD / ||tD|| with tD = slot1 - slot0 -- so the update with that column
+// too is v - C(:, k) (D(:, k) . slot1), without applying J0^{-1} and the columns a
+// second time.  Committed and counted as end_small_kernel does; with no
+// iteration pending the update is v.  64 rows per workgroup, four groups of
+// columns; the last workgroup to get there counts (*ticket goes back to 0).
+// One launch each for both halves, where the two updates took seven: 25 us of
+// the 100 that an iteration of 16 filaments of 20 and 2,000 blobs took.
+__global__ __launch_bounds__(256) void step_commit_kernel(const double* __restrict__ y, double* __restrict__ C,
+                                                          double* __restrict__ D, int64_t ld, int n, int kmax,
+                                                          const double* __restrict__ h, double* __restrict__ slot0,
+                                                          const double* __restrict__ slot1,
+                                                          const double* __restrict__ sums,
+                                                          const double* __restrict__ gate, int32_t* d_iter,
+                                                          int32_t* pending, int32_t* ticket,
+                                                          double* __restrict__ update) {
+    __shared__ double part[4][64];
+    const int l = (int)threadIdx.x & 63, q = (int)threadIdx.x >> 6;
+    const int r = (int)blockIdx.x * 64 + l;
+    const int it = *d_iter;
+    const bool due = *pending != 0;
+    const int k = it < kmax ? it : kmax;
+    const int cq = (k + 3) / 4;
+    const int c0 = q * cq, c1 = c0 + cq < k ? c0 + cq : k;
+    double s0 = 0.0, s1 = 0.0;
+    if (r < n) {
+        int c = c0;
+        for (; c + 8 <= c1; c += 8) {  // eight loads in flight per batch
+            double a[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) a[u] = C[(int64_t)(c + u) * ld + r];
+#pragma unroll
+            for (int u = 0; u < 8; u += 2) {
+                s0 += a[u] * h[c + u];
+                s1 += a[u + 1] * h[c + u + 1];
+            }
+        }
+        for (; c < c1; ++c) s0 += C[(int64_t)c * ld + r] * h[c];
+    }
+    part[q][l] = s0 + s1;
+    __syncthreads();
+    if (q == 0 && r < n) {
+        const double v = y[r] - ((part[0][l] + part[1][l]) + (part[2][l] + part[3][l]));
+        if (due && gate[0] > 1.0 && it < kmax) {
+            const double nrm = __builtin_sqrt(sums[0]);
+            const double inv = nrm > 0.0 ? 1.0 / nrm : 0.0;
+            const double e = slot1[r], cn = v * inv;
+            C[(int64_t)it * ld + r] = cn;
+            D[(int64_t)it * ld + r] = (e - slot0[r]) * inv;
+            slot0[r] = e;
+            update[r] = v - cn * (inv * sums[1]);
+        } else {
+            update[r] = v;
+        }
+    }
+    // every thread of the workgroup has used what it read of *d_iter and *pending
+    if (threadIdx.x == 0 && atomicAdd(ticket, 1) == (int)gridDim.x - 1) {
+        *ticket = 0;
+        if (due) {
+            *d_iter = it + 1;
+            *pending = 0;
+        }
     }
 }
 
@@ -516,18 +644,39 @@ __global__ __launch_bounds__(256) void body_balance_kernel(ResidualArgs a, doubl
     if (threadIdx.x < 6) err[s * per + 6 * nsw + threadIdx.x] = sm[threadIdx.x][0];
 }
 
+// out[0] = max |e|/tolerance, out[1] = nonfinite flag, and the bookkeeping
+// (book: see tfs::broyden_set_bookkeeping, may be null).
+__device__ __forceinline__ void residual_flags(double ratio, double nonfinite, double* __restrict__ out,
+                                               int32_t* __restrict__ book, int book_max) {
+    out[0] = ratio;
+    out[1] = nonfinite;
+    // one more iteration, unless the iterations had stopped; stop once the
+    // residual is small enough, not finite, or book_max iterations have run
+    if (book && !book[2]) {
+        book[0] += 1;
+        book[1] = nonfinite != 0.0 ? 0 : 1;
+        if (nonfinite != 0.0) book[2] = 2;
+        else if (!(ratio > 1.0) || book[0] >= book_max) book[2] = 1;
+    }
+}
+
 // One thread per segment (then one per body): 3 position and 3 Lie-algebra
 // residuals in the reference's storage order (mobility_solver.cpp:2661-2946),
 // evaluated without contraction in the reference's operation order.
 // partial[2*block] = max |e|/tolerance, partial[2*block+1] = 1 if any residual
-// of the block is not finite.
-__global__ __launch_bounds__(256) void residual_kernel(ResidualArgs a, double* __restrict__ err,
-                                                       double* __restrict__ partial) {
+// of the block is not finite.  A launch of one workgroup (up to kResidualOne
+// threads, a power of two) goes on to the flags itself: 4 us less than a
+// launch of their own.
+constexpr int kResidualOne = 1024;
+__global__ __launch_bounds__(kResidualOne) void residual_kernel(ResidualArgs a, double* __restrict__ err,
+                                                                double* __restrict__ partial,
+                                                                double* __restrict__ out, int32_t* __restrict__ book,
+                                                                int book_max) {
 #pragma clang fp contract(off)
-    __shared__ double sm[256];
-    __shared__ double sn[256];
+    __shared__ double sm[kResidualOne];
+    __shared__ double sn[kResidualOne];
     const int64_t nsegs = (int64_t)a.nswim * a.nfil * a.nseg;
-    const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const double c1 = -4.0 / 3.0, c2 = 1.0 / 3.0, c3 = -2.0 / 3.0;
     // per-swimmer stride of the Broyden vector
     const int64_t per = 6 * ((int64_t)a.nfil * a.nseg + 1) + 3LL * a.nblob;
@@ -627,21 +776,23 @@ __global__ __launch_bounds__(256) void residual_kernel(ResidualArgs a, double* _
     sm[threadIdx.x] = ratio;
     sn[threadIdx.x] = nonfinite;
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
+    for (int w = (int)blockDim.x / 2; w > 0; w >>= 1) {
         if (threadIdx.x < w) {
             sm[threadIdx.x] = fmax(sm[threadIdx.x], sm[threadIdx.x + w]);
             sn[threadIdx.x] = fmax(sn[threadIdx.x], sn[threadIdx.x + w]);
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
+    if (threadIdx.x != 0) return;
+    if (gridDim.x == 1) {
+        residual_flags(sm[0], sn[0], out, book, book_max);
+    } else {
         partial[2 * blockIdx.x] = sm[0];
         partial[2 * blockIdx.x + 1] = sn[0];
     }
 }
 
-// out[0] = max ratio, out[1] = nonfinite flag over nb partial pairs (one block).
-// (book: see tfs::broyden_set_bookkeeping, may be null)
+// The flags over nb partial pairs (one workgroup).
 __global__ __launch_bounds__(256) void residual_finish_kernel(const double* __restrict__ partial, int nb,
                                                               double* __restrict__ out, int32_t* __restrict__ book,
                                                               int book_max) {
@@ -662,19 +813,7 @@ __global__ __launch_bounds__(256) void residual_finish_kernel(const double* __re
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        out[0] = sm[0];
-        out[1] = sn[0];
-        // one more iteration, unless the iterations had stopped; stop once the
-        // residual is small enough, not finite, or book_max iterations have run
-        if (book && !book[2]) {
-            const bool nonfinite = sn[0] != 0.0;
-            book[0] += 1;
-            book[1] = nonfinite ? 0 : 1;
-            if (nonfinite) book[2] = 2;
-            else if (!(sm[0] > 1.0) || book[0] >= book_max) book[2] = 1;
-        }
-    }
+    if (threadIdx.x == 0) residual_flags(sm[0], sn[0], out, book, book_max);
 }
 
 int check(hipError_t e, const char* where) { return e == hipSuccess ? TFS_OK : hip_fail(e, where); }
@@ -732,6 +871,15 @@ hipMemcpyKind to_device(const tfs_broyden* b) {
     return host_mem(b) ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
 }
 
+// The free bodies' part of y = alpha J0^{-1} x, once y has the blocks' part.
+int apply_coupling(tfs_broyden* b, const double* x, double* y, double alpha) {
+    if (!b->coupled) return TFS_OK;
+    hipLaunchKernelGGL(coupling_apply_kernel, dim3(b->cpl_swim), dim3(256), 0, b->stream, (const double*)b->W,
+                       (const double*)b->BJ, (const double*)b->Sinv, b->cpl_fil, b->cpl_n6, b->cpl_blobs, x, y,
+                       alpha);
+    return check(hipGetLastError(), "J0^{-1} body coupling");
+}
+
 int apply_jinv(tfs_broyden* b, const double* x, double* y, double alpha) {
     if (b->max_block >= 64)
         hipLaunchKernelGGL(block_gemv_wide_kernel, dim3(b->nblocks), dim3(1024), 0, b->stream, b->J, b->mat_off,
@@ -740,13 +888,7 @@ int apply_jinv(tfs_broyden* b, const double* x, double* y, double alpha) {
         hipLaunchKernelGGL(block_gemv_kernel, dim3(b->nblocks), dim3(128), 0, b->stream, b->J, b->mat_off,
                            b->row_off, b->sizes, x, y, alpha);
     int rc = check(hipGetLastError(), "J0^{-1}");
-    if (!rc && b->coupled) {
-        hipLaunchKernelGGL(coupling_apply_kernel, dim3(b->cpl_swim), dim3(256), 0, b->stream, (const double*)b->W,
-                           (const double*)b->BJ, (const double*)b->Sinv, b->cpl_fil, b->cpl_n6, b->cpl_blobs, x, y,
-                           alpha);
-        rc = check(hipGetLastError(), "J0^{-1} body coupling");
-    }
-    return rc;
+    return rc ? rc : apply_coupling(b, x, y, alpha);
 }
 
 // out = -c J0^{-1} e - C(:, 0:iter) (D(:, 0:iter)^T e)
@@ -838,7 +980,7 @@ int tfs_broyden_create(const tfs_broyden_desc* desc, tfs_broyden** out) {
     if (e == hipSuccess) e = hipMalloc(&b->sizes, sizeof(int32_t) * D.num_blocks);
     if (e == hipSuccess) e = hipMalloc(&b->piv, sizeof(int32_t) * D.n);
     if (e == hipSuccess) e = hipMalloc(&b->status, sizeof(int32_t) * D.num_blocks);
-    if (e == hipSuccess) e = hipMalloc(&b->d_iter, sizeof(int32_t));
+    if (e == hipSuccess) e = hipMalloc(&b->d_iter, 2 * sizeof(int32_t));  // and a ticket
     if (e == hipSuccess) e = hipHostMalloc((void**)&b->host_scal, 64, hipHostMallocDefault);
     if (e == hipSuccess) {
         double* p = b->arena;
@@ -847,6 +989,7 @@ int tfs_broyden_create(const tfs_broyden_desc* desc, tfs_broyden** out) {
             p += round32(parts[i]);
         }
         e = hipMemsetAsync(b->arena, 0, total * 8, b->stream);
+        if (e == hipSuccess) e = hipMemsetAsync(b->d_iter, 0, 2 * sizeof(int32_t), b->stream);
     }
     if (e == hipSuccess)
         e = hipMemcpyAsync(b->mat_off, moff.data(), sizeof(int64_t) * D.num_blocks, hipMemcpyHostToDevice, b->stream);
@@ -1213,7 +1356,8 @@ static int errors_enqueue(tfs_broyden* b, const tfs_broyden_state* st, int32_t s
     if (!rc && ((nsegs && (!a.x || !a.xm1 || !a.u || !a.v || (a.bdf2 && (!a.xm2 || !a.um1)))) || !a.bx ||
                 !a.bxm1 || !a.bu || !a.bv || (a.bdf2 && (!a.bxm2 || !a.bum1))))
         rc = fail(TFS_ERR_OUT_OF_MEMORY, "tfs_broyden_compute_errors: staging");
-    const int blocks = (int)((nseg_tot + nb + nblob_tot + 255) / 256);
+    const int64_t rows = nseg_tot + nb + nblob_tot;
+    const int blocks = rows <= kResidualOne ? 1 : (int)((rows + 255) / 256);
     if (!rc && 2LL * blocks > std::max<int64_t>((int64_t)b->G * (b->max_iter + 1), 2LL * b->RB))
         rc = fail(TFS_ERR_INVALID_ARGUMENT, "tfs_broyden_compute_errors: state larger than the engine");
     if (!rc && a.free_bfe) {
@@ -1221,9 +1365,13 @@ static int errors_enqueue(tfs_broyden* b, const tfs_broyden_state* st, int32_t s
         rc = check(hipGetLastError(), "force and torque balance");
     }
     if (!rc) {
-        hipLaunchKernelGGL(residual_kernel, dim3(blocks), dim3(256), 0, b->stream, a, b->slot[slot], b->partial);
-        hipLaunchKernelGGL(residual_finish_kernel, dim3(1), dim3(256), 0, b->stream, b->partial, blocks,
+        int threads = 256;
+        while (blocks == 1 && threads < rows) threads *= 2;
+        hipLaunchKernelGGL(residual_kernel, dim3(blocks), dim3(threads), 0, b->stream, a, b->slot[slot], b->partial,
                            b->scal + 2, b->book, b->book_max);
+        if (blocks > 1)
+            hipLaunchKernelGGL(residual_finish_kernel, dim3(1), dim3(256), 0, b->stream, b->partial, blocks,
+                               b->scal + 2, b->book, b->book_max);
         rc = check(hipGetLastError(), "residual");
     }
     if (!rc && copy_flags)
@@ -1300,6 +1448,33 @@ int tfs::broyden_dev_end_of_iter(tfs_broyden* b, int32_t* pending) {
                        (const int32_t*)b->d_iter, b->max_iter, (const int32_t*)pending);
     hipLaunchKernelGGL(advance_count_kernel, dim3(1), dim3(64), 0, b->stream, b->d_iter, pending);
     return check(hipGetLastError(), "end of iteration");
+}
+
+bool tfs::broyden_dev_step_supported(const tfs_broyden* b, int max_iter) {
+    return b->n <= kEndSmall && b->max_iter > 1 && max_iter <= b->max_iter;
+}
+
+int tfs::broyden_dev_step_begin(tfs_broyden* b) {
+    return check(hipMemcpyAsync(b->slot[1], b->slot[0], (size_t)b->n * 8, hipMemcpyDeviceToDevice, b->stream),
+                 "first residual");
+}
+
+int tfs::broyden_dev_step(tfs_broyden* b, int32_t* pending, double* update) {
+    const int n = b->n, kmax = b->max_iter - 1;
+    const double* e = b->slot[1];
+    hipLaunchKernelGGL(step_parts_kernel, dim3((unsigned)(b->nblocks + kmax + 1)), dim3(1024), 0, b->stream,
+                       (const double*)b->J, (const int64_t*)b->mat_off, (const int32_t*)b->row_off,
+                       (const int32_t*)b->sizes, b->nblocks, e, b->tC, -b->desc.confidence, (const double*)b->D,
+                       (int64_t)b->ld, kmax, n, b->h, (const int32_t*)b->d_iter, (const double*)b->slot[0],
+                       b->scal + 4);
+    int rc = check(hipGetLastError(), "Broyden step");
+    if (!rc) rc = apply_coupling(b, e, b->tC, -b->desc.confidence);
+    if (rc) return rc;
+    hipLaunchKernelGGL(step_commit_kernel, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, b->stream,
+                       (const double*)b->tC, b->C, b->D, (int64_t)b->ld, n, kmax, (const double*)b->h, b->slot[0], e,
+                       (const double*)(b->scal + 4), (const double*)(b->scal + 2), b->d_iter, pending, b->d_iter + 1,
+                       update);
+    return check(hipGetLastError(), "Broyden step");
 }
 
 void tfs::broyden_dev_finish(tfs_broyden* b, int32_t iter, int32_t latest) {

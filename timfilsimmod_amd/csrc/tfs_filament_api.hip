@@ -365,10 +365,8 @@ __global__ void initial_guess_kernel(FilState S, FilParams P, int nt) {
     robot_arm(S, P, f);
 }
 
-// filament::internal_forces_and_torques, one thread per segment.
-__global__ void forces_kernel(FilState S, FilParams P, int nt, double* __restrict__ out) {
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= (int64_t)P.nfil * P.nseg) return;
+// filament::internal_forces_and_torques of segment g.
+__device__ void segment_forces(const FilState& S, const FilParams& P, int nt, int64_t g, double* __restrict__ out) {
     const int f = (int)(g / P.nseg), i = (int)(g % P.nseg), N = P.nseg;
     const int nm = 3 * (N + 1);
     const double* mult = S.mult + (int64_t)f * nm;
@@ -433,6 +431,11 @@ __global__ void forces_kernel(FilState S, FilParams P, int nt, double* __restric
         out[6 * g + k] = F[k];
         out[6 * g + 3 + k] = T[k];
     }
+}
+
+__global__ void forces_kernel(FilState S, FilParams P, int nt, double* __restrict__ out) {
+    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (g < (int64_t)P.nfil * P.nseg) segment_forces(S, P, nt, g, out);
 }
 
 __device__ __forceinline__ void put3(double* J, int64_t ld, int r, int c, const M3& B) {
@@ -565,14 +568,10 @@ __global__ __launch_bounds__(64) void jacobian_kernel(FilState S, FilParams P, i
     }
 }
 
-// filament::update (filament.cpp:1896-1930), one thread per segment: the
-// segment's Lie-algebra element and orientation, and its three multiplier
-// entries (segment 0 also the clamp's); the robot arm follows in
-// robot_arm_kernel.
-__global__ void update_kernel(FilState S, FilParams P, const double* __restrict__ du,
-                              const int32_t* __restrict__ stop) {
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= (int64_t)P.nfil * P.nseg || (stop && *stop)) return;
+// filament::update (filament.cpp:1896-1930) of segment g: its Lie-algebra
+// element and orientation, and its three multiplier entries (segment 0 also
+// the clamp's); the robot arm follows.
+__device__ void segment_update(const FilState& S, const FilParams& P, const double* __restrict__ du, int64_t g) {
     const int N = P.nseg, n6 = 6 * N;
     const int f = (int)(g / N), i = (int)(g % N);
     const int swim = f / P.fil_per_swim, fs = f % P.fil_per_swim;
@@ -607,17 +606,30 @@ __global__ void update_kernel(FilState S, FilParams P, const double* __restrict_
     store_q(S.q + 4 * g, qmul(lie_exp(S.u + 3 * g), load_q(S.qm1 + 4 * g)));
 }
 
+__global__ void update_kernel(FilState S, FilParams P, const double* __restrict__ du,
+                              const int32_t* __restrict__ stop) {
+    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (g < (int64_t)P.nfil * P.nseg && !(stop && *stop)) segment_update(S, P, du, g);
+}
+
 __global__ void robot_arm_kernel(FilState S, FilParams P) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f >= P.nfil) return;
     robot_arm(S, P, f);
 }
 
-// The robot arm for filaments of at most 64 segments: one wave per filament,
-// lane i the segment's step 0.5 DL (t_{i-1} + t_i), the positions x_0 plus an
-// inclusive scan of the steps over the lanes.
-__global__ __launch_bounds__(64) void robot_arm_wave_kernel(FilState S, FilParams P) {
+// The update, the robot arm and (out not null) the forces after it, for
+// filaments of at most 64 segments: one wave per filament, a lane per segment.
+// One launch: each of the three is bound by its launch (4 us).
+//
+// The robot arm: lane i the segment's step 0.5 DL (t_{i-1} + t_i), the
+// positions x_0 plus an inclusive scan of the steps over the lanes.
+__global__ __launch_bounds__(64) void advance_wave_kernel(FilState S, FilParams P, const double* __restrict__ du,
+                                                         const int32_t* __restrict__ stop, int nt,
+                                                         double* __restrict__ out) {
     const int f = blockIdx.x, i = threadIdx.x, N = P.nseg;
+    if (i < N && !(stop && *stop)) segment_update(S, P, du, (int64_t)f * N + i);
+    __syncthreads();  // the other lanes' multipliers and orientations, and x_0
     const int64_t s0 = (int64_t)f * N;
     double t[3] = {0.0, 0.0, 0.0};
     if (i < N) tangent(load_q(S.q + 4 * (s0 + i)), t);
@@ -638,6 +650,7 @@ __global__ __launch_bounds__(64) void robot_arm_wave_kernel(FilState S, FilParam
 #pragma unroll
         for (int k = 0; k < 3; ++k) S.x[3 * (s0 + i) + k] = S.x[3 * s0 + k] + d[k];
     }
+    if (out && i < N) segment_forces(S, P, nt, s0 + i, out);
 }
 
 // rigid_body::initial_guess (rigid_body.cpp:395-447), one thread per body.
@@ -1099,6 +1112,26 @@ unsigned grid_for(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
 }  // namespace
 
+// The state's update by du (device) and, where the filaments are short enough
+// for one launch, the forces at step nt after it (f_segs, device, may be null:
+// not wanted; see update_gives_forces).
+static hipError_t launch_update(tfs_filament* h, const double* du, int nt, double* f_segs) {
+    if (h->S.bx)
+        hipLaunchKernelGGL(body_update_kernel, dim3(grid_for(h->desc.num_swim, 64)), dim3(64), 0, h->stream, h->S,
+                           h->P, (int)h->desc.num_swim, du, h->update_stop);
+    if (h->P.nseg <= 64) {
+        hipLaunchKernelGGL(advance_wave_kernel, dim3((unsigned)h->P.nfil), dim3(64), 0, h->stream, h->S, h->P, du,
+                           h->update_stop, nt, f_segs);
+    } else {
+        hipLaunchKernelGGL(update_kernel, dim3(grid_for(num_segs(h), 256)), dim3(256), 0, h->stream, h->S, h->P, du,
+                           h->update_stop);
+        hipLaunchKernelGGL(robot_arm_kernel, dim3(grid_for(h->P.nfil, 64)), dim3(64), 0, h->stream, h->S, h->P);
+    }
+    return hipGetLastError();
+}
+
+static bool update_gives_forces(const tfs_filament* h) { return h->P.nseg <= 64; }
+
 extern "C" {
 
 int tfs_filament_create(const tfs_filament_desc* desc, tfs_filament** out) {
@@ -1297,20 +1330,7 @@ int tfs_filament_update(tfs_filament* h, const double* update) {
         e = hipMemcpyAsync(st, update, 8 * n, hipMemcpyHostToDevice, h->stream);
         du = st;
     }
-    if (e == hipSuccess && h->S.bx) {
-        hipLaunchKernelGGL(body_update_kernel, dim3(grid_for(h->desc.num_swim, 64)), dim3(64), 0, h->stream, h->S,
-                           h->P, (int)h->desc.num_swim, du, h->update_stop);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) {
-        hipLaunchKernelGGL(update_kernel, dim3(grid_for(num_segs(h), 256)), dim3(256), 0, h->stream, h->S, h->P, du,
-                           h->update_stop);
-        if (h->P.nseg <= 64)
-            hipLaunchKernelGGL(robot_arm_wave_kernel, dim3((unsigned)h->P.nfil), dim3(64), 0, h->stream, h->S, h->P);
-        else
-            hipLaunchKernelGGL(robot_arm_kernel, dim3(grid_for(h->P.nfil, 64)), dim3(64), 0, h->stream, h->S, h->P);
-        e = hipGetLastError();
-    }
+    if (e == hipSuccess) e = launch_update(h, du, 0, nullptr);
     if (e == hipSuccess && host) e = hipStreamSynchronize(h->stream);
     return check(e, "tfs_filament_update");
 }
@@ -1747,9 +1767,10 @@ int tfs_elastic_step(tfs_elastic* e, int32_t nt, tfs_elastic_stats* stats) {
     };
     // forces -> velocities -> residual in `slot` (enqueue_only: the residual's
     // flags are left for tfs::broyden_errors_result, nothing waits)
-    auto evaluate = [&](int slot, int32_t* too_large, bool enqueue_only = false, bool copy_flags = true) -> int {
+    auto evaluate = [&](int slot, int32_t* too_large, bool enqueue_only = false, bool copy_flags = true,
+                        bool have_forces = false) -> int {
         int rc = e->free_bodies ? tfs_filament_blob_positions(fh, e->x_blobs) : TFS_OK;
-        if (!rc) rc = tfs_filament_forces(fh, nt, e->f_segs);
+        if (!rc && !have_forces) rc = tfs_filament_forces(fh, nt, e->f_segs);
         if (!rc) rc = order(s_fil, s_vel);
         tfs_solve_stats vs{};
         if (!rc && e->rpy) {
@@ -1799,9 +1820,9 @@ int tfs_elastic_step(tfs_elastic* e, int32_t nt, tfs_elastic_stats* stats) {
         const int rc0 = tfs::rpy_near_reserve(rpyh, 0, rpyh->desc.num_segs + rpyh->desc.num_blobs);
         if (rc0) return rc0;
     }
-    auto evaluate_checked = [&](int slot, int32_t* too_large) -> int {
+    auto evaluate_checked = [&](int slot, int32_t* too_large, bool have_forces = false) -> int {
         for (int attempt = 0; attempt < 8; ++attempt) {
-            int rc = evaluate(slot, too_large);
+            int rc = evaluate(slot, too_large, false, true, have_forces);
             bool overflow = false;
             if (!rc) rc = tfs::rpy_near_check(rpyh, s_bro, &overflow);
             if (rc || !overflow) return rc;
@@ -1852,14 +1873,19 @@ int tfs_elastic_step(tfs_elastic* e, int32_t nt, tfs_elastic_stats* stats) {
     }
     if (!rc) rc = tfs_broyden_start(D.broyden, nullptr);
     // find_update -> the state's update (device_count: the engine's iteration
-    // count read on the device)
+    // count read on the device, and with `step` the end of the last iteration
+    // before it); those get the forces with the update
+    const bool step = tfs::broyden_dev_supported(D.broyden) && tfs::broyden_dev_step_supported(D.broyden, D.max_iter);
+    auto dev_update = [&](double* du) -> int {
+        return step ? tfs::broyden_dev_step(D.broyden, e->d_flags + 1, du)
+                    : tfs::broyden_dev_find_update(D.broyden, du);
+    };
     auto advance = [&](bool device_count) -> int {
         int rc2;
         if (e->rpy) {
             // the filament and body entries to the filament layout, the blob
             // entries onto the blob forces
-            rc2 = device_count ? tfs::broyden_dev_find_update(D.broyden, e->bfe_du)
-                               : tfs_broyden_find_update(D.broyden, e->bfe_du);
+            rc2 = device_count ? dev_update(e->bfe_du) : tfs_broyden_find_update(D.broyden, e->bfe_du);
             if (!rc2) rc2 = order(s_bro, s_fil);
             for (int64_t s = 0; s < nswim && !rc2; ++s)
                 rc2 = check(hipMemcpyAsync(e->du + s * (fil * n6 + 6), e->bfe_du + s * e->per, 8 * (fil * n6 + 6),
@@ -1872,11 +1898,14 @@ int tfs_elastic_step(tfs_elastic* e, int32_t nt, tfs_elastic_stats* stats) {
                 rc2 = check(hipGetLastError(), "blob force update");
             }
         } else {
-            rc2 = device_count ? tfs::broyden_dev_find_update(D.broyden, e->du)
-                               : tfs_broyden_find_update(D.broyden, e->du);
+            rc2 = device_count ? dev_update(e->du) : tfs_broyden_find_update(D.broyden, e->du);
         }
         if (!rc2 && !e->rpy) rc2 = order(s_bro, s_fil);
-        if (!rc2) rc2 = tfs_filament_update(fh, e->du);
+        if (!rc2 && device_count)
+            rc2 = check(launch_update(fh, e->du, (int)nt, update_gives_forces(fh) ? e->f_segs : nullptr),
+                        "tfs_elastic_step: update");
+        else if (!rc2)
+            rc2 = tfs_filament_update(fh, e->du);
         return rc2;
     };
     int32_t iter = 0;
@@ -1916,9 +1945,9 @@ int tfs_elastic_step(tfs_elastic* e, int32_t nt, tfs_elastic_stats* stats) {
             if (ce != hipSuccess) return hip_fail(ce, "tfs_elastic_step: begin capture");
             fh->update_stop = e->d_flags + 2;
             tfs::broyden_set_bookkeeping(D.broyden, e->d_flags, D.max_iter);
-            int rc2 = tfs::broyden_dev_end_of_iter(D.broyden, e->d_flags + 1);
+            int rc2 = which == 1 || !step ? tfs::broyden_dev_end_of_iter(D.broyden, e->d_flags + 1) : TFS_OK;
             if (!rc2 && which == 0) rc2 = advance(true);
-            if (!rc2 && which == 0) rc2 = evaluate(1, nullptr, true, false);
+            if (!rc2 && which == 0) rc2 = evaluate(1, nullptr, true, false, update_gives_forces(fh));
             tfs::broyden_set_bookkeeping(D.broyden, nullptr, 0);
             fh->update_stop = nullptr;
             hipError_t ee = hipStreamEndCapture(s_fil, &G.g[which]);
@@ -1929,6 +1958,7 @@ int tfs_elastic_step(tfs_elastic* e, int32_t nt, tfs_elastic_stats* stats) {
         };
         const bool roomy = rpyh->near[0].cap >= rpyh->desc.num_segs + rpyh->desc.num_blobs;
         rc = tfs::broyden_dev_begin(D.broyden);
+        if (!rc && step) rc = tfs::broyden_dev_step_begin(D.broyden);
         if (!rc) {
             hipLaunchKernelGGL(set_flags_kernel, dim3(1), dim3(64), 0, s_fil, e->d_flags, 0, 0, 0);
             rc = check(hipGetLastError(), "tfs_elastic_step: bookkeeping");
@@ -1985,7 +2015,29 @@ int tfs_elastic_step(tfs_elastic* e, int32_t nt, tfs_elastic_stats* stats) {
         if (!rc) tfs::broyden_dev_finish(D.broyden, iter, 1);
         if (!rc && stop == 2) rc = fail(TFS_ERR_NON_FINITE, "tfs_broyden_compute_errors: residual not finite");
     }
-    while (!graph_mode && !rc && big && iter < D.max_iter) {
+    // the same launches one by one, counted by the host
+    const bool counted = !graph_mode && !rc && big && step;
+    if (counted) {
+        rc = tfs::broyden_dev_begin(D.broyden);
+        if (!rc) rc = tfs::broyden_dev_step_begin(D.broyden);
+    }
+    auto set_pending = [&]() -> int {
+        hipLaunchKernelGGL(set_flags_kernel, dim3(1), dim3(64), 0, s_bro, e->d_flags, iter, iter > 0 ? 1 : 0, 0);
+        return check(hipGetLastError(), "tfs_elastic_step: bookkeeping");
+    };
+    while (counted && !rc && big && iter < D.max_iter) {
+        rc = set_pending();
+        if (!rc) rc = advance(true);
+        if (!rc) rc = evaluate_checked(1, &big, update_gives_forces(fh));
+        iter++;
+        e->eager_iters++;
+    }
+    if (counted && !rc && iter > 0) {
+        rc = set_pending();
+        if (!rc) rc = tfs::broyden_dev_end_of_iter(D.broyden, e->d_flags + 1);
+        if (!rc) tfs::broyden_dev_finish(D.broyden, iter, 1);
+    }
+    while (!graph_mode && !counted && !rc && big && iter < D.max_iter) {
         rc = advance(false);
         if (!rc) rc = evaluate_checked(1, &big);
         if (!rc) rc = tfs_broyden_end_of_iter(D.broyden, nullptr, big);

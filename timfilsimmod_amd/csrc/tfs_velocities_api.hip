@@ -335,7 +335,7 @@ int build_free_direct(tfs_velocities* v) {
         hipLaunchKernelGGL(kref_column_kernel, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, st,
                            (const double*)v->body_refs, nb, k, v->xpad);
         rc = check(hipGetLastError(), "K_ref column");
-        if (!rc) rc = check(k_symv_dense(v->Ainv, v->n_pad, v->xpad, v->ypad, v->sym_partial, v->chunks, st), "A K_ref");
+        if (!rc) rc = check(k_symv_dense(v->Ainv, v->n_pad, v->xpad, v->ypad, v->n_pad, v->sym_partial, v->chunks, st), "A K_ref");
         if (!rc) rc = check(hipMemcpyAsync(v->Z + k * n_pad, v->ypad, 8 * n_pad, hipMemcpyDeviceToDevice, st), "Z");
         if (!rc) {
             hipLaunchKernelGGL(kref_transpose_kernel, dim3(1), dim3(256), 0, st, (const double*)v->body_refs, nb,
@@ -527,21 +527,43 @@ int compute(tfs_velocities* v, const double* x_segs, const double* f_segs, const
     // With device memory the segment forces are read in place, the segment
     // velocities are summed straight into the caller's array, and the small
     // inputs arrive in one copy launch; a direct solve needs no warm start.
+    // One with prescribed body velocities reads the segments and the bodies
+    // and writes the blob forces in place too, so that blobs that did not move
+    // leave nothing to copy (two launches of about 4 us each).
     const bool dev = v->desc.memory == TFS_MEMORY_DEVICE;
     const bool direct_fixed = v->direct && !free_bodies;
+    const bool in_place = dev && direct_fixed;
+    struct InPlace {
+        tfs_rpy* h = nullptr;
+        double* own = nullptr;
+        ~InPlace() {
+            if (!h) return;
+            h->x_segs = own;
+            (void)tfs_rpy_positions_changed(h);
+        }
+    } segs;
+    if (in_place && ns) {
+        segs.h = h;
+        segs.own = h->x_segs;
+        h->x_segs = const_cast<double*>(x_segs);  // read only: nothing is uploaded to it below
+    }
+    const double* xb_in = in_place ? x_bodies : v->d_bodies;
+    const double* vb_in = in_place ? bodies : v->d_bodies + 3 * v->nswim;
     const double* fs_in = dev && ns ? f_segs : h->f_segs;
     double* vs_out = dev && ns ? v_segs : h->v_segs;
     double* sol = free_bodies ? v->d_sol : h->f_blobs;
     if (!rc && dev) {
         CopyList L;
-        L.add(x_blobs, h->x_blobs, 3 * nb);
-        if (ns) L.add(x_segs, h->x_segs, 3 * ns);
-        if (!v->direct) L.add(f_blobs, sol, 3 * nb);
-        if (free_bodies && !v->direct) L.add(v_bodies_io, sol + 3 * nb, 6 * v->nswim);
-        L.add(x_bodies, v->d_bodies, 3 * v->nswim);
-        if (bodies) L.add(bodies, v->d_bodies + 3 * v->nswim, 6 * v->nswim);
-        if (q_bodies) L.add(q_bodies, v->d_q, 4 * v->nswim);
-        rc = check(copy_list(L, st), "inputs");
+        if (!in_place || blobs_moved) L.add(x_blobs, h->x_blobs, 3 * nb);
+        if (!in_place) {
+            if (ns) L.add(x_segs, h->x_segs, 3 * ns);
+            if (!v->direct) L.add(f_blobs, sol, 3 * nb);
+            if (free_bodies && !v->direct) L.add(v_bodies_io, sol + 3 * nb, 6 * v->nswim);
+            L.add(x_bodies, v->d_bodies, 3 * v->nswim);
+            if (bodies) L.add(bodies, v->d_bodies + 3 * v->nswim, 6 * v->nswim);
+            if (q_bodies) L.add(q_bodies, v->d_q, 4 * v->nswim);
+        }
+        if (!in_place || blobs_moved) rc = check(copy_list(L, st), "inputs");
     } else if (!rc) {
         rc = check(hipMemcpyAsync(h->x_blobs, x_blobs, 24 * nb, kin, st), "blob positions");
         if (!rc && ns) rc = check(hipMemcpyAsync(h->x_segs, x_segs, 24 * ns, kin, st), "segment positions");
@@ -564,6 +586,7 @@ int compute(tfs_velocities* v, const double* x_segs, const double* f_segs, const
     if (!rc) v->have_blobs = true;
     if (!rc && blobs_moved) v->direct_valid = false;
     if (!rc && direct_fixed && !v->direct_valid) rc = build_direct(v, v->rpy->x_blobs);
+    double* fb_solved = in_place ? f_blobs : direct_fixed ? v->ypad : h->f_blobs;  // (ypad: made by build_direct)
     if (!rc && free_bodies) {
         hipLaunchKernelGGL(free_rhs_kernel, dim3((unsigned)v->nswim), dim3(256), 0, st, h->x_segs, fs_in,
                            h->v_blobs, nb, (int)v->desc.segs_per_swim, v->d_bodies,
@@ -573,7 +596,7 @@ int compute(tfs_velocities* v, const double* x_segs, const double* f_segs, const
     } else if (!rc) {
         // the direct solve reads its right-hand side from the padded vector
         hipLaunchKernelGGL(blob_rhs_kernel, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, st, h->v_blobs,
-                           h->x_blobs, v->d_bodies, v->d_bodies + 3 * v->nswim, (int)nb, v->desc.blobs_per_swim,
+                           h->x_blobs, xb_in, vb_in, (int)nb, v->desc.blobs_per_swim,
                            ns > 0 ? 1 : 0, direct_fixed ? v->xpad : v->d_rhs);
         rc = check(hipGetLastError(), "blob rhs");
     }
@@ -587,7 +610,9 @@ int compute(tfs_velocities* v, const double* x_segs, const double* f_segs, const
                                (const double*)v->d_q, v->xpad, v->small + 8);
             rc = check(hipGetLastError(), "body frame");
         }
-        if (!rc) rc = check(k_symv_dense(v->Ainv, v->n_pad, v->xpad, v->ypad, v->sym_partial, v->chunks, st), "direct solve");
+        if (!rc)
+            rc = check(k_symv_dense(v->Ainv, v->n_pad, v->xpad, v->ypad, v->n_pad, v->sym_partial, v->chunks, st),
+                       "direct solve");
         if (!rc) {
             hipLaunchKernelGGL(free_direct_velocity_kernel, dim3(1), dim3(256), 0, st, (const double*)v->body_refs,
                                (int)nb, (const double*)v->ypad, (const double*)(v->small + 8),
@@ -603,8 +628,9 @@ int compute(tfs_velocities* v, const double* x_segs, const double* f_segs, const
             stats->converged = 1;
         }
     } else if (!rc && v->direct) {
-        // blob forces = M_bb^{-1} rhs, left in ypad (its first 3 nb entries)
-        rc = check(k_symv_dense(v->Ainv, v->n_pad, v->xpad, v->ypad, v->sym_partial, v->chunks, st), "direct solve");
+        // blob forces = M_bb^{-1} rhs
+        rc = check(k_symv_dense(v->Ainv, v->n_pad, v->xpad, fb_solved, 3 * (int)nb, v->sym_partial, v->chunks, st),
+                   "direct solve");
         if (stats) {
             *stats = tfs_solve_stats{};
             stats->converged = 1;
@@ -616,10 +642,11 @@ int compute(tfs_velocities* v, const double* x_segs, const double* f_segs, const
             rc = check(hipMemcpyAsync(h->f_blobs, sol, 24 * nb, hipMemcpyDeviceToDevice, st), "blob forces");
     }
     const std::string solve_msg = solve_rc ? g_last_error : std::string();
-    const double* fb_solved = direct_fixed ? v->ypad : h->f_blobs;
     // Msb_mult '+='
     if (!rc && ns) rc = tfs_rpy_apply(h, TFS_BLOCK_SB, nullptr, fb_solved, vs_out, nullptr);
-    if (!rc && dev) {
+    if (!rc && in_place) {
+        // the blob forces are where they belong
+    } else if (!rc && dev) {
         CopyList L;
         L.add(fb_solved, f_blobs, 3 * nb);
         if (free_bodies) L.add(sol + 3 * nb, v_bodies_io, 6 * v->nswim);
