@@ -216,22 +216,26 @@ __device__ __forceinline__ void pair_near(double* __restrict__ v, double dx, dou
 // evaluated in T (double, or float as the reference's Real = float build
 // does).  Accumulates into v the velocity (VT = 3) or velocity and angular
 // velocity (VT = 6) of particle i due to the force (FS = 3) or force and
-// torque (FS = 6) f on particle j, given their separation (dx, dy, dz) =
-// xi - xj and heights zi, zj above the wall; `same` marks i and j as one
-// particle (the wall self-mobility).  Distinct particles take the unbounded
-// far-field form plus the image corrections; as in the reference, the
-// rotation-translation wall terms enter with the opposite sign to the
-// paper's printed alternating-tensor convention.
+// torque (FS = 6) on particle j, f being those over 6 pi, given their
+// separation (dx, dy, dz) = xi - xj and heights zi, zj above the wall; `same`
+// marks i and j as one particle (the wall self-mobility).  Distinct particles
+// take the unbounded far-field form plus the image corrections; as in the
+// reference, the rotation-translation wall terms enter with the opposite sign
+// to the paper's printed alternating-tensor convention.
+//
+// Bound by the FP64 operations, so they are arranged for few of them: the
+// horizontal separation is common to the particle and the image (at (xj, yj,
+// -zj), R = (dx, dy, zi + zj), p = 1/|R|, e = R p), so each vector has one
+// coefficient; and the image weight h = zj / (zi + zj) only ever comes with
+// e_z: h e_z = zj p and (1 - h) e_z = zi p, which leaves no division.
 template <typename T, int VT, int FS>
 __device__ inline void pair_wall(T* __restrict__ v, bool same, T dx, T dy, T dz, T zi, T zj,
                                  const T* __restrict__ f) {
-    const double PI = 3.14159265358979323846;
-    const T k6 = T(1.0 / (6.0 * PI)), k8 = T(1.0 / (8.0 * PI));
     if (same) {
         const T g1 = T(1) / zi, g3 = g1 * g1 * g1, g4 = g3 * g1, g5 = g4 * g1;
-        const T tpar = k6 - (T(9.0) * g1 - T(2.0) * g3 + g5) * (k6 / T(16.0));
-        const T tperp = k6 - (T(9.0) * g1 - T(4.0) * g3 + g5) * (k6 / T(8.0));
-        const T cpl = g4 * (k6 * T(3.0) / T(32.0));
+        const T tpar = T(1) - (T(9.0) * g1 - T(2.0) * g3 + g5) * T(1.0 / 16.0);
+        const T tperp = T(1) - (T(9.0) * g1 - T(4.0) * g3 + g5) * T(1.0 / 8.0);
+        const T cpl = g4 * T(3.0 / 32.0);
         v[0] += tpar * f[0];
         v[1] += tpar * f[1];
         v[2] += tperp * f[2];
@@ -243,8 +247,8 @@ __device__ inline void pair_wall(T* __restrict__ v, bool same, T dx, T dy, T dz,
             v[3] -= cpl * f[1];
             v[4] += cpl * f[0];
             if constexpr (FS == 6) {
-                const T rpar = k8 - g3 * (k6 * T(15.0) / T(64.0));
-                const T rperp = k8 - g3 * (k6 * T(3.0) / T(32.0));
+                const T rpar = T(0.75) - g3 * T(15.0 / 64.0);
+                const T rperp = T(0.75) - g3 * T(3.0 / 32.0);
                 v[3] += rpar * f[3];
                 v[4] += rpar * f[4];
                 v[5] += rperp * f[5];
@@ -252,82 +256,58 @@ __device__ inline void pair_wall(T* __restrict__ v, bool same, T dx, T dy, T dz,
         }
         return;
     }
-    // unbounded far field between the particles
-    {
-        const T q = rsqrt_refined(dx * dx + dy * dy + dz * dz);
-        const T ux = dx * q, uy = dy * q, uz = dz * q;
-        const T uf = ux * f[0] + uy * f[1] + uz * f[2];
-        const T ca = k8 * q, cb = T(1.0) + (T(2.0) / T(3.0)) * q * q, cc = (T(1.0) - T(2.0) * q * q) * uf;
-        v[0] += ca * (cb * f[0] + cc * ux);
-        v[1] += ca * (cb * f[1] + cc * uy);
-        v[2] += ca * (cb * f[2] + cc * uz);
-        const T c2 = ca * q;
-        if constexpr (FS == 6) {
-            v[0] += c2 * (f[4] * uz - f[5] * uy);
-            v[1] += c2 * (f[5] * ux - f[3] * uz);
-            v[2] += c2 * (f[3] * uy - f[4] * ux);
-        }
-        if constexpr (VT == 6) {
-            v[3] += c2 * (f[1] * uz - f[2] * uy);
-            v[4] += c2 * (f[2] * ux - f[0] * uz);
-            v[5] += c2 * (f[0] * uy - f[1] * ux);
-            if constexpr (FS == 6) {
-                const T c3 = T(0.5) * c2 * q, ut = ux * f[3] + uy * f[4] + uz * f[5];
-                v[3] += c3 * (T(3.0) * ut * ux - f[3]);
-                v[4] += c3 * (T(3.0) * ut * uy - f[4]);
-                v[5] += c3 * (T(3.0) * ut * uz - f[5]);
-            }
-        }
-    }
-    // image corrections: separation from the image of j at (xj, yj, -zj)
-    const T Rx = dx, Ry = dy, Rz = zi + zj;
-    const T p1 = rsqrt_refined(Rx * Rx + Ry * Ry + Rz * Rz);
-    const T p2 = p1 * p1, p3 = p2 * p1, p4 = p3 * p1, p5 = p4 * p1;
-    const T ex = Rx * p1, ey = Ry * p1, ez = Rz * p1, ez2 = ez * ez;
-    const T h = zj / Rz;
-    const T ef = ex * f[0] + ey * f[1] + ez * f[2];
-    {
-        const T t0 = -(T(0.75) * p1 * (T(1.0) + T(2.0) * h * (T(1.0) - h) * ez2) +
-                            T(0.5) * (p3 * (T(1.0) - T(3.0) * ez2) - p5 * (T(1.0) - T(5.0) * ez2)));
-        const T t12 = -(T(0.75) * p1 * (T(1.0) - T(6.0) * h * (T(1.0) - h) * ez2) - T(1.5) * p3 * (T(1.0) - T(5.0) * ez2) +
-                             T(2.5) * p5 * (T(1.0) - T(7.0) * ez2)) * ef +
-                           ez * f[2] *
-                               (T(1.5) * h * p1 * (T(1.0) - T(6.0) * (T(1.0) - h) * ez2) - T(3.0) * p3 * (T(1.0) - T(5.0) * ez2) +
-                                T(5.0) * p5 * (T(2.0) - T(7.0) * ez2));
-        const T t3 = (T(1.5) * h * p1 - T(5.0) * p5) * ef;
-        const T t4 = -((T(3.0) * h * h * p1 + T(3.0) * p3) * ez2 + (T(2.0) - T(15.0) * ez2) * p5) * f[2];
-        v[0] += k6 * (t0 * f[0] + t12 * ex);
-        v[1] += k6 * (t0 * f[1] + t12 * ey);
-        v[2] += k6 * (t0 * f[2] + (t12 + t3) * ez + t4);
-    }
-    if constexpr (VT == 6) {
-        const T u0 = T(0.75) * p2;
-        const T u12 = f[2] * (T(9.0) * h * ez2 * p2 + (T(1.5) - T(15.0) * ez2) * p4) - ez * ef * (T(4.5) * h * p2 - T(7.5) * p4);
-        const T u3 = -T(1.5) * ez * (h * p2 - p4);
-        v[3] -= k6 * (u0 * (f[1] * ez - f[2] * ey) - u12 * ey + u3 * f[1]);
-        v[4] -= k6 * (u0 * (f[2] * ex - f[0] * ez) + u12 * ex - u3 * f[0]);
-        v[5] -= k6 * u0 * (f[0] * ey - f[1] * ex);
-        if constexpr (FS == 6) {
-            const T et = ex * f[3] + ey * f[4] + ez * f[5];
-            const T w0 = p3 * (T(0.375) - T(2.25) * ez2), w1 = -T(1.125) * p3 * et, w2 = T(2.25) * ez * p3 * et;
-            const T w3 = T(2.25) * p3 * (ex * f[4] - ey * f[3]);
-            v[3] += k6 * (w0 * f[3] + w1 * ex - w3 * ey);
-            v[4] += k6 * (w0 * f[4] + w1 * ey + w3 * ex);
-            v[5] += k6 * (w0 * f[5] + w1 * ez + w2);
-        }
-    }
+    const T Rz = zi + zj, s2 = dx * dx + dy * dy;
+    const T q = rsqrt_refined(s2 + dz * dz), p = rsqrt_refined(s2 + Rz * Rz);
+    const T q2 = q * q, q3 = q2 * q;
+    const T p2 = p * p, p3 = p2 * p, p4 = p2 * p2, p5 = p4 * p;
+    const T fh = dx * f[0] + dy * f[1];          // horizontal part of both d . f and R . f
+    const T A = q * (T(0.75) + T(0.5) * q2), B = q3 * (T(0.75) - T(1.5) * q2) * (fh + dz * f[2]);
+    const T C = T(0.75) * q3;
+    const T ez = Rz * p, ez2 = ez * ez, zt = zj * p, et = zi * p;   // e_z, h e_z, (1 - h) e_z
+    const T ef = p * (fh + Rz * f[2]);
+    const T he = zt * et, ee = et * ez, zp = T(1.5) * (zt * p), p75 = T(0.75) * p, p55 = T(5.0) * p5;
+    const T y5 = T(1.0) - T(5.0) * ez2, y7 = T(1.0) - T(7.0) * ez2, y15 = T(1.5) - T(15.0) * ez2;
+    const T p3y = p3 * y5, p4e = p4 * ez;
+    // coefficient of the force, and of e (its horizontal and vertical parts)
+    const T t0 = A - (p75 * (T(1.0) + T(2.0) * he) + T(0.5) * (p3 * (T(1.0) - T(3.0) * ez2) - p5 * y5));
+    const T t1 = f[2] * (zp * (T(1.0) - T(6.0) * ee) + ez * (p55 * (y7 + T(1.0)) - T(3.0) * p3y)) -
+                 ef * (p75 * (T(1.0) - T(6.0) * he) - T(1.5) * p3y + T(0.5) * p55 * y7);
+    T vz = t0 * f[2] + B * dz + t1 * ez + ef * (zp - p55 * ez) -
+           f[2] * (T(2.0) * (zp * zt) + T(3.0) * (p3 * ez2) + p5 * (y15 + T(0.5)));
+    T ch = t1;
+    const T u0 = T(0.75) * p2, M2 = u0 * p - C, Cz = C * dz;
     if constexpr (FS == 6) {
-        // translation from torque: transpose of the rotation-from-force block
-        // seen from j (image weight 1 - h, e_x and e_y reversed)
-        const T hh = T(1.0) - h, fx = -ex, fy = -ey;
-        const T ext = fx * f[4] - fy * f[3];
-        const T q0 = T(0.75) * p2;
-        const T q1 = (T(9.0) * hh * ez2 * p2 + (T(1.5) - T(15.0) * ez2) * p4) * ext;
-        const T q2 = -ez * (T(4.5) * hh * p2 - T(7.5) * p4) * ext;
-        const T q3 = -T(1.5) * ez * (hh * p2 - p4);
-        v[0] -= k6 * (q0 * (f[5] * fy - f[4] * ez) + q2 * fx - q3 * f[4]);
-        v[1] -= k6 * (q0 * (f[3] * ez - f[5] * fx) + q2 * fy + q3 * f[3]);
-        v[2] -= k6 * (q0 * (f[4] * fx - f[3] * fy) + q2 * ez + q1);
+        // translation from torque
+        const T sp = dx * f[4] - dy * f[3], s = p * sp;
+        const T ep2 = et * p2, c2 = s * (T(4.5) * ep2 - T(7.5) * p4e);
+        const T M1 = Cz + u0 * ez - T(1.5) * (ep2 - p4e), m = M2 * f[5];
+        ch += c2;
+        v[0] += M1 * f[4] + m * dy;
+        v[1] -= M1 * f[3] + m * dx;
+        vz += M2 * sp + s * (T(9.0) * (ee * p2) + y15 * p4) - c2 * ez;
+    }
+    const T P = B + p * ch;
+    v[0] += t0 * f[0] + P * dx;
+    v[1] += t0 * f[1] + P * dy;
+    v[2] += vz;
+    if constexpr (VT == 6) {
+        const T zp2 = zt * p2;
+        const T N1 = Cz - u0 * ez + T(1.5) * (zp2 - p4e);
+        T n = u0 * f[2] + f[2] * (T(9.0) * (zp2 * ez) + y15 * p4) - ef * (T(4.5) * zp2 - T(7.5) * p4e);
+        if constexpr (FS == 6) {
+            const T th = dx * f[3] + dy * f[4];
+            const T tt = p * (th + Rz * f[5]), w = T(1.125) * p3;
+            const T E = T(1.125) * (q3 * q2) * (th + dz * f[5]);
+            const T T1 = p3 * (T(0.375) - T(2.25) * ez2) - T(0.5) * C, w1 = w * tt, Q = E - w1 * p;
+            n -= T(2.0) * w * (p * (dx * f[4] - dy * f[3]));
+            v[3] += T1 * f[3] + Q * dx;
+            v[4] += T1 * f[4] + Q * dy;
+            v[5] += T1 * f[5] + E * dz + w1 * ez;
+        }
+        const T N2 = p * n - C * f[2];
+        v[3] += N1 * f[1] + N2 * dy;
+        v[4] -= N1 * f[0] + N2 * dx;
+        v[5] -= M2 * (dy * f[0] - dx * f[1]);
     }
 }
 

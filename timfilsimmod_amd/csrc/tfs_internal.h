@@ -251,9 +251,10 @@ hipError_t launch_matvec_reduce(int precision, int seg_dof, const TileShape& sha
 
 // Half-space domain (no-slip wall at z = 0): the wall pair kernel (FP64, or
 // FP32 tiles from fixed-point separations) over a work list of
-// kWallBlock-target tiles (one target per lane), then the reduce kernel
-// without near-pair terms.
+// kWallTile-target tiles (one target per lane, the waves of a workgroup
+// dividing the sources), then the reduce kernel without near-pair terms.
 constexpr int kWallBlock = 256;
+constexpr int kWallTile = 64;
 hipError_t launch_wall_pairs(int precision, int seg_dof, const MatvecArgs& a, const MatvecTile* d_tiles, int n_tiles,
                              const MatvecItem* d_items, int n_items, double* partial, hipStream_t stream,
                              hipEvent_t ev_begin, hipEvent_t ev_end);
