@@ -113,7 +113,9 @@ int arnoldi_blocks(int64_t n);
 // Nothing happens while *skip (if given) is nonzero.
 hipError_t k_scale_precond(const double* w, const double* dev_scale, double host_scale, double* v, double* out,
                            const PrecondArgs& P, const SaddleDims& d, const int32_t* skip, hipStream_t s);
-hipError_t k_precond(const double* in, double* out, const PrecondArgs& P, const SaddleDims& d, hipStream_t s);
+// (nothing where stopped is given and *stopped >= all)
+hipError_t k_precond(const double* in, double* out, const PrecondArgs& P, const SaddleDims& d, hipStream_t s,
+                     const int32_t* stopped = nullptr, int all = 0);
 // Block preconditioner set-up (kind 1).  fil_blk / patch_blk receive the
 // blocks of D (to be inverted in place by k_batched_inverse); k_fil_schur then
 // forms fil_dk and fil_sinv from the inverted filament blocks.
@@ -149,16 +151,21 @@ struct EnsArgs {
     int mstride = 0;
     double* scal = nullptr;
     int32_t* stop = nullptr;
-    int32_t* nstop = nullptr;         // bodies that stopped since it was cleared
+    int32_t* nstop = nullptr;         // bodies that do not run (any more)
+    const int32_t* map = nullptr;     // operator index of each Krylov index
+    const double* w_op = nullptr;     // w = A z in the operator layout
+    double* v_op = nullptr;           // v_{j+1} in the operator layout
     const double* abs_tol = nullptr;  // per body
     double *pa = nullptr, *pb = nullptr;
     int64_t pstride = 0;
     int64_t* stamps = nullptr;        // per body: wall clock of its last stop (may be null)
 };
 // Gram-Schmidt step j of every running body, G x nbody workgroups per launch:
-// passes = 2 (CGS2, three launches) or 1 (CGS, two launches).
+// passes = 2 (CGS2, three launches) or 1 (CGS, two launches).  w is taken from
+// the operator layout (w_op).
 hipError_t k_ens_arnoldi_step(const EnsArgs& e, int j, int G, int passes, hipStream_t s);
-// Close step j of every running body; with write_next, v_{j+1} into the basis.
+// Close step j of every running body; with write_next, v_{j+1} into the basis
+// and the operator layout (v_op).
 hipError_t k_ens_close(const EnsArgs& e, int j, bool write_next, int G, hipStream_t s);
 // v_0 = r / ||r|| and g = (||r||, 0, ...) for every running body (r in the Krylov layout).
 hipError_t k_ens_open(const EnsArgs& e, const double* r, const double* rnorm, int G, hipStream_t s);

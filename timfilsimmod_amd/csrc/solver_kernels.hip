@@ -764,7 +764,9 @@ __global__ __launch_bounds__(256) void arnoldi_close_next_kernel(
 // D = I/(6 pi mu a) (mobility_solver.cpp:1040-1116).  Blob rows are scaled by
 // 6 pi mu a_b.  Filament waves first, then a grid-stride over blob entries.
 __global__ __launch_bounds__(256) void precond_kernel(const double* __restrict__ in, double* __restrict__ out,
-                                                     PrecondArgs P, SaddleDims d) {
+                                                     PrecondArgs P, SaddleDims d,
+                                                     const int32_t* __restrict__ stopped, int all) {
+    if (stopped && *stopped >= all) return;
     if (P.kind == 1) {
         block_precond_body(P, d, in, 1.0, nullptr, out);
         return;
@@ -1287,9 +1289,18 @@ __device__ __forceinline__ ArnoldiArgs ens_slice(const EnsArgs& e, int b, int nc
     return ArnoldiArgs{e.V + e.koff[b], e.ld, ncols, e.w + e.koff[b], (int)(e.koff[b + 1] - e.koff[b]), nullptr};
 }
 
+// The first projection takes its slice of w from the operator layout.
 __global__ __launch_bounds__(256) void ens_dots_kernel(EnsArgs e, int ncols, int to_pb) {
     const int b = blockIdx.y;
     if (e.stop[b]) return;
+    const int64_t o = e.koff[b], n = e.koff[b + 1] - o;
+    for (int64_t r0 = (int64_t)blockIdx.x * kSlice; r0 < n; r0 += (int64_t)gridDim.x * kSlice)
+#pragma unroll
+        for (int q = 0; q < kSlice / 256; ++q) {
+            const int64_t r = r0 + q * 256 + threadIdx.x;
+            if (r < n) e.w[o + r] = e.w_op[e.map[o + r]];
+        }
+    __syncthreads();
     slice_dots(ens_slice(e, b, ncols), (to_pb ? e.pb : e.pa) + (int64_t)b * e.pstride, blockIdx.x, gridDim.x);
 }
 
@@ -1329,7 +1340,8 @@ __global__ __launch_bounds__(256) void ens_update_sumsq_kernel(EnsArgs e, int nc
 
 // Closes step j of every running body (||w|| from its partial sums, Givens,
 // estimate, stop flag; the body's workgroup 0) and, with write_next, writes
-// v_{j+1} = w / ||w|| into column j + 1 of its basis.  A body that stops here
+// v_{j+1} = w / ||w|| into column j + 1 of its basis and into the operator
+// layout.  A body that stops here
 // is counted in *nstop and stamped (wall clock) in stamps[b].
 __global__ __launch_bounds__(256) void ens_close_kernel(EnsArgs e, int j, int write_next) {
     __shared__ double nrm;
@@ -1355,7 +1367,10 @@ __global__ __launch_bounds__(256) void ens_close_kernel(EnsArgs e, int j, int wr
         const int64_t o = e.koff[b], n = e.koff[b + 1] - o;
         double* v = e.V + (int64_t)(j + 1) * e.ld + o;
         const double* w = e.w + o;
-        for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < n; r += (int64_t)gridDim.x * 256) v[r] = w[r] * sc;
+        for (int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x; r < n; r += (int64_t)gridDim.x * 256) {
+            v[r] = w[r] * sc;
+            e.v_op[e.map[o + r]] = w[r] * sc;
+        }
     }
 }
 
@@ -1382,14 +1397,30 @@ __global__ __launch_bounds__(256) void ens_permute_kernel(const double* __restri
 }
 
 // out[b] = ||v_b|| over body b's rows (one workgroup per body, fixed order).
-__global__ __launch_bounds__(256) void ens_norms_kernel(const double* __restrict__ v, const int64_t* __restrict__ koff,
-                                                        double* __restrict__ out) {
-    __shared__ double sh[4];
-    const int b = blockIdx.x;
-    double s = 0.0;
-    for (int64_t i = koff[b] + threadIdx.x; i < koff[b + 1]; i += 256) s += v[i] * v[i];
-    s = block_sum256(s, sh);
-    if (threadIdx.x == 0) out[b] = __builtin_sqrt(s);
+// Bound by the loads in flight: four per thread of 1024 (36 us with one per
+// thread of 256, six bodies of up to 44,000 rows).
+__global__ __launch_bounds__(1024) void ens_norms_kernel(const double* __restrict__ v,
+                                                         const int64_t* __restrict__ koff, double* __restrict__ out) {
+    __shared__ double sh[16];
+    const int b = blockIdx.x, tid = (int)threadIdx.x;
+    const int64_t hi = koff[b + 1];
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    int64_t i = koff[b] + tid;
+    for (; i + 3 * 1024 < hi; i += 4 * 1024) {
+        double x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = v[i + u * 1024];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s[u] += x[u] * x[u];
+    }
+    for (; i < hi; i += 1024) s[0] += v[i] * v[i];
+    const double t = wave_sum((s[0] + s[1]) + (s[2] + s[3]));
+    if ((tid & (kWave - 1)) == 0) sh[tid / kWave] = t;
+    __syncthreads();
+    if (tid != 0) return;
+    double all = 0.0;
+    for (int w = 0; w < 16; ++w) all += sh[w];
+    out[b] = __builtin_sqrt(all);
 }
 
 // Iterations of body b in the cycle just run: the stopping step, all m if it
@@ -1565,8 +1596,9 @@ hipError_t k_sub(const double* x, const double* y, double* out, int n, hipStream
     hipLaunchKernelGGL(sub_kernel, dim3(blocks_for(n)), dim3(256), 0, s, x, y, out, n);
     return hipGetLastError();
 }
-hipError_t k_precond(const double* in, double* out, const PrecondArgs& P, const SaddleDims& d, hipStream_t s) {
-    hipLaunchKernelGGL(precond_kernel, dim3(blocks_for(precond_work(P, d))), dim3(256), 0, s, in, out, P, d);
+hipError_t k_precond(const double* in, double* out, const PrecondArgs& P, const SaddleDims& d, hipStream_t s,
+                     const int32_t* stopped, int all) {
+    hipLaunchKernelGGL(precond_kernel, dim3(blocks_for(precond_work(P, d))), dim3(256), 0, s, in, out, P, d, stopped, all);
     return hipGetLastError();
 }
 hipError_t k_fil_blocks(const double* x_segs, int nfil, int nseg, double a_seg, double mu, double* fil_blk,
@@ -1691,7 +1723,7 @@ hipError_t k_ens_permute(const double* src, double* dst, const int32_t* map, int
     return hipGetLastError();
 }
 hipError_t k_ens_norms(const double* v, const int64_t* koff, int nbody, double* out, hipStream_t s) {
-    hipLaunchKernelGGL(ens_norms_kernel, dim3((unsigned)nbody), dim3(256), 0, s, v, koff, out);
+    hipLaunchKernelGGL(ens_norms_kernel, dim3((unsigned)nbody), dim3(1024), 0, s, v, koff, out);
     return hipGetLastError();
 }
 hipError_t k_ens_update(const EnsArgs& e, int m, double* y, int32_t* kdone, double* out, int G, hipStream_t s) {

@@ -67,6 +67,12 @@ hipError_t k_fill(double* p, double v, int64_t n, hipStream_t s) {
 // body -- and the Krylov vectors live in the bodies' own layout, body b's
 // unknowns contiguous at koff[b]; map[i] is the operator index of Krylov
 // index i.
+// Steps of a captured piece of a lock-step cycle.  The next piece is launched
+// before the host has looked at the last one's count of stopped bodies, so up
+// to two pieces run empty once every body has stopped (28 us a step): short
+// pieces, of which each costs the copy and the event after it (10 us).
+constexpr int kEnsPiece = 5;
+
 struct EnsState {
     int nbody = 0;
     std::vector<int32_t> fil, blob;   // per body
@@ -92,9 +98,18 @@ struct EnsState {
     std::vector<double> relres;
     // captured cycles (one per precision) and the pointers / values they hold
     bool use_graphs = true;
-    hipGraph_t graph[2] = {nullptr, nullptr};
-    hipGraphExec_t exec[2] = {nullptr, nullptr};
+    std::vector<hipGraph_t> graph[2];     // kEnsPiece steps each
+    std::vector<hipGraphExec_t> exec[2];
     std::vector<uintptr_t> key[2];
+    hipEvent_t piece_done[2] = {nullptr, nullptr};
+    void drop_graphs(int p) {
+        for (hipGraphExec_t x : exec[p])
+            if (x) (void)hipGraphExecDestroy(x);
+        for (hipGraph_t g : graph[p])
+            if (g) (void)hipGraphDestroy(g);
+        exec[p].clear();
+        graph[p].clear();
+    }
     int64_t graph_launches = 0, eager_cycles = 0;
 };
 
@@ -646,6 +661,9 @@ EnsArgs ens_args(tfs_solver* s) {
     a.scal = E.scal;
     a.stop = E.stop;
     a.nstop = E.nstop;
+    a.map = E.d_map;
+    a.w_op = s->w;
+    a.v_op = s->t;
     a.abs_tol = E.abs_tol;
     a.pa = E.pa;
     a.pb = E.pb;
@@ -667,9 +685,10 @@ int ens_norms(tfs_solver* s, const double* v, std::vector<double>& norms) {
 }
 
 // Lock-step steps j0 <= j < j1 of the current cycle (no host round trip):
-// w = A z with the stopped bodies' work skipped, w to the Krylov layout, the
-// Gram-Schmidt step (twice in FP64 solves, once in the inner solve of mixed
-// refinement) and close of every running body, v_{j+1} and z = P^{-1} v_{j+1}.
+// w = A z with the stopped bodies' work skipped, the Gram-Schmidt step (twice in
+// FP64 solves, once in the inner solve of mixed refinement) and close of every
+// running body, which take w from the operator layout and put v_{j+1} there,
+// and z = P^{-1} v_{j+1}.
 int ens_enqueue_steps(tfs_solver* s, int precision, int j0, int j1) {
     EnsState& E = *s->ens;
     const EnsArgs a = ens_args(s);
@@ -678,22 +697,18 @@ int ens_enqueue_steps(tfs_solver* s, int precision, int j0, int j1) {
         s->rpy->body_skip = E.stop;
         int rc = apply_A(s, s->z, s->w, precision, nullptr);
         s->rpy->body_skip = nullptr;
-        if (!rc) rc = check(k_ens_permute(s->w, E.w, E.d_map, E.ntot, false, s->stream), "w to the Krylov layout");
         if (!rc)
             rc = check(k_ens_arnoldi_step(a, j, E.G, precision == TFS_PRECISION_FP64 ? 2 : 1, s->stream),
                        "lock-step Arnoldi");
         if (!rc) rc = check(k_ens_close(a, j, j + 1 < m, E.G, s->stream), "lock-step close");
-        if (!rc && j + 1 < m) {
-            rc = check(k_ens_permute(E.V + (int64_t)(j + 1) * E.ldv, s->t, E.d_map, E.ntot, true, s->stream),
-                       "v to the operator layout");
-            if (!rc) rc = check(k_precond(s->t, s->z, precond_args(s), s->dims, s->stream), "preconditioner");
-        }
+        if (!rc && j + 1 < m)
+            rc = check(k_precond(s->t, s->z, precond_args(s), s->dims, s->stream, E.nstop, E.nbody), "preconditioner");
         if (rc) return rc;
     }
     return TFS_OK;
 }
 
-// The m steps of a cycle as one hipGraph, captured again only when something
+// The m steps of a cycle as hipGraphs of kEnsPiece steps, captured again only when something
 // the launches hold by value or pointer changed (the work list, partial
 // buffer, near-pair lists, fixed-point positions).
 int ens_cycle_graph(tfs_solver* s, int precision) {
@@ -720,35 +735,31 @@ int ens_cycle_graph(tfs_solver* s, int precision) {
                                         (uintptr_t)sh.symmetric,
                                         (uintptr_t)s->precond_kind,
                                         (uintptr_t)s->npatch};
-    if (E.exec[precision] && E.key[precision] == key) return TFS_OK;
-    if (E.exec[precision]) (void)hipGraphExecDestroy(E.exec[precision]);
-    if (E.graph[precision]) (void)hipGraphDestroy(E.graph[precision]);
-    E.exec[precision] = nullptr;
-    E.graph[precision] = nullptr;
+    if (!E.exec[precision].empty() && E.key[precision] == key) return TFS_OK;
+    E.drop_graphs(precision);
+    for (hipEvent_t& ev : E.piece_done)
+        if (!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess)
+            return fail(TFS_ERR_HIP, "lock-step cycle: events");
     const bool prof = h->profiling, timing = h->body_timing;
-    h->profiling = false;
+    h->profiling = false;  // timing events and stamps are not captured
     h->body_timing = false;
-    hipError_t e = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);
-    if (e != hipSuccess) {
-        h->profiling = prof;
-        h->body_timing = timing;
-        return hip_fail(e, "lock-step cycle: begin capture");
+    hipError_t e = hipSuccess;
+    for (int j0 = 0; j0 < s->m && !rc && e == hipSuccess; j0 += kEnsPiece) {
+        e = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);
+        if (e != hipSuccess) break;
+        hipGraph_t g = nullptr;
+        hipGraphExec_t x = nullptr;
+        rc = ens_enqueue_steps(s, precision, j0, std::min(s->m, j0 + kEnsPiece));
+        e = hipStreamEndCapture(s->stream, &g);
+        if (!rc && e == hipSuccess) e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
+        if (g) E.graph[precision].push_back(g);
+        if (x) E.exec[precision].push_back(x);
     }
-    rc = ens_enqueue_steps(s, precision, 0, s->m);
-    hipError_t e2 = hipStreamEndCapture(s->stream, &E.graph[precision]);
     h->profiling = prof;
     h->body_timing = timing;
-    if (rc || e2 != hipSuccess) {
-        if (E.graph[precision]) (void)hipGraphDestroy(E.graph[precision]);
-        E.graph[precision] = nullptr;
-        return rc ? rc : hip_fail(e2, "lock-step cycle: end capture");
-    }
-    e = hipGraphInstantiate(&E.exec[precision], E.graph[precision], nullptr, nullptr, 0);
-    if (e != hipSuccess) {
-        (void)hipGraphDestroy(E.graph[precision]);
-        E.graph[precision] = nullptr;
-        E.exec[precision] = nullptr;
-        return hip_fail(e, "lock-step cycle: instantiate");
+    if (rc || e != hipSuccess) {
+        E.drop_graphs(precision);
+        return rc ? rc : hip_fail(e, "lock-step cycle: capture");
     }
     E.key[precision] = key;
     return TFS_OK;
@@ -795,7 +806,7 @@ int gmres_batched(tfs_solver* s, int precision, const double* rhs, double* x, do
         // open the cycle: stop flags, H = 0, v_0 = r / ||r||, z = P^{-1} v_0
         for (int b = 0; b < nb; ++b) E.h_i32[b] = active[b] ? 0 : kEnsInactive;
         rc = check(hipMemcpyAsync(E.stop, E.h_i32, 4LL * nb, hipMemcpyHostToDevice, s->stream), "stop flags");
-        if (!rc) rc = check(k_fill_int(E.nstop, 0, 1, s->stream), "stop count");
+        if (!rc) rc = check(k_fill_int(E.nstop, nb - n_active, 1, s->stream), "stop count");
         if (!rc) rc = check(k_fill(E.H, 0.0, (int64_t)nb * E.hstride, s->stream), "H");
         if (!rc) rc = check(k_ens_open(a, E.rk, E.norms, E.G, s->stream), "v0");
         if (!rc) rc = check(k_ens_permute(E.V, s->t, E.d_map, E.ntot, true, s->stream), "v0 to the operator layout");
@@ -804,7 +815,17 @@ int gmres_batched(tfs_solver* s, int precision, const double* rhs, double* x, do
         int launched = m;
         if (E.use_graphs) {
             rc = ens_cycle_graph(s, precision);
-            if (!rc) rc = check(hipGraphLaunch(E.exec[precision], s->stream), "lock-step cycle graph");
+            launched = 0;
+            for (size_t p = 0; p < E.exec[precision].size() && !rc; ++p) {
+                hipError_t e = hipGraphLaunch(E.exec[precision][p], s->stream);
+                if (e == hipSuccess) e = hipMemcpyAsync(E.h_i32 + nb, E.nstop, 4, hipMemcpyDeviceToHost, s->stream);
+                if (e == hipSuccess) e = hipEventRecord(E.piece_done[p & 1], s->stream);
+                launched = std::min(m, launched + kEnsPiece);
+                if (e == hipSuccess && p > 0) e = hipEventSynchronize(E.piece_done[(p - 1) & 1]);
+                if (e != hipSuccess) rc = hip_fail(e, "lock-step cycle graph");
+                // (the count only grows: a later piece's copy may be there already)
+                else if (p > 0 && __atomic_load_n(E.h_i32 + nb, __ATOMIC_RELAXED) >= nb) break;
+            }
             if (rc) return rc;
             E.graph_launches++;
         } else {
@@ -818,7 +839,7 @@ int gmres_batched(tfs_solver* s, int precision, const double* rhs, double* x, do
                 if (!rc) rc = check(hipStreamSynchronize(s->stream), "stop count");
                 if (rc) return rc;
                 launched = j1;
-                if (E.h_i32[nb] >= n_active) break;
+                if (E.h_i32[nb] >= nb) break;
             }
         }
         // x += P^{-1} V y per body
@@ -949,8 +970,8 @@ void free_ens(tfs_solver* s) {
     EnsState* E = s->ens;
     if (!E) return;
     for (int p = 0; p < 2; ++p) {
-        if (E->exec[p]) (void)hipGraphExecDestroy(E->exec[p]);
-        if (E->graph[p]) (void)hipGraphDestroy(E->graph[p]);
+        E->drop_graphs(p);
+        if (E->piece_done[p]) (void)hipEventDestroy(E->piece_done[p]);
     }
     if (E->arena) (void)hipFree(E->arena);
     if (E->h_i32) (void)hipHostFree(E->h_i32);
