@@ -59,7 +59,8 @@ def handle(ns, nb, precision):
 
 
 @pytest.mark.parametrize("precision", [P32, P64])
-@pytest.mark.parametrize("ns,nb,cluster", [(1, 0, 0), (0, 3, 2), (130, 71, 20), (700, 500, 170), (511, 1, 30),
+@pytest.mark.parametrize("ns,nb,cluster", [(1, 0, 0), (0, 3, 2), (16, 1, 9), (130, 71, 20), (340, 300, 170),
+                                           (340, 301, 170), (700, 500, 170), (511, 1, 30),
                                            (6100, 45, 30), (3300, 3100, 60), (4000, 2600, 170)])
 def test_sizes_and_clusters(ns, nb, cluster, precision):
     print(f"case ns={ns} nb={nb} cluster={cluster} precision={precision}", flush=True)

@@ -1,0 +1,47 @@
+"""Uploads and downloads of host memory that a kernel reaches (pinned arrays from
+16 KB to 1 MB) and that it does not (smaller and larger ones, pageable arrays, a
+view that starts inside a pinned array): the same evaluation from each, bit for
+bit, and again from other values (nothing is kept from the first)."""
+import numpy as np
+import pytest
+
+from timfilsimmod_amd import _lib as L
+from timfilsimmod_amd.mobility import PinnedArray, RpyHandle
+
+pytestmark = pytest.mark.gpu
+
+
+def evaluate(h, arrays, vs, vb):
+    for what, a in zip((L.SEG_POSITIONS, L.BLOB_POSITIONS, L.SEG_FORCES, L.BLOB_FORCES), arrays):
+        h.upload(what, a)
+    h.evaluate()
+    h.download(L.SEG_VELOCITIES, vs)
+    h.download(L.BLOB_VELOCITIES, vb)
+    h.sync()
+    return vs.copy(), vb.copy()
+
+
+# x_segs 24 ns, f_segs 48 ns, blobs 24 nb bytes: all below 16 KB, on both sides of it, all kernels, above 1 MB
+@pytest.mark.parametrize("ns,nb", [(5, 7), (341, 683), (342, 682), (3000, 1500), (21846, 800)])
+def test_pinned_equals_pageable(ns, nb):
+    print(f"case ns={ns} nb={nb}", flush=True)
+    rng = np.random.default_rng(ns)
+    lens = (3 * ns, 3 * nb, 6 * ns, 3 * nb, 6 * ns, 3 * nb)
+    pinned = [PinnedArray(n + 3) for n in lens]
+    h = RpyHandle(ns, nb, seg_dof=6, precision=L.PRECISION_FP64, bs_accumulate=True)
+    try:
+        for _ in range(2):
+            box = 2.0 * (ns + nb) ** (1 / 3)
+            plain = [rng.uniform(-box, box, lens[0]), rng.uniform(-box, box, lens[1]), rng.normal(size=lens[2]),
+                     rng.normal(size=lens[3])]
+            want = evaluate(h, plain, np.zeros(lens[4]), np.zeros(lens[5]))
+            for off in (0, 3):
+                views = [p.array[off:off + n] for p, n in zip(pinned, lens)]
+                for v, a in zip(views, plain):
+                    v[:] = a
+                got = evaluate(h, views[:4], views[4], views[5])
+                assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    finally:
+        h.close()
+        for p in pinned:
+            p.free()

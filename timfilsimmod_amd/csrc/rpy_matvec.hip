@@ -1059,8 +1059,7 @@ __global__ __launch_bounds__(BLOCK) void rpy_pairs_persistent_kernel(const Matve
 // of 12,800 + 9,000 particles and 74 us for twelve of 1,000-29,000 (164 and 620
 // with one workgroup per body for the boxes and the conversion, the frame
 // computed on the host, and a counting sort with a one-workgroup scan for the
-// cells).  Small problems take the same path: testing every pair instead (bit
-// masks) was 26 against 45 us at 5,794 particles and no faster at 64.
+// cells).  Small FP64 problems test every pair instead (near_small_kernel).
 //
 // Cells have side h >= (1 + 1e-5) max(ai + aj), so every pair that either
 // arithmetic (FP64, or FP32 fixed point, whose r^2 errs by well under 1e-5
@@ -1469,6 +1468,68 @@ __global__ __launch_bounds__(256) void near_grid_kernel(MatvecArgs a, int n, dou
             }
             e[j + 1] = v;
         }
+    }
+}
+
+// The FP64 lists of small problems by testing every pair of a body in one launch:
+// four targets per wave, whose lanes take 64 sources at a time (four batches'
+// loads in flight); a ballot places the near ones, so the lists come out in
+// increasing order.  Grid (16 targets each, bodies).  *max_cnt is zero before
+// (geometry_clear_kernel's job otherwise).
+__global__ __launch_bounds__(256) void near_small_kernel(MatvecArgs a, const int4* __restrict__ ranges,
+                                                        int32_t* __restrict__ cnt, int32_t* __restrict__ idx, int cap,
+                                                        int32_t* __restrict__ max_cnt) {
+    constexpr int REC = rec_len<double, 3>(), U = 4, Q = 4;
+    const int4 r = ranges[blockIdx.y];
+    const int m = (r.y - r.x) + (r.w - r.z);
+    const int lane = (int)threadIdx.x & 63;
+    const int t0 = ((int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) * U;
+    if (t0 >= m) return;
+    double xi[U][3], sum_seg[U], sum_blob[U];
+    int32_t* e[U];
+    int n[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int p = body_particle(r, a.ns, t0 + u < m ? t0 + u : m - 1);
+        const int cls = p < a.ns ? 0 : 1;
+        load_target(a, cls, cls == 0 ? p : p - a.ns, xi[u]);
+        const double ai = cls == 0 ? a.a_seg : a.a_blob;
+        sum_seg[u] = (ai + a.a_seg) * (ai + a.a_seg);
+        sum_blob[u] = (ai + a.a_blob) * (ai + a.a_blob);
+        e[u] = idx + (int64_t)p * cap;
+        n[u] = 0;
+    }
+    for (int s0 = 0; s0 < m; s0 += 64 * Q) {
+        double rec[Q][REC];
+        int src[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int t = s0 + 64 * q + lane;
+            src[q] = body_particle(r, a.ns, t < m ? t : m - 1);
+            const int cls = src[q] < a.ns ? 0 : 1;
+            stage_source<double, 3>(rec[q], a, cls, cls == 0 ? src[q] : src[q] - a.ns, false);
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const bool in = s0 + 64 * q + lane < m;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                double ddx, ddy, ddz;
+                const double r2 = separation(xi[u], rec[q], ddx, ddy, ddz);
+                const bool near = in && !(r2 > (src[q] < a.ns ? sum_seg[u] : sum_blob[u]));
+                const uint64_t hits = __ballot(near);
+                const int k = n[u] + __popcll(hits & ((uint64_t(1) << lane) - 1));
+                if (near && k < cap && t0 + u < m) e[u][k] = src[q];
+                n[u] += __popcll(hits);
+            }
+        }
+    }
+    if (lane != 0) return;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if (t0 + u >= m) continue;
+        cnt[body_particle(r, a.ns, t0 + u)] = n[u];
+        if (n[u] > cap) atomicMax(max_cnt, n[u]);
     }
 }
 
@@ -2018,6 +2079,12 @@ hipError_t build_near_list(int precision, const MatvecArgs& a, const GeometryArg
                            const NearList& near, hipStream_t stream) {
     const int n = a.ns + a.nb;
     if (n <= 0) return hipSuccess;
+    if (precision == 0 && n <= kNearSmallMax) {
+        hipLaunchKernelGGL(near_small_kernel, dim3((unsigned)((g.largest + 15) / 16), (unsigned)g.nbody), dim3(256), 0,
+                           stream, a, reinterpret_cast<const int4*>(g.ranges), near.cnt, near.idx, near.cap,
+                           near.max_cnt);
+        return hipGetLastError();
+    }
     size_grid(grid, n);
     if (!grid.fill) TFS_HIP_CHECK(hipMalloc(&grid.fill, sizeof(int32_t) * grid.table));
     if (!grid.nodes) TFS_HIP_CHECK(hipMalloc(&grid.nodes, sizeof(int4) * n));

@@ -72,11 +72,11 @@ struct tfs_rpy {
     tfs::NearGrid grid;
     int domain = 0;  // TFS_DOMAIN_UNBOUNDED or TFS_DOMAIN_HALF_SPACE
     // Fixed-point positions for FP32 tiles (valid with the near lists), their
-    // frame, and the event after its read-back into host_int[0..5].
+    // frame, and the number of its latest read-back into host_int.
     int4* x_fx = nullptr;
     bool fx_valid = false;
     tfs::GeomFrame* d_frame = nullptr;  // carved out of `arena`
-    hipEvent_t frame_read = nullptr;
+    int32_t frame_number = 0;
     double* d_body_box = nullptr;    // kBoxShares, or one per body: min xyz, max xyz
     int32_t* d_body_range = nullptr; // 4 per body (BodyRange), for the box and conversion kernels
     size_t body_cap = 0;

@@ -134,6 +134,13 @@ struct TileShape {
 // particle (n^2 entries of 4 bytes), so that none can overflow.
 constexpr int kNearRoomyMax = 6144;
 
+// Up to this many particles the FP64 lists come from testing every pair in one
+// launch instead of three.  An evaluation at new positions, device memory, us,
+// pairs / grid: 520 particles 28.5 / 30.6, 1,320 36.0 / 33.0, 2,320 49.9 / 40.7.
+// FP32 tiles need two launches for the fixed-point positions anyway, which fill
+// the grid too: 520 particles 36.6 / 33.9.
+constexpr int kNearSmallMax = 640;
+
 // The symmetric form's kinds, two target particles per lane or one (bodies
 // where two would leave too few workgroups); the waves of its workgroups, and
 // the 64-particle tiles of a panel; the longest run of source tiles of one
@@ -221,9 +228,9 @@ size_t build_sym_worklist(const std::vector<BodyRange>& bodies, int kind, int se
 // Rebuilds `near` for the given precision: every pair of particles of one
 // body whose squared separation, in the pair kernel's own arithmetic for that
 // precision, is <= (ai+aj)^2.  With `fixed` the bodies' fixed-point frame and
-// positions are made first (precision 1).  Enqueues only: *near.max_cnt and
-// the frame are on the device once the stream gets there.  Allocates what
-// `grid` lacks.
+// positions are made first (precision 1).  Enqueues only: *near.max_cnt, zero
+// before, and the frame are on the device once the stream gets there.
+// Allocates what `grid` lacks.
 hipError_t build_near_list(int precision, const MatvecArgs& a, const GeometryArgs& g, bool fixed, NearGrid& grid,
                            const NearList& near, hipStream_t stream);
 // The fixed-point frame and positions alone.

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -46,6 +47,47 @@ hipError_t copy_list(const CopyList& list, hipStream_t stream) {
     const int64_t g = (list.longest + 255) / 256;
     hipLaunchKernelGGL(copy_list_kernel, dim3((unsigned)(g < 1024 ? g : 1024)), dim3(256), 0, stream, list);
     return hipGetLastError();
+}
+
+// A pinned array of this many bytes is copied by a kernel.  Below, the runtime
+// writes it without a copy engine (40 segments + 50 blobs, the whole evaluation:
+// 80 us, 88 with kernels); above is not measured (614 KB is, where both uploads
+// and downloads gain).
+constexpr size_t kKernelCopyMin = size_t(16) << 10, kKernelCopyMax = size_t(1) << 20;
+
+// Whether a kernel can read or write `bytes` at the host address p: all of it
+// in one pinned allocation (pageable memory is not), of a size where the copy
+// engines' hand-over costs more than the transfer.
+static bool kernel_reaches(const void* p, size_t bytes, void** device) {
+    if (bytes < kKernelCopyMin || bytes > kKernelCopyMax || reinterpret_cast<uintptr_t>(p) % sizeof(double)) return false;
+    const char* c = static_cast<const char*>(p);
+    hipPointerAttribute_t first, last;
+    const bool known = hipPointerGetAttributes(&first, c) == hipSuccess &&
+                       hipPointerGetAttributes(&last, c + bytes - 1) == hipSuccess;
+    if (!known) (void)hipGetLastError();
+    if (!known || first.type != hipMemoryTypeHost || last.type != hipMemoryTypeHost || !first.devicePointer ||
+        static_cast<char*>(last.devicePointer) != static_cast<char*>(first.devicePointer) + (bytes - 1))
+        return false;
+    *device = first.devicePointer;
+    return true;
+}
+
+// len doubles between a caller's array (host or device memory) and the device.
+// A small pinned array is copied by a kernel that goes to host memory itself:
+// the runtime's copies of such arrays wait about 10 us each time the queue and
+// the copy engine take turns.  A whole evaluation from pinned arrays, FP64,
+// copies / kernels: 320 segments + 2,000 blobs 113 / 85 us, 2,140 + 3,333 152 /
+// 120, 12,800 + 9,000 694 / 656.
+static hipError_t copy_array(double* dst, const double* src, size_t len, bool host, bool to_device, hipStream_t stream) {
+    const size_t bytes = len * sizeof(double);
+    if (!host) return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, stream);
+    void* reached = nullptr;
+    if (!kernel_reaches(to_device ? src : dst, bytes, &reached))
+        return hipMemcpyAsync(dst, src, bytes, to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, stream);
+    CopyList L;
+    if (to_device) L.add(static_cast<const double*>(reached), dst, (int64_t)len);
+    else L.add(src, static_cast<double*>(reached), (int64_t)len);
+    return copy_list(L, stream);
 }
 
 // s.chunk for ~per_cu items per CU over a body of ns segments and nb blobs
@@ -333,9 +375,43 @@ static GeometryArgs geometry_args(const tfs_rpy* h) {
     return g;
 }
 
+// host_int: a GeomFrame in words 0-5, its number, deferred list checks in 8-9.
+constexpr int kFrameSeq = 6;
+static_assert(sizeof(GeomFrame) == 6 * sizeof(int32_t), "the frame's number comes after it");
+
 // Enqueues the read-back of the frame into pinned memory.
 static hipError_t read_frame(tfs_rpy* h) {
     return hipMemcpyAsync(h->host_int, h->d_frame, sizeof(GeomFrame), hipMemcpyDeviceToHost, h->stream);
+}
+
+// The same for a host that looks on: the frame, then the number of this
+// read-back behind it; the counts start from zero again.
+__global__ static void publish_frame_kernel(GeomFrame* __restrict__ frame, GeomFrame* __restrict__ host,
+                                            int32_t* seq, int32_t number) {
+    if (threadIdx.x != 0) return;
+    *host = *frame;
+    frame->max_cnt[0] = frame->max_cnt[1] = 0;
+    __hip_atomic_store(seq, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ static void clear_count_kernel(int32_t* count) {
+    if (threadIdx.x == 0) *count = 0;
+}
+
+// Waits for a published frame: by looking (the next kernel is running
+// meanwhile; an event in between would hold that up by 5 us and wake the host
+// 10 us late), and after a while, where the queue has much before it, by
+// waiting for the stream, which also tells of errors.
+static hipError_t await_frame(tfs_rpy* h) {
+    const int32_t* seq = h->host_int + kFrameSeq;
+    const auto t0 = std::chrono::steady_clock::now();
+    for (int spins = 0;; ++spins) {
+        if (__atomic_load_n(seq, __ATOMIC_ACQUIRE) == h->frame_number) return hipSuccess;
+        if ((spins & 63) == 63 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
+    }
+    const hipError_t e = hipStreamSynchronize(h->stream);
+    if (e != hipSuccess) return e;
+    return __atomic_load_n(seq, __ATOMIC_ACQUIRE) == h->frame_number ? hipSuccess : hipErrorUnknown;
 }
 
 static const GeomFrame& frame_of(const tfs_rpy* h) { return *reinterpret_cast<const GeomFrame*>(h->host_int); }
@@ -406,17 +482,29 @@ static int near_open(tfs_rpy* h, int precision, bool* open) {
                                    geometry_args(h), fixed, h->grid, nl, h->stream);
     if (h->defer_near_check) {
         // a capacity of every particle cannot overflow: nothing to check
+        // (and a count past it cannot come up, so the zero stays)
         const bool roomy = nl.cap >= nt;
         if (e == hipSuccess && !roomy)
             e = hipMemcpyAsync(h->host_int + 8 + precision, nl.max_cnt, sizeof(int32_t), hipMemcpyDeviceToHost, h->stream);
+        if (e == hipSuccess && !roomy) {
+            hipLaunchKernelGGL(clear_count_kernel, dim3(1), dim3(64), 0, h->stream, nl.max_cnt);
+            e = hipGetLastError();
+        }
         if (e != hipSuccess) return hip_fail(e, "near-pair lists");
         h->near_valid[precision] = true;
         h->near_pending[precision] = !roomy;
         return TFS_OK;
     }
-    if (e == hipSuccess && !h->frame_read) e = hipEventCreateWithFlags(&h->frame_read, hipEventDisableTiming);
-    if (e == hipSuccess) e = read_frame(h);
-    if (e == hipSuccess) e = hipEventRecord(h->frame_read, h->stream);
+    if (e == hipSuccess) {
+        void* host = nullptr;
+        e = hipHostGetDevicePointer(&host, h->host_int, 0);
+        if (e == hipSuccess) {
+            int32_t* words = static_cast<int32_t*>(host);
+            hipLaunchKernelGGL(publish_frame_kernel, dim3(1), dim3(64), 0, h->stream, h->d_frame,
+                               reinterpret_cast<GeomFrame*>(words), words + kFrameSeq, ++h->frame_number);
+            e = hipGetLastError();
+        }
+    }
     if (e != hipSuccess) return hip_fail(e, "near-pair lists");
     *open = true;
     return TFS_OK;
@@ -427,7 +515,7 @@ static int near_open(tfs_rpy* h, int precision, bool* open) {
 static int near_close(tfs_rpy* h, int precision) {
     NearList& nl = h->near[precision];
     for (int attempt = 0; attempt < 8; ++attempt) {
-        hipError_t e = hipEventSynchronize(h->frame_read);
+        const hipError_t e = await_frame(h);
         if (e != hipSuccess) return hip_fail(e, "near-pair lists");
         const GeomFrame& f = frame_of(h);
         if (precision == 1) {
@@ -670,6 +758,7 @@ int tfs_rpy_create(const tfs_rpy_desc* desc, tfs_rpy** out) {
         tfs_rpy_destroy(h);
         return hip_fail(e, "tfs_rpy_create: pinned scratch");
     }
+    std::memset(h->host_int, 0, 64);
     *out = h;
     return TFS_OK;
 }
@@ -694,7 +783,6 @@ int tfs_rpy_destroy(tfs_rpy* h) {
     if (h->x_fx) hipFree(h->x_fx);
     if (h->d_body_box) hipFree(h->d_body_box);
     if (h->d_body_range) hipFree(h->d_body_range);
-    if (h->frame_read) hipEventDestroy(h->frame_read);
     if (h->host_int) hipHostFree(h->host_int);
     if (h->blob_rep) hipFree(h->blob_rep);
     free_stage(h->f32);
@@ -727,10 +815,7 @@ int tfs_rpy_upload(tfs_rpy* h, int32_t what, const double* src) {
     if (len == 0) return TFS_OK;
     if (!src) return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_upload: null source");
     if (what == TFS_SEG_POSITIONS || what == TFS_BLOB_POSITIONS) invalidate_near(h);
-    hipError_t e = hipMemcpyAsync(dev, src, len * sizeof(double),
-                                  h->desc.memory == TFS_MEMORY_HOST ? hipMemcpyHostToDevice
-                                                                    : hipMemcpyDeviceToDevice,
-                                  h->stream);
+    const hipError_t e = copy_array(dev, src, len, h->desc.memory == TFS_MEMORY_HOST, true, h->stream);
     return e == hipSuccess ? TFS_OK : hip_fail(e, "tfs_rpy_upload");
 }
 
@@ -744,10 +829,7 @@ int tfs_rpy_download(tfs_rpy* h, int32_t what, double* dst) {
     if (rc) return rc;
     if (len == 0) return TFS_OK;
     if (!dst) return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_download: null destination");
-    hipError_t e = hipMemcpyAsync(dst, dev, len * sizeof(double),
-                                  h->desc.memory == TFS_MEMORY_HOST ? hipMemcpyDeviceToHost
-                                                                    : hipMemcpyDeviceToDevice,
-                                  h->stream);
+    const hipError_t e = copy_array(dst, dev, len, h->desc.memory == TFS_MEMORY_HOST, false, h->stream);
     return e == hipSuccess ? TFS_OK : hip_fail(e, "tfs_rpy_download");
 }
 
@@ -1509,6 +1591,7 @@ int tfs_rpy_apply_noalloc(const tfs_rpy_desc* desc, uint32_t blocks, const doubl
     grid.table = 1024;
     while (grid.table < 2 * n) grid.table <<= 1;
     GeomFrame host{};
+    hipLaunchKernelGGL(clear_count_kernel, dim3(1), dim3(64), 0, st, near.max_cnt);
     e = build_near_list(D.precision, a, g, f32, grid, near, st);
     if (e == hipSuccess) e = hipMemcpyAsync(&host, frame, sizeof(host), hipMemcpyDeviceToHost, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
