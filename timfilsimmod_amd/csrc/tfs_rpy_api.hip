@@ -49,17 +49,15 @@ hipError_t copy_list(const CopyList& list, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// A pinned array of this many bytes is copied by a kernel.  Below, the runtime
-// writes it without a copy engine (40 segments + 50 blobs, the whole evaluation:
-// 80 us, 88 with kernels); above is not measured (614 KB is, where both uploads
-// and downloads gain).
-constexpr size_t kKernelCopyMin = size_t(16) << 10, kKernelCopyMax = size_t(1) << 20;
+// Up to this many bytes a pinned array is copied by a kernel (measured up to
+// 614 KB, where both uploads and downloads gain).
+constexpr size_t kKernelCopyMax = size_t(1) << 20;
 
 // Whether a kernel can read or write `bytes` at the host address p: all of it
 // in one pinned allocation (pageable memory is not), of a size where the copy
 // engines' hand-over costs more than the transfer.
 static bool kernel_reaches(const void* p, size_t bytes, void** device) {
-    if (bytes < kKernelCopyMin || bytes > kKernelCopyMax || reinterpret_cast<uintptr_t>(p) % sizeof(double)) return false;
+    if (bytes == 0 || bytes > kKernelCopyMax || reinterpret_cast<uintptr_t>(p) % sizeof(double)) return false;
     const char* c = static_cast<const char*>(p);
     hipPointerAttribute_t first, last;
     const bool known = hipPointerGetAttributes(&first, c) == hipSuccess &&
@@ -76,7 +74,7 @@ static bool kernel_reaches(const void* p, size_t bytes, void** device) {
 // A small pinned array is copied by a kernel that goes to host memory itself:
 // the runtime's copies of such arrays wait about 10 us each time the queue and
 // the copy engine take turns.  A whole evaluation from pinned arrays, FP64,
-// copies / kernels: 320 segments + 2,000 blobs 113 / 85 us, 2,140 + 3,333 152 /
+// copies / kernels: 320 segments + 2,000 blobs 113 / 80 us, 2,140 + 3,333 152 /
 // 120, 12,800 + 9,000 694 / 656.
 static hipError_t copy_array(double* dst, const double* src, size_t len, bool host, bool to_device, hipStream_t stream) {
     const size_t bytes = len * sizeof(double);
@@ -405,7 +403,10 @@ __global__ static void clear_count_kernel(int32_t* count) {
 static hipError_t await_frame(tfs_rpy* h) {
     const int32_t* seq = h->host_int + kFrameSeq;
     const auto t0 = std::chrono::steady_clock::now();
-    for (int spins = 0;; ++spins) {
+    // (the fewest particles from host memory: nothing else is queued, and the
+    // stream's own wait is as quick: 320 + 200 particles 66 us, 68-82 by looking)
+    const bool look = h->desc.memory != TFS_MEMORY_HOST || h->desc.num_segs + h->desc.num_blobs > kNearSmallMax;
+    for (int spins = 0; look; ++spins) {
         if (__atomic_load_n(seq, __ATOMIC_ACQUIRE) == h->frame_number) return hipSuccess;
         if ((spins & 63) == 63 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
     }
@@ -660,6 +661,14 @@ int run_matvec(tfs_rpy* h, uint32_t blocks, int precision, CView fs, CView fb, V
         if (rc) return rc;
         ps.item_stamps = h->d_item_stamps;
         h->stamped_plan = p;
+    }
+    // Few particles from host memory: the host has little to hide the wait behind
+    // and goes on sooner with nothing queued meanwhile (320 segments + 2,000
+    // blobs: 80 us against 86; with device memory it is 46 against 42).
+    if (near_unread && h->desc.memory == TFS_MEMORY_HOST && h->desc.num_segs + h->desc.num_blobs <= 4096) {
+        err = near_close(h, precision);
+        if (err) return err;
+        near_unread = false;
     }
     const int n_tiles = (int)p->tiles.size(), n_items = (int)p->items.size();
     hipError_t e = wall ? launch_wall_pairs(precision, h->desc.seg_dof, a, p->d_tiles, n_tiles, p->d_items, n_items,
