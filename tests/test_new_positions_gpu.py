@@ -120,3 +120,32 @@ def test_refused_positions_and_the_ones_after_them(ns, nb):
         assert rel(evaluate(h, ns, nb, far, xb + 1e5, fs, fb), oracle_all(far, xb + 1e5, fs, fb)) <= TOLS[P32]
     finally:
         h.close()
+
+
+@pytest.mark.parametrize("radius", [1e-9, 3e-7, 1.0, 4e5])
+def test_one_particle_of_any_radius(radius):
+    """Force and torque on a particle by itself, whose extent gives the
+    fixed-point scale no bound: neither the staged torques (times the scale's
+    square) nor the third power of 1/r may leave a float's range."""
+    print(f"case radius={radius}", flush=True)
+    fs = np.array([0.3, -0.7, 0.2, 1.0, 0.4, -0.5])
+    got = {}
+    for precision in (P32, P64):
+        h = RpyHandle(1, 0, seg_dof=6, precision=precision, bs_accumulate=True, seg_radius=radius, blob_radius=radius)
+        try:
+            got[precision] = evaluate(h, 1, 0, np.array([radius, 0.0, 0.0]), np.zeros(0), fs, np.zeros(0))
+        finally:
+            h.close()
+    exact = np.concatenate([fs[:3] / (6 * np.pi * radius), fs[3:] / (8 * np.pi * radius**3)])
+    for precision, v in got.items():
+        for part in (slice(0, 3), slice(3, 6)):
+            assert rel(v[part], exact[part]) <= TOLS[precision]
+
+
+def test_radii_too_small_for_the_scale_are_refused():
+    h = RpyHandle(1, 0, seg_dof=6, precision=P32, bs_accumulate=True, seg_radius=1e-13, blob_radius=1e-13)
+    try:
+        with pytest.raises(Exception, match="1024"):
+            evaluate(h, 1, 0, np.zeros(3), np.zeros(0), np.ones(6), np.zeros(0))
+    finally:
+        h.close()

@@ -1266,7 +1266,8 @@ __global__ __launch_bounds__(256) void geometry_clear_kernel(MatvecArgs a, const
 // lambda * (largest half-extent) <= 2^30 - 2, so every coordinate and every
 // difference of two fits an int32, and lambda amin < 2^40, so that the third
 // power of 1/r at the clamp r = ai + aj is no denormal float (a particle on
-// its own, bodies of coincident particles).  Returns lambda, 0
+// its own, bodies of coincident particles), and lambda <= 2^60, so that the
+// lambda^2 of a staged torque stays far inside a float.  Returns lambda, 0
 // with *status set where the positions are not finite or the step 1/lambda is
 // not below 2^-19 amin, and the centre of body `own`.  Every workgroup of the
 // launch works it out for itself from the few hundred boxes.
@@ -1321,6 +1322,7 @@ __device__ double fixed_frame(const double* __restrict__ box, int nbody, int sha
     int ea;
     (void)frexp(amin, &ea);
     k = k < 40 - ea ? k : 40 - ea;
+    k = k < 60 ? k : 60;
     if (ldexp(1.0, -k) > ldexp(amin, -19)) {
         *status = kFrameTooLarge;
         return 0.0;

@@ -426,8 +426,8 @@ static int alloc_fixed(tfs_rpy* h) {
 // Fixed-point coordinates for FP32 tiles.  Each body is centred on its
 // bounding box; lambda = 2^k is the largest power of two with
 // lambda * (largest half-extent) <= 2^30 - 2, so every coordinate and every
-// difference of two fits an int32 (2^40 / the smallest radius where the bodies
-// are smaller than that).  The quantisation step 1/lambda must stay
+// difference of two fits an int32 (2^40 / the smallest radius or 2^60 where the
+// bodies are smaller than that).  The quantisation step 1/lambda must stay
 // below 2^-19 of the smallest radius (a body within ~1024 radii of its
 // centre); larger bodies are refused in FP32.  Synchronises the stream.
 int ensure_fixed(tfs_rpy* h) {
