@@ -161,3 +161,45 @@ def test_graph_of_a_subset_survives_a_larger_evaluation():
         g.close()
     finally:
         h.close()
+
+
+def test_large_ensembles_take_the_form_within_the_buffer_limit():
+    """Sixty-four uneven bodies: a tile's slots are one per run of source tiles, so
+    the form's buffer stays inside the 4 GiB it may take (beside it, lists and
+    positions of ~200 bytes per particle); so with one body of 170,000 particles,
+    and not with one of 400,000."""
+    import torch
+
+    from timfilsimmod_amd.ensemble import make_ensemble
+
+    e = make_ensemble(64)
+    for seg_dof in (3, 6):
+        kw = dict(seg_dof=seg_dof, precision=P32, bs_accumulate=True)
+        h, plain = (RpyHandle(e.num_segs, e.num_blobs, **kw) for _ in range(2))
+        try:
+            for x in (h, plain):
+                x.set_bodies(e.segs_per_body, e.blobs_per_body)
+                load(x, e.x_segs, e.x_blobs, e.f_segs, e.f_blobs)
+            plain.set_symmetric(P32, False)
+            print(f"case 64 bodies dof={seg_dof}", flush=True)
+            torch.cuda.synchronize()
+            before = torch.cuda.mem_get_info()[0]
+            h.evaluate()
+            got = read(h, e.num_segs, e.num_blobs)
+            used = (before - torch.cuda.mem_get_info()[0]) / 2**30
+            plain.evaluate()
+            want = read(plain, e.num_segs, e.num_blobs)
+            print(f"  {used:.2f} GiB, rel diff {rel(got, want):.2e}", flush=True)
+            assert rel(got, want) <= TOLS[P32] and not np.array_equal(got, want)
+            assert used <= 4.0 + 200 * (e.num_segs + e.num_blobs) / 2**30
+            if seg_dof == 3:
+                assert h.symmetric(P32) and h.symmetric(P64)
+        finally:
+            h.close()
+            plain.close()
+    for n, takes in ((170_000, True), (400_000, False)):
+        h = RpyHandle(n, 0, seg_dof=3, precision=P32, bs_accumulate=True)
+        try:
+            assert h.symmetric(P32) == takes
+        finally:
+            h.close()

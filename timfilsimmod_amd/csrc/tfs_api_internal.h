@@ -95,6 +95,7 @@ struct tfs_rpy {
     // take: -1 while the shape is the default, where the handle may choose it
     // by its size, else 0 (off) or the kind that the autotuner found fastest.
     int sym_pick[2] = {-1, -1};
+    int sym_size = 0;               // the kind by size for the present bodies, or 0
     bool graph_made = false;        // a captured graph may hold `partial`: replaced buffers stay
     std::vector<double*> retired;   // until the handle goes
     // Stop flag passed to the kernels of later evaluations (set by a solver

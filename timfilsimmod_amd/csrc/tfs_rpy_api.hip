@@ -145,19 +145,27 @@ static bool panels_fill(const std::vector<BodyRange>& bodies, int num_cus) {
     return items >= 4.0 * (num_cus > 0 ? num_cus : 256);
 }
 
-// The symmetric form's partial slots for these bodies, at most.
-static double sym_slot_count(const std::vector<BodyRange>& bodies, int kind) {
-    double slots = 0.0;
-    const int panel = sym_panel(kind);
+// Whether the symmetric form's partial slots for these bodies stay within
+// kSymMaxPartialBytes (at 8 bytes a value: a handle's one buffer serves both
+// precisions).  A tile has a slot for each panel before its own and one for each
+// run of source tiles from its own on, runs of 1 to kSymMaxRun tiles; where
+// neither extreme settles it, the work list does (64 uneven bodies of 4,100 to
+// 27,700 particles: 736,138 slots, 1.05 GiB with 3 components; 4.6 GiB if every
+// run were one tile).
+static bool sym_fits(const std::vector<BodyRange>& bodies, int kind, int seg_dof, int num_cus) {
+    double least = 0.0, most = 0.0;
+    const double panel = sym_panel(kind);
     for (const BodyRange& b : bodies) {
         const double t = double((b.seg_end - b.seg_begin + 63) / 64 + (b.blob_end - b.blob_begin + 63) / 64);
-        slots += t * (t + 0.5 * (t / panel) + 2.0) * 0.6;
+        least += std::max(0.0, 0.5 * t * t * (1.0 / panel + 1.0 / kSymMaxRun) - t);
+        most += 0.5 * t * (t * (1.0 / panel + 1.0) + 3.0);
     }
-    return slots;
-}
-
-static bool sym_fits(const std::vector<BodyRange>& bodies, int kind, int seg_dof) {
-    return sym_slot_count(bodies, kind) * seg_dof * 64 * sizeof(double) <= kSymMaxPartialBytes;
+    const double limit = kSymMaxPartialBytes / (seg_dof * 64.0 * sizeof(double));
+    if (most <= limit) return true;
+    if (least > limit) return false;
+    std::vector<MatvecTile> tiles;
+    std::vector<MatvecItem> items;
+    return (double)build_sym_worklist(bodies, kind, seg_dof, num_cus, 0, 0, tiles, items) <= limit;
 }
 
 // The shape of a handle that none was set for: the symmetric form for 3-DOF
@@ -165,15 +173,15 @@ static bool sym_fits(const std::vector<BodyRange>& bodies, int kind, int seg_dof
 // (measured on MI355X, 12,800 segments + 9,000 blobs: 0.187 ms per FP32 launch
 // against 0.266 for the best source-split shape, 0.313 ms per FP64 launch
 // against 0.432), else default_shape.
-static TileShape preferred_shape(int precision, int ns, int nb, int num_cus, int seg_dof,
-                                 const std::vector<BodyRange>& bodies) {
-    if (seg_dof == 3 && sym_fits(bodies, kSymWide, seg_dof) &&
-        panels_fill({BodyRange{0, ns, 0, nb}}, num_cus)) {
+// (ns, nb: the largest body; wide_fits: sym_fits of all of them.)
+static TileShape preferred_shape(int precision, int ns, int nb, int num_cus, int seg_dof, int num_bodies,
+                                 bool wide_fits) {
+    if (seg_dof == 3 && wide_fits && panels_fill({BodyRange{0, ns, 0, nb}}, num_cus)) {
         TileShape s{256, 1, 0, 0, 0};
         s.symmetric = kSymWide;
         return s;
     }
-    return default_shape(precision, ns, nb, num_cus, seg_dof, (int)bodies.size());
+    return default_shape(precision, ns, nb, num_cus, seg_dof, num_bodies);
 }
 
 // Without the split: 512-target tiles, ~16 items per CU (short items even
@@ -279,15 +287,27 @@ bool symmetric_applies(const tfs_rpy* h, uint32_t blocks) {
 // rotations: 1,600 + 2,600 particles FP32 31 / 30, FP64 41 / 40; 2,461 + 3,333
 // 44 / 42, 64 / 57; 6,000 + 4,500 109 / 100, 171 / 155; 12,800 + 9,000 392 /
 // 340, 693 / 560; twelve uneven bodies 3,480 / 2,830, 6,250 / 4,750.
-static int sym_by_size(const tfs_rpy* h) {
+static int sym_by_size(const tfs_rpy* h, bool wide_fits) {
     const double cus = h->num_cus > 0 ? h->num_cus : 256;
-    if (panels_fill(h->bodies, h->num_cus) && sym_fits(h->bodies, kSymWide, h->desc.seg_dof)) return kSymWide;
+    if (wide_fits && panels_fill(h->bodies, h->num_cus)) return kSymWide;
     double pairs = 0.0;
     for (const BodyRange& b : h->bodies) {
         const double t = double((b.seg_end - b.seg_begin + 63) / 64 + (b.blob_end - b.blob_begin + 63) / 64);
         pairs += t * (t + 1.0) / 2.0;
     }
-    return pairs >= 8.0 * cus && sym_fits(h->bodies, kSymNarrow, h->desc.seg_dof) ? kSymNarrow : 0;
+    return pairs >= 8.0 * cus && sym_fits(h->bodies, kSymNarrow, h->desc.seg_dof, h->num_cus) ? kSymNarrow : 0;
+}
+
+// What follows from the body list alone, once per list: the kind above, and the
+// shapes that no caller chose.
+static void choose_by_size(tfs_rpy* h) {
+    const bool wide_fits = sym_fits(h->bodies, kSymWide, h->desc.seg_dof, h->num_cus);
+    h->sym_size = sym_by_size(h, wide_fits);
+    int ns = 0, nb = 0;
+    largest_body(h, &ns, &nb);
+    for (int pr = 0; pr < 2; ++pr)
+        if (!h->shape_chosen[pr])
+            h->shape[pr] = preferred_shape(pr, ns, nb, h->num_cus, h->desc.seg_dof, (int)h->bodies.size(), wide_fits);
 }
 
 TileShape effective_shape(const tfs_rpy* h, int precision, uint32_t blocks) {
@@ -295,7 +315,7 @@ TileShape effective_shape(const tfs_rpy* h, int precision, uint32_t blocks) {
     const bool applies = symmetric_applies(h, blocks);
     if (!sh.symmetric) {
         const int pick = h->sym_pick[precision];
-        const int kind = !applies || sh.persistent > 0 ? 0 : pick < 0 ? sym_by_size(h) : pick;
+        const int kind = !applies || sh.persistent > 0 ? 0 : pick < 0 ? h->sym_size : pick;
         if (!kind) return sh;
         TileShape s{64 * kSymWaves, 1, 0, 0, 0};
         s.symmetric = kind;
@@ -757,10 +777,8 @@ int tfs_rpy_create(const tfs_rpy_desc* desc, tfs_rpy** out) {
         tfs_rpy_destroy(h);
         return hip_fail(e, "tfs_rpy_create: clear");
     }
-    for (int pr = 0; pr < 2; ++pr)
-        h->shape[pr] = preferred_shape(pr, desc->num_segs, desc->num_blobs, cus, desc->seg_dof,
-                                       {BodyRange{0, desc->num_segs, 0, desc->num_blobs}});
     h->bodies.push_back(BodyRange{0, desc->num_segs, 0, desc->num_blobs});
+    choose_by_size(h);
     e = hipHostMalloc((void**)&h->host_int, 64, hipHostMallocDefault);
     if (e != hipSuccess) {
         tfs_rpy_destroy(h);
@@ -1054,11 +1072,7 @@ int tfs_rpy_set_bodies(tfs_rpy* h, int32_t num_bodies, const int32_t* segs_per_b
     h->bodies = bodies;
     h->body_table_valid = false;
     invalidate_near(h);
-    int lns = 0, lnb = 0;
-    largest_body(h, &lns, &lnb);
-    for (int pr = 0; pr < 2; ++pr)
-        if (!h->shape_chosen[pr])
-            h->shape[pr] = preferred_shape(pr, lns, lnb, h->num_cus, h->desc.seg_dof, h->bodies);
+    choose_by_size(h);
     return TFS_OK;
 }
 
@@ -1161,14 +1175,14 @@ int tfs_rpy_autotune(tfs_rpy* h, int32_t precision, uint32_t blocks, int32_t rep
     };
     // The symmetric form: as the shape of 3-DOF handles, behind the default
     // shape of 6-DOF ones.
-    if (symmetric_applies(h, blocks) && sym_fits(h->bodies, kSymWide, h->desc.seg_dof)) {
+    if (symmetric_applies(h, blocks) && sym_fits(h->bodies, kSymWide, h->desc.seg_dof, h->num_cus)) {
         if (h->desc.seg_dof == 3) {
             TileShape sym{256, 1, 0, 0, 0};
             sym.symmetric = kSymWide;
             time_shape(sym);
         } else {
             for (int kind : {kSymWide, kSymNarrow}) {
-                if (rc || !sym_fits(h->bodies, kind, h->desc.seg_dof)) continue;
+                if (rc || !sym_fits(h->bodies, kind, h->desc.seg_dof, h->num_cus)) continue;
                 h->sym_pick[precision] = kind;
                 time_shape(default_shape(precision, ns, nb, h->num_cus, h->desc.seg_dof, (int)h->bodies.size()));
             }
