@@ -96,6 +96,7 @@ struct tfs_rpy {
     // by its size, else 0 (off) or the kind that the autotuner found fastest.
     int sym_pick[2] = {-1, -1};
     int sym_size = 0;               // the kind by size for the present bodies, or 0
+    bool sized = false;             // that and the shapes that no caller chose are made
     bool graph_made = false;        // a captured graph may hold `partial`: replaced buffers stay
     std::vector<double*> retired;   // until the handle goes
     // Stop flag passed to the kernels of later evaluations (set by a solver
@@ -195,7 +196,7 @@ bool symmetric_applies(const tfs_rpy* h, uint32_t blocks);
 // The launch shape of one evaluation: the handle's shape, the symmetric form
 // where the handle has no chosen shape and its size favours it, or the default
 // source-split shape where a symmetric shape does not apply.
-TileShape effective_shape(const tfs_rpy* h, int precision, uint32_t blocks);
+TileShape effective_shape(tfs_rpy* h, int precision, uint32_t blocks);
 // Positions changed: the near-pair lists must be rebuilt before the next matvec.
 void invalidate_near(tfs_rpy* h);
 // Builds the near-pair list of `precision` (and, for FP32, the fixed-point

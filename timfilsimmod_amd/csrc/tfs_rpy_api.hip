@@ -298,9 +298,13 @@ static int sym_by_size(const tfs_rpy* h, bool wide_fits) {
     return pairs >= 8.0 * cus && sym_fits(h->bodies, kSymNarrow, h->desc.seg_dof, h->num_cus) ? kSymNarrow : 0;
 }
 
-// What follows from the body list alone, once per list: the kind above, and the
-// shapes that no caller chose.
+// What follows from the body list alone: the kind above, and the shapes that no
+// caller chose.  Once per list, at the first call that looks at them (a count of
+// the work list takes milliseconds at 100,000 particles, and a handle that is
+// given bodies needs none of its particles as one body).
 static void choose_by_size(tfs_rpy* h) {
+    if (h->sized) return;
+    h->sized = true;
     const bool wide_fits = sym_fits(h->bodies, kSymWide, h->desc.seg_dof, h->num_cus);
     h->sym_size = sym_by_size(h, wide_fits);
     int ns = 0, nb = 0;
@@ -310,7 +314,8 @@ static void choose_by_size(tfs_rpy* h) {
             h->shape[pr] = preferred_shape(pr, ns, nb, h->num_cus, h->desc.seg_dof, (int)h->bodies.size(), wide_fits);
 }
 
-TileShape effective_shape(const tfs_rpy* h, int precision, uint32_t blocks) {
+TileShape effective_shape(tfs_rpy* h, int precision, uint32_t blocks) {
+    choose_by_size(h);
     const TileShape& sh = h->shape[precision];
     const bool applies = symmetric_applies(h, blocks);
     if (!sh.symmetric) {
@@ -778,7 +783,6 @@ int tfs_rpy_create(const tfs_rpy_desc* desc, tfs_rpy** out) {
         return hip_fail(e, "tfs_rpy_create: clear");
     }
     h->bodies.push_back(BodyRange{0, desc->num_segs, 0, desc->num_blobs});
-    choose_by_size(h);
     e = hipHostMalloc((void**)&h->host_int, 64, hipHostMallocDefault);
     if (e != hipSuccess) {
         tfs_rpy_destroy(h);
@@ -994,6 +998,7 @@ static int set_shape(tfs_rpy* h, const char* fn, int32_t precision, int32_t bloc
         return fail(TFS_ERR_INVALID_ARGUMENT,
                     std::string(fn) + ": chunk must be a positive multiple of block (or, without the split, a "
                                       "divisor of it of at least 32)");
+    choose_by_size(h);
     const int pers = h->shape[precision].persistent;
     if (split && pers > 0)
         return fail(TFS_ERR_INVALID_ARGUMENT, std::string(fn) + ": the source split has no persistent form");
@@ -1016,6 +1021,7 @@ int tfs_rpy_set_symmetric(tfs_rpy* h, int32_t precision, int32_t enable) {
     if (!h) return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_set_symmetric: null handle");
     if (precision != 0 && precision != 1)
         return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_set_symmetric: unknown precision");
+    choose_by_size(h);
     if (!enable) {
         h->sym_pick[precision] = 0;
         if (h->shape[precision].symmetric) {
@@ -1040,6 +1046,7 @@ int tfs_rpy_set_symmetric(tfs_rpy* h, int32_t precision, int32_t enable) {
 int tfs_rpy_get_symmetric(tfs_rpy* h, int32_t precision, int32_t* enabled) {
     if (!h || !enabled || (precision != 0 && precision != 1))
         return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_get_symmetric: bad arguments");
+    choose_by_size(h);
     *enabled = h->shape[precision].symmetric ? 1 : 0;
     return TFS_OK;
 }
@@ -1072,7 +1079,7 @@ int tfs_rpy_set_bodies(tfs_rpy* h, int32_t num_bodies, const int32_t* segs_per_b
     h->bodies = bodies;
     h->body_table_valid = false;
     invalidate_near(h);
-    choose_by_size(h);
+    h->sized = false;
     return TFS_OK;
 }
 
@@ -1139,6 +1146,7 @@ int tfs_graph_destroy(tfs_graph* g) {
 int tfs_rpy_autotune(tfs_rpy* h, int32_t precision, uint32_t blocks, int32_t reps, double* best_ms) {
     if (!h || (precision != 0 && precision != 1) || reps < 1 || (blocks & ~TFS_BLOCK_ALL))
         return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_autotune: bad arguments");
+    choose_by_size(h);
     const int saved_precision = h->desc.precision;
     h->desc.precision = precision;
     hipEvent_t e0, e1;
@@ -1230,6 +1238,7 @@ int tfs_rpy_autotune(tfs_rpy* h, int32_t precision, uint32_t blocks, int32_t rep
 int tfs_rpy_set_persistent(tfs_rpy* h, int32_t precision, int32_t workgroups_per_cu) {
     if (!h || (precision != 0 && precision != 1) || workgroups_per_cu < 0 || workgroups_per_cu > 64)
         return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_set_persistent: bad arguments");
+    choose_by_size(h);
     if (workgroups_per_cu > 0 && (h->shape[precision].split || h->shape[precision].symmetric)) {
         // the split and the symmetric form have no persistent form: a default
         // shape gives way to the plain default
@@ -1250,6 +1259,7 @@ int tfs_rpy_set_persistent(tfs_rpy* h, int32_t precision, int32_t workgroups_per
 int tfs_rpy_get_tile_shape(tfs_rpy* h, int32_t precision, int32_t shape[4]) {
     if (!h || !shape || (precision != 0 && precision != 1))
         return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_get_tile_shape: bad arguments");
+    choose_by_size(h);
     const TileShape& s = h->shape[precision];
     shape[0] = s.block;
     shape[1] = s.per_thread;
@@ -1261,6 +1271,7 @@ int tfs_rpy_get_tile_shape(tfs_rpy* h, int32_t precision, int32_t shape[4]) {
 int tfs_rpy_get_source_split(tfs_rpy* h, int32_t precision, int32_t* split) {
     if (!h || !split || (precision != 0 && precision != 1))
         return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_get_source_split: bad arguments");
+    choose_by_size(h);
     *split = h->shape[precision].split;
     return TFS_OK;
 }
