@@ -1,7 +1,7 @@
 """New positions: the fixed-point frame of FP32 tiles and the overlapping-pair
 lists against the FP64 oracle, from one particle on: particles by the hundred
-in one place (lists sorted from LDS, by rank and by insertion, capacities
-grown), independent bodies in the same place and bodies without particles, positions that are refused and the ones after
+in one place (lists sorted from LDS and by rank, or made in order, capacities
+grown), thousands of them, coincident ones and cells with more particles than a walk visits, independent bodies in the same place and bodies without particles, positions that are refused and the ones after
 them, lists rebuilt while an earlier capacity is in use.
 
 Tolerances: the matvec's bars, 1e-12 (FP64 sums of n terms in another order)
@@ -147,5 +147,78 @@ def test_radii_too_small_for_the_scale_are_refused():
     try:
         with pytest.raises(Exception, match="1024"):
             evaluate(h, 1, 0, np.zeros(3), np.zeros(0), np.ones(6), np.zeros(0))
+    finally:
+        h.close()
+
+
+def seconds(run):
+    import time
+
+    t0 = time.perf_counter()
+    out = run()
+    return out, time.perf_counter() - t0
+
+
+# a list of one entry per particle of the body, beside a second body as crowded
+@pytest.mark.parametrize("precision", [P32, P64])
+@pytest.mark.parametrize("ns,nb,spread", [(1500, 1500, 0.5), (700, 1, 1e-3), (2500, 3600, 0.3)])
+def test_thousands_in_one_place(ns, nb, spread, precision):
+    """Every particle overlaps every other: the lists' cost stays a pass over the
+    body for each target (milliseconds for all; their lengths squared, moved one
+    by one, would be seconds)."""
+    print(f"case ns={ns} nb={nb} spread={spread} precision={precision}", flush=True)
+    rng = np.random.default_rng(ns)
+    xs, xb = spread * rng.uniform(-1, 1, 3 * ns), spread * rng.uniform(-1, 1, 3 * nb)
+    fs, fb = rng.normal(size=6 * ns), rng.normal(size=3 * nb)
+    h = handle(ns, nb, precision)
+    try:
+        evaluate(h, ns, nb, xs, xb, fs, fb)                       # grows the lists
+        got, took = seconds(lambda: evaluate(h, ns, nb, xs, xb, fs, fb))
+        want = oracle_all(xs, xb, fs, fb)
+        print(f"  rel err {rel(got, want):.2e}, {took * 1e3:.1f} ms", flush=True)
+        assert rel(got, want) <= TOLS[precision]
+        assert took < 0.25
+        assert np.array_equal(evaluate(h, ns, nb, xs, xb, fs, fb), got)
+    finally:
+        h.close()
+
+
+@pytest.mark.parametrize("precision", [P32, P64])
+@pytest.mark.parametrize("bodies", [1, 2])
+def test_small_particles_crowd_a_cell(bodies, precision):
+    """Cells take their side from the larger radius: thousands of small blobs in
+    each, nearly none of which overlap."""
+    print(f"case bodies={bodies} precision={precision}", flush=True)
+    rng = np.random.default_rng(3)
+    ns, nb, kw = 20, 4000, dict(a_seg=1.0, a_blob=0.02)
+    parts = [(rng.uniform(-3, 3, 3 * ns), rng.uniform(-2, 2, 3 * nb), rng.normal(size=6 * ns), rng.normal(size=3 * nb))
+             for _ in range(bodies)]
+    h = RpyHandle(ns * bodies, nb * bodies, seg_dof=6, precision=precision, bs_accumulate=True, seg_radius=1.0,
+                  blob_radius=0.02)
+    try:
+        if bodies > 1:
+            h.set_bodies([ns] * bodies, [nb] * bodies)
+        got = evaluate(h, ns * bodies, nb * bodies, *(np.concatenate([p[k] for p in parts]) for k in range(4)))
+        each = [O.full_mobility(*p, seg_dof=6, bs_accumulate=True, **kw) for p in parts]
+        want = np.concatenate([e[0] for e in each] + [e[1] for e in each])
+        print(f"  rel err {rel(got, want):.2e}", flush=True)
+        assert rel(got, want) <= TOLS[precision]
+    finally:
+        h.close()
+
+
+def test_positions_that_are_not_finite_in_fp64():
+    """FP64 does not look at the positions: an evaluation of such ones ends as
+    soon as any other and says so in its velocities."""
+    ns, nb = 3000, 1000
+    xs, xb, fs, fb = cloud(ns, nb, 4, 5)
+    h = handle(ns, nb, P64)
+    try:
+        want = evaluate(h, ns, nb, xs, xb, fs, fb)
+        evaluate(h, ns, nb, np.full(3 * ns, np.nan), xb, fs, fb)  # grows the lists
+        got, took = seconds(lambda: evaluate(h, ns, nb, np.full(3 * ns, np.nan), xb, fs, fb))
+        print(f"case ns={ns} nb={nb}: {took * 1e3:.1f} ms", flush=True)
+        assert np.all(np.isnan(got.reshape(-1, 3)[:2 * ns:2])) and took < 0.25
+        assert np.array_equal(evaluate(h, ns, nb, xs, xb, fs, fb), want)
     finally:
         h.close()

@@ -1376,71 +1376,103 @@ __global__ __launch_bounds__(256) void geometry_place_kernel(MatvecArgs a, const
 // entries are distinct), from LDS for up to 64 of them, so the lists are the
 // same on every run.  cnt is the full count, entries past cap are dropped and
 // *max_cnt gets any count above cap.
+//
+// Crowded places (a bucket longer than `walk` particles, or a list of more than
+// 256): the target's lanes test all of its body's particles
+// in order instead, 32 at a time, so that no cell and no list, whatever the
+// positions (coincident, not finite), takes more than a walk of those lengths
+// and one pass over the body: a launch costs at most about what the pair kernel
+// does.  Sorting such a list by itself would take a lane as many dependent moves
+// as its length squared.
 constexpr int kNearLds = 64, kRankPer = 8;
 template <typename T>
 __global__ __launch_bounds__(256) void near_grid_kernel(MatvecArgs a, int n, double inv_h, uint32_t mask,
+                                                       const int4* __restrict__ ranges, int walk,
                                                        const int32_t* __restrict__ head,
                                                        const int4* __restrict__ nodes,
                                                        const int32_t* __restrict__ body_of, int32_t* __restrict__ cnt,
                                                        int32_t* idx, int cap, int32_t* __restrict__ max_cnt) {
     constexpr bool F32 = sizeof(T) == 4;
     constexpr int REC = rec_len<T, 3>();
-    __shared__ int32_t found[8];
+    __shared__ int32_t found[8], crowded[8];
     __shared__ int32_t list[8][kNearLds + 1];
     const int s = (int)(threadIdx.x >> 5);
     const int tg = (int)blockIdx.x * 8 + s;
     const int lane = (int)(threadIdx.x & 31);
     const double lam = F32 ? *a.lam : 1.0;
     if (!(lam > 0.0)) return;  // no frame: uniform over the launch
-    if (threadIdx.x < 8) found[threadIdx.x] = 0;
+    if (threadIdx.x < 8) found[threadIdx.x] = crowded[threadIdx.x] = 0;
     __syncthreads();
     int32_t* e = idx + (int64_t)tg * cap;
-    if (tg < n && lane < 27) {
-        const int cls = tg < a.ns ? 0 : 1;
-        using XT = typename std::conditional<F32, int32_t, double>::type;
-        XT xi[3];
-        load_target(a, cls, cls == 0 ? tg : tg - a.ns, xi);
-        const int4 own = nodes[tg];
+    const bool in = tg < n;
+    // (past the end: the last target's, so that the loads go out together)
+    const int tc = in ? tg : n - 1;
+    const int cls = tc < a.ns ? 0 : 1;
+    const int4 own = nodes[tc];
+    using XT = typename std::conditional<F32, int32_t, double>::type;
+    XT xi[3];
+    load_target(a, cls, cls == 0 ? tc : tc - a.ns, xi);
+    const int body = body_of ? body_of[tc] : 0;
+    const double ai = cls == 0 ? a.a_seg : a.a_blob;
+    const T sum_seg = T(lam * lam * ((ai + a.a_seg) * (ai + a.a_seg)));
+    const T sum_blob = T(lam * lam * ((ai + a.a_blob) * (ai + a.a_blob)));
+    auto is_near = [&](int j) {
+        const int jcls = j < a.ns ? 0 : 1;
+        T rec[REC];
+        stage_source<T, 3>(rec, a, jcls, jcls == 0 ? j : j - a.ns, false);
+        T ddx, ddy, ddz;
+        const T r2 = separation(xi, rec, ddx, ddy, ddz);
+        return !(r2 > (jcls == 0 ? sum_seg : sum_blob));
+    };
+    if (in && lane < 27) {
         const int nx = own.x + lane % 3 - 1, ny = own.y + (lane / 3) % 3 - 1, nz = own.z + lane / 9 - 1;
-        const int body = body_of ? body_of[tg] : 0;
-        const double ai = cls == 0 ? a.a_seg : a.a_blob;
-        const T sum_seg = T(lam * lam * ((ai + a.a_seg) * (ai + a.a_seg)));
-        const T sum_blob = T(lam * lam * ((ai + a.a_blob) * (ai + a.a_blob)));
-        for (int j = head[body_cell_hash(nx, ny, nz, body, mask)]; j >= 0;) {
+        int j = head[body_cell_hash(nx, ny, nz, body, mask)];
+        for (int left = walk; j >= 0 && left > 0; --left) {
             const int4 nd = nodes[j];
             // the bucket may also hold other cells (and bodies): visit j from its own only
-            if (nd.x == nx && nd.y == ny && nd.z == nz && (!body_of || body_of[j] == body)) {
-                const int jcls = j < a.ns ? 0 : 1;
-                T rec[REC];
-                stage_source<T, 3>(rec, a, jcls, jcls == 0 ? j : j - a.ns, false);
-                T ddx, ddy, ddz;
-                const T r2 = separation(xi, rec, ddx, ddy, ddz);
-                if (!(r2 > (jcls == 0 ? sum_seg : sum_blob))) {
-                    const int k = atomicAdd(&found[s], 1);
-                    if (k < kNearLds) list[s][k] = j;
-                    if (k < cap) e[k] = j;
-                }
+            if (nd.x == nx && nd.y == ny && nd.z == nz && (!body_of || body_of[j] == body) && is_near(j)) {
+                const int k = atomicAdd(&found[s], 1);
+                if (k < kNearLds) list[s][k] = j;
+                if (k < cap) e[k] = j;
             }
             j = nd.w;
         }
+        if (j >= 0) crowded[s] = 1;
     }
     __syncthreads();
-    const int total = tg < n ? found[s] : 0;
-    if (tg < n && lane == 0) {
+    int total = in ? found[s] : 0;
+    const bool scan = in && (crowded[s] || total > 32 * kRankPer);
+    if (scan) {
+        const int shift = (int)(threadIdx.x & 32);  // the target's half of the wave
+        const int4 r = ranges[body];
+        const int m = (r.y - r.x) + (r.w - r.z);
+        total = 0;
+        for (int t0 = 0; t0 < m; t0 += 32) {
+            const int t = t0 + lane;
+            const int j = body_particle(r, a.ns, t < m ? t : m - 1);
+            const bool near = t < m && is_near(j);
+            const uint32_t hits = (uint32_t)(__ballot(near) >> shift);
+            const int k = total + __popc(hits & ((1u << lane) - 1u));
+            if (near && k < cap) e[k] = j;
+            total += __popc(hits);
+        }
+    }
+    if (in && lane == 0) {
         cnt[tg] = total;
         if (total > cap) atomicMax(max_cnt, total);
     }
-    const int c = total < cap ? total : cap;
-    if (total <= kNearLds) {
+    if (!scan && total <= kNearLds) {
         for (int i = lane; i < total; i += 32) {
             const int32_t v = list[s][i];
-            int r = 0;
-            for (int j = 0; j < total; ++j) r += list[s][j] < v ? 1 : 0;
-            if (r < cap) e[r] = v;
+            int q = 0;
+            for (int j = 0; j < total; ++j) q += list[s][j] < v ? 1 : 0;
+            if (q < cap) e[q] = v;
         }
     }
-    if (!__syncthreads_or(total > kNearLds)) return;
+    const bool by_rank = !scan && total > kNearLds;
+    if (!__syncthreads_or(by_rank)) return;
     // longer lists: ranked against what the barrier above made readable
+    const int c = total < cap ? total : cap;
     int32_t val[kRankPer];
     int rank[kRankPer];
 #pragma unroll
@@ -1448,29 +1480,18 @@ __global__ __launch_bounds__(256) void near_grid_kernel(MatvecArgs a, int n, dou
         const int i = lane + 32 * q;
         val[q] = 0;
         rank[q] = -1;
-        if (total > kNearLds && c <= 32 * kRankPer && i < c) {
+        if (by_rank && i < c) {
             const int32_t v = e[i];
-            int r = 0;
-            for (int j = 0; j < c; ++j) r += e[j] < v ? 1 : 0;
+            int below = 0;
+            for (int j = 0; j < c; ++j) below += e[j] < v ? 1 : 0;
             val[q] = v;
-            rank[q] = r;
+            rank[q] = below;
         }
     }
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < kRankPer; ++q)
         if (rank[q] >= 0) e[rank[q]] = val[q];
-    if (total > kNearLds && c > 32 * kRankPer && lane == 0) {
-        for (int i = 1; i < c; ++i) {
-            const int32_t v = e[i];
-            int j = i - 1;
-            while (j >= 0 && e[j] > v) {
-                e[j + 1] = e[j];
-                --j;
-            }
-            e[j + 1] = v;
-        }
-    }
 }
 
 // The FP64 lists of small problems by testing every pair of a body in one launch:
@@ -2097,12 +2118,14 @@ hipError_t build_near_list(int precision, const MatvecArgs& a, const GeometryArg
     const uint32_t mask = (uint32_t)grid.table - 1;
     const unsigned gl = (unsigned)((n + 7) / 8);   // 8 targets of 32 lanes per workgroup
     const int32_t* body_of = g.nbody > 1 ? grid.body_of : nullptr;
+    // a step of the walk waits for the one before, a pass takes 32 particles at once
+    const int walk = std::max(256, g.largest / 32);
     if (precision == 0)
-        hipLaunchKernelGGL(near_grid_kernel<double>, dim3(gl), dim3(256), 0, stream, a, n, inv_h, mask, grid.fill,
-                           grid.nodes, body_of, near.cnt, near.idx, near.cap, near.max_cnt);
+        hipLaunchKernelGGL(near_grid_kernel<double>, dim3(gl), dim3(256), 0, stream, a, n, inv_h, mask,
+                           reinterpret_cast<const int4*>(g.ranges), walk, grid.fill, grid.nodes, body_of, near.cnt, near.idx, near.cap, near.max_cnt);
     else
-        hipLaunchKernelGGL(near_grid_kernel<float>, dim3(gl), dim3(256), 0, stream, a, n, inv_h, mask, grid.fill,
-                           grid.nodes, body_of, near.cnt, near.idx, near.cap, near.max_cnt);
+        hipLaunchKernelGGL(near_grid_kernel<float>, dim3(gl), dim3(256), 0, stream, a, n, inv_h, mask,
+                           reinterpret_cast<const int4*>(g.ranges), walk, grid.fill, grid.nodes, body_of, near.cnt, near.idx, near.cap, near.max_cnt);
     return hipGetLastError();
 }
 
