@@ -222,3 +222,28 @@ def test_positions_that_are_not_finite_in_fp64():
         assert np.array_equal(evaluate(h, ns, nb, xs, xb, fs, fb), want)
     finally:
         h.close()
+
+
+@pytest.mark.parametrize("precision", [P32, P64])
+@pytest.mark.parametrize("num_bodies", [1024, 1025, 70_000])
+def test_more_bodies_than_a_grid_has_rows(num_bodies, precision):
+    """Bodies of one segment each, all in one place: each its own mobility only;
+    then most of them empty (FP64: the small problem's one launch)."""
+    print(f"case bodies={num_bodies} precision={precision}", flush=True)
+    rng = np.random.default_rng(num_bodies)
+    a = 1.0
+    for ns in (num_bodies, 300):
+        xs, fs = rng.uniform(-5, 5, 3 * ns), rng.normal(size=6 * ns)
+        h = handle(ns, 0, precision)
+        try:
+            h.set_bodies([1] * ns + [0] * (num_bodies - ns), [0] * num_bodies)
+            for _ in range(2):
+                got = evaluate(h, ns, 0, xs, np.zeros(0), fs, np.zeros(0)).reshape(ns, 6)
+                f = fs.reshape(ns, 6)
+                assert rel(got[:, :3], f[:, :3] / (6 * np.pi * a)) <= TOLS[precision]
+                assert rel(got[:, 3:], f[:, 3:] / (8 * np.pi * a**3)) <= TOLS[precision]
+                xs = xs[::-1].copy()
+        finally:
+            h.close()
+        if num_bodies < 2000:
+            break

@@ -1209,9 +1209,10 @@ __device__ __forceinline__ uint32_t body_cell_hash(int cx, int cy, int cz, int b
 }
 
 // Empties the grid (head, table entries, may be null), clears *max_cnt and,
-// with BOX, writes box[blockIdx.y gridDim.x + blockIdx.x]: the bounds (min
-// xyz, max xyz) of the workgroup's share of body blockIdx.y, NaN if any of its
-// coordinates is not finite.  Workgroups of 256.
+// with BOX, writes box[blockIdx.x gridDim.y + blockIdx.y]: the bounds (min
+// xyz, max xyz) of the workgroup's share of body blockIdx.x, NaN if any of its
+// coordinates is not finite.  Workgroups of 256.  (Bodies are counted in x here
+// and below: a grid's y ends at 65,535.)
 template <bool BOX>
 __global__ __launch_bounds__(256) void geometry_clear_kernel(MatvecArgs a, const int4* __restrict__ ranges,
                                                             double* __restrict__ box, int32_t* __restrict__ head,
@@ -1219,17 +1220,17 @@ __global__ __launch_bounds__(256) void geometry_clear_kernel(MatvecArgs a, const
     const int tid = (int)threadIdx.x;
     const int block = (int)(blockIdx.y * gridDim.x + blockIdx.x);
     if (head)
-        for (int i = (block * 256 + tid) * 4; i < table; i += (int)(gridDim.x * gridDim.y) * 1024)
+        for (int64_t i = ((int64_t)block * 256 + tid) * 4; i < table; i += (int64_t)(gridDim.x * gridDim.y) * 1024)
             *reinterpret_cast<int4*>(head + i) = make_int4(-1, -1, -1, -1);
     if (block == 0 && tid == 0) *max_cnt = 0;
     if constexpr (BOX) {
         __shared__ double red[4][6];
-        const int4 r = ranges[blockIdx.y];
+        const int4 r = ranges[blockIdx.x];
         const int m = (r.y - r.x) + (r.w - r.z);
         double lo[3] = {__builtin_inf(), __builtin_inf(), __builtin_inf()};
         double hi[3] = {-__builtin_inf(), -__builtin_inf(), -__builtin_inf()};
         bool bad = false;
-        for (int t = (int)blockIdx.x * 256 + tid; t < m; t += (int)gridDim.x * 256) {
+        for (int t = (int)blockIdx.y * 256 + tid; t < m; t += (int)gridDim.y * 256) {
             double x[3];
             particle_pos(a, body_particle(r, a.ns, t), x);
 #pragma unroll
@@ -1256,7 +1257,7 @@ __global__ __launch_bounds__(256) void geometry_clear_kernel(MatvecArgs a, const
         if (tid < 6) {
             double v = red[0][tid];
             for (int w = 1; w < 4; ++w) v = tid < 3 ? __builtin_fmin(v, red[w][tid]) : __builtin_fmax(v, red[w][tid]);
-            box[6 * (int64_t)block + tid] = any_bad ? __builtin_nan("") : v;
+            box[6 * ((int64_t)blockIdx.x * gridDim.y + blockIdx.y) + tid] = any_bad ? __builtin_nan("") : v;
         }
     }
 }
@@ -1269,17 +1270,20 @@ __global__ __launch_bounds__(256) void geometry_clear_kernel(MatvecArgs a, const
 // its own, bodies of coincident particles), and lambda <= 2^60, so that the
 // lambda^2 of a staged torque stays far inside a float.  Returns lambda, 0
 // with *status set where the positions are not finite or the step 1/lambda is
-// not below 2^-19 amin, and the centre of body `own`.  Every workgroup of the
-// launch works it out for itself from the few hundred boxes.
+// not below 2^-19 amin, and the centre of body `own`.  Every workgroup of
+// geometry_place_kernel works it out for itself from up to kFrameBodies boxes;
+// more bodies have geometry_frame_kernel do it once.
+constexpr int kFrameBodies = 1024;  // at least kBoxShares: more have one box each
+template <int THREADS>
 __device__ double fixed_frame(const double* __restrict__ box, int nbody, int shares, int own, double amin,
                               double* centre, int* status) {
-    __shared__ double wave_ext[4], own_centre[3];
+    __shared__ double wave_ext[THREADS / 64], own_centre[3];
     const int tid = (int)threadIdx.x;
     int width = 1;  // lanes per body
     while (width < shares && width < 64) width <<= 1;
     double ext = 0.0;
     bool bad = false;
-    for (int b = tid / width; b < nbody; b += 256 / width) {
+    for (int b = tid / width; b < nbody; b += THREADS / width) {
         double lo[3] = {__builtin_inf(), __builtin_inf(), __builtin_inf()};
         double hi[3] = {-__builtin_inf(), -__builtin_inf(), -__builtin_inf()};
         for (int g = tid % width; g < shares; g += width) {
@@ -1309,7 +1313,7 @@ __device__ double fixed_frame(const double* __restrict__ box, int nbody, int sha
     for (int off = 32; off > 0; off >>= 1) ext = __builtin_fmax(ext, __shfl_xor(ext, off, 64));
     if ((tid & 63) == 0) wave_ext[tid >> 6] = ext;
     const bool any_bad = __syncthreads_or(bad);
-    for (int w = 0; w < 4; ++w) ext = __builtin_fmax(ext, wave_ext[w]);
+    for (int w = 0; w < THREADS / 64; ++w) ext = __builtin_fmax(ext, wave_ext[w]);
     for (int k = 0; k < 3; ++k) centre[k] = own_centre[k];
     *status = any_bad ? kFrameNonFinite : ext < 1e300 ? 0 : kFrameTooLarge;
     if (*status) return 0.0;
@@ -1330,31 +1334,52 @@ __device__ double fixed_frame(const double* __restrict__ box, int nbody, int sha
     return ldexp(1.0, k);
 }
 
-// FIXED: X = rint(lambda (x - c_body)) of every particle, and the frame.
+// One box per body.
+__global__ __launch_bounds__(1024) void geometry_frame_kernel(const double* __restrict__ box, int nbody, double amin,
+                                                             GeomFrame* __restrict__ frame) {
+    double centre[3];
+    int status;
+    const double lam = fixed_frame<1024>(box, nbody, 1, -1, amin, centre, &status);
+    if (threadIdx.x == 0) {
+        frame->lam = lam;
+        frame->status = status;
+    }
+}
+
+// FIXED: X = rint(lambda (x - c_body)) of every particle, and the frame (shares
+// = 0: it is there already, and each body has one box).
 // head not null: every particle into the grid, each bucket a list linked
 // through nodes[p] = (cell, next particle or -1), newest first (the order
 // varies between runs; near_grid_kernel sorts what it finds).  body_of (may be
-// null) gets each particle's body.  Grid (workgroups per body, bodies).
+// null) gets each particle's body.  Grid (bodies, workgroups per body).
 template <bool FIXED>
 __global__ __launch_bounds__(256) void geometry_place_kernel(MatvecArgs a, const int4* __restrict__ ranges,
                                                             const double* __restrict__ box, int shares, double amin,
                                                             int4* __restrict__ fixed, GeomFrame* __restrict__ frame,
                                                             double inv_h, uint32_t mask, int32_t* __restrict__ head,
                                                             int4* __restrict__ nodes, int32_t* __restrict__ body_of) {
-    const int body = (int)blockIdx.y;
+    const int body = (int)blockIdx.x;
     const int4 r = ranges[body];
     const int m = (r.y - r.x) + (r.w - r.z);
     double centre[3] = {0.0, 0.0, 0.0}, lam = 0.0;
     if constexpr (FIXED) {
         int status;
-        lam = fixed_frame(box, (int)gridDim.y, shares, body, amin, centre, &status);
-        if (blockIdx.x == 0 && body == 0 && threadIdx.x == 0) {
-            frame->lam = lam;
-            frame->status = status;
+        if (shares == 0) {
+            lam = frame->lam;
+            status = frame->status;
+            const double* q = box + 6 * (int64_t)body;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) centre[k] = q[k] <= q[3 + k] ? 0.5 * (q[k] + q[3 + k]) : 0.0;
+        } else {
+            lam = fixed_frame<256>(box, (int)gridDim.x, shares, body, amin, centre, &status);
+            if (blockIdx.y == 0 && body == 0 && threadIdx.x == 0) {
+                frame->lam = lam;
+                frame->status = status;
+            }
         }
         if (status) return;  // the same in every workgroup
     }
-    for (int t = (int)(blockIdx.x * 256 + threadIdx.x); t < m; t += (int)gridDim.x * 256) {
+    for (int t = (int)(blockIdx.y * 256 + threadIdx.x); t < m; t += (int)gridDim.y * 256) {
         const int p = body_particle(r, a.ns, t);
         double x[3];
         particle_pos(a, p, x);
@@ -1497,16 +1522,16 @@ __global__ __launch_bounds__(256) void near_grid_kernel(MatvecArgs a, int n, dou
 // The FP64 lists of small problems by testing every pair of a body in one launch:
 // four targets per wave, whose lanes take 64 sources at a time (four batches'
 // loads in flight); a ballot places the near ones, so the lists come out in
-// increasing order.  Grid (16 targets each, bodies).  *max_cnt is zero before
+// increasing order.  Grid (bodies, 16 targets each).  *max_cnt is zero before
 // (geometry_clear_kernel's job otherwise).
 __global__ __launch_bounds__(256) void near_small_kernel(MatvecArgs a, const int4* __restrict__ ranges,
                                                         int32_t* __restrict__ cnt, int32_t* __restrict__ idx, int cap,
                                                         int32_t* __restrict__ max_cnt) {
     constexpr int REC = rec_len<double, 3>(), U = 4, Q = 4;
-    const int4 r = ranges[blockIdx.y];
+    const int4 r = ranges[blockIdx.x];
     const int m = (r.y - r.x) + (r.w - r.z);
     const int lane = (int)threadIdx.x & 63;
-    const int t0 = ((int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) * U;
+    const int t0 = ((int)blockIdx.y * 4 + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6)) * U;
     if (t0 >= m) return;
     double xi[U][3], sum_seg[U], sum_blob[U];
     int32_t* e[U];
@@ -2073,21 +2098,30 @@ static void launch_geometry(const MatvecArgs& a, const GeometryArgs& g, bool fix
     const int4* ranges = reinterpret_cast<const int4*>(g.ranges);
     int32_t* head = grid ? grid->fill : nullptr;
     const int table = grid ? grid->table : 0;
-    const int shares = box_shares(g.nbody, g.largest);
+    const double amin = std::min(a.a_seg, a.a_blob);
+    int shares = box_shares(g.nbody, g.largest);
     if (fixed)
-        hipLaunchKernelGGL(geometry_clear_kernel<true>, dim3((unsigned)shares, (unsigned)g.nbody), dim3(256), 0, stream,
+        hipLaunchKernelGGL(geometry_clear_kernel<true>, dim3((unsigned)g.nbody, (unsigned)shares), dim3(256), 0, stream,
                            a, ranges, g.box, head, table, max_cnt);
     else
         hipLaunchKernelGGL(geometry_clear_kernel<false>, dim3((unsigned)std::max(1, table / 4096)), dim3(256), 0,
                            stream, a, ranges, g.box, head, table, max_cnt);
     const int per_body = std::max(1, std::min((g.largest + 255) / 256, std::max(1, 4096 / g.nbody)));
-    const dim3 place((unsigned)per_body, (unsigned)g.nbody);
+    const dim3 place((unsigned)g.nbody, (unsigned)per_body);
+    if (fixed && g.nbody > kFrameBodies) {
+        // (every box in every workgroup is the square of the bodies: an evaluation
+        // of 20,000 bodies of 40 at new positions took 1,835 us, 980 so; the
+        // launch takes 1.6 us more where there are 300)
+        hipLaunchKernelGGL(geometry_frame_kernel, dim3(1), dim3(1024), 0, stream, (const double*)g.box, g.nbody, amin,
+                           g.frame);
+        shares = 0;
+    }
     const uint32_t mask = (uint32_t)table - 1;
     int4* nodes = grid ? grid->nodes : nullptr;
     int32_t* body_of = grid && g.nbody > 1 ? grid->body_of : nullptr;
     if (fixed)
         hipLaunchKernelGGL(geometry_place_kernel<true>, place, dim3(256), 0, stream, a, ranges, (const double*)g.box,
-                           shares, std::min(a.a_seg, a.a_blob), g.fixed, g.frame, inv_h, mask, head, nodes, body_of);
+                           shares, amin, g.fixed, g.frame, inv_h, mask, head, nodes, body_of);
     else
         hipLaunchKernelGGL(geometry_place_kernel<false>, place, dim3(256), 0, stream, a, ranges, (const double*)g.box,
                            shares, 0.0, g.fixed, g.frame, inv_h, mask, head, nodes, body_of);
@@ -2103,7 +2137,7 @@ hipError_t build_near_list(int precision, const MatvecArgs& a, const GeometryArg
     const int n = a.ns + a.nb;
     if (n <= 0) return hipSuccess;
     if (precision == 0 && n <= kNearSmallMax) {
-        hipLaunchKernelGGL(near_small_kernel, dim3((unsigned)((g.largest + 15) / 16), (unsigned)g.nbody), dim3(256), 0,
+        hipLaunchKernelGGL(near_small_kernel, dim3((unsigned)g.nbody, (unsigned)((g.largest + 15) / 16)), dim3(256), 0,
                            stream, a, reinterpret_cast<const int4*>(g.ranges), near.cnt, near.idx, near.cap,
                            near.max_cnt);
         return hipGetLastError();
