@@ -122,6 +122,39 @@ def test_refused_positions_and_the_ones_after_them(ns, nb):
         h.close()
 
 
+@pytest.mark.parametrize("device", [False, True])
+@pytest.mark.parametrize("ns,nb", [(200, 100), (5000, 1500)])
+def test_profile_counts_no_refused_evaluation(ns, nb, device):
+    print(f"case ns={ns} nb={nb} device={device}", flush=True)
+    import torch
+
+    put = (lambda a: torch.tensor(a, device="cuda")) if device else (lambda a: a)
+    xs, xb, fs, fb = (put(a) for a in cloud(ns, nb, 4, 5))
+    bad = put(np.full(3 * ns, np.nan))
+    torch.cuda.synchronize()
+    h = RpyHandle(ns, nb, seg_dof=6, precision=P32, bs_accumulate=True, seg_radius=1.0, blob_radius=1.2,
+                  memory=L.MEMORY_DEVICE if device else L.MEMORY_HOST)
+    try:
+        for what, a in ((L.SEG_POSITIONS, xs), (L.BLOB_POSITIONS, xb), (L.SEG_FORCES, fs), (L.BLOB_FORCES, fb)):
+            h.upload(what, a)
+        h.profile(True)
+        h.evaluate()
+        ms, launches = h.profile_read()[P32]
+        assert launches == 1 and ms > 0
+        for _ in range(2):
+            h.upload(L.SEG_POSITIONS, bad)
+            with pytest.raises(Exception, match="finite"):
+                h.evaluate()
+            assert h.profile_read()[P32] == (0.0, 0)
+        h.upload(L.SEG_POSITIONS, xs)
+        for _ in range(3):
+            h.evaluate()
+        again, launches = h.profile_read()[P32]
+        assert launches == 3 and 0 < again < 30 * ms + 1.0
+    finally:
+        h.close()
+
+
 @pytest.mark.parametrize("radius", [1e-9, 3e-7, 1.0, 4e5])
 def test_one_particle_of_any_radius(radius):
     """Force and torque on a particle by itself, whose extent gives the
