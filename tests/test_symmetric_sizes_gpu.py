@@ -203,3 +203,27 @@ def test_large_ensembles_take_the_form_within_the_buffer_limit():
             assert h.symmetric(P32) == takes
         finally:
             h.close()
+
+
+def test_many_small_bodies_keep_the_directed_form():
+    """Bodies that leave their 64-particle tiles mostly empty, or have few tiles,
+    take the directed form bit for bit; the same particles in bodies that fill
+    them do not."""
+    for bodies, takes in (([(20, 30)] * 1000, False), ([(64, 64)] * 1000, False), ([(129, 65)] * 300, False),
+                          ([(640, 640)] * 40, True)):
+        ns, nb = sum(s for s, _ in bodies), sum(b for _, b in bodies)
+        xs, xb, fs, fb = cloud(ns, nb, 6)
+        h, plain = (RpyHandle(ns, nb, seg_dof=6, precision=P64, bs_accumulate=True) for _ in range(2))
+        try:
+            print(f"case {len(bodies)} bodies of {bodies[0]}", flush=True)
+            for x in (h, plain):
+                x.set_bodies([s for s, _ in bodies], [b for _, b in bodies])
+                load(x, xs, xb, fs, fb)
+            plain.set_symmetric(P64, False)
+            h.evaluate()
+            plain.evaluate()
+            a, b = read(h, ns, nb), read(plain, ns, nb)
+            assert rel(a, b) <= 1e-12 and np.array_equal(a, b) != takes
+        finally:
+            h.close()
+            plain.close()

@@ -132,17 +132,21 @@ TileShape default_shape(int precision, int ns, int nb, int num_cus, int seg_dof,
     return s;
 }
 
-// Whether bodies of these sizes give every CU ~4 items of the symmetric form's
-// panels (12,800 segments + 9,000 blobs: 3,741 pairs of groups of four tiles
-// for 256 CUs).
+// Tiles of 64 particles of one class in a body.
+static double tiles_of(const BodyRange& b) {
+    return double((b.seg_end - b.seg_begin + 63) / 64 + (b.blob_end - b.blob_begin + 63) / 64);
+}
+
+// Whether the bodies' pairs of four-tile groups come to four per CU (one body
+// of 11,300 particles; 12,800 segments + 9,000 blobs have 3,741 for 256 CUs):
+// where two particles per lane leave enough work to spread evenly.
 static bool panels_fill(const std::vector<BodyRange>& bodies, int num_cus) {
-    double items = 0.0;
+    double pairs = 0.0;
     for (const BodyRange& b : bodies) {
-        const long tiles = (b.seg_end - b.seg_begin + 63L) / 64 + (b.blob_end - b.blob_begin + 63L) / 64;
-        const double groups = double((tiles + 3) / 4);
-        items += groups * (groups + 1.0) / 2.0;
+        const double groups = std::ceil(tiles_of(b) / 4.0);
+        pairs += groups * (groups + 1.0) / 2.0;
     }
-    return items >= 4.0 * (num_cus > 0 ? num_cus : 256);
+    return pairs >= 4.0 * (num_cus > 0 ? num_cus : 256);
 }
 
 // Whether the symmetric form's partial slots for these bodies stay within
@@ -156,7 +160,7 @@ static bool sym_fits(const std::vector<BodyRange>& bodies, int kind, int seg_dof
     double least = 0.0, most = 0.0;
     const double panel = sym_panel(kind);
     for (const BodyRange& b : bodies) {
-        const double t = double((b.seg_end - b.seg_begin + 63) / 64 + (b.blob_end - b.blob_begin + 63) / 64);
+        const double t = tiles_of(b);
         least += std::max(0.0, 0.5 * t * t * (1.0 / panel + 1.0 / kSymMaxRun) - t);
         most += 0.5 * t * (t * (1.0 / panel + 1.0) + 3.0);
     }
@@ -279,22 +283,39 @@ bool symmetric_applies(const tfs_rpy* h, uint32_t blocks) {
 }
 
 // The symmetric form's kind that a handle without a chosen shape takes by its
-// size, or 0.  Two particles per lane where the bodies' panels fill the device;
-// one per lane (twice as many, smaller items) from 8 pairs of tiles per CU on,
-// about 4,100 particles in one body; below that the launch is bound by its
-// longest item and the finest directed shape (one wave per 64 x 32 pairs) is
-// as fast.  Measured on MI355X per evaluation, directed / symmetric, us, with
-// rotations: 1,600 + 2,600 particles FP32 31 / 30, FP64 41 / 40; 2,461 + 3,333
-// 44 / 42, 64 / 57; 6,000 + 4,500 109 / 100, 171 / 155; 12,800 + 9,000 392 /
-// 340, 693 / 560; twelve uneven bodies 3,480 / 2,830, 6,250 / 4,750.
+// size, or 0.  Measured on MI355X, us per evaluation, directed / wide / narrow
+// (two or one particle per lane); "6" with rotations, "3" without.
+//
+// How many bodies fill their tiles: a pair of tiles costs 64 x 64 steps however
+// many particles they hold, a directed tile one step per source that is there.
+// The symmetric form is the faster one from 1.8 of the latter to one of the
+// former on (2 for large full tiles; 6 FP32, 3 FP64): 1,000 bodies of 20 + 30
+// (0.5) 27 / 58 / 50, 24 / 49 / 43; 1,000 of 128 + 128 (1.60) 105 / 131 / 118,
+// 94 / 107 / 101; 200 of 256 + 256 (1.78) 73 / 91 / 88, 72 / 89 / 72; 40 of
+// 200 + 2,000 (1.86) 151 / 137 / 133, 232 / 181 / 177; 64 of 512 + 512 (1.88)
+// 85 / 97 / 85, 88 / 82 / 73.
+//
+// How much there is: narrow from 8 pairs of tiles per CU on, about 4,100
+// particles in one body, below which the launch is bound by its longest item
+// and the finest directed shape (one wave per 64 x 32 pairs) is as fast; wide
+// where panels_fill.  3 FP32: 1,600 + 2,600 particles 23 / 28 / 23, 4,000 +
+// 3,000 38 / 40 / 37, 6,000 + 5,500 81 / 74 / 72, 9,000 + 7,000 143 / 119 / 120,
+// 12,800 + 9,000 255 / 202 / 208.  3 FP64: 32 / 34 / 29, 60 / 56 / 54, 132 / 111
+// / 112, 241 / 189 / 197, 426 / 327 / 344.  6 FP64: 44 / 49 / 41, 90 / 85 / 84,
+// 192 / 171 / 171, 399 / 309 / 313, 680 / 550 / 563.  6 FP32: 30 / 43 / 31, 54 /
+// 68 / 60, 114 / 119 / 112, 224 / 201 / 194, 383 / 352 / 340 -- here the form
+// costs up to a tenth up to 9,000 particles, and is taken for its error, which
+// is a quarter smaller (2,460 + 3,333: 1.2e-7 against 1.5e-7).
 static int sym_by_size(const tfs_rpy* h, bool wide_fits) {
     const double cus = h->num_cus > 0 ? h->num_cus : 256;
-    if (wide_fits && panels_fill(h->bodies, h->num_cus)) return kSymWide;
-    double pairs = 0.0;
+    double pairs = 0.0, directed = 0.0;
     for (const BodyRange& b : h->bodies) {
-        const double t = double((b.seg_end - b.seg_begin + 63) / 64 + (b.blob_end - b.blob_begin + 63) / 64);
+        const double t = tiles_of(b);
         pairs += t * (t + 1.0) / 2.0;
+        directed += t * ((b.seg_end - b.seg_begin) + (double)(b.blob_end - b.blob_begin)) / 64.0;
     }
+    if (directed < 1.8 * pairs) return 0;
+    if (wide_fits && panels_fill(h->bodies, h->num_cus)) return kSymWide;
     return pairs >= 8.0 * cus && sym_fits(h->bodies, kSymNarrow, h->desc.seg_dof, h->num_cus) ? kSymNarrow : 0;
 }
 
