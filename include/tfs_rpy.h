@@ -211,7 +211,8 @@ int tfs_rpy_body_times(tfs_rpy *h, double *ms_per_body);
  * replayed by tfs_graph_launch on the handle's stream (no counterpart in the
  * reference, which launches kernels one by one, rpy_mobility_solver.cu:258-337).
  * The work list, partial buffer and near-pair lists are fixed at capture:
- * re-create the graph after positions change. */
+ * re-create the graph after positions change.  A graph ends with its handle:
+ * launching it then is refused, destroying it is not. */
 typedef struct tfs_graph tfs_graph;
 int tfs_rpy_graph_create(tfs_rpy *h, uint32_t blocks, int32_t evaluations, tfs_graph **out);
 int tfs_graph_launch(tfs_graph *g);

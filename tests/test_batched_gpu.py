@@ -106,3 +106,21 @@ def test_graph_replays_match_eager_every_time(persistent):
         g.close()
     finally:
         h.close()
+
+
+def test_a_graph_ends_with_its_handle():
+    ns, nb = 300, 200
+    rng = np.random.default_rng(1)
+    h = RpyHandle(ns, nb, seg_dof=6, precision=L.PRECISION_FP64, bs_accumulate=True)
+    for what, n in ((L.SEG_POSITIONS, 3 * ns), (L.BLOB_POSITIONS, 3 * nb), (L.SEG_FORCES, 6 * ns), (L.BLOB_FORCES, 3 * nb)):
+        h.upload(what, rng.uniform(-9, 9, n))
+    first, second, third = (h.graph(L.BLOCK_ALL) for _ in range(3))
+    second.launch()
+    second.close()
+    first.launch()
+    third.launch()
+    h.close()
+    with pytest.raises(RuntimeError, match="destroyed"):
+        first.launch()
+    first.close()
+    del third

@@ -99,6 +99,7 @@ struct tfs_rpy {
     bool sized = false;             // that and the shapes that no caller chose are made
     bool graph_made = false;        // a captured graph may hold `partial`: replaced buffers stay
     std::vector<double*> retired;   // until the handle goes
+    std::vector<tfs_graph*> graphs; // tfs_rpy_graph_create's
     // Stop flag passed to the kernels of later evaluations (set by a solver
     // around its speculative Krylov iterations; null otherwise).
     const int32_t* skip_flag = nullptr;

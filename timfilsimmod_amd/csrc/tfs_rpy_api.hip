@@ -736,6 +736,21 @@ int run_matvec(tfs_rpy* h, uint32_t blocks, int precision, CView fs, CView fb, V
 
 using namespace tfs;
 
+// Ends with its handle (whose stream, arrays and partial sums it uses): one
+// destroyed later has nothing left to wait for.
+struct tfs_graph {
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+    tfs_rpy* owner = nullptr;
+    void end() {
+        if (exec) hipGraphExecDestroy(exec);
+        if (graph) hipGraphDestroy(graph);
+        exec = nullptr;
+        graph = nullptr;
+        owner = nullptr;
+    }
+};
+
 extern "C" {
 
 const char* tfs_last_error(void) { return g_last_error.c_str(); }
@@ -817,6 +832,7 @@ int tfs_rpy_create(const tfs_rpy_desc* desc, tfs_rpy** out) {
 int tfs_rpy_destroy(tfs_rpy* h) {
     if (!h) return TFS_OK;
     if (h->stream) hipStreamSynchronize(h->stream);
+    for (tfs_graph* g : h->graphs) g->end();
     for (auto& kv : h->plans) {
         hipFree(kv.second.d_tiles);
         hipFree(kv.second.d_items);
@@ -1104,12 +1120,6 @@ int tfs_rpy_set_bodies(tfs_rpy* h, int32_t num_bodies, const int32_t* segs_per_b
     return TFS_OK;
 }
 
-struct tfs_graph {
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    hipStream_t stream = nullptr;
-};
-
 int tfs_rpy_graph_create(tfs_rpy* h, uint32_t blocks, int32_t evaluations, tfs_graph** out) {
     if (!h || !out || evaluations < 1 || (blocks & ~TFS_BLOCK_ALL))
         return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_graph_create: bad arguments");
@@ -1124,7 +1134,6 @@ int tfs_rpy_graph_create(tfs_rpy* h, uint32_t blocks, int32_t evaluations, tfs_g
     h->profiling = false;
     h->graph_made = true;
     tfs_graph* g = new tfs_graph();
-    g->stream = h->stream;
     e = hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) {
         h->profiling = prof;
@@ -1145,21 +1154,27 @@ int tfs_rpy_graph_create(tfs_rpy* h, uint32_t blocks, int32_t evaluations, tfs_g
         delete g;
         return hip_fail(e, "tfs_rpy_graph_create: instantiate");
     }
+    g->owner = h;
+    h->graphs.push_back(g);
     *out = g;
     return TFS_OK;
 }
 
 int tfs_graph_launch(tfs_graph* g) {
     if (!g) return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_graph_launch: null graph");
-    hipError_t e = hipGraphLaunch(g->exec, g->stream);
+    if (!g->owner) return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_graph_launch: the graph's handle was destroyed");
+    hipError_t e = hipGraphLaunch(g->exec, g->owner->stream);
     return e == hipSuccess ? TFS_OK : hip_fail(e, "tfs_graph_launch");
 }
 
 int tfs_graph_destroy(tfs_graph* g) {
     if (!g) return TFS_OK;
-    hipStreamSynchronize(g->stream);
-    if (g->exec) hipGraphExecDestroy(g->exec);
-    if (g->graph) hipGraphDestroy(g->graph);
+    if (g->owner) {
+        hipStreamSynchronize(g->owner->stream);
+        auto& own = g->owner->graphs;
+        own.erase(std::find(own.begin(), own.end(), g));
+        g->end();
+    }
     delete g;
     return TFS_OK;
 }
