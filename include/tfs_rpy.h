@@ -198,7 +198,8 @@ int tfs_rpy_get_source_split(tfs_rpy *h, int32_t precision, int32_t *split);
  * Handles that no shape was set for also evaluate this way, with either kind of
  * segments, wherever their size favours it (from about 4,100 particles on);
  * the shape that the functions here report is then the one such a handle falls
- * back to, and setting any shape ends it. */
+ * back to, and setting any shape ends it -- except the one that was reported
+ * after tfs_rpy_autotune, which brings back what the autotuner kept. */
 int tfs_rpy_set_symmetric(tfs_rpy *h, int32_t precision, int32_t enable);
 /* 1 if the precision's current shape is the symmetric form. */
 int tfs_rpy_get_symmetric(tfs_rpy *h, int32_t precision, int32_t *enabled);

@@ -205,6 +205,31 @@ def test_large_ensembles_take_the_form_within_the_buffer_limit():
             h.close()
 
 
+def test_the_autotuned_shape_set_again_gives_the_same_results():
+    """6-DOF handles report the directed shape behind the symmetric form: setting
+    what was reported after the autotuner brings its choice back, and switching
+    the form off or setting another shape does not."""
+    ns, nb = 12800, 9000                         # symmetric by a fifth
+    xs, xb, fs, fb = cloud(ns, nb, 4)
+    h = RpyHandle(ns, nb, seg_dof=6, precision=P64, bs_accumulate=True)
+    try:
+        load(h, xs, xb, fs, fb)
+        h.autotune(P64, reps=1)
+        h.evaluate()
+        tuned, s = read(h, ns, nb), h.tile_shape(P64)
+        put = h.set_split_shape if s["split"] else h.set_tile_shape
+        other = (h.set_tile_shape, (256, 2, 1024))
+        for first, args in (other, (h.set_symmetric, (False,))):
+            first(P64, *args)
+            h.evaluate()
+            assert not np.array_equal(read(h, ns, nb), tuned)
+            put(P64, s["block"], s["per_thread"], s["chunk"])
+            h.evaluate()
+            assert np.array_equal(read(h, ns, nb), tuned)
+    finally:
+        h.close()
+
+
 def test_many_small_bodies_keep_the_directed_form():
     """Bodies that leave their 64-particle tiles mostly empty, or have few tiles,
     take the directed form bit for bit; the same particles in bodies that fill

@@ -95,6 +95,8 @@ struct tfs_rpy {
     // take: -1 while the shape is the default, where the handle may choose it
     // by its size, else 0 (off) or the kind that the autotuner found fastest.
     int sym_pick[2] = {-1, -1};
+    tfs::TileShape tuned[2];        // what the autotuner left, for a caller who sets it again
+    int tuned_pick[2] = {0, 0};
     int sym_size = 0;               // the kind by size for the present bodies, or 0
     bool sized = false;             // that and the shapes that no caller chose are made
     bool graph_made = false;        // a captured graph may hold `partial`: replaced buffers stay

@@ -1041,7 +1041,11 @@ static int set_shape(tfs_rpy* h, const char* fn, int32_t precision, int32_t bloc
         return fail(TFS_ERR_INVALID_ARGUMENT, std::string(fn) + ": the source split has no persistent form");
     h->shape[precision] = TileShape{block, per_thread, chunk, pers, split};
     h->shape_chosen[precision] = true;
-    h->sym_pick[precision] = 0;
+    // the shape that the autotuner's choice is reported as stands for that choice
+    const TileShape& tuned = h->tuned[precision];
+    const bool as_tuned = !pers && block == tuned.block && per_thread == tuned.per_thread && chunk == tuned.chunk &&
+                          split == tuned.split;
+    h->sym_pick[precision] = as_tuned ? h->tuned_pick[precision] : 0;
     return TFS_OK;
 }
 
@@ -1267,6 +1271,8 @@ int tfs_rpy_autotune(tfs_rpy* h, int32_t precision, uint32_t blocks, int32_t rep
     h->shape[precision] = best;
     h->shape_chosen[precision] = true;
     h->sym_pick[precision] = best_pick;
+    h->tuned[precision] = best;
+    h->tuned_pick[precision] = best_pick;
     if (best_ms) *best_ms = best_t;
     return rc;
 }
