@@ -252,3 +252,38 @@ def test_many_small_bodies_keep_the_directed_form():
         finally:
             h.close()
             plain.close()
+
+
+def test_autotune_tries_both_kinds_without_rotations():
+    """Twelve bodies of 320 + 2,000 particles with 3-DOF segments, FP64: one
+    particle per lane, the handle's own choice, is a tenth faster than two or the
+    directed shapes; the autotuner keeps it, or has found something faster."""
+    import time
+
+    bodies = [(320, 2000)] * 12
+    ns, nb = (sum(b[k] for b in bodies) for k in (0, 1))
+    xs, xb, fs, fb = cloud(ns, nb, 6)
+    own, tuned = (RpyHandle(ns, nb, seg_dof=3, precision=P64, bs_accumulate=True) for _ in range(2))
+    try:
+        for h in (own, tuned):
+            h.set_bodies([s for s, _ in bodies], [b for _, b in bodies])
+            load(h, xs, xb, fs, fb)
+            h.evaluate()
+        want = read(own, ns, nb)
+        assert np.array_equal(read(tuned, ns, nb), want)
+        ms = 1e9
+        for _ in range(5):
+            t0 = time.perf_counter()
+            for _ in range(20):
+                own.evaluate()
+            own.sync()
+            ms = min(ms, (time.perf_counter() - t0) * 50)
+        best = tuned.autotune(P64, reps=20)
+        print(f"case own {ms * 1e3:.1f} us, tuned {best * 1e3:.1f}, shape {tuned.tile_shape(P64)}", flush=True)
+        tuned.evaluate()
+        got = read(tuned, ns, nb)
+        assert rel(got, want) <= 1e-12
+        assert np.array_equal(got, want) or best < ms
+    finally:
+        own.close()
+        tuned.close()

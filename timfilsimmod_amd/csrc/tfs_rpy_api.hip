@@ -1202,8 +1202,8 @@ int tfs_rpy_autotune(tfs_rpy* h, int32_t precision, uint32_t blocks, int32_t rep
     int ns = 0, nb = 0;
     largest_body(h, &ns, &nb);
     const double pairs = double(ns + nb) * double(ns + nb);
+    int best_pick = h->sym_pick[precision];  // (kept if nothing could be timed)
     h->sym_pick[precision] = 0;
-    int best_pick = 0;
     auto time_shape = [&](const TileShape& sh) {
         h->shape[precision] = sh;
         rc = tfs_rpy_evaluate(h, blocks);  // builds the plan; warm-up
@@ -1221,19 +1221,17 @@ int tfs_rpy_autotune(tfs_rpy* h, int32_t precision, uint32_t blocks, int32_t rep
             best_pick = h->sym_pick[precision];
         }
     };
-    // The symmetric form: as the shape of 3-DOF handles, behind the default
-    // shape of 6-DOF ones.
-    if (symmetric_applies(h, blocks) && sym_fits(h->bodies, kSymWide, h->desc.seg_dof, h->num_cus)) {
-        if (h->desc.seg_dof == 3) {
+    // The symmetric form, both kinds: the wide one as the shape of 3-DOF handles,
+    // otherwise behind the default shape.
+    for (int kind : {kSymWide, kSymNarrow}) {
+        if (rc || !symmetric_applies(h, blocks) || !sym_fits(h->bodies, kind, h->desc.seg_dof, h->num_cus)) continue;
+        if (h->desc.seg_dof == 3 && kind == kSymWide) {
             TileShape sym{256, 1, 0, 0, 0};
             sym.symmetric = kSymWide;
             time_shape(sym);
         } else {
-            for (int kind : {kSymWide, kSymNarrow}) {
-                if (rc || !sym_fits(h->bodies, kind, h->desc.seg_dof, h->num_cus)) continue;
-                h->sym_pick[precision] = kind;
-                time_shape(default_shape(precision, ns, nb, h->num_cus, h->desc.seg_dof, (int)h->bodies.size()));
-            }
+            h->sym_pick[precision] = kind;
+            time_shape(default_shape(precision, ns, nb, h->num_cus, h->desc.seg_dof, (int)h->bodies.size()));
             h->sym_pick[precision] = 0;
         }
     }
