@@ -199,7 +199,9 @@ int tfs_rpy_get_source_split(tfs_rpy *h, int32_t precision, int32_t *split);
  * segments, wherever their size favours it (from about 4,100 particles on);
  * the shape that the functions here report is then the one such a handle falls
  * back to, and setting any shape ends it -- except the one that was reported
- * after tfs_rpy_autotune, which brings back what the autotuner kept. */
+ * after tfs_rpy_autotune, which brings back what the autotuner kept; enable =
+ * 0 ends it as well, and with 6-DOF segments and no shape set since, enable = 1
+ * then gives the handle its own choice back. */
 int tfs_rpy_set_symmetric(tfs_rpy *h, int32_t precision, int32_t enable);
 /* 1 if the precision's current shape is the symmetric form. */
 int tfs_rpy_get_symmetric(tfs_rpy *h, int32_t precision, int32_t *enabled);

@@ -230,6 +230,30 @@ def test_the_autotuned_shape_set_again_gives_the_same_results():
         h.close()
 
 
+def test_a_six_dof_handle_switched_off_gets_its_own_choice_back():
+    ns, nb = 2500, 2300
+    h = RpyHandle(ns, nb, seg_dof=6, precision=P64, bs_accumulate=True)
+    try:
+        load(h, *cloud(ns, nb, 4))
+        with pytest.raises(RuntimeError):
+            h.set_symmetric(P64)                 # cannot be set, only left
+        results = []
+        for enable in (None, False, True, False):
+            if enable is not None:
+                h.set_symmetric(P64, enable)
+            h.evaluate()
+            results.append(read(h, ns, nb))
+        own, off = results[:2]
+        assert rel(own, off) <= 1e-12 and not np.array_equal(own, off)
+        assert np.array_equal(results[2], own) and np.array_equal(results[3], off)
+        s = h.tile_shape(P64)
+        (h.set_split_shape if s["split"] else h.set_tile_shape)(P64, s["block"], s["per_thread"], s["chunk"])
+        with pytest.raises(RuntimeError):
+            h.set_symmetric(P64)                 # a shape was set
+    finally:
+        h.close()
+
+
 def test_many_small_bodies_keep_the_directed_form():
     """Bodies that leave their 64-particle tiles mostly empty, or have few tiles,
     take the directed form bit for bit; the same particles in bodies that fill

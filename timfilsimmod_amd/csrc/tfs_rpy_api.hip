@@ -1073,6 +1073,10 @@ int tfs_rpy_set_symmetric(tfs_rpy* h, int32_t precision, int32_t enable) {
         }
         return TFS_OK;
     }
+    if (h->desc.seg_dof == 6 && h->sym_pick[precision] == 0 && !h->shape_chosen[precision]) {  // was switched off
+        h->sym_pick[precision] = -1;
+        return TFS_OK;
+    }
     if (h->desc.seg_dof != 3)
         return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_set_symmetric: the symmetric form needs 3-DOF segments");
     if (h->shape[precision].persistent > 0)
