@@ -102,6 +102,9 @@ int tfs_rpy_upload(tfs_rpy *h, int32_t what, const double *src);
 /* copy_{segment,blob}_velocities_to_host (rpy_mobility_solver.cu:177-205):
  * `what` is TFS_SEG_VELOCITIES / TFS_BLOB_VELOCITIES. Asynchronous. */
 int tfs_rpy_download(tfs_rpy *h, int32_t what, double *dst);
+/* How many of those, of a host-memory handle, a kernel made by itself: arrays of
+ * up to 1 MB in one pinned allocation (others go to the copy engines). */
+int tfs_rpy_kernel_copies(tfs_rpy *h, int64_t *copies);
 
 /* evaluate_{segment_segment,segment_blob,blob_blob,blob_segment,full}_mobility
  * (rpy_mobility_solver.cu:258-337) on the uploaded positions/forces, into the

@@ -75,6 +75,7 @@ def test_null_handles_are_errors_not_crashes():
     out = ctypes.c_int32(7)
     assert lib.tfs_rpy_get_symmetric(None, 1, ctypes.byref(out)) == L.TFS_ERR_INVALID_ARGUMENT
     assert out.value == 7
+    assert lib.tfs_rpy_kernel_copies(None, ctypes.byref(ctypes.c_int64())) == L.TFS_ERR_INVALID_ARGUMENT
 
 
 def test_create_reports_missing_device_on_cpu_host():

@@ -1,7 +1,8 @@
 """Uploads and downloads of host memory that a kernel reaches (pinned arrays of up
 to 1 MB, whole ones and views inside them) and that it does not (larger ones,
 pageable arrays): the same evaluation from each, bit for bit, and again from
-other values (nothing is kept from the first)."""
+other values (nothing is kept from the first); the kernel's copies are counted,
+one for every array that it reaches and none for the others."""
 import numpy as np
 import pytest
 
@@ -34,13 +35,18 @@ def test_pinned_equals_pageable(ns, nb):
             box = 2.0 * (ns + nb) ** (1 / 3)
             plain = [rng.uniform(-box, box, lens[0]), rng.uniform(-box, box, lens[1]), rng.normal(size=lens[2]),
                      rng.normal(size=lens[3])]
+            before = h.kernel_copies()
             want = evaluate(h, plain, np.zeros(lens[4]), np.zeros(lens[5]))
+            assert h.kernel_copies() == before
             for off in (0, 3):
                 views = [p.array[off:off + n] for p, n in zip(pinned, lens)]
                 for v, a in zip(views, plain):
                     v[:] = a
                 got = evaluate(h, views[:4], views[4], views[5])
                 assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+                reached = sum(8 * n <= 1 << 20 for n in lens)
+                assert h.kernel_copies() == before + reached
+                before += reached
     finally:
         h.close()
         for p in pinned:

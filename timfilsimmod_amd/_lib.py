@@ -69,6 +69,7 @@ SIGNATURES = {
     "tfs_rpy_destroy": (ctypes.c_int, [_vp]),
     "tfs_rpy_upload": (ctypes.c_int, [_vp, _i32, _vp]),
     "tfs_rpy_download": (ctypes.c_int, [_vp, _i32, _vp]),
+    "tfs_rpy_kernel_copies": (ctypes.c_int, [_vp, ctypes.POINTER(ctypes.c_int64)]),
     "tfs_rpy_evaluate": (ctypes.c_int, [_vp, _u32]),
     "tfs_rpy_apply": (ctypes.c_int, [_vp, _u32, _vp, _vp, _vp, _vp]),
     "tfs_rpy_sync": (ctypes.c_int, [_vp]),

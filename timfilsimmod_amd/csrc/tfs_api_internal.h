@@ -81,6 +81,7 @@ struct tfs_rpy {
     int32_t* d_body_range = nullptr; // 4 per body (BodyRange), for the box and conversion kernels
     size_t body_cap = 0;
     int32_t* host_int = nullptr;  // pinned scratch
+    int64_t kernel_copies = 0;    // of pinned arrays (tfs_rpy_kernel_copies)
     double* blob_rep = nullptr;   // device blob repulsion staging (tfs_rpy_barrier_forces, host memory)
     // Persistent launches with timing: per-item stamps of the last launch and
     // the plan they belong to.

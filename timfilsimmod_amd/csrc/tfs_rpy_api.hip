@@ -76,15 +76,17 @@ static bool kernel_reaches(const void* p, size_t bytes, void** device) {
 // the copy engine take turns.  A whole evaluation from pinned arrays, FP64,
 // copies / kernels: 320 segments + 2,000 blobs 113 / 80 us, 2,140 + 3,333 152 /
 // 120, 12,800 + 9,000 694 / 656.
-static hipError_t copy_array(double* dst, const double* src, size_t len, bool host, bool to_device, hipStream_t stream) {
+static hipError_t copy_array(tfs_rpy* h, double* dst, const double* src, size_t len, bool to_device) {
     const size_t bytes = len * sizeof(double);
-    if (!host) return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, stream);
+    const hipStream_t stream = h->stream;
+    if (h->desc.memory != TFS_MEMORY_HOST) return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, stream);
     void* reached = nullptr;
     if (!kernel_reaches(to_device ? src : dst, bytes, &reached))
         return hipMemcpyAsync(dst, src, bytes, to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, stream);
     CopyList L;
     if (to_device) L.add(static_cast<const double*>(reached), dst, (int64_t)len);
     else L.add(src, static_cast<double*>(reached), (int64_t)len);
+    h->kernel_copies++;
     return copy_list(L, stream);
 }
 
@@ -882,7 +884,7 @@ int tfs_rpy_upload(tfs_rpy* h, int32_t what, const double* src) {
     if (len == 0) return TFS_OK;
     if (!src) return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_upload: null source");
     if (what == TFS_SEG_POSITIONS || what == TFS_BLOB_POSITIONS) invalidate_near(h);
-    const hipError_t e = copy_array(dev, src, len, h->desc.memory == TFS_MEMORY_HOST, true, h->stream);
+    const hipError_t e = copy_array(h, dev, src, len, true);
     return e == hipSuccess ? TFS_OK : hip_fail(e, "tfs_rpy_upload");
 }
 
@@ -896,8 +898,14 @@ int tfs_rpy_download(tfs_rpy* h, int32_t what, double* dst) {
     if (rc) return rc;
     if (len == 0) return TFS_OK;
     if (!dst) return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_download: null destination");
-    const hipError_t e = copy_array(dst, dev, len, h->desc.memory == TFS_MEMORY_HOST, false, h->stream);
+    const hipError_t e = copy_array(h, dst, dev, len, false);
     return e == hipSuccess ? TFS_OK : hip_fail(e, "tfs_rpy_download");
+}
+
+int tfs_rpy_kernel_copies(tfs_rpy* h, int64_t* copies) {
+    if (!h || !copies) return fail(TFS_ERR_INVALID_ARGUMENT, "tfs_rpy_kernel_copies: null argument");
+    *copies = h->kernel_copies;
+    return TFS_OK;
 }
 
 int tfs_rpy_evaluate(tfs_rpy* h, uint32_t blocks) {

@@ -81,6 +81,12 @@ class RpyHandle:
     def download(self, what: int, dst):
         L.check(L.lib().tfs_rpy_download(self.h, what, L.ptr(dst)))
 
+    def kernel_copies(self) -> int:
+        """Uploads and downloads of pinned arrays that a kernel made, so far."""
+        out = ctypes.c_int64()
+        L.check(L.lib().tfs_rpy_kernel_copies(self.h, ctypes.byref(out)))
+        return out.value
+
     def evaluate(self, blocks: int = L.BLOCK_ALL):
         L.check(L.lib().tfs_rpy_evaluate(self.h, blocks))
 
