@@ -54,19 +54,26 @@ hipError_t copy_list(const CopyList& list, hipStream_t stream) {
 constexpr size_t kKernelCopyMax = size_t(1) << 20;
 
 // Whether a kernel can read or write `bytes` at the host address p: all of it
-// in one pinned allocation (pageable memory is not), of a size where the copy
-// engines' hand-over costs more than the transfer.
+// in one pinned allocation (pageable memory is not, nor is an array of which
+// only some pages were registered), of a size where the copy engines' hand-over
+// costs more than the transfer.
 static bool kernel_reaches(const void* p, size_t bytes, void** device) {
     if (bytes == 0 || bytes > kKernelCopyMax || reinterpret_cast<uintptr_t>(p) % sizeof(double)) return false;
-    const char* c = static_cast<const char*>(p);
-    hipPointerAttribute_t first, last;
-    const bool known = hipPointerGetAttributes(&first, c) == hipSuccess &&
-                       hipPointerGetAttributes(&last, c + bytes - 1) == hipSuccess;
-    if (!known) (void)hipGetLastError();
-    if (!known || first.type != hipMemoryTypeHost || last.type != hipMemoryTypeHost || !first.devicePointer ||
-        static_cast<char*>(last.devicePointer) != static_cast<char*>(first.devicePointer) + (bytes - 1))
+    hipPointerAttribute_t at;
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();
         return false;
-    *device = first.devicePointer;
+    }
+    if (at.type != hipMemoryTypeHost || !at.devicePointer) return false;
+    if (hipMemGetAddressRange(&base, &size, static_cast<hipDeviceptr_t>(at.devicePointer)) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    const uintptr_t lo = reinterpret_cast<uintptr_t>(base), d = reinterpret_cast<uintptr_t>(at.devicePointer);
+    if (!base || d < lo || d - lo > size || bytes > size - (d - lo)) return false;
+    *device = at.devicePointer;
     return true;
 }
 
