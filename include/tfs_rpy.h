@@ -195,11 +195,12 @@ int tfs_rpy_get_source_split(tfs_rpy *h, int32_t precision, int32_t *split);
  * precisions; set for 3-DOF segments only (refused otherwise); evaluations whose
  * blocks lack SS, SB or BS, and the half-space domain, take the default
  * source-split shape instead.  No persistent form.  The default shape (both
- * precisions) of a handle with 3-DOF segments whose (largest) body's groups of
- * four tiles pair into at least four items per CU (e.g. 12,800 segments + 9,000
- * blobs: 3,741 items); enable = 0 selects the source-split default instead.
- * Handles that no shape was set for also evaluate this way, with either kind of
- * segments, wherever their size favours it (from about 4,100 particles on);
+ * precisions) of a handle with 3-DOF segments whose largest body has at least
+ * four pairs of four-tile groups per CU (about 11,300 particles; 12,800 segments
+ * + 9,000 blobs have 3,741 pairs); enable = 0 selects the source-split default
+ * instead.  Handles that no shape was set for also evaluate this way, with either
+ * kind of segments, wherever their size favours it (from about 4,100 particles
+ * on, in bodies that fill their tiles; not many small ones);
  * the shape that the functions here report is then the one such a handle falls
  * back to, and setting any shape ends it -- except the one that was reported
  * after tfs_rpy_autotune, which brings back what the autotuner kept; enable =

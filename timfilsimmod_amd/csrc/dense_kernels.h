@@ -40,10 +40,11 @@ struct DenseWork {
 // trailing update and the column panel are 64^3-FMA tile products, one
 // workgroup per tile.  work.status[k] = 1 if step k met a singular pivot.
 hipError_t k_spd_inverse_blocked(double* A, int n_pad, const DenseWork& work, hipStream_t stream);
-// y = A x for a symmetric n_pad x n_pad A (n_pad a multiple of 64; x and y
-// of n_pad entries) from its lower triangle: per 64 x 64 tile the row sums
-// and, off the diagonal, the column sums into partial (chunks x n_pad,
-// chunks = n_pad / 64), then summed in a fixed order.
+// y = A x for a symmetric n_pad x n_pad A (n_pad a multiple of 64; x of n_pad
+// entries) from its lower triangle: per 64 x 64 tile the row sums and, off the
+// diagonal, the column sums into partial (chunks x n_pad, chunks = n_pad / 64),
+// then summed in a fixed order.  Only the first n_out <= n_pad entries of y are
+// written (a caller's array need not be padded).
 hipError_t k_symv_dense(const double* A, int n_pad, const double* x, double* y, int n_out, double* partial, int chunks,
                         hipStream_t stream);
 

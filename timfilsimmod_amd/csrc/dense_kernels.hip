@@ -107,8 +107,8 @@ __global__ __launch_bounds__(256) void block_gauss_jordan_kernel(double* __restr
 // The same for blocks of up to WAVES x ROWS rows and 64 x COLS columns: the
 // block stays in registers, lane l holding columns l, l + 64, ... of rows w,
 // w + WAVES, ... of its wave w.  Rows are not moved: each step takes the
-// largest entry of its column (by its first 12 bits, the lowest row among
-// equals) among the rows that were no pivot yet, and the block is written back
+// largest entry of its column (by its exponent and first 12 mantissa bits, so
+// within 0.025% of the largest; the lowest row among equals) among the rows that were no pivot yet, and the block is written back
 // by the order in which they were.  Two barriers a step: the wave that holds
 // the pivot row puts it, scaled, into LDS; after the update the lane that holds
 // the next column puts that there and its rows' largest into a maximum over

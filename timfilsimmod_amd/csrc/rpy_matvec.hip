@@ -631,12 +631,15 @@ __device__ __forceinline__ void sym_particle(const MatvecTile& tl, const MatvecA
     }
 }
 
-// Parts of a stage after each of which the sums are put down into FP64: an FP32
-// sum of the sources takes at most 64 particles' terms, and a lane's own at
-// most 64 (32 with rotations, whose terms add four times to a component and
-// not twice).  The length of these chains sets the FP32 error: 12,800 segments
-// + 9,000 blobs with rotations, 2.1e-7 with one part, 1.2e-7 with four (5%
-// slower).
+// Parts of a stage.  After each, a lane's own sums go to FP64 and the sources'
+// sums to an LDS set of their own, in the evaluation type; the sets of all waves
+// and parts are added in FP64.  An FP32 chain so has at most 64 particles' terms
+// (a lane's own 32 where there are two parts: two particles per lane, and always
+// with rotations, whose terms add four times to a component and not twice); in
+// panels whose two tiles differ the second one's chain is added to the first
+// one's, 32 terms each.  The length of these chains sets the FP32 error: 12,800
+// segments + 9,000 blobs with rotations, 2.1e-7 with one part, 1.2e-7 with four
+// (5% slower).
 template <typename T, int DOF, int R>
 constexpr int sym_parts() {
     return sizeof(T) == 4 ? (DOF == 6 ? 2 : R) : 1;
