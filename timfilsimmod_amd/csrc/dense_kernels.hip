@@ -108,11 +108,12 @@ __global__ __launch_bounds__(256) void block_gauss_jordan_kernel(double* __restr
 // block stays in registers, lane l holding columns l, l + 64, ... of rows w,
 // w + WAVES, ... of its wave w.  Rows are not moved: each step takes the
 // largest entry of its column (by its exponent and first 12 mantissa bits, so
-// within 0.025% of the largest; the lowest row among equals) among the rows that were no pivot yet, and the block is written back
-// by the order in which they were.  Two barriers a step: the wave that holds
-// the pivot row puts it, scaled, into LDS; after the update the lane that holds
-// the next column puts that there and its rows' largest into a maximum over
-// the waves (keys of three steps in turn, the one after next cleared).
+// within 0.025% of the largest; the lowest row among equals) among the rows
+// that were no pivot yet, and the block is written back by the order in which
+// they were.  Two barriers a step: the wave that holds the pivot row puts it,
+// scaled, into LDS; after the update the lane that holds the next column puts
+// that there and its rows' largest into a maximum over the waves (keys of three
+// steps in turn, the one after next cleared).
 //
 // Bound by the steps' latency and by what every wave does again (the search,
 // the barriers).  Sixteen blocks of 120 x 120: 182 us with sixteen waves (209
